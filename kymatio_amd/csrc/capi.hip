@@ -281,6 +281,7 @@ static int launch_call(const Scat2DPlan<T>& p, const Launch2D& l, int mode, cons
                        void* out, const void* dS, void* gx, long long img_elems, void* ws, long long i0, int nimg,
                        uintptr_t base, Launch2DCall<T>* c) {
     Scat2DArgs<T> a = p.args(l, base);
+    a.fold = mode != 0 || img_elems >= p.ws_img;
     a.x = static_cast<const T*>(x);
     a.filt = static_cast<const T*>(filt);
     a.ws = static_cast<cpx<T>*>(ws);
@@ -302,10 +303,16 @@ static int launch_call(const Scat2DPlan<T>& p, const Launch2D& l, int mode, cons
     return KYM_OK;
 }
 
-// Images per chunk of a forward over `batch` images with ws_bytes of workspace.
+// Images per chunk of a forward over `batch` images with ws_bytes of workspace,
+// and the workspace elements per image.  A workspace that holds no image with
+// its gin slots but one without them runs without the fold launches.
 template <class T>
-static int chunk_of(const Scat2DPlan<T>& p, int mode, long long batch, long long ws_bytes, long long* chunk) {
-    const long long img_elems = mode == 0 ? p.ws_img : p.ws_img_train;
+static int chunk_of(const Scat2DPlan<T>& p, int mode, long long batch, long long ws_bytes, long long* chunk,
+                    long long* elems) {
+    const long long cs = (long long)sizeof(cpx<T>);
+    const bool folds = mode != 0 || ws_bytes >= p.ws_img * cs;
+    const long long img_elems = mode != 0 ? p.ws_img_train : folds ? p.ws_img : p.ws_img_base;
+    *elems = img_elems;
     const long long per = img_elems * (long long)sizeof(cpx<T>);
     if (mode != 0 && !p.trainable) return fail(KYM_ERR_UNSUPPORTED, p.train_error);
     long long c = per > 0 ? ws_bytes / per : batch;
@@ -329,9 +336,8 @@ template <class T>
 static int run2d(const Scat2DPlan<T>& p, int mode, const void* x, const void* filt, void* out, const void* dS,
                  void* gx, long long batch, void* ws, long long ws_bytes, hipStream_t stream, uintptr_t base,
                  LaunchProfile* prof, ChunkStreams* cs = nullptr) {
-    const long long img_elems = mode == 0 ? p.ws_img : p.ws_img_train;
-    long long chunk = 0;
-    int rc = chunk_of(p, mode, batch, ws_bytes, &chunk);
+    long long chunk = 0, img_elems = 0;
+    int rc = chunk_of(p, mode, batch, ws_bytes, &chunk, &img_elems);
     if (rc != KYM_OK) return rc;
     const std::vector<Launch2D>& launches = mode == 2 ? p.bwd_launches : p.launches;
     const int ns = chunk_streams(cs, p.tune.streams, mode, batch, &chunk);
@@ -344,6 +350,7 @@ static int run2d(const Scat2DPlan<T>& p, int mode, const void* x, const void* fi
         const hipStream_t st = si ? cs->aux[si - 1] : stream;
         void* wsk = static_cast<char*>(ws) + (mode == 0 ? si * chunk : i0) * img_elems * (long long)sizeof(cpx<T>);
         for (const Launch2D& l : launches) {
+            if (l.kind == K2_FOLD && mode == 0 && img_elems < p.ws_img) continue;
             Launch2DCall<T> c;
             rc = launch_call(p, l, mode, x, filt, out, dS, gx, img_elems, wsk, i0, nimg, base, &c);
             if (rc != KYM_OK) return rc;
@@ -415,8 +422,8 @@ extern "C" int kym_scat2d_forward_noalloc(void* plan, const void* x, const void*
     int cur = 0;
     KYM_HIP_TRY(hipGetDevice(&cur));
     if (cur != h->device) return fail(KYM_ERR_TYPE, "plan was created for another device");
-    const long long per_image = h->pf ? h->pf->ws_img * (long long)sizeof(cpx<float>)
-                                      : h->pd->ws_img * (long long)sizeof(cpx<double>);
+    const long long per_image = h->pf ? h->pf->ws_img_base * (long long)sizeof(cpx<float>)
+                                      : h->pd->ws_img_base * (long long)sizeof(cpx<double>);
     if (per_image > KYM_NOALLOC_SCRATCH_BYTES)
         return fail(KYM_ERR_VALUE, "kym_scat2d_forward_noalloc: one image needs " + std::to_string(per_image) +
                                        " bytes of workspace, more than the " +
@@ -530,16 +537,17 @@ template <class T>
 static int add_plan_chain(hipGraph_t g, const Scat2DPlan<T>& p, const void* x, const void* filt, void* out,
                           long long batch, void* ws, long long ws_bytes, uintptr_t base,
                           const int* dev_count = nullptr) {
-    long long chunk = 0;
-    int rc = chunk_of(p, 0, batch, ws_bytes, &chunk);
+    long long chunk = 0, img_elems = 0;
+    int rc = chunk_of(p, 0, batch, ws_bytes, &chunk, &img_elems);
     if (rc != KYM_OK) return rc;
     if (dev_count && batch > 0x7fffffffll) return fail(KYM_ERR_VALUE, "maximum batch too large");
     hipGraphNode_t prev = nullptr;
     for (long long i0 = 0; i0 < batch; i0 += chunk) {
         const int nimg = (int)std::min(chunk, batch - i0);
         for (const Launch2D& l : p.launches) {
+            if (l.kind == K2_FOLD && img_elems < p.ws_img) continue;
             Launch2DCall<T> c;
-            rc = launch_call(p, l, 0, x, filt, out, nullptr, nullptr, p.ws_img, ws, i0, nimg, base, &c);
+            rc = launch_call(p, l, 0, x, filt, out, nullptr, nullptr, img_elems, ws, i0, nimg, base, &c);
             if (rc != KYM_OK) return rc;
             c.a.dev_count = dev_count;
             c.a.max_count = (int)batch;

@@ -34,7 +34,7 @@ static void emu_spec(const Launch2D& l, const Scat2DArgs<T>& a, int t, cpx<T>* l
 template <class T>
 static int emu_forward2d(int M, int N, int J, int L, int max_order, int pre_pad, long long lds_limit, const void* x,
                          const void* filt, void* out, long long batch, long long chunk, long long* info,
-                         const int* tune = nullptr, int ntune = 0) {
+                         const int* tune = nullptr, int ntune = 0, bool folds = true) {
     Scat2DPlan<T> p;
     int* fields[7] = {&p.tune.max_pow2, &p.tune.node_threads, &p.tune.col_block, &p.tune.row_block,
                       &p.tune.pass_threads, &p.tune.streams, &p.tune.pair};
@@ -66,12 +66,16 @@ static int emu_forward2d(int M, int N, int J, int L, int max_order, int pre_pad,
     }
     if (!x) return 0;
     if (chunk <= 0 || chunk > batch) chunk = batch;
-    std::vector<cpx<T>> ws((size_t)(p.ws_img * chunk) + 1);
+    const long long ws_img = folds ? p.ws_img : p.ws_img_base;
+    std::vector<cpx<T>> ws((size_t)(ws_img * chunk) + 1);
     std::vector<cpx<T>> lds(p.max_lds / sizeof(cpx<T>) + 1);
     for (long long i0 = 0; i0 < batch; i0 += chunk) {
         const int nimg = (int)std::min(chunk, batch - i0);
         for (const Launch2D& l : p.launches) {
+            if (l.kind == K2_FOLD && !folds) continue;
             Scat2DArgs<T> a = p.args(l, base);
+            a.ws_img = ws_img;
+            a.fold = folds;
             a.x = static_cast<const T*>(x);
             a.filt = static_cast<const T*>(filt);
             a.ws = ws.data();
@@ -193,6 +197,18 @@ extern "C" int kym_emu_scat2d_taps(int M, int N, int J, int L, int max_order, in
                                    long long lds_limit, long long* desc, int n) {
     if (dtype == 0) return emu_taps2d<float>(M, N, J, L, max_order, pre_pad, lds_limit, desc, n);
     return emu_taps2d<double>(M, N, J, L, max_order, pre_pad, lds_limit, desc, n);
+}
+
+// As kym_emu_scat2d_forward with the workspace layout without gin slots
+// (every node gathers by itself).
+extern "C" int kym_emu_scat2d_forward_nofold(int M, int N, int J, int L, int max_order, int pre_pad, int dtype,
+                                             long long lds_limit, const void* x, const void* filt, void* out,
+                                             long long batch, long long chunk, long long* info) {
+    if (dtype == 0)
+        return emu_forward2d<float>(M, N, J, L, max_order, pre_pad, lds_limit, x, filt, out, batch, chunk, info,
+                                    nullptr, 0, false);
+    return emu_forward2d<double>(M, N, J, L, max_order, pre_pad, lds_limit, x, filt, out, batch, chunk, info, nullptr,
+                                 0, false);
 }
 
 // As kym_emu_scat2d_forward with plan tuning choices (kym_scat2d_create_tuned).

@@ -60,6 +60,9 @@ struct Node2D {
     int fir;         // 0 spectral leaf; 1 FIR leaf in the LDS node kernel; 2 FIR row pass + K2_FIR_COLS (big nodes)
     int fwd;         // 1 = forward FFT of the modulus is formed (children or spectral leaf need it)
     long long tslot; // fir == 2: row-filtered field (H_r x ow reals), -1 none
+    // deep periodisations: slot of the gathered input P_k(U_parent f) written by
+    // K2_FOLD (H_r x W_r, natural order), -1 where the node gathers by itself
+    long long gin;
 };
 
 // FP32 plans form every leaf in space, FP64 plans spectrally (compile-time,
@@ -76,6 +79,26 @@ struct FirAxis {
     int lo, cnt;
     long long band_off;
     int kmax, pad_;
+};
+
+// Periodisation from which LDS nodes get their input from K2_FOLD.  Below it
+// the gather's few aliases per point cost less than the child's round trip
+// through the workspace.  Measured from k = 16 / 8 / 4 / 2: 8 images of 512 x
+// 512 J=6 3752 / 3234 / 3193 / 3294 us, 6 of 150 x 203 J=4 245 / 232 / 243 /
+// 259 us, 32 of 128 x 128 J=4 forward + backward 944 / 934 / 966 / 1098 us, 64
+// of 256 x 256 J=3 (k <= 4) 1362 / 1362 / 1649 / 2389 us.
+#ifndef KYM_FOLD_MIN_K
+#define KYM_FOLD_MIN_K 8
+#endif
+
+// A tile of K2_FOLD: the children of np parents (one resolution) under nf
+// wavelets of theirs, all at resolution res with one periodisation k;
+// child[p * nf + q] is parent p's child under wavelet q.
+#define KYM_FOLD_TILE 4
+struct FoldTile {
+    int res, k, np, nf;
+    int parent[KYM_FOLD_TILE];
+    int child[KYM_FOLD_TILE * KYM_FOLD_TILE];
 };
 
 template <class T>
@@ -100,6 +123,7 @@ struct Scat2DArgs {
     int C, oh, ow;
     int img0;   // first image of this chunk
     int ntask;  // tasks in this launch
+    int fold;   // 1: the workspace holds the nodes' gin slots (K2_FOLD ran)
     // training
     int save;        // forward: store u into each node's save slot
     const T* dS;     // backward: dL/dS, same layout as out
@@ -426,6 +450,112 @@ KYM_HD KYM_INL void gather_whole(cpx<T>* dst, const cpx<T>* U, const T* f, int H
         }
     }
     gather_block(dst, W, 0, U, f, W * k, H, W, k, tid, nth);
+}
+
+// ------------------------------------------------------------------ fold
+// Gathers of deep periodisations as a pass of their own (K2_FOLD).
+//
+// A child of k aliases per axis reads its parent's whole spectrum and filter,
+// k^2 values of each per output.  In the child's own workgroup (a few hundred
+// points, up to 1024 aliases each) every thread walks that chain alone and
+// each child reads the parent again.  Here a task is one output row y0 of a
+// tile of np x nf children (np same-resolution parents, nf of their wavelets:
+// the filters are shared by the parents, so one value of each serves the
+// whole tile): 256 threads walk the k parent rows y0 + a H in contiguous
+// pieces.  Thread t sums, over rows and over the columns t, t + stripe, ...,
+// every product of the tile in registers; the stripe is a multiple of the
+// child's width, so all these columns fold onto column t mod W, and the last
+// stripe / W partial sums per point meet in LDS.  A 4 x 4 tile reads
+// (4 * 8 + 4 * 4) / 16 = 3 bytes per product instead of 12 (8 by sibling
+// pairs); the bytes from L2 and MALL are what bounds it.
+// Measured: 8 images of 512 x 512, J = 6 (20 x 20 and 40 x 40 children of
+// 640 x 640 parents, 136 workgroups a launch before): 7.93 -> 3.23 ms.
+#define KYM_FOLD_THREADS 256
+KYM_HD KYM_INL constexpr int fold_stripe(int W) { return W * (KYM_FOLD_THREADS / W); }
+
+template <int P, int F, class T>
+KYM_HD KYM_INL void fold_tile(const Scat2DArgs<T>& a, const FoldTile& tl, cpx<T>* wsi, int y0, cpx<T>* part, int tid,
+                              int nth) {
+    const int H = a.H[tl.res], W = a.W[tl.res], k = tl.k, Wp = W * k, stripe = fold_stripe(W);
+    const cpx<T>* U[P];
+    const T* f[F];
+#pragma unroll
+    for (int p = 0; p < P; ++p) U[p] = wsi + a.nodes[tl.parent[p]].slot + (long long)y0 * Wp;
+#pragma unroll
+    for (int q = 0; q < F; ++q) f[q] = a.filt + a.filt_off[a.nodes[tl.child[q]].filt] + (long long)y0 * Wp;
+    const int rstep = H * Wp;
+    for (int t = tid; t < stripe; t += nth) {
+        cpx<T> acc[P][F];
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+#pragma unroll
+            for (int q = 0; q < F; ++q) acc[p][q] = {T(0), T(0)};
+        for (int x = t; x < Wp; x += stripe) {
+            // k is even: two rows of loads in flight
+            for (int al = 0; al < k; al += 2) {
+                const int i0 = al * rstep + x, i1 = i0 + rstep;
+                cpx<T> u0[P], u1[P];
+                T f0[F], f1[F];
+#pragma unroll
+                for (int p = 0; p < P; ++p) {
+                    u0[p] = kym_ldg(U[p] + i0);
+                    u1[p] = kym_ldg(U[p] + i1);
+                }
+#pragma unroll
+                for (int q = 0; q < F; ++q) {
+                    f0[q] = kym_ldg(f[q] + i0);
+                    f1[q] = kym_ldg(f[q] + i1);
+                }
+#pragma unroll
+                for (int p = 0; p < P; ++p)
+#pragma unroll
+                    for (int q = 0; q < F; ++q) {
+                        acc[p][q].re += u0[p].re * f0[q];
+                        acc[p][q].im += u0[p].im * f0[q];
+                        acc[p][q].re += u1[p].re * f1[q];
+                        acc[p][q].im += u1[p].im * f1[q];
+                    }
+            }
+        }
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+#pragma unroll
+            for (int q = 0; q < F; ++q) part[(p * F + q) * stripe + t] = acc[p][q];
+    }
+    wg_barrier();
+    const T scale = T(1) / T(k * k);
+    for (int i = tid; i < P * F * W; i += nth) {
+        const int pq = i / W, x = i - pq * W;
+        const cpx<T>* s = part + pq * stripe + x;
+        cpx<T> v = s[0];
+        for (int c = W; c < stripe; c += W) v = v + s[c];
+        wsi[a.nodes[tl.child[pq]].gin + (long long)y0 * W + x] = v * scale;
+    }
+}
+
+// task -> (image, tile, output row).
+template <class T>
+KYM_HD void body_fold(const Scat2DArgs<T>& a, int task, cpx<T>* lds, int tid, int nth) {
+    const int per = a.ngroup * a.nblk;
+    const int il = task / per, rem = task - il * per;
+    const int gi = rem / a.nblk, y0 = rem - gi * a.nblk;
+    const FoldTile& tl = reinterpret_cast<const FoldTile*>(a.group)[gi];
+    cpx<T>* wsi = a.ws + il * a.ws_img;
+    switch (tl.np * 8 + tl.nf) {  // the plan's tiles: P x F with P = F or P = 1
+        case 8 * 4 + 4: fold_tile<4, 4>(a, tl, wsi, y0, lds, tid, nth); break;
+        case 8 * 3 + 3: fold_tile<3, 3>(a, tl, wsi, y0, lds, tid, nth); break;
+        case 8 * 2 + 2: fold_tile<2, 2>(a, tl, wsi, y0, lds, tid, nth); break;
+        case 8 * 1 + 4: fold_tile<1, 4>(a, tl, wsi, y0, lds, tid, nth); break;
+        case 8 * 1 + 3: fold_tile<1, 3>(a, tl, wsi, y0, lds, tid, nth); break;
+        case 8 * 1 + 2: fold_tile<1, 2>(a, tl, wsi, y0, lds, tid, nth); break;
+        default: fold_tile<1, 1>(a, tl, wsi, y0, lds, tid, nth); break;
+    }
+}
+
+// The gathered input of a node from its gin slot.
+template <class T>
+KYM_HD KYM_INL void load_gin(cpx<T>* dst, const cpx<T>* src, int n, int tid, int nth) {
+    copy_batched<4>(n, [&](int i) { return kym_ldg(src + i); }, [&](int i, cpx<T> v) { dst[i] = v; }, tid, nth);
 }
 
 template <class T>
@@ -1009,7 +1139,8 @@ KYM_HD void node_body(const Scat2DArgs<T>& a, const G& g, const Node2D& nd, int 
         }
     } else {
         const Node2D& pn = a.nodes[nd.parent];
-        gather_whole(lds, wsi + pn.slot, a.filt + a.filt_off[nd.filt], g.H, g.W, nd.k, tid, nth);
+        if (nd.k >= KYM_FOLD_MIN_K && a.fold && nd.gin >= 0) load_gin(lds, wsi + nd.gin, g.H * g.W, tid, nth);
+        else gather_whole(lds, wsi + pn.slot, a.filt + a.filt_off[nd.filt], g.H, g.W, nd.k, tid, nth);
         wg_barrier();
         node_after_gather(a, g, nd, il, lds, tid, nth);
         return;
@@ -1151,7 +1282,10 @@ KYM_HD KYM_INL void body_lds_pair_s(const Scat2DArgs<T>& a, int task, cpx<T>* ld
     const T* fa = a.filt + a.filt_off[na.filt];
     const T* fb = a.filt + a.filt_off[nb.filt];
     const T scale = T(1) / T(na.k * na.k);
-    switch (na.k) {  // the plan pairs k = 2^i <= 32
+    if (na.k >= KYM_FOLD_MIN_K && a.fold && na.gin >= 0) {
+        load_gin(buf, a.ws + il * a.ws_img + na.gin, H * W, tid, NT);
+        load_gin(stash, a.ws + il * a.ws_img + nb.gin, H * W, tid, NT);
+    } else switch (na.k) {  // the plan pairs k = 2^i <= 32
         case 1: gather_pair_s<1, H, W, NT>(buf, stash, U, fa, fb, scale, tid); break;
         case 2: gather_pair_s<2, H, W, NT>(buf, stash, U, fa, fb, scale, tid); break;
         case 4: gather_pair_s<4, H, W, NT>(buf, stash, U, fa, fb, scale, tid); break;
@@ -1638,7 +1772,7 @@ inline int pass_spec_id(int H, int W, int cb, int rb, int want_threads, int* thr
 
 enum Kind2D {
     K2_LDS_NODE = 0, K2_LEAF, K2_ROOT_ROWS, K2_ICOL, K2_ROWS_MOD, K2_FWD_COLS, K2_LEAF_ICOL, K2_LEAF_ROWS, K2_FIR_COLS,
-    K2_ICOL_PAIR
+    K2_ICOL_PAIR, K2_FOLD
 };
 
 template <class T, int KIND, class P>
@@ -1701,6 +1835,7 @@ KYM_HD KYM_INL void dispatch_body2d(int kind, const Scat2DArgs<T>& a, int task, 
         case K2_LEAF_ICOL: body_leaf_icol<T, MAXP>(a, task, lds, tid, nth); break;
         case K2_LEAF_ROWS: body_leaf_rows<T, MAXP>(a, task, lds, tid, nth); break;
         case K2_FIR_COLS: body_fir_cols<T, MAXP>(a, task, lds, tid, nth); break;
+        case K2_FOLD: body_fold<T>(a, task, lds, tid, nth); break;
         default: break;
     }
 }

@@ -49,6 +49,9 @@ struct Scat2DPlan {
     // tree
     std::vector<Node2D> nodes;
     long long ws_img = 0;  // complex elements of workspace per image
+    // the same without the gin slots (which come last): a workspace that holds
+    // only this runs without the K2_FOLD launches, every node gathering itself
+    long long ws_img_base = 0;
     std::vector<Launch2D> launches;
     // training: forward with saving, then the backward launches
     long long ws_img_train = 0;  // complex elements per image (layout extends the inference one)
@@ -99,6 +102,48 @@ struct Scat2DPlan {
             if (2 * R + 1 < n) { f.lo = -R; f.cnt = 2 * R + 1; }
         }
         return f;
+    }
+
+    size_t fold_lds(int r) const {
+        return (size_t)KYM_FOLD_TILE * KYM_FOLD_TILE * fold_stripe(W[r]) * sizeof(cpx<T>);
+    }
+
+    // Tiles of the fold launch of resolution r: siblings under wavelets of one
+    // scale, by parents of one scale (whose children share the filters).
+    std::vector<FoldTile> fold_tiles(int r) const {
+        // [parent][scale] -> children in theta order
+        std::vector<std::vector<int>> sets;  // one per (parent, filter scale)
+        std::vector<int> par;
+        for (size_t i = 0; i < nodes.size(); ++i) {
+            const Node2D& nd = nodes[i];
+            if (nd.res != r || nd.gin < 0) continue;
+            if (par.empty() || par.back() != nd.parent) { par.push_back(nd.parent); sets.emplace_back(); }
+            sets.back().push_back((int)i);
+        }
+        auto width = [](int n) { return n % 4 == 0 ? 4 : n % 3 == 0 ? 3 : n % 2 == 0 ? 2 : 1; };
+        std::vector<FoldTile> tiles;
+        for (size_t s = 0; s < sets.size();) {
+            // parents of one scale: consecutive sets whose first children have one filter
+            size_t e = s + 1;
+            while (e < sets.size() && sets[e].size() == sets[s].size() &&
+                   nodes[sets[e][0]].filt == nodes[sets[s][0]].filt && nodes[par[e]].res == nodes[par[s]].res)
+                ++e;
+            const int nset = (int)(e - s), nch = (int)sets[s].size();
+            const int F = width(nch);
+            const int P = nset % F == 0 ? F : 1;  // square tiles, or one parent at a time
+            for (int p0 = 0; p0 < nset; p0 += P)
+                for (int q0 = 0; q0 < nch; q0 += F) {
+                    FoldTile t = {};
+                    t.res = r; t.k = nodes[sets[s][0]].k; t.np = P; t.nf = F;
+                    for (int p = 0; p < P; ++p) {
+                        t.parent[p] = par[s + p0 + p];
+                        for (int q = 0; q < F; ++q) t.child[p * F + q] = sets[s + p0 + p][q0 + q];
+                    }
+                    tiles.push_back(t);
+                }
+            s = e;
+        }
+        return tiles;
     }
 
     bool build(int M_, int N_, int J_, int L_, int max_order_, int pre_pad_, size_t lds_limit_, KymError* e) {
@@ -259,6 +304,17 @@ struct Scat2DPlan {
             const long long align = 256 / (long long)cs;
             ws_img = (ws_img + align - 1) / align * align;
         }
+        // gathered inputs of LDS nodes with a deep periodisation (K2_FOLD)
+        ws_img_base = ws_img;
+        for (auto& nd : nodes) {
+            nd.gin = -1;
+            if (nd.big || nd.order == 0 || nd.k < KYM_FOLD_MIN_K || W[nd.res] > KYM_FOLD_THREADS ||
+                fold_lds(nd.res) > lds_limit)
+                continue;
+            nd.gin = ws_img;
+            const long long align = 256 / (long long)cs;
+            ws_img = (ws_img + (long long)H[nd.res] * W[nd.res] + align - 1) / align * align;
+        }
         // training layout: save slot (u) and gsave slot (dL/dX) for every non-root node,
         // leaf dL/dY slot where the leaf is not formed in the node kernel, and
         // the root's dL/dpad(x); children as node-index ranges.
@@ -392,6 +448,14 @@ struct Scat2DPlan {
             const Node2D& n0 = nodes[ids[0]];
             const int r = n0.res;
             const size_t elems = (size_t)H[r] * W[r];
+            const std::vector<FoldTile> tiles = n0.big ? std::vector<FoldTile>() : fold_tiles(r);
+            if (!tiles.empty()) {
+                push(K2_FOLD, {ids[0]}, H[r], 1, KYM_FOLD_THREADS, fold_lds(r));
+                Launch2D& lf = launches.back();
+                lf.group_off = blob.add(sizeof(FoldTile) * tiles.size());
+                std::memcpy(blob.at<char>(lf.group_off), tiles.data(), sizeof(FoldTile) * tiles.size());
+                lf.ngroup = (int)tiles.size();
+            }
             if (!n0.big) {
                 const size_t lds = fir ? node_lds(n0) : (elems + (n0.leaf_mode == 0 ? leaf_elems : 0)) * cs;
                 // sibling pairs: the nodes sorted by parent, every parent with an even
@@ -629,6 +693,7 @@ struct Scat2DPlan {
         a.M = pre_pad ? Mp : M; a.N = pre_pad ? Np : N;
         a.top = top; a.left = left; a.pre_pad = pre_pad;
         a.ws_img = ws_img;
+        a.fold = 1;
         a.C = C; a.oh = oh; a.ow = ow;
         return a;
     }

@@ -3,6 +3,8 @@ harness libkymatio_emu.so, against the golden vectors and the oracle.  This
 checks the plan, the digit-reversal maps, the twiddles and every index
 formula of the 2D kernels (both the all-in-LDS route and, with a tiny LDS
 cap, the column/row multi-pass route) without a GPU."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -139,3 +141,26 @@ def test_backward_fp32_compiled_nodes(emu, shape, J, tune):
     g = xt.grad.numpy()
     assert np.abs(out - S.detach().numpy()).max() <= 1e-5 * np.abs(S.detach().numpy()).max()
     assert np.abs(gx - g).max() <= 1e-5 * np.abs(g).max()
+
+
+@pytest.mark.parametrize('shape,J,L,dt', [((64, 48), 4, 8, np.float32), ((40, 64), 4, 6, np.float32),
+                                          ((32, 90), 5, 5, np.float32), ((64, 64), 4, 3, np.float64),
+                                          ((33, 70), 5, 2, np.float64)])
+def test_fold_pass_matches_gathers(emu, shape, J, L, dt):
+    """Deep periodisations (k >= 8) summed by the fold pass, over tiles of 4,
+    3, 2 and 1 parents and wavelets, against the same nodes gathering by
+    themselves (the route of a workspace without room for the inputs)."""
+    Mp, Np = compute_padding(shape[0], shape[1], J)
+    f = pack_filters_2d(filter_bank(Mp, Np, J, L)).astype(dt)
+    x = np.random.default_rng(J * L).standard_normal((2,) + shape).astype(dt)
+    out, info = emu.scat2d(x, J, shape, f, L=L)
+    g = emu.with_taps(f, J, shape, L)
+    ref = np.zeros_like(out)
+    fn = emu.lib.kym_emu_scat2d_forward_nofold
+    fn.argtypes, fn.restype = emu.lib.kym_emu_scat2d_forward.argtypes, ctypes.c_int
+    i9 = (ctypes.c_longlong * 9)()
+    rc = fn(shape[0], shape[1], J, L, 2, 0, 0 if dt == np.float32 else 1, 160 * 1024, x.ctypes.data, g.ctypes.data,
+            ref.ctypes.data, 2, 0, i9)
+    assert rc == 0
+    # k^2 <= 256 products per point in another order: sqrt(256) eps of the largest term
+    assert channel_rel_err(out, ref) < (1e-5 if dt == np.float32 else 1e-13)
