@@ -295,9 +295,11 @@ static int launch_call(const Scat2DPlan<T>& p, const Launch2D& l, int mode, cons
     if (ntask > (1ll << 30)) return fail(KYM_ERR_VALUE, "too many tasks in one launch");
     a.ntask = (int)ntask;
     c->grid = (unsigned)((ntask + 7) / 8 * 8);
-    c->threads = (unsigned)l.threads;
+    const bool many = l.many_threads && ntask > KYM_MANY_TASKS;
+    const int threads = many ? l.many_threads : l.threads;
+    c->threads = (unsigned)threads;
     c->lds = l.lds_bytes;
-    c->k = pick_scat2d<T>(l.kind, l.threads, p.pclass, l.spec);
+    c->k = pick_scat2d<T>(l.kind, threads, p.pclass, many ? l.many_spec : l.spec);
     if (!c->k) return fail(KYM_ERR_UNSUPPORTED, "no kernel for launch kind");
     c->a = a;
     return KYM_OK;

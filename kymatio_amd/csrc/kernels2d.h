@@ -105,6 +105,8 @@ template <class T, int KIND, int MAXP>
 Scat2DKernel<T> pick_scat2d_nt(int threads) {
     if (threads >= 1024) return k_scat2d<T, KIND, 1024, MAXP>;
     if (threads >= 512) return k_scat2d<T, KIND, 512, MAXP>;
+    if constexpr (KIND == K2_LDS_NODE || KIND == K2B_NODE)
+        if (threads == 64) return k_scat2d<T, KIND, 64, MAXP>;
     return k_scat2d<T, KIND, 256, MAXP>;
 }
 

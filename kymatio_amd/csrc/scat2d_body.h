@@ -1686,7 +1686,8 @@ KYM_HD void body_fwd_cols(const P& fp, const Scat2DArgs<T>& a, int task, cpx<T>*
     X(9, 68, 68, 34, 34, 256, 1)       \
     X(10, 20, 20, 10, 10, 256, 2)      \
     X(11, 40, 40, 10, 10, 256, 2)      \
-    X(12, 80, 80, 10, 10, 512, 2)
+    X(12, 80, 80, 10, 10, 512, 2)      \
+    X(13, 20, 20, 10, 10, 64, 0)
 
 // want_threads = 0: the first (default) specialisation of these sizes.
 inline int node_spec_id(int H, int W, int HJ, int WJ, int want_threads, int* threads, int want_pair = 0) {

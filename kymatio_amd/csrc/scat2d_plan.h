@@ -19,7 +19,20 @@ struct Launch2D {
     long long model_bytes;  // algorithmic HBM bytes per image (stage-boundary model)
     int spec;               // compile-time specialisation id, -1 = run-time sizes
     int pair = 0;           // 1: a task is a sibling pair (group lists 2 ngroup node ids)
+    // small LDS nodes: threads (and specialisation) of a launch of more than
+    // KYM_MANY_TASKS workgroups, 0 = the same
+    int many_threads = 0, many_spec = -1;
 };
+
+// Workgroups from which a launch of small nodes uses one wave per node.  Up to
+// there every node of a launch runs at once at 256 threads (8 workgroups on
+// each of 256 CUs), so more threads only shorten it (one 32 x 32 image alone:
+// 68 us against 72 us); beyond, a 400-point node leaves most of 256 threads
+// idle in its FFT passes (80 radix-5 butterflies a pass) and waits at barriers
+// that one wave does not have (384 images of 32 x 32 J=2: 217 -> 150 us).
+#define KYM_MANY_TASKS 2048
+// Points up to which one wave per node is used.
+#define KYM_WAVE_NODE 640
 
 // Tuning choices of a plan (0 = the built-in heuristic).  Any non-default
 // choice turns the compile-time specialisations off for what it affects.
@@ -354,6 +367,16 @@ struct Scat2DPlan {
         launches.clear();
         max_lds = 0;
         max_threads = 256;
+        // one wave per node where the launch's nodes are small and many
+        auto many_waves = [&](Launch2D& l) {
+            const size_t elems = (size_t)H[l.res] * W[l.res];
+            if (tune.node_threads || elems > KYM_WAVE_NODE || l.pair) return;
+            int nt = 0;
+            const int sid = l.spec >= 0 ? node_spec_id(H[l.res], W[l.res], H[J], W[J], 64, &nt, 0) : -1;
+            if (l.spec >= 0 && sid < 0) return;
+            l.many_threads = 64;
+            l.many_spec = sid;
+        };
         auto add_group = [&](const std::vector<int>& ids) {
             size_t o = blob.add(sizeof(int) * ids.size());
             std::memcpy(blob.at<char>(o), ids.data(), sizeof(int) * ids.size());
@@ -500,6 +523,7 @@ struct Scat2DPlan {
                     launches.back().lds_bytes = lds + cs * kym_tw_elems(H[r], W[r]);  // + twiddles
                     max_lds = std::max(max_lds, launches.back().lds_bytes);
                 }
+                many_waves(launches.back());
             } else {
                 int cb = col_blk(H[r]);
                 const int rb = row_blk(r);
@@ -624,6 +648,7 @@ struct Scat2DPlan {
                     launches.back().lds_bytes = lds + tw;
                     max_lds = std::max(max_lds, launches.back().lds_bytes);
                 }
+                many_waves(launches.back());
             } else {
                 int cb = col_blk(H[r]);
                 int rb = std::max(1, std::min(tune.row_block ? tune.row_block : 16,

@@ -196,3 +196,19 @@ def test_list_output_meta():
     for o, r, c in zip(out, ref, range(arr.shape[-3])):
         assert o['j'] == r['j'] and o['n'] == r['n'] and o['theta'] == r['theta']
         assert torch.equal(o['coef'], arr[:, c])
+
+
+@pytest.mark.parametrize('shape,J,B', [((32, 32), 2, 80), ((28, 34), 2, 70), ((24, 24), 3, 130)])
+def test_many_small_nodes_match_few(shape, J, B):
+    """Launches of more than 2048 small nodes run them one wave each, smaller
+    launches with 256 threads: the same coefficients and gradients."""
+    sc = Scattering2D(J, shape).to(DEV)
+    x = torch.randn((B,) + shape, device=DEV, generator=torch.Generator(DEV).manual_seed(B)).requires_grad_()
+    w = torch.randn(sc(x[:1]).shape[1:], device=DEV, generator=torch.Generator(DEV).manual_seed(1))
+    many = sc(x)
+    gmany, = torch.autograd.grad((many * w).sum(), x)
+    few = torch.cat([sc(x[i:i + 4]) for i in range(0, B, 4)])
+    gfew, = torch.autograd.grad((few * w).sum(), x)
+    # the same butterflies in the same order, only spread over other threads
+    assert (many - few).abs().max() <= 1e-6 * few.abs().max()
+    assert (gmany - gfew).abs().max() <= 1e-5 * gfew.abs().max()
