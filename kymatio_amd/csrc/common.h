@@ -113,6 +113,46 @@ template <> KYM_HD KYM_INL float kym_sqrt<float>(float v) {
 }
 template <> KYM_HD KYM_INL double kym_sqrt<double>(double v) { return sqrt(v); }
 
+// Run-time divisors.  Dividing by a run-time int costs about 30 instructions
+// on the vector units, as much as a small butterfly; with m = floor(2^32 / d)
+// + 1 the quotient is the high half of n m, exact while n d < 2^32 (indices
+// within a workgroup's LDS stay far below).  FInt is an int of a launch's
+// sizes that carries its m; IntC is a compile-time one, so bodies shared by
+// run-time and compile-time sizes write i / W for both.
+// Measured (with the run-time passes' twiddles in LDS and one copy of each
+// transform per kernel, 120 -> 61 KB of code for a run-time node): 48 images of
+// 224 x 224 J=3 1275 -> 1102 us, 6 of 150 x 203 J=4 232 -> 222 us; compiled
+// nodes 384 of 32 x 32 J=2 150 -> 123 us (122 -> 64 registers).
+KYM_HD KYM_INL constexpr unsigned div_magic(int d) { return d > 1 ? 0xFFFFFFFFu / (unsigned)d + 1u : 0u; }
+struct FInt {
+    int d;
+    unsigned m;  // div_magic(d)
+    KYM_HD KYM_INL operator int() const { return d; }
+};
+KYM_HD KYM_INL FInt fast_int(int d) { return {d, div_magic(d)}; }
+KYM_HD KYM_INL int div_by(int n, unsigned m) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return m ? (int)__umulhi((unsigned)n, m) : n;
+#else
+    return m ? (int)(((unsigned long long)(unsigned)n * m) >> 32) : n;
+#endif
+}
+KYM_HD KYM_INL int operator/(int n, FInt f) { return div_by(n, f.m); }
+KYM_HD KYM_INL int operator%(int n, FInt f) { return n - div_by(n, f.m) * f.d; }
+template <int N>
+struct IntC {
+    KYM_HD KYM_INL constexpr operator int() const { return N; }
+};
+// v - 1 and v / 2 + 1 as divisors of the same kind
+KYM_HD KYM_INL FInt minus_one(FInt v) { return fast_int(v.d - 1); }
+template <int N> KYM_HD KYM_INL IntC<N - 1> minus_one(IntC<N>) { return {}; }
+KYM_HD KYM_INL int minus_one(int v) { return v - 1; }
+KYM_HD KYM_INL FInt half_of(FInt v) { return fast_int(v.d / 2); }
+KYM_HD KYM_INL int half_of(int v) { return v / 2; }
+KYM_HD KYM_INL FInt half_plus_one(FInt v) { return fast_int(v.d / 2 + 1); }
+template <int N> KYM_HD KYM_INL IntC<N / 2 + 1> half_plus_one(IntC<N>) { return {}; }
+KYM_HD KYM_INL int half_plus_one(int v) { return v / 2 + 1; }
+
 // numpy-style 'reflect' index (edge sample not repeated), any pad width.
 KYM_HD KYM_INL int reflect_index(int i, int n) {
     if (n == 1) return 0;

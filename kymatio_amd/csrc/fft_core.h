@@ -27,7 +27,19 @@ struct FftLen {
     const cpx<T>* tw;          // n entries
     const int* rev;            // n entries: storage position -> natural index
     const int* irev;           // n entries: natural index -> storage position (inverse of rev)
+    // div_magic of n and, per pass q, of its butterflies n / rad[q] and of the
+    // product rad[0] ... rad[q - 1]
+    unsigned mn, mnb[KYM_MAX_RADICES], mlp[KYM_MAX_RADICES];
+    KYM_HD KYM_INL FInt size() const { return {n, mn}; }
 };
+
+// TWL: the twiddle table was copied to LDS (plain loads), else it is read
+// from global memory.
+template <bool TWL, class T>
+KYM_HD KYM_INL cpx<T> tw_at(const cpx<T>* tw, int i) {
+    if constexpr (TWL) return tw[i];
+    else return kym_ldg(tw + i);
+}
 
 // ---------------------------------------------------------------- butterflies
 template <bool INV, class T> KYM_HD KYM_INL void dft2(cpx<T>* v) {
@@ -159,17 +171,18 @@ struct Batch {
     bool tfast;
 };
 
-template <int R, bool INV, class T>
-KYM_HD void dit_pass(cpx<T>* buf, const FftLen<T>& fl, int Lp, const Batch& bt, int tid, int nth) {
-    const int n = fl.n, nb = n / R, L = Lp * R, tstep = n / L;
+// q: the pass's index in fl.rad; mtr: div_magic(bt.ntr), used when bt.tfast.
+template <int R, bool INV, bool TWL, class T>
+KYM_HD KYM_INL void dit_pass(cpx<T>* buf, const FftLen<T>& fl, const cpx<T>* tw, int q, int Lp, const Batch& bt, unsigned mtr,
+                     int tid, int nth) {
+    const int n = fl.n, L = Lp * R, nb = div_by(n, div_magic(R)), tstep = nb / FInt{Lp, fl.mlp[q]};
     const int total = nb * bt.ntr;
-    const cpx<T>* tw = fl.tw;
+    const FInt dtr = bt.tfast ? FInt{bt.ntr, mtr} : FInt{nb, fl.mnb[q]}, dlp = {Lp, fl.mlp[q]};
     for (int f = tid; f < total; f += nth) {
-        int u, t;
-        if (bt.tfast) { t = f % bt.ntr; u = f / bt.ntr; }
-        else { u = f % nb; t = f / nb; }
-        const int b = u / Lp, j = u - b * Lp;
-        cpx<T>* p = buf + (size_t)t * bt.ts + (size_t)(b * L + j) * bt.es;
+        const int hi = f / dtr, lo = f - hi * dtr;
+        const int t = bt.tfast ? lo : hi, u = bt.tfast ? hi : lo;
+        const int b = u / dlp, j = u - b * Lp;
+        cpx<T>* p = buf + (t * bt.ts + (b * L + j) * bt.es);
         const int st = Lp * bt.es;
         cpx<T> v[R];
 #pragma unroll
@@ -177,7 +190,7 @@ KYM_HD void dit_pass(cpx<T>* buf, const FftLen<T>& fl, int Lp, const Batch& bt, 
         if (j != 0) {
 #pragma unroll
             for (int m = 1; m < R; ++m) {
-                const cpx<T> w = kym_ldg(tw + j * m * tstep);
+                const cpx<T> w = tw_at<TWL>(tw, j * m * tstep);
                 v[m] = INV ? cmulc(v[m], w) : cmul(v[m], w);
             }
         }
@@ -187,17 +200,17 @@ KYM_HD void dit_pass(cpx<T>* buf, const FftLen<T>& fl, int Lp, const Batch& bt, 
     }
 }
 
-template <int R, bool INV, class T>
-KYM_HD void dif_pass(cpx<T>* buf, const FftLen<T>& fl, int L, const Batch& bt, int tid, int nth) {
-    const int n = fl.n, nb = n / R, Ls = L / R, tstep = n / L;
+template <int R, bool INV, bool TWL, class T>
+KYM_HD KYM_INL void dif_pass(cpx<T>* buf, const FftLen<T>& fl, const cpx<T>* tw, int q, int L, const Batch& bt, unsigned mtr,
+                     int tid, int nth) {
+    const int n = fl.n, Ls = div_by(L, div_magic(R)), nb = div_by(n, div_magic(R)), tstep = nb / FInt{Ls, fl.mlp[q]};
     const int total = nb * bt.ntr;
-    const cpx<T>* tw = fl.tw;
+    const FInt dtr = bt.tfast ? FInt{bt.ntr, mtr} : FInt{nb, fl.mnb[q]}, dls = {Ls, fl.mlp[q]};
     for (int f = tid; f < total; f += nth) {
-        int u, t;
-        if (bt.tfast) { t = f % bt.ntr; u = f / bt.ntr; }
-        else { u = f % nb; t = f / nb; }
-        const int b = u / Ls, j = u - b * Ls;
-        cpx<T>* p = buf + (size_t)t * bt.ts + (size_t)(b * L + j) * bt.es;
+        const int hi = f / dtr, lo = f - hi * dtr;
+        const int t = bt.tfast ? lo : hi, u = bt.tfast ? hi : lo;
+        const int b = u / dls, j = u - b * Ls;
+        cpx<T>* p = buf + (t * bt.ts + (b * L + j) * bt.es);
         const int st = Ls * bt.es;
         cpx<T> v[R];
 #pragma unroll
@@ -206,7 +219,7 @@ KYM_HD void dif_pass(cpx<T>* buf, const FftLen<T>& fl, int L, const Batch& bt, i
         if (j != 0) {
 #pragma unroll
             for (int m = 1; m < R; ++m) {
-                const cpx<T> w = kym_ldg(tw + j * m * tstep);
+                const cpx<T> w = tw_at<TWL>(tw, j * m * tstep);
                 v[m] = INV ? cmulc(v[m], w) : cmul(v[m], w);
             }
         }
@@ -220,10 +233,10 @@ KYM_HD void dif_pass(cpx<T>* buf, const FftLen<T>& fl, int L, const Batch& bt, i
 // cost registers for every path through the kernel).
 #define KYM_RADIX_SWITCH(R_, CALL)                                   \
     switch (R_) {                                                    \
-        case 2: CALL(2); break;                                      \
-        case 4: CALL(4); break;                                      \
-        case 8: CALL(8); break;                                      \
-        case 16: CALL(16); break;                                    \
+        case 2: { CALL(2); } break;                                      \
+        case 4: { CALL(4); } break;                                      \
+        case 8: { CALL(8); } break;                                      \
+        case 16: { CALL(16); } break;                                    \
         case 3: if constexpr (MAXP >= 3) { CALL(3); } break;         \
         case 5: if constexpr (MAXP >= 5) { CALL(5); } break;         \
         case 7: if constexpr (MAXP >= 7) { CALL(7); } break;         \
@@ -251,12 +264,15 @@ KYM_HD KYM_INL int kym_max_odd_prime(int n) {
 KYM_HD KYM_INL int kym_prime_class(int maxp) { return maxp <= 7 ? 7 : maxp <= 17 ? 17 : 31; }
 
 // Full DIT transform (digit-reversed in, natural out); barrier after each pass.
-template <bool INV, int MAXP, class T>
-KYM_HD void fft_dit(cpx<T>* buf, const FftLen<T>& fl, const Batch& bt, int tid, int nth) {
+// TWL: tw is fl's twiddle table copied to LDS (else fl.tw is read).
+template <bool INV, int MAXP, bool TWL = false, class T>
+KYM_HD KYM_INL void fft_dit(cpx<T>* buf, const FftLen<T>& fl, const Batch& bt, int tid, int nth, const cpx<T>* tw = nullptr) {
     int Lp = 1;
+    if (!TWL) tw = fl.tw;
+    const unsigned mtr = bt.tfast ? div_magic(bt.ntr) : 0;
     for (int q = 0; q < fl.nrad; ++q) {
         const int R = fl.rad[q];
-#define KYM_DIT_CALL(RR) dit_pass<RR, INV, T>(buf, fl, Lp, bt, tid, nth)
+#define KYM_DIT_CALL(RR) dit_pass<RR, INV, TWL, T>(buf, fl, tw, q, Lp, bt, mtr, tid, nth)
         KYM_RADIX_SWITCH(R, KYM_DIT_CALL)
 #undef KYM_DIT_CALL
         Lp *= R;
@@ -265,15 +281,16 @@ KYM_HD void fft_dit(cpx<T>* buf, const FftLen<T>& fl, const Batch& bt, int tid, 
 }
 
 // Full DIF transform (natural in, digit-reversed out); barrier after each pass.
-template <bool INV, int MAXP, class T>
-KYM_HD void fft_dif(cpx<T>* buf, const FftLen<T>& fl, const Batch& bt, int tid, int nth) {
+template <bool INV, int MAXP, bool TWL = false, class T>
+KYM_HD KYM_INL void fft_dif(cpx<T>* buf, const FftLen<T>& fl, const Batch& bt, int tid, int nth, const cpx<T>* tw = nullptr) {
     int L = fl.n;
+    if (!TWL) tw = fl.tw;
+    const unsigned mtr = bt.tfast ? div_magic(bt.ntr) : 0;
     for (int q = fl.nrad - 1; q >= 0; --q) {
         const int R = fl.rad[q];
-#define KYM_DIF_CALL(RR) dif_pass<RR, INV, T>(buf, fl, L, bt, tid, nth)
+#define KYM_DIF_CALL(RR) dif_pass<RR, INV, TWL, T>(buf, fl, tw, q, L, bt, mtr, tid, nth); L = div_by(L, div_magic(RR))
         KYM_RADIX_SWITCH(R, KYM_DIF_CALL)
 #undef KYM_DIF_CALL
-        L /= R;
         wg_barrier();
     }
 }

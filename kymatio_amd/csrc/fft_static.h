@@ -35,14 +35,6 @@ KYM_HD KYM_INL int kym_rev_s(int p) {
     return value;
 }
 
-// TWL: the twiddle table was copied to LDS (plain loads), else it is read
-// from global memory.
-template <bool TWL, class T>
-KYM_HD KYM_INL cpx<T> tw_at(const cpx<T>* tw, int i) {
-    if constexpr (TWL) return tw[i];
-    else return kym_ldg(tw + i);
-}
-
 template <int R, bool INV, int N, int LP, int NTR, int ES, int TS, bool TFAST, int NT, class T, bool TWL = false>
 KYM_HD KYM_INL void dit_pass_s(cpx<T>* buf, const cpx<T>* tw, int tid) {
     constexpr int NB = N / R, L = LP * R, TSTEP = N / L, TOTAL = NB * NTR, ST = LP * ES;

@@ -111,6 +111,13 @@ struct LenTable {
                 *err = "FFT length " + std::to_string(n) + " has a prime factor above 31 (unsupported)";
                 return false;
             }
+            f.mn = div_magic(n);
+            for (int q = 0, lp = 1; q < f.nrad; ++q) {
+                const int R = f.rad[q] > 1 ? f.rad[q] : 1;
+                f.mnb[q] = div_magic(n / R);
+                f.mlp[q] = div_magic(lp);
+                lp *= R;
+            }
             tw_off[i] = b.add(sizeof(cpx<T>) * n);
             rev_off[i] = b.add(sizeof(int) * n);
             irev_off[i] = b.add(sizeof(int) * n);

@@ -190,8 +190,8 @@ KYM_HD KYM_INL cpx<T> gather_periodized_k(const cpx<T>* U, const T* f, int Wp, i
 // dst[y * ncols + c] = scale * P_k(U * f)[y][c0 + c] for y < H, c < ncols.
 // E = 8 / K elements per thread and round: their 2 K^2 loads each are all
 // issued before the first use, so the memory latency is paid once per round.
-template <int K, class T>
-KYM_HD KYM_INL void gather_block_k(cpx<T>* dst, int ncols, int c0, const cpx<T>* U, const T* f, int H, int W,
+template <int K, class T, class NC>
+KYM_HD KYM_INL void gather_block_k(cpx<T>* dst, NC ncols, int c0, const cpx<T>* U, const T* f, int H, int W,
                                    T scale, int tid, int nth) {
     constexpr int E = K >= 8 ? 1 : 8 / K;
     const int Wp = W * K;  // the parent's row length
@@ -225,12 +225,13 @@ KYM_HD KYM_INL void gather_block_k(cpx<T>* dst, int ncols, int c0, const cpx<T>*
 // points directly.  Results equal the plain gather's up to rounding.
 KYM_HD KYM_INL constexpr int herm_pairs(int H, int W) { return (H / 2 - 1) * (W - 1) + W + 1 + H / 2; }
 
-// Point of pair p; returns false for the pairs gathered directly.
-KYM_HD KYM_INL bool herm_point(int p, int H, int W, int* y, int* x) {
+// Point of pair p (W1 = W - 1); returns false for the pairs gathered directly.
+template <class D>
+KYM_HD KYM_INL bool herm_point(int p, int H, int W, D W1, int* y, int* x) {
     const int na = (H / 2 - 1) * (W - 1);
     if (p < na) {
-        *y = 1 + p / (W - 1);
-        *x = 1 + p - (*y - 1) * (W - 1);
+        *y = 1 + p / W1;
+        *x = 1 + p - (*y - 1) * W1;
         return true;
     }
     p -= na;
@@ -301,20 +302,17 @@ KYM_HD KYM_INL void herm_block(cpx<T>* d, cpx<T>* m, const cpx<T>* U, const T* c
 template <int K, int NF, class T>
 KYM_HD KYM_INL void herm_gather(cpx<T>* d, cpx<T>* m, const cpx<T>* U, const T* const* fs, int H, int W, int y,
                                 int x) {
-    constexpr int NC = K < 4 ? 1 : K / 4;
-    if constexpr (K <= 4) {
+    static_assert(K <= 4, "deeper periodisations are not gathered by mirror pairs");
 #pragma unroll
-        for (int a0 = 0; a0 < (K + 1) / 2; ++a0) herm_block<K, NF>(d, m, U, fs, H, W, y, x, a0, 0);
-    } else {  // rolled loops over the row and chunk pairs: the body is already 32 alias terms
-        for (int a0 = 0; a0 < K / 2; ++a0)
-            for (int c0 = 0; c0 < NC / 2; ++c0) herm_block<K, NF>(d, m, U, fs, H, W, y, x, a0, c0);
-    }
+    for (int a0 = 0; a0 < (K + 1) / 2; ++a0) herm_block<K, NF>(d, m, U, fs, H, W, y, x, a0, 0);
 }
 
 // dst[y W + x] = scale P_K(U f)[y][x] for the whole H x W child.
-template <int K, class T>
-KYM_HD KYM_INL void gather_herm_k(cpx<T>* dst, const cpx<T>* U, const T* f, int H, int W, T scale, int tid,
+template <int K, class T, class WD>
+KYM_HD KYM_INL void gather_herm_k(cpx<T>* dst, const cpx<T>* U, const T* f, int H, WD Wd, T scale, int tid,
                                   int nth) {
+    const int W = Wd;
+    const auto W1 = minus_one(Wd);
     // pairs per thread and round: one from K = 2 on (A/B on MI355X at 256x256
     // J=3: two pairs per round 266 us per 136x136 launch, one 257 us, four 287 us)
     constexpr int E = K >= 2 ? 1 : 2;
@@ -326,18 +324,13 @@ KYM_HD KYM_INL void gather_herm_k(cpx<T>* dst, const cpx<T>* U, const T* f, int 
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             d[e] = m[e] = {T(0), T(0)};
-            const bool h = herm_point(p0 + e * nth < np ? p0 + e * nth : p0, H, W, &y[e], &x[e]);
+            const bool h = herm_point(p0 + e * nth < np ? p0 + e * nth : p0, H, W, W1, &y[e], &x[e]);
             if (h) {
                 herm_gather<K, 1>(&d[e], &m[e], U, fs, H, W, y[e], x[e]);
             } else {
                 const int ym = y[e] == 0 ? 0 : H - y[e], xm = x[e] == 0 ? 0 : W - x[e];
-                if constexpr (K <= 4) {
-                    d[e] = gather_periodized_k<K>(U, f, Wp, H, W, y[e], x[e]);
-                    m[e] = gather_periodized_k<K>(U, f, Wp, H, W, ym, xm);
-                } else {  // rolled: K^2 terms
-                    d[e] = gather_periodized(U, f, Wp, H, W, K, y[e], x[e]);
-                    m[e] = gather_periodized(U, f, Wp, H, W, K, ym, xm);
-                }
+                d[e] = gather_periodized_k<K>(U, f, Wp, H, W, y[e], x[e]);
+                m[e] = gather_periodized_k<K>(U, f, Wp, H, W, ym, xm);
             }
         }
 #pragma unroll
@@ -351,8 +344,8 @@ KYM_HD KYM_INL void gather_herm_k(cpx<T>* dst, const cpx<T>* U, const T* f, int 
 }
 
 // Wp = W k is the parent's row length.
-template <class T>
-KYM_HD KYM_INL void gather_block(cpx<T>* dst, int ncols, int c0, const cpx<T>* U, const T* f, int Wp, int H, int W, int k,
+template <class T, class NC>
+KYM_HD KYM_INL void gather_block(cpx<T>* dst, NC ncols, int c0, const cpx<T>* U, const T* f, int Wp, int H, int W, int k,
                          int tid, int nth) {
     const T scale = T(1) / T(k * k);
     switch (k) {
@@ -391,8 +384,8 @@ KYM_HD KYM_INL void gather_periodized_pair_k(const cpx<T>* U, const T* fa, const
 }
 
 // gather_block for two siblings (same parent, same k) into dsta and dstb.
-template <int K, class T>
-KYM_HD KYM_INL void gather_block_pair_k(cpx<T>* dsta, cpx<T>* dstb, int ncols, int c0, const cpx<T>* U, const T* fa,
+template <int K, class T, class NC>
+KYM_HD KYM_INL void gather_block_pair_k(cpx<T>* dsta, cpx<T>* dstb, NC ncols, int c0, const cpx<T>* U, const T* fa,
                                         const T* fb, int H, int W, T scale, int tid, int nth) {
     constexpr int E = K >= 4 ? 1 : 4 / K;
     const int Wp = W * K;  // the parent's row length
@@ -421,8 +414,8 @@ KYM_HD KYM_INL void gather_block_pair_k(cpx<T>* dsta, cpx<T>* dstb, int ncols, i
 }
 
 // Returns false for a k without a pair gather (the plan pairs k = 2 and 4).
-template <class T>
-KYM_HD KYM_INL bool gather_block_pair(cpx<T>* dsta, cpx<T>* dstb, int ncols, int c0, const cpx<T>* U, const T* fa,
+template <class T, class NC>
+KYM_HD KYM_INL bool gather_block_pair(cpx<T>* dsta, cpx<T>* dstb, NC ncols, int c0, const cpx<T>* U, const T* fa,
                                       const T* fb, int H, int W, int k, int tid, int nth) {
     const T scale = T(1) / T(k * k);
     switch (k) {
@@ -434,18 +427,16 @@ KYM_HD KYM_INL bool gather_block_pair(cpx<T>* dsta, cpx<T>* dstb, int ncols, int
 }
 
 // The whole H x W child spectrum (a node in LDS): by mirror pairs where the
-// sizes are even and K is a power of two up to 32, else gather_block.
-template <class T>
-KYM_HD KYM_INL void gather_whole(cpx<T>* dst, const cpx<T>* U, const T* f, int H, int W, int k, int tid, int nth) {
+// sizes are even and k is at most 4, else gather_block (deeper ones come from
+// K2_FOLD where the workspace holds them).
+template <class T, class WD>
+KYM_HD KYM_INL void gather_whole(cpx<T>* dst, const cpx<T>* U, const T* f, int H, WD W, int k, int tid, int nth) {
     const T scale = T(1) / T(k * k);
     if (H % 2 == 0 && W % 2 == 0 && H >= 2 && W >= 2) {
         switch (k) {
             case 1: gather_herm_k<1>(dst, U, f, H, W, scale, tid, nth); return;
             case 2: gather_herm_k<2>(dst, U, f, H, W, scale, tid, nth); return;
             case 4: gather_herm_k<4>(dst, U, f, H, W, scale, tid, nth); return;
-            case 8: gather_herm_k<8>(dst, U, f, H, W, scale, tid, nth); return;
-            case 16: gather_herm_k<16>(dst, U, f, H, W, scale, tid, nth); return;
-            case 32: gather_herm_k<32>(dst, U, f, H, W, scale, tid, nth); return;
             default: break;
         }
     }
@@ -592,11 +583,14 @@ struct DynGeom {
     static constexpr int STAGE = KYM_STAGE_MAX;
     // modulus / restaging as separate sweeps (stage_modulus, restage_complex)
     static constexpr bool FUSED_INV = false, FUSED_FWD = false;
-    int H, W, HJ, WJ;
+    FInt H, W, HJ, WJ;
     const FftLen<T>* fH;
     const FftLen<T>* fW;
     const FftLen<T>* fHJ;
     const FftLen<T>* fWJ;
+    // twiddle tables of H and W in LDS (load_twiddles)
+    const cpx<T>* twH;
+    const cpx<T>* twW;
     KYM_HD const int* revH() const { return fH->rev; }
     KYM_HD const int* revW() const { return fW->rev; }
     KYM_HD const int* revHJ() const { return fHJ->rev; }
@@ -604,12 +598,12 @@ struct DynGeom {
     KYM_HD int rh(int p) const { return kym_ldg(fH->rev + p); }
     KYM_HD int rw(int p) const { return kym_ldg(fW->rev + p); }
     KYM_HD KYM_INL void inv2d(cpx<T>* b, int tid, int nth) const {
-        fft_dif<true, MAXP>(b, *fW, Batch{H, 1, W, false}, tid, nth);
-        fft_dif<true, MAXP>(b, *fH, Batch{W, W, 1, true}, tid, nth);
+        fft_dif<true, MAXP, true>(b, *fW, Batch{H, 1, W, false}, tid, nth, twW);
+        fft_dif<true, MAXP, true>(b, *fH, Batch{W, W, 1, true}, tid, nth, twH);
     }
     KYM_HD KYM_INL void fwd2d(cpx<T>* b, int tid, int nth) const {
-        fft_dit<false, MAXP>(b, *fW, Batch{H, 1, W, false}, tid, nth);
-        fft_dit<false, MAXP>(b, *fH, Batch{W, W, 1, true}, tid, nth);
+        fft_dit<false, MAXP, true>(b, *fW, Batch{H, 1, W, false}, tid, nth, twW);
+        fft_dit<false, MAXP, true>(b, *fH, Batch{W, W, 1, true}, tid, nth, twH);
     }
     KYM_HD KYM_INL void leaf_inv2d(cpx<T>* b, int tid, int nth) const {
         fft_dif<true, MAXP>(b, *fWJ, Batch{HJ, 1, WJ, false}, tid, nth);
@@ -692,7 +686,7 @@ struct StatGeom {
 // Leaf: periodise U (H x W, natural, row stride W) times phi into `B`
 // (HJ x WJ), inverse FFT, real part, unpad, store into the output channel.
 template <class T, class G>
-KYM_HD void leaf_body(const Scat2DArgs<T>& a, const G& g, const cpx<T>* U, const T* phi, int kk, int ch, int img,
+KYM_HD KYM_INL void leaf_body(const Scat2DArgs<T>& a, const G& g, const cpx<T>* U, const T* phi, int kk, int ch, int img,
                       cpx<T>* B, int tid, int nth) {
     const T inv_k2 = T(1) / T(kk * kk);
     for (int i = tid; i < g.HJ * g.WJ; i += nth) {
@@ -724,7 +718,7 @@ KYM_HD void leaf_body(const Scat2DArgs<T>& a, const G& g, const cpx<T>* U, const
 // then all write after a barrier.  The CPU harness runs one thread, which
 // stages through a host array instead.
 template <class T, class G>
-KYM_HD void stage_modulus(const G& g, cpx<T>* lds, cpx<T>* sv, T inv_n, int tid, int nth) {
+KYM_HD KYM_INL void stage_modulus(const G& g, cpx<T>* lds, cpx<T>* sv, T inv_n, int tid, int nth) {
     const int n = g.H * g.W, rs = g.W + 1;
     T* R = reinterpret_cast<T*>(lds);
 #if !defined(__HIP_DEVICE_COMPILE__)
@@ -764,7 +758,7 @@ KYM_HD void stage_modulus(const G& g, cpx<T>* lds, cpx<T>* sv, T inv_n, int tid,
 
 // R (natural reals) -> digit-reversed complex buffer, ready for a forward DIT.
 template <class T, class G>
-KYM_HD void restage_complex(const G& g, cpx<T>* lds, int tid, int nth) {
+KYM_HD KYM_INL void restage_complex(const G& g, cpx<T>* lds, int tid, int nth) {
     const int n = g.H * g.W, rs = g.W + 1;
     const T* R = reinterpret_cast<const T*>(lds);
 #if !defined(__HIP_DEVICE_COMPILE__)
@@ -848,7 +842,7 @@ KYM_HD KYM_INL void fir_band(T* band, const T* filt, const FirAxis& f, int tid, 
 // A rows past nrows repeat row nrows - 1 and B columns past ow are read as
 // they are: they only reach outputs that are not stored.
 template <class T, class OUT>
-KYM_HD void fir_rows_mma(const T* R, int rs, int nrows, int W, int kl, int ow, const FirAxis& fx, const T* Bx,
+KYM_HD KYM_INL void fir_rows_mma(const T* R, int rs, int nrows, int W, int kl, int ow, const FirAxis& fx, const T* Bx,
                          OUT out, int tid, int nth) {
     const int lane = lane_id(tid), wv = wave_id(tid), nw = wave_count(nth);
     const int nmt = (nrows + 15) >> 4, nnt = (ow + 15) >> 4;
@@ -976,7 +970,7 @@ KYM_HD void fir_rows_mma_split(const T* R, int rs, int nrows, int W, int kl, int
 // for y < oh, x < ow (Tb row stride ts), into o[y * ow + x].  Ay = fir_band(.., H, kl, c, cnt).
 // Same k-step segments as the row pass, with the window along p.
 template <class T>
-KYM_HD void fir_cols_mma(const T* Tb, int ts, int H, int kl, int oh, int ow, const FirAxis& fy, const T* Ay, T* o,
+KYM_HD KYM_INL void fir_cols_mma(const T* Tb, int ts, int H, int kl, int oh, int ow, const FirAxis& fy, const T* Ay, T* o,
                          int tid, int nth) {
     const int lane = lane_id(tid), wv = wave_id(tid), nw = wave_count(nth);
     const int nmt = (oh + 15) >> 4, nnt = (ow + 15) >> 4;
@@ -1032,7 +1026,7 @@ KYM_HD void fir_cols_mma(const T* Tb, int ts, int H, int kl, int oh, int ow, con
 // samples its 16 outputs touch (the whole circle when the taps cover it).
 // Callers barrier before reusing the buffer.
 template <class T, class G>
-KYM_HD void fir_leaf_lds(const Scat2DArgs<T>& a, const G& g, const Node2D& nd, T* R, int img, int tid, int nth) {
+KYM_HD KYM_INL void fir_leaf_lds(const Scat2DArgs<T>& a, const G& g, const Node2D& nd, T* R, int img, int tid, int nth) {
     const int r = nd.res, ow = a.ow, oh = a.oh, kl = nd.leaf_k;
     const int H = g.H, W = g.W, rs = W + 1, ts = fir_tstride(W, ow);
     const FirAxis fy = a.fir[2 * r], fx = a.fir[2 * r + 1];
@@ -1052,46 +1046,54 @@ KYM_HD void fir_leaf_lds(const Scat2DArgs<T>& a, const G& g, const Node2D& nd, T
 // A whole node in LDS: root (pad + forward FFT) or order 1/2 (gather +
 // periodise, inverse FFT, modulus, forward FFT); then the optional store of
 // the spectrum for the children and the optional in-kernel leaf.
-// A node of order >= 1 from its gathered spectrum in `lds` (natural
-// order): inverse FFT, modulus, leaf, forward FFT and slot if needed.
+
+// Order >= 1, from the gathered spectrum in `lds` (natural order): inverse
+// FFT and modulus, which leaves the real field R (FP32) or the modulus in
+// digit-reversed complex storage (FP64).
 template <class T, class G>
-KYM_HD KYM_INL void node_after_gather(const Scat2DArgs<T>& a, const G& g, const Node2D& nd, int il, cpx<T>* lds, int tid,
-                              int nth) {
-    const int img = a.img0 + il;
-    cpx<T>* wsi = a.ws + il * a.ws_img;
-    {
-        const T inv_n = T(1) / T(g.H * g.W);
-        cpx<T>* sv = (a.save && nd.save >= 0) ? wsi + nd.save : nullptr;
-        if constexpr (kym_fir<T>) {
-            T* R = reinterpret_cast<T*>(lds);
-            if constexpr (G::FUSED_INV) {
-                g.inv2d_modulus(lds, R, inv_n, sv, tid);
-            } else {
-                g.inv2d(lds, tid, nth);
-                stage_modulus<T>(g, lds, sv, inv_n, tid, nth);
-            }
-            fir_leaf_lds(a, g, nd, R, img, tid, nth);
-            if (nd.fwd) {
-                if constexpr (G::FUSED_FWD) {
-                    g.fwd2d_real(lds, R, tid);
-                } else {
-                    restage_complex<T>(g, lds, tid, nth);
-                    g.fwd2d(lds, tid, nth);
-                }
-            }
+KYM_HD KYM_INL void node_modulus(const Scat2DArgs<T>& a, const G& g, const Node2D& nd, int il, cpx<T>* lds, int tid,
+                                 int nth) {
+    const T inv_n = T(1) / T(g.H * g.W);
+    cpx<T>* sv = (a.save && nd.save >= 0) ? a.ws + il * a.ws_img + nd.save : nullptr;
+    if constexpr (kym_fir<T>) {
+        T* R = reinterpret_cast<T*>(lds);
+        if constexpr (G::FUSED_INV) {
+            g.inv2d_modulus(lds, R, inv_n, sv, tid);
         } else {
             g.inv2d(lds, tid, nth);
-            for (int i = tid; i < g.H * g.W; i += nth) {
-                const cpx<T> v = lds[i];
-                if (sv) sv[i] = v;
-                lds[i] = {kym_sqrt(v.re * v.re + v.im * v.im) * inv_n, T(0)};
-            }
-            wg_barrier();
+            stage_modulus<T>(g, lds, sv, inv_n, tid, nth);
+        }
+    } else {
+        g.inv2d(lds, tid, nth);
+        for (int i = tid; i < g.H * g.W; i += nth) {
+            const cpx<T> v = lds[i];
+            if (sv) sv[i] = v;
+            lds[i] = {kym_sqrt(v.re * v.re + v.im * v.im) * inv_n, T(0)};
+        }
+        wg_barrier();
+    }
+}
+
+// From the node's real field: leaf, forward FFT and slot if needed.
+template <class T, class G>
+KYM_HD KYM_INL void node_finish(const Scat2DArgs<T>& a, const G& g, const Node2D& nd, int il, cpx<T>* lds, int tid,
+                                int nth) {
+    const int img = a.img0 + il;
+    if constexpr (kym_fir<T>) {
+        T* R = reinterpret_cast<T*>(lds);
+        fir_leaf_lds(a, g, nd, R, img, tid, nth);
+        if (!nd.fwd) return;
+        if constexpr (G::FUSED_FWD) {
+            g.fwd2d_real(lds, R, tid);
+        } else {
+            restage_complex<T>(g, lds, tid, nth);
             g.fwd2d(lds, tid, nth);
         }
+    } else {
+        g.fwd2d(lds, tid, nth);
     }
     if (nd.slot >= 0 && nd.fwd) {
-        cpx<T>* dst = wsi + nd.slot;
+        cpx<T>* dst = a.ws + il * a.ws_img + nd.slot;
         for (int i = tid; i < g.H * g.W; i += nth) dst[i] = lds[i];
     }
     if (!kym_fir<T> && nd.leaf_mode == 0)
@@ -1100,11 +1102,10 @@ KYM_HD KYM_INL void node_after_gather(const Scat2DArgs<T>& a, const G& g, const 
 }
 
 template <class T, class G>
-KYM_HD void node_body(const Scat2DArgs<T>& a, const G& g, const Node2D& nd, int il, cpx<T>* lds, int tid, int nth) {
-    const int img = a.img0 + il;
-    cpx<T>* wsi = a.ws + il * a.ws_img;
+KYM_HD KYM_INL void node_body(const Scat2DArgs<T>& a, const G& g, const Node2D& nd, int il, cpx<T>* lds, int tid,
+                              int nth) {
     if (nd.order == 0) {
-        const T* xin = a.x + (long long)img * a.M * a.N;
+        const T* xin = a.x + (long long)(a.img0 + il) * a.M * a.N;
         if constexpr (kym_fir<T>) {
             T* R = reinterpret_cast<T*>(lds);
             const int rs = g.W + 1;
@@ -1119,63 +1120,32 @@ KYM_HD void node_body(const Scat2DArgs<T>& a, const G& g, const Node2D& nd, int 
                     R[y * rs + x] = v;
                 },
                 tid, nth);
-            wg_barrier();
-            fir_leaf_lds(a, g, nd, R, img, tid, nth);
-            if constexpr (G::FUSED_FWD) {
-                g.fwd2d_real(lds, R, tid);
-            } else {
-                restage_complex<T>(g, lds, tid, nth);
-                g.fwd2d(lds, tid, nth);
-            }
         } else {
             const int* rH = g.revH();
             const int* rW = g.revW();
             for (int i = tid; i < g.H * g.W; i += nth) {
                 const int py = i / g.W, px = i - py * g.W;
-                lds[i] = {input_pixel(a, xin, rH[py], rW[px]), T(0)};
+                lds[i] = {input_pixel(a, xin, kym_ldg(rH + py), kym_ldg(rW + px)), T(0)};
             }
-            wg_barrier();
-            g.fwd2d(lds, tid, nth);
         }
-    } else {
-        const Node2D& pn = a.nodes[nd.parent];
-        if (nd.k >= KYM_FOLD_MIN_K && a.fold && nd.gin >= 0) load_gin(lds, wsi + nd.gin, g.H * g.W, tid, nth);
-        else gather_whole(lds, wsi + pn.slot, a.filt + a.filt_off[nd.filt], g.H, g.W, nd.k, tid, nth);
         wg_barrier();
-        node_after_gather(a, g, nd, il, lds, tid, nth);
-        return;
+    } else {
+        const cpx<T>* wsi = a.ws + il * a.ws_img;
+        if (nd.k >= KYM_FOLD_MIN_K && a.fold && nd.gin >= 0) load_gin(lds, wsi + nd.gin, g.H * g.W, tid, nth);
+        else gather_whole(lds, wsi + a.nodes[nd.parent].slot, a.filt + a.filt_off[nd.filt], g.H, g.W, nd.k, tid, nth);
+        wg_barrier();
+        node_modulus(a, g, nd, il, lds, tid, nth);
     }
-    if (nd.slot >= 0 && nd.fwd) {
-        cpx<T>* dst = wsi + nd.slot;
-        for (int i = tid; i < g.H * g.W; i += nth) dst[i] = lds[i];
-    }
-    if (!kym_fir<T> && nd.leaf_mode == 0)
-        leaf_body(a, g, lds, a.filt + a.filt_off[nd.leaf_filt], nd.leaf_k, nd.leaf_ch, img, lds + g.H * g.W, tid,
-                  nth);
+    node_finish(a, g, nd, il, lds, tid, nth);
 }
 
-template <class T, int MAXP>
-KYM_HD DynGeom<T, MAXP> dyn_geom(const Scat2DArgs<T>& a, int r) {
-    const int J = a.J;
-    return DynGeom<T, MAXP>{a.H[r], a.W[r], a.H[J], a.W[J], &a.lens[a.lenH[r]], &a.lens[a.lenW[r]],
-                            &a.lens[a.lenH[J]], &a.lens[a.lenW[J]]};
-}
-
-// A whole node in LDS.  task -> (image of chunk, node of group).
-template <class T, int MAXP>
-KYM_HD void body_lds_node(const Scat2DArgs<T>& a, int task, cpx<T>* lds, int tid, int nth) {
-    const int il = task / a.ngroup, gi = task - il * a.ngroup;
-    const Node2D& nd = a.nodes[a.group[gi]];
-    node_body(a, dyn_geom<T, MAXP>(a, nd.res), nd, il, lds, tid, nth);
-}
-
-// The same with compile-time sizes (the plan only selects it when the
-// launch's node and leaf sizes equal the template's).
-// Complex elements at the start of a compile-time kernel's LDS that hold
-// twiddle tables (lengths h and w; one table when equal), kept 16-byte aligned.
+// Complex elements at the start of a node's LDS that hold twiddle tables
+// (lengths h and w; one table when equal), kept 16-byte aligned.
 KYM_HD constexpr int kym_tw_elems(int h, int w) { return ((w + (h != w ? h : 0)) + 1) / 2 * 2; }
 
-// Copies the twiddles of lengths fh->n and fw->n to tw (LDS); barrier.
+// Copies the twiddles of lengths fh->n and fw->n to tw (LDS); barrier.  (The
+// bodies' own barriers would cover the copy, but without this one the 80 x 80
+// backward node takes 64 instead of 57 registers and 76 instead of 64 us.)
 template <class T>
 KYM_HD KYM_INL void load_twiddles(cpx<T>* tw, const FftLen<T>* fh, const FftLen<T>* fw, int h, int w, int tid,
                                   int nth) {
@@ -1184,6 +1154,32 @@ KYM_HD KYM_INL void load_twiddles(cpx<T>* tw, const FftLen<T>* fh, const FftLen<
         for (int i = tid; i < h; i += nth) tw[w + i] = kym_ldg(fh->tw + i);
     wg_barrier();
 }
+
+// tw: LDS for the twiddles of the node's sizes (nullptr: a body that
+// transforms leaves only).
+template <class T, int MAXP>
+KYM_HD DynGeom<T, MAXP> dyn_geom(const Scat2DArgs<T>& a, int r, cpx<T>* tw, int tid, int nth) {
+    const int J = a.J;
+    const FftLen<T>* fH = &a.lens[a.lenH[r]];
+    const FftLen<T>* fW = &a.lens[a.lenW[r]];
+    const FftLen<T>* fHJ = &a.lens[a.lenH[J]];
+    const FftLen<T>* fWJ = &a.lens[a.lenW[J]];
+    if (tw) load_twiddles(tw, fH, fW, fH->n, fW->n, tid, nth);
+    return DynGeom<T, MAXP>{fH->size(), fW->size(), fHJ->size(), fWJ->size(), fH, fW, fHJ, fWJ,
+                            tw + (fH->n != fW->n ? fW->n : 0), tw};
+}
+
+// A whole node in LDS (after its twiddles).  task -> (image of chunk, node of group).
+template <class T, int MAXP>
+KYM_HD KYM_INL void body_lds_node(const Scat2DArgs<T>& a, int task, cpx<T>* lds, int tid, int nth) {
+    const int il = task / a.ngroup, gi = task - il * a.ngroup;
+    const Node2D& nd = a.nodes[a.group[gi]];
+    const auto g = dyn_geom<T, MAXP>(a, nd.res, lds, tid, nth);
+    node_body(a, g, nd, il, lds + kym_tw_elems(g.H, g.W), tid, nth);
+}
+
+// The same with compile-time sizes (the plan only selects it when the
+// launch's node and leaf sizes equal the template's).
 
 template <class T, int H, int W, int HJ, int WJ, int NT>
 KYM_HD void body_lds_node_s(const Scat2DArgs<T>& a, int task, cpx<T>* lds, int tid) {
@@ -1209,7 +1205,7 @@ KYM_HD KYM_INL void gather_pair_s(cpx<T>* da, cpx<T>* db, const cpx<T>* U, const
     constexpr int np = herm_pairs(H, W), Wp = W * K;
     for (int p = tid; p < np; p += NT) {
         int y, x;
-        const bool h = herm_point(p, H, W, &y, &x);
+        const bool h = herm_point(p, H, W, W - 1, &y, &x);
         const int ym = y == 0 ? 0 : H - y, xm = x == 0 ? 0 : W - x;
         cpx<T> d[2] = {{T(0), T(0)}, {T(0), T(0)}}, m[2] = {{T(0), T(0)}, {T(0), T(0)}};
         if (h) {
@@ -1228,16 +1224,10 @@ KYM_HD KYM_INL void gather_pair_s(cpx<T>* da, cpx<T>* db, const cpx<T>* U, const
                     vb.re += uv.re * wb;
                     vb.im += uv.im * wb;
                 };
-                if constexpr (K <= 4) {
 #pragma unroll
-                    for (int al = 0; al < K; ++al)
+                for (int al = 0; al < K; ++al)
 #pragma unroll
-                        for (int b = 0; b < K; ++b) term(al, b);
-                } else {  // K^2 terms: rows rolled, four columns per step
-                    for (int al = 0; al < K; ++al)
-#pragma unroll 4
-                        for (int b = 0; b < K; ++b) term(al, b);
-                }
+                    for (int b = 0; b < K; ++b) term(al, b);
                 if (s) { m[0] = va; m[1] = vb; } else { d[0] = va; d[1] = vb; }
             }
         }
@@ -1285,20 +1275,26 @@ KYM_HD KYM_INL void body_lds_pair_s(const Scat2DArgs<T>& a, int task, cpx<T>* ld
     if (na.k >= KYM_FOLD_MIN_K && a.fold && na.gin >= 0) {
         load_gin(buf, a.ws + il * a.ws_img + na.gin, H * W, tid, NT);
         load_gin(stash, a.ws + il * a.ws_img + nb.gin, H * W, tid, NT);
-    } else switch (na.k) {  // the plan pairs k = 2^i <= 32
+    } else switch (na.k) {
         case 1: gather_pair_s<1, H, W, NT>(buf, stash, U, fa, fb, scale, tid); break;
         case 2: gather_pair_s<2, H, W, NT>(buf, stash, U, fa, fb, scale, tid); break;
         case 4: gather_pair_s<4, H, W, NT>(buf, stash, U, fa, fb, scale, tid); break;
-        case 8: gather_pair_s<8, H, W, NT>(buf, stash, U, fa, fb, scale, tid); break;
-        case 16: gather_pair_s<16, H, W, NT>(buf, stash, U, fa, fb, scale, tid); break;
-        default: gather_pair_s<32, H, W, NT>(buf, stash, U, fa, fb, scale, tid); break;
+        default:
+            gather_block(buf, IntC<W>(), 0, U, fa, W * na.k, H, W, na.k, tid, NT);
+            gather_block(stash, IntC<W>(), 0, U, fb, W * na.k, H, W, na.k, tid, NT);
     }
     wg_barrier();
-    node_after_gather(a, g, na, il, buf, tid, NT);
-    wg_barrier();
-    for (int i = tid; i < H * W; i += NT) buf[i] = stash[i];
-    wg_barrier();
-    node_after_gather(a, g, nb, il, buf, tid, NT);
+#pragma unroll 1
+    for (int second = 0; second < 2; ++second) {  // one copy of the node's code for both
+        const Node2D& nd = second ? nb : na;
+        if (second) {
+            wg_barrier();
+            for (int i = tid; i < H * W; i += NT) buf[i] = stash[i];
+            wg_barrier();
+        }
+        node_modulus(a, g, nd, il, buf, tid, NT);
+        node_finish(a, g, nd, il, buf, tid, NT);
+    }
 }
 
 // Leaf from a spectrum kept in the workspace.  task -> (image, node).
@@ -1309,7 +1305,7 @@ KYM_HD void body_leaf(const Scat2DArgs<T>& a, int task, cpx<T>* lds, int tid, in
     const int r = nd.res;
     const cpx<T>* U = a.ws + il * a.ws_img + nd.slot;
     const T* phi = a.filt + a.filt_off[nd.leaf_filt];
-    leaf_body(a, dyn_geom<T, MAXP>(a, r), U, phi, nd.leaf_k, nd.leaf_ch, a.img0 + il, lds, tid, nth);
+    leaf_body(a, dyn_geom<T, MAXP>(a, r, nullptr, tid, nth), U, phi, nd.leaf_k, nd.leaf_ch, a.img0 + il, lds, tid, nth);
 }
 
 // ------------------------------------------------------------------ pass FFTs
@@ -1317,20 +1313,26 @@ KYM_HD void body_leaf(const Scat2DArgs<T>& a, int task, cpx<T>* lds, int tid, in
 // column pass) or nr rows (row pass).  DynPass takes the lengths at run time;
 // StatPass fixes lengths, block sizes and thread count at compile time (the
 // plan selects it only when every block of the launch is full).
-template <class T, int MAXP>
+// Bodies take the sizes through the pass, as divisors of its kind (FInt, IntC).
+// TWL: tw is the twiddle table of the pass's direction in LDS.
+template <class T, int MAXP, bool TWL>
 struct DynPass {
     static constexpr bool FUSED = false;
+    const cpx<T>* tw;
+    KYM_HD KYM_INL FInt len(const FftLen<T>& f) const { return f.size(); }
+    KYM_HD KYM_INL FInt lenH(const FftLen<T>& f) const { return f.size(); }
+    KYM_HD KYM_INL FInt cols(int nc) const { return fast_int(nc); }
     KYM_HD KYM_INL void col_inv(cpx<T>* b, const FftLen<T>& f, int nc, int tid, int nth) const {
-        fft_dif<true, MAXP>(b, f, Batch{nc, nc, 1, true}, tid, nth);
+        fft_dif<true, MAXP, TWL>(b, f, Batch{nc, nc, 1, true}, tid, nth, tw);
     }
     KYM_HD KYM_INL void col_fwd(cpx<T>* b, const FftLen<T>& f, int nc, int tid, int nth) const {
-        fft_dit<false, MAXP>(b, f, Batch{nc, nc, 1, true}, tid, nth);
+        fft_dit<false, MAXP, TWL>(b, f, Batch{nc, nc, 1, true}, tid, nth, tw);
     }
     KYM_HD KYM_INL void row_inv(cpx<T>* b, const FftLen<T>& f, int nr, int tid, int nth) const {
-        fft_dif<true, MAXP>(b, f, Batch{nr, 1, f.n, false}, tid, nth);
+        fft_dif<true, MAXP, TWL>(b, f, Batch{nr, 1, f.n, false}, tid, nth, tw);
     }
     KYM_HD KYM_INL void row_fwd(cpx<T>* b, const FftLen<T>& f, int nr, int tid, int nth) const {
-        fft_dit<false, MAXP>(b, f, Batch{nr, 1, f.n, false}, tid, nth);
+        fft_dit<false, MAXP, TWL>(b, f, Batch{nr, 1, f.n, false}, tid, nth, tw);
     }
 };
 
@@ -1339,6 +1341,9 @@ template <class T, int H, int W, int CB, int RB, int NT>
 struct StatPass {
     const cpx<T>* twH;
     const cpx<T>* twW;
+    KYM_HD KYM_INL IntC<W> len(const FftLen<T>&) const { return {}; }
+    KYM_HD KYM_INL IntC<H> lenH(const FftLen<T>&) const { return {}; }
+    KYM_HD KYM_INL IntC<CB> cols(int) const { return {}; }
     KYM_HD KYM_INL void col_inv(cpx<T>* b, const FftLen<T>&, int, int tid, int) const {
         fft_dif_s<true, H, CB, CB, 1, true, NT, true>(b, twH, tid);
     }
@@ -1391,7 +1396,7 @@ KYM_HD void fir_rows_to_slot(const Scat2DArgs<T>& a, const Node2D& nd, const T* 
     T* red = (!in_lds && fir_rows_split(a.blk, ow)) ? Bx : nullptr;
     wg_barrier();  // also: R complete
     T* Tg = reinterpret_cast<T*>(wsi + nd.tslot);
-    auto out = [&](int p, int x, float v) { Tg[(long long)rev[r0 + p] * ow + x] = v; };
+    auto out = [&](int p, int x, float v) { Tg[(long long)kym_ldg(rev + r0 + p) * ow + x] = v; };
     // separate calls, so that each reads its band through a known address space
     if (in_lds) fir_rows_mma(R, rs, nr, W, kl, ow, fx, Bx, out, tid, nth);
     else if (red) fir_rows_mma_split(R, rs, nr, W, kl, ow, fx, a.filt + fx.band_off, out, tid, nth, red);
@@ -1401,9 +1406,9 @@ KYM_HD void fir_rows_to_slot(const Scat2DArgs<T>& a, const Node2D& nd, const T* 
 // The row spectra of a real field are Hermitian along x (row[W - x] =
 // conj(row[x])), so the row passes store columns x <= W / 2 only and the
 // forward column pass (body_fwd_cols) writes the other half by symmetry.
-template <class T>
-KYM_HD KYM_INL void store_half_rows(cpx<T>* dst, const cpx<T>* src, int nr, int W, int tid, int nth) {
-    const int Wh = W / 2 + 1;
+template <class T, class WD>
+KYM_HD KYM_INL void store_half_rows(cpx<T>* dst, const cpx<T>* src, int nr, WD W, int tid, int nth) {
+    const auto Wh = half_plus_one(W);
     for (int i = tid; i < nr * Wh; i += nth) {
         const int rr = i / Wh, x = i - rr * Wh;
         dst[(long long)rr * W + x] = src[rr * W + x];
@@ -1419,9 +1424,10 @@ KYM_HD void body_root_rows(const P& fp, const Scat2DArgs<T>& a, int task, cpx<T>
     const int il = task / a.nblk, rb = task - il * a.nblk;
     const int img = a.img0 + il;
     const Node2D& nd = a.nodes[0];
-    const int H = a.H[0], W = a.W[0];
     const FftLen<T>& fH = a.lens[a.lenH[0]];
     const FftLen<T>& fW = a.lens[a.lenW[0]];
+    const int H = a.H[0];
+    const auto W = fp.len(fW);
     const int r0 = rb * a.blk, nr = (H - r0 < a.blk) ? H - r0 : a.blk;
     const T* xin = a.x + (long long)img * a.M * a.N;
     if constexpr (kym_fir<T>) {
@@ -1431,7 +1437,7 @@ KYM_HD void body_root_rows(const P& fp, const Scat2DArgs<T>& a, int task, cpx<T>
             nr * W,
             [&](int i) {
                 const int rr = i / W, x = i - rr * W;
-                return input_pixel(a, xin, fH.rev[r0 + rr], x);
+                return input_pixel(a, xin, kym_ldg(fH.rev + r0 + rr), x);
             },
             [&](int i, T v) {
                 const int rr = i / W, x = i - rr * W;
@@ -1441,7 +1447,7 @@ KYM_HD void body_root_rows(const P& fp, const Scat2DArgs<T>& a, int task, cpx<T>
         wg_barrier();
         for (int i = tid; i < nr * W; i += nth) {
             const int rr = i / W, px = i - rr * W;
-            lds[i] = {R[rr * rs + fW.rev[px]], T(0)};
+            lds[i] = {R[rr * rs + kym_ldg(fW.rev + px)], T(0)};
         }
         fir_rows_to_slot(a, nd, R, rs, nr, r0, fH.rev, a.ws + il * a.ws_img, R + nr * rs, tid, nth);
     } else {
@@ -1449,7 +1455,7 @@ KYM_HD void body_root_rows(const P& fp, const Scat2DArgs<T>& a, int task, cpx<T>
             nr * W,
             [&](int i) {
                 const int rr = i / W, px = i - rr * W;
-                return input_pixel(a, xin, fH.rev[r0 + rr], fW.rev[px]);
+                return input_pixel(a, xin, kym_ldg(fH.rev + r0 + rr), kym_ldg(fW.rev + px));
             },
             [&](int i, T v) { lds[i] = {v, T(0)}; }, tid, nth);
     }
@@ -1460,14 +1466,14 @@ KYM_HD void body_root_rows(const P& fp, const Scat2DArgs<T>& a, int task, cpx<T>
 
 // Gather + inverse column DIF.  Shared by big nodes (filter psi, slot) and
 // big leaves (filter phi, leaf_slot).  task -> (image, node, column block).
-template <class T, class P>
+template <class T, class P, class NC>
 KYM_HD KYM_INL void icol_common(const P& fp, const Scat2DArgs<T>& a, const cpx<T>* U, const T* f, int Wp, int H, int W, int k,
-                        const FftLen<T>& fH, cpx<T>* dst, int c0, int nc, cpx<T>* lds, int tid, int nth) {
+                        const FftLen<T>& fH, cpx<T>* dst, int c0, NC nc, cpx<T>* lds, int tid, int nth) {
     gather_block(lds, nc, c0, U, f, Wp, H, W, k, tid, nth);
     wg_barrier();
     fp.col_inv(lds, fH, nc, tid, nth);
     for (int i = tid; i < H * nc; i += nth) {
-        const int p = i / nc, c = i - (i / nc) * nc;
+        const int p = i / nc, c = i - p * nc;
         dst[(long long)p * W + c0 + c] = lds[i];
     }
 }
@@ -1480,7 +1486,8 @@ KYM_HD void body_icol(const P& fp, const Scat2DArgs<T>& a, int task, cpx<T>* lds
     const Node2D& nd = a.nodes[a.group[gi]];
     const Node2D& pn = a.nodes[nd.parent];
     const int r = nd.res, H = a.H[r], W = a.W[r];
-    const int c0 = cb * a.blk, nc = (W - c0 < a.blk) ? W - c0 : a.blk;
+    const int c0 = cb * a.blk;
+    const auto nc = fp.cols((W - c0 < a.blk) ? W - c0 : a.blk);
     cpx<T>* wsi = a.ws + il * a.ws_img;
     icol_common<T>(fp, a, wsi + pn.slot, a.filt + a.filt_off[nd.filt], a.W[pn.res], H, W, nd.k, a.lens[a.lenH[r]],
                 wsi + nd.slot, c0, nc, lds, tid, nth);
@@ -1500,7 +1507,8 @@ KYM_HD void body_icol_pair(const P& fp, const Scat2DArgs<T>& a, int task, cpx<T>
     const Node2D& nb = a.nodes[a.group[2 * gi + 1]];
     const Node2D& pn = a.nodes[na.parent];
     const int r = na.res, H = a.H[r], W = a.W[r];
-    const int c0 = cb * a.blk, nc = a.blk;
+    const int c0 = cb * a.blk;
+    const auto nc = fp.cols(a.blk);
     cpx<T>* wsi = a.ws + il * a.ws_img;
     cpx<T>* la = lds;
     cpx<T>* lb = lds + H * nc;
@@ -1513,7 +1521,7 @@ KYM_HD void body_icol_pair(const P& fp, const Scat2DArgs<T>& a, int task, cpx<T>
     cpx<T>* da = wsi + na.slot;
     cpx<T>* db = wsi + nb.slot;
     for (int i = tid; i < H * nc; i += nth) {
-        const int p = i / nc, c = i - (i / nc) * nc;
+        const int p = i / nc, c = i - p * nc;
         da[(long long)p * W + c0 + c] = la[i];
         db[(long long)p * W + c0 + c] = lb[i];
     }
@@ -1521,13 +1529,14 @@ KYM_HD void body_icol_pair(const P& fp, const Scat2DArgs<T>& a, int task, cpx<T>
 
 template <class T, int MAXP>
 KYM_HD void body_leaf_icol(const Scat2DArgs<T>& a, int task, cpx<T>* lds, int tid, int nth) {
-    const DynPass<T, MAXP> fp;
+    const DynPass<T, MAXP, false> fp{nullptr};
     const int per = a.ngroup * a.nblk;
     const int il = task / per, rem = task - il * per;
     const int gi = rem / a.nblk, cb = rem - gi * a.nblk;
     const Node2D& nd = a.nodes[a.group[gi]];
     const int J = a.J, HJ = a.H[J], WJ = a.W[J];
-    const int c0 = cb * a.blk, nc = (WJ - c0 < a.blk) ? WJ - c0 : a.blk;
+    const int c0 = cb * a.blk;
+    const auto nc = fp.cols((WJ - c0 < a.blk) ? WJ - c0 : a.blk);
     cpx<T>* wsi = a.ws + il * a.ws_img;
     icol_common<T>(fp, a, wsi + nd.slot, a.filt + a.filt_off[nd.leaf_filt], a.W[nd.res], HJ, WJ, nd.leaf_k,
                 a.lens[a.lenH[J]], wsi + nd.leaf_slot, c0, nc, lds, tid, nth);
@@ -1542,8 +1551,9 @@ KYM_HD void body_rows_mod(const P& fp, const Scat2DArgs<T>& a, int task, cpx<T>*
     const int il = task / per, rem = task - il * per;
     const int gi = rem / a.nblk, rb = rem - gi * a.nblk;
     const Node2D& nd = a.nodes[a.group[gi]];
-    const int r = nd.res, H = a.H[r], W = a.W[r];
+    const int r = nd.res, H = a.H[r];
     const FftLen<T>& fW = a.lens[a.lenW[r]];
+    const auto W = fp.len(fW);
     const int r0 = rb * a.blk, nr = (H - r0 < a.blk) ? H - r0 : a.blk;
     cpx<T>* wsi = a.ws + il * a.ws_img;
     cpx<T>* buf = wsi + nd.slot + (long long)r0 * W;
@@ -1569,7 +1579,7 @@ KYM_HD void body_rows_mod(const P& fp, const Scat2DArgs<T>& a, int task, cpx<T>*
         lds[i] = {m, T(0)};
         if constexpr (kym_fir<T>) {
             const int rr = i / W, px = i - rr * W;
-            R[rr * rs + fW.rev[px]] = m;
+            R[rr * rs + kym_ldg(fW.rev + px)] = m;
         }
     }
     wg_barrier();
@@ -1586,7 +1596,8 @@ KYM_HD void body_fir_cols(const Scat2DArgs<T>& a, int task, cpx<T>* lds, int tid
     if constexpr (kym_fir<T>) {
         const int il = task / a.ngroup, gi = task - il * a.ngroup;
         const Node2D& nd = a.nodes[a.group[gi]];
-        const int r = nd.res, H = a.H[r], W = a.W[r], ow = a.ow, oh = a.oh, kl = nd.leaf_k;
+        const int r = nd.res, H = a.H[r], W = a.W[r], oh = a.oh, kl = nd.leaf_k;
+        const FInt ow = fast_int(a.ow);
         const FirAxis fy = a.fir[2 * r];
         const int ts = fir_tstride(W, ow), kym = fir_kmax(H, kl, fy.cnt);
         T* Tb = reinterpret_cast<T*>(lds);
@@ -1641,7 +1652,8 @@ KYM_HD void body_fwd_cols(const P& fp, const Scat2DArgs<T>& a, int task, cpx<T>*
     const Node2D& nd = a.nodes[a.group[gi]];
     const int r = nd.res, H = a.H[r], W = a.W[r];
     const FftLen<T>& fH = a.lens[a.lenH[r]];
-    const int c0 = cb * a.blk, nc = (W - c0 < a.blk) ? W - c0 : a.blk;
+    const int c0 = cb * a.blk;
+    const auto nc = fp.cols((W - c0 < a.blk) ? W - c0 : a.blk);
     cpx<T>* spec = a.ws + il * a.ws_img + nd.slot;
     const cpx<T>* buf = spec + c0;
     copy_batched<8>(
@@ -1824,15 +1836,42 @@ KYM_HD void dispatch_pass_spec(int id, const Scat2DArgs<T>& a, int task, cpx<T>*
     }
 }
 
+// Twiddles of a run-time-sized pass (columns: H, rows: W) at the start of its
+// LDS; returns the elements they take (pass_tw_elems).
+KYM_HD KYM_INL constexpr int pass_tw_elems(int n) { return (n + 1) / 2 * 2; }
+template <bool COLS, class T>
+KYM_HD KYM_INL int pass_twiddles(const Scat2DArgs<T>& a, cpx<T>* lds, int tid, int nth) {
+    const int r = a.nodes[a.group[0]].res;
+    const FftLen<T>& f = a.lens[COLS ? a.lenH[r] : a.lenW[r]];
+    for (int i = tid; i < f.n; i += nth) lds[i] = kym_ldg(f.tw + i);
+    return pass_tw_elems(f.n);
+}
+
 template <class T, int MAXP>
 KYM_HD KYM_INL void dispatch_body2d(int kind, const Scat2DArgs<T>& a, int task, cpx<T>* lds, int tid, int nth) {
     switch (kind) {
         case K2_LDS_NODE: body_lds_node<T, MAXP>(a, task, lds, tid, nth); break;
         case K2_LEAF: body_leaf<T, MAXP>(a, task, lds, tid, nth); break;
-        case K2_ROOT_ROWS: body_root_rows<T>(DynPass<T, MAXP>(), a, task, lds, tid, nth); break;
-        case K2_ICOL: body_icol<T>(DynPass<T, MAXP>(), a, task, lds, tid, nth); break;
-        case K2_ROWS_MOD: body_rows_mod<T>(DynPass<T, MAXP>(), a, task, lds, tid, nth); break;
-        case K2_FWD_COLS: body_fwd_cols<T>(DynPass<T, MAXP>(), a, task, lds, tid, nth); break;
+        case K2_ROOT_ROWS: {
+            const int n = pass_twiddles<false>(a, lds, tid, nth);
+            body_root_rows<T>(DynPass<T, MAXP, true>{lds}, a, task, lds + n, tid, nth);
+            break;
+        }
+        case K2_ICOL: {
+            const int n = pass_twiddles<true>(a, lds, tid, nth);
+            body_icol<T>(DynPass<T, MAXP, true>{lds}, a, task, lds + n, tid, nth);
+            break;
+        }
+        case K2_ROWS_MOD: {
+            const int n = pass_twiddles<false>(a, lds, tid, nth);
+            body_rows_mod<T>(DynPass<T, MAXP, true>{lds}, a, task, lds + n, tid, nth);
+            break;
+        }
+        case K2_FWD_COLS: {
+            const int n = pass_twiddles<true>(a, lds, tid, nth);
+            body_fwd_cols<T>(DynPass<T, MAXP, true>{lds}, a, task, lds + n, tid, nth);
+            break;
+        }
         case K2_LEAF_ICOL: body_leaf_icol<T, MAXP>(a, task, lds, tid, nth); break;
         case K2_LEAF_ROWS: body_leaf_rows<T, MAXP>(a, task, lds, tid, nth); break;
         case K2_FIR_COLS: body_fir_cols<T, MAXP>(a, task, lds, tid, nth); break;

@@ -227,7 +227,7 @@ KYM_HD KYM_INL bool grad_alias_ok(const Scat2DArgs<T>& a, const Node2D& nd) {
 
 // Leaf gradient into B (HJ x WJ, natural), scaled by 1 / (n_J kl^2).
 template <class T, class G>
-KYM_HD void leaf_grad(const Scat2DArgs<T>& a, const G& g, const Node2D& nd, int img, cpx<T>* B, int tid, int nth) {
+KYM_HD KYM_INL void leaf_grad(const Scat2DArgs<T>& a, const G& g, const Node2D& nd, int img, cpx<T>* B, int tid, int nth) {
     const T* d = a.dS + ((long long)img * a.C + nd.leaf_ch) * a.oh * a.ow;
     const int* rH = g.revHJ();
     const int* rW = g.revWJ();
@@ -247,7 +247,7 @@ KYM_HD void leaf_grad(const Scat2DArgs<T>& a, const G& g, const Node2D& nd, int 
 
 // A whole node's backward in LDS.
 template <class T, class G>
-KYM_HD void bwd_node_body(const Scat2DArgs<T>& a, const G& g, const Node2D& nd, int il, cpx<T>* lds, int tid,
+KYM_HD KYM_INL void bwd_node_body(const Scat2DArgs<T>& a, const G& g, const Node2D& nd, int il, cpx<T>* lds, int tid,
                           int nth) {
     const int img = a.img0 + il;
     cpx<T>* wsi = a.ws + il * a.ws_img;
@@ -264,7 +264,8 @@ KYM_HD void bwd_node_body(const Scat2DArgs<T>& a, const G& g, const Node2D& nd, 
         // the points (y, x), (y, x + W/2), (y + H/2, x), (y + H/2, x + W/2)
         // share their child and leaf reads (one base point per thread and
         // round; nodes without children keep the plain loop)
-        const int hh = g.H / 2, hw = g.W / 2, nb = hh * hw;
+        const int hh = g.H / 2, nb = hh * (g.W / 2);
+        const auto hw = half_of(g.W);
         for (int i = tid; i < nb; i += nth) {
             const int y = i / hw, x = i - y * hw;
             cpx<T> gu[1][4];
@@ -323,7 +324,8 @@ template <class T, int MAXP>
 KYM_HD void body_bwd_node(const Scat2DArgs<T>& a, int task, cpx<T>* lds, int tid, int nth) {
     const int il = task / a.ngroup, gi = task - il * a.ngroup;
     const Node2D& nd = a.nodes[a.group[gi]];
-    bwd_node_body(a, dyn_geom<T, MAXP>(a, nd.res), nd, il, lds, tid, nth);
+    const auto g = dyn_geom<T, MAXP>(a, nd.res, lds, tid, nth);
+    bwd_node_body(a, g, nd, il, lds + kym_tw_elems(g.H, g.W), tid, nth);
 }
 
 // A node's backward with compile-time sizes (FP32): twiddles of both lengths
@@ -368,7 +370,7 @@ template <class T, int MAXP>
 KYM_HD void body_bwd_leafg(const Scat2DArgs<T>& a, int task, cpx<T>* lds, int tid, int nth) {
     const int il = task / a.ngroup, gi = task - il * a.ngroup;
     const Node2D& nd = a.nodes[a.group[gi]];
-    const auto g = dyn_geom<T, MAXP>(a, nd.res);
+    const auto g = dyn_geom<T, MAXP>(a, nd.res, nullptr, tid, nth);
     leaf_grad(a, g, nd, a.img0 + il, lds, tid, nth);
     cpx<T>* dst = a.ws + il * a.ws_img + nd.gslot;
     for (int i = tid; i < g.HJ * g.WJ; i += nth) dst[i] = lds[i];
@@ -382,7 +384,8 @@ KYM_HD void body_bwd_gcols(const P& fp, const Scat2DArgs<T>& a, int task, cpx<T>
     const int gi = rem / a.nblk, cb = rem - gi * a.nblk;
     const Node2D& nd = a.nodes[a.group[gi]];
     const int r = nd.res, H = a.H[r], W = a.W[r], J = a.J;
-    const int c0 = cb * a.blk, nc = (W - c0 < a.blk) ? W - c0 : a.blk;
+    const int c0 = cb * a.blk;
+    const auto nc = fp.cols((W - c0 < a.blk) ? W - c0 : a.blk);
     cpx<T>* wsi = a.ws + il * a.ws_img;
     constexpr int E = 2;  // elements (base points) per thread and round
     if (nd.child_end > nd.child_begin && grad_alias_ok(a, nd)) {
@@ -425,7 +428,7 @@ KYM_HD void body_bwd_gcols(const P& fp, const Scat2DArgs<T>& a, int task, cpx<T>
     fp.col_inv(lds, a.lens[a.lenH[r]], nc, tid, nth);
     cpx<T>* dst = wsi + nd.slot;
     for (int i = tid; i < H * nc; i += nth) {
-        const int p = i / nc, c = i - (i / nc) * nc;
+        const int p = i / nc, c = i - p * nc;
         dst[(long long)p * W + c0 + c] = lds[i];
     }
 }
@@ -438,9 +441,10 @@ KYM_HD void body_bwd_grows(const P& fp, const Scat2DArgs<T>& a, int task, cpx<T>
     const int il = task / per, rem = task - il * per;
     const int gi = rem / a.nblk, rb = rem - gi * a.nblk;
     const Node2D& nd = a.nodes[a.group[gi]];
-    const int r = nd.res, H = a.H[r], W = a.W[r];
+    const int r = nd.res, H = a.H[r];
     const FftLen<T>& fW = a.lens[a.lenW[r]];
     const FftLen<T>& fH = a.lens[a.lenH[r]];
+    const auto W = fp.len(fW);
     const int r0 = rb * a.blk, nr = (H - r0 < a.blk) ? H - r0 : a.blk;
     cpx<T>* wsi = a.ws + il * a.ws_img;
     const cpx<T>* src = wsi + nd.slot + (long long)r0 * W;
@@ -451,7 +455,7 @@ KYM_HD void body_bwd_grows(const P& fp, const Scat2DArgs<T>& a, int task, cpx<T>
         T* gp = reinterpret_cast<T*>(wsi + nd.gpad);
         for (int i = tid; i < nr * W; i += nth) {
             const int rr = i / W, px = i - rr * W;
-            gp[(long long)fH.rev[r0 + rr] * W + fW.rev[px]] = lds[i].re;
+            gp[(long long)kym_ldg(fH.rev + r0 + rr) * W + kym_ldg(fW.rev + px)] = lds[i].re;
         }
         return;
     }
@@ -478,7 +482,8 @@ KYM_HD void body_bwd_gfcols(const P& fp, const Scat2DArgs<T>& a, int task, cpx<T
     const int gi = rem / a.nblk, cb = rem - gi * a.nblk;
     const Node2D& nd = a.nodes[a.group[gi]];
     const int r = nd.res, H = a.H[r], W = a.W[r];
-    const int c0 = cb * a.blk, nc = (W - c0 < a.blk) ? W - c0 : a.blk;
+    const int c0 = cb * a.blk;
+    const auto nc = fp.cols((W - c0 < a.blk) ? W - c0 : a.blk);
     cpx<T>* buf = a.ws + il * a.ws_img + nd.gsave + c0;
     copy_batched_pred<8>(
         H * nc,
@@ -547,9 +552,21 @@ KYM_HD KYM_INL void dispatch_bwd2d(int kind, const Scat2DArgs<T>& a, int task, c
     switch (kind) {
         case K2B_NODE: body_bwd_node<T, MAXP>(a, task, lds, tid, nth); break;
         case K2B_LEAFG: body_bwd_leafg<T, MAXP>(a, task, lds, tid, nth); break;
-        case K2B_GCOLS: body_bwd_gcols<T>(DynPass<T, MAXP>(), a, task, lds, tid, nth); break;
-        case K2B_GROWS: body_bwd_grows<T>(DynPass<T, MAXP>(), a, task, lds, tid, nth); break;
-        case K2B_GFCOLS: body_bwd_gfcols<T>(DynPass<T, MAXP>(), a, task, lds, tid, nth); break;
+        case K2B_GCOLS: {
+            const int n = pass_twiddles<true>(a, lds, tid, nth);
+            body_bwd_gcols<T>(DynPass<T, MAXP, true>{lds}, a, task, lds + n, tid, nth);
+            break;
+        }
+        case K2B_GROWS: {
+            const int n = pass_twiddles<false>(a, lds, tid, nth);
+            body_bwd_grows<T>(DynPass<T, MAXP, true>{lds}, a, task, lds + n, tid, nth);
+            break;
+        }
+        case K2B_GFCOLS: {
+            const int n = pass_twiddles<true>(a, lds, tid, nth);
+            body_bwd_gfcols<T>(DynPass<T, MAXP, true>{lds}, a, task, lds + n, tid, nth);
+            break;
+        }
         case K2B_FOLD: body_bwd_fold<T, MAXP>(a, task, lds, tid, nth); break;
         default: break;
     }

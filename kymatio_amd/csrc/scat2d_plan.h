@@ -297,9 +297,10 @@ struct Scat2DPlan {
                 specs && sizeof(T) == 4 &&
                 node_spec_id(H[nd.res], W[nd.res], H[J], W[J], node_threads(elems), &spec_threads, 0) >= 0 &&
                 node_lds(nd) + cs * kym_tw_elems(H[nd.res], W[nd.res]) <= lds_limit;
-            const bool fits = node_lds(nd) <= lds_limit &&
+            const size_t tw = cs * kym_tw_elems(H[nd.res], W[nd.res]);
+            const bool fits = node_lds(nd) + tw <= lds_limit &&
                               (!fir || elems <= (size_t)KYM_STAGE_MAX * node_threads(elems) || spec_fit);
-            if (fits) { nd.big = 0; nd.leaf_mode = ((elems + leaf_elems) * cs <= lds_limit) ? 0 : 1; }
+            if (fits) { nd.big = 0; nd.leaf_mode = ((elems + leaf_elems) * cs + tw <= lds_limit) ? 0 : 1; }
             else { nd.big = 1; nd.leaf_mode = (leaf_elems * cs <= lds_limit) ? 1 : 2; }
             nd.fir = fir ? (nd.big ? 2 : 1) : 0;
             nd.fwd = (has_children[i] || !fir) ? 1 : 0;
@@ -513,15 +514,12 @@ struct Scat2DPlan {
                         return;
                     }
                 }
-                push(K2_LDS_NODE, ids, 1, 0, node_threads(elems), lds);
+                push(K2_LDS_NODE, ids, 1, 0, node_threads(elems), lds + cs * kym_tw_elems(H[r], W[r]));
                 int nt = 0;
                 const int sid = node_spec_id(H[r], W[r], H[J], W[J], tune.node_threads, &nt, 0);
-                if (specs && sizeof(T) == 4 && sid >= 0 && (n0.fir == 1 || n0.leaf_mode == 0) &&
-                    lds + cs * kym_tw_elems(H[r], W[r]) <= lds_limit) {
+                if (specs && sizeof(T) == 4 && sid >= 0 && (n0.fir == 1 || n0.leaf_mode == 0)) {
                     launches.back().spec = sid;
                     launches.back().threads = nt;
-                    launches.back().lds_bytes = lds + cs * kym_tw_elems(H[r], W[r]);  // + twiddles
-                    max_lds = std::max(max_lds, launches.back().lds_bytes);
                 }
                 many_waves(launches.back());
             } else {
@@ -541,7 +539,8 @@ struct Scat2DPlan {
                                      ? pass_spec_id(H[r], W[r], cb, rb, want, &pnt) : -1;
                 if (tune.pass_threads && tune.pass_threads != 256 && psid < 0) no_pass_spec = true;
                 auto pass = [&](int kind, int nblk, int blk, size_t lds) {
-                    push(kind, ids, nblk, blk, 256, lds);
+                    const bool cols = kind == K2_ICOL || kind == K2_FWD_COLS;
+                    push(kind, ids, nblk, blk, 256, lds + cs * pass_tw_elems(cols ? H[r] : W[r]));
                     const size_t tw = cs * kym_tw_elems(H[r], W[r]);
                     if (psid >= 0 && lds + tw <= lds_limit) {
                         launches.back().spec = psid;
@@ -637,16 +636,13 @@ struct Scat2DPlan {
             if (!leafg.empty()) push(K2B_LEAFG, leafg, 1, 0, node_threads(leaf_elems), leaf_elems * cs);
             if (!n0.big) {
                 const size_t lds = (elems + (n0.leaf_mode == 0 ? leaf_elems : 0)) * cs;
-                push(K2B_NODE, ids, 1, 0, node_threads(elems), lds);
+                push(K2B_NODE, ids, 1, 0, node_threads(elems), lds + cs * kym_tw_elems(H[r], W[r]));
                 // compile-time sizes as in the forward (one node per workgroup)
                 int nt = 0;
                 const int sid = node_spec_id(H[r], W[r], H[J], W[J], tune.node_threads, &nt, 0);
-                const size_t tw = cs * kym_tw_elems(H[r], W[r]);
-                if (specs && sizeof(T) == 4 && sid >= 0 && lds + tw <= lds_limit) {
+                if (specs && sizeof(T) == 4 && sid >= 0) {
                     launches.back().spec = sid;
                     launches.back().threads = nt;
-                    launches.back().lds_bytes = lds + tw;
-                    max_lds = std::max(max_lds, launches.back().lds_bytes);
                 }
                 many_waves(launches.back());
             } else {
@@ -672,7 +668,7 @@ struct Scat2DPlan {
                     if (psid < 0 && !tune.col_block && !tune.row_block && (psid = spec_for(8, 8)) >= 0) cb = rb = 8;
                 }
                 auto bpass = [&](int kind, int nblk, int blk, size_t lds) {
-                    push(kind, ids, nblk, blk, 256, lds);
+                    push(kind, ids, nblk, blk, 256, lds + cs * pass_tw_elems(kind == K2B_GROWS ? W[r] : H[r]));
                     const size_t tw = cs * kym_tw_elems(H[r], W[r]);
                     if (psid >= 0 && lds + tw <= lds_limit) {
                         launches.back().spec = psid;
