@@ -275,6 +275,7 @@ extern "C" int kym_emu_scat1d_forward(int N, int N_pad, int pad_left, int log2_s
                 a.ntask = (int)(batch * l.ngroup);
                 for (int t = 0; t < a.ntask; ++t) {
                     if (l.kind == 0 && l.spec >= 0) dispatch_node1d_spec<T, true>(l.spec, a, t, lds.data(), 0);
+                    else if (l.kind == 1 && l.spec >= 0) dispatch_bwd_node1d_spec<T, true>(l.spec, a, t, lds.data(), 0);
                     else if (l.kind == 0) body_node1d<T, 31>(a, t, lds.data(), 0, 1);
                     else if (l.kind == 1) body_bwd_node1d<T, 31>(a, t, lds.data(), 0, 1);
                     else body_bwd_fold1d<T>(a, t, 0, 1);

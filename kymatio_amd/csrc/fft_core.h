@@ -30,16 +30,15 @@ struct FftLen {
     // div_magic of n and, per pass q, of its butterflies n / rad[q] and of the
     // product rad[0] ... rad[q - 1]
     unsigned mn, mnb[KYM_MAX_RADICES], mlp[KYM_MAX_RADICES];
+    // the twiddles in the order the passes read them from global memory: pass q
+    // takes exp(-2 pi i j m / (Lp rad[q])) at ptw[poff[q] + (m - 1) Lp + j], so
+    // neighbouring butterflies read neighbouring entries (from tw, element m of
+    // a wave's butterflies lies m n / L entries apart: for the 8192-point
+    // transform up to 60 cache lines a load)
+    const cpx<T>* ptw;
+    int poff[KYM_MAX_RADICES];
     KYM_HD KYM_INL FInt size() const { return {n, mn}; }
 };
-
-// TWL: the twiddle table was copied to LDS (plain loads), else it is read
-// from global memory.
-template <bool TWL, class T>
-KYM_HD KYM_INL cpx<T> tw_at(const cpx<T>* tw, int i) {
-    if constexpr (TWL) return tw[i];
-    else return kym_ldg(tw + i);
-}
 
 // ---------------------------------------------------------------- butterflies
 template <bool INV, class T> KYM_HD KYM_INL void dft2(cpx<T>* v) {
@@ -176,7 +175,7 @@ template <int R, bool INV, bool TWL, class T>
 KYM_HD KYM_INL void dit_pass(cpx<T>* buf, const FftLen<T>& fl, const cpx<T>* tw, int q, int Lp, const Batch& bt, unsigned mtr,
                      int tid, int nth) {
     const int n = fl.n, L = Lp * R, nb = div_by(n, div_magic(R)), tstep = nb / FInt{Lp, fl.mlp[q]};
-    const int total = nb * bt.ntr;
+    const int total = nb * bt.ntr, off = TWL ? 0 : fl.poff[q];
     const FInt dtr = bt.tfast ? FInt{bt.ntr, mtr} : FInt{nb, fl.mnb[q]}, dlp = {Lp, fl.mlp[q]};
     for (int f = tid; f < total; f += nth) {
         const int hi = f / dtr, lo = f - hi * dtr;
@@ -190,7 +189,7 @@ KYM_HD KYM_INL void dit_pass(cpx<T>* buf, const FftLen<T>& fl, const cpx<T>* tw,
         if (j != 0) {
 #pragma unroll
             for (int m = 1; m < R; ++m) {
-                const cpx<T> w = tw_at<TWL>(tw, j * m * tstep);
+                const cpx<T> w = TWL ? tw[j * m * tstep] : kym_ldg(tw + off + (m - 1) * Lp + j);
                 v[m] = INV ? cmulc(v[m], w) : cmul(v[m], w);
             }
         }
@@ -204,7 +203,7 @@ template <int R, bool INV, bool TWL, class T>
 KYM_HD KYM_INL void dif_pass(cpx<T>* buf, const FftLen<T>& fl, const cpx<T>* tw, int q, int L, const Batch& bt, unsigned mtr,
                      int tid, int nth) {
     const int n = fl.n, Ls = div_by(L, div_magic(R)), nb = div_by(n, div_magic(R)), tstep = nb / FInt{Ls, fl.mlp[q]};
-    const int total = nb * bt.ntr;
+    const int total = nb * bt.ntr, off = TWL ? 0 : fl.poff[q];
     const FInt dtr = bt.tfast ? FInt{bt.ntr, mtr} : FInt{nb, fl.mnb[q]}, dls = {Ls, fl.mlp[q]};
     for (int f = tid; f < total; f += nth) {
         const int hi = f / dtr, lo = f - hi * dtr;
@@ -219,7 +218,7 @@ KYM_HD KYM_INL void dif_pass(cpx<T>* buf, const FftLen<T>& fl, const cpx<T>* tw,
         if (j != 0) {
 #pragma unroll
             for (int m = 1; m < R; ++m) {
-                const cpx<T> w = tw_at<TWL>(tw, j * m * tstep);
+                const cpx<T> w = TWL ? tw[j * m * tstep] : kym_ldg(tw + off + (m - 1) * Ls + j);
                 v[m] = INV ? cmulc(v[m], w) : cmul(v[m], w);
             }
         }
@@ -264,11 +263,11 @@ KYM_HD KYM_INL int kym_max_odd_prime(int n) {
 KYM_HD KYM_INL int kym_prime_class(int maxp) { return maxp <= 7 ? 7 : maxp <= 17 ? 17 : 31; }
 
 // Full DIT transform (digit-reversed in, natural out); barrier after each pass.
-// TWL: tw is fl's twiddle table copied to LDS (else fl.tw is read).
+// TWL: tw is fl's twiddle table copied to LDS (else fl.ptw is read).
 template <bool INV, int MAXP, bool TWL = false, class T>
 KYM_HD KYM_INL void fft_dit(cpx<T>* buf, const FftLen<T>& fl, const Batch& bt, int tid, int nth, const cpx<T>* tw = nullptr) {
     int Lp = 1;
-    if (!TWL) tw = fl.tw;
+    if (!TWL) tw = fl.ptw;
     const unsigned mtr = bt.tfast ? div_magic(bt.ntr) : 0;
     for (int q = 0; q < fl.nrad; ++q) {
         const int R = fl.rad[q];
@@ -284,7 +283,7 @@ KYM_HD KYM_INL void fft_dit(cpx<T>* buf, const FftLen<T>& fl, const Batch& bt, i
 template <bool INV, int MAXP, bool TWL = false, class T>
 KYM_HD KYM_INL void fft_dif(cpx<T>* buf, const FftLen<T>& fl, const Batch& bt, int tid, int nth, const cpx<T>* tw = nullptr) {
     int L = fl.n;
-    if (!TWL) tw = fl.tw;
+    if (!TWL) tw = fl.ptw;
     const unsigned mtr = bt.tfast ? div_magic(bt.ntr) : 0;
     for (int q = fl.nrad - 1; q >= 0; --q) {
         const int R = fl.rad[q];
@@ -351,4 +350,15 @@ inline bool kym_factor(int n, int* rad, int* nrad, int max_pow2 = 16) {
     for (int i = 0; i < rl.nrad; ++i) rad[i] = rl.rad[i];
     *nrad = rl.nrad;
     return true;
+}
+
+// Offset of pass Q's entries in FftLen::ptw (DIT order; a first pass has none).
+KYM_HD constexpr int kym_ptw_off(const RadList& rl, int Q) {
+    int off = 0, lp = 1;
+    for (int q = 0; q < Q; ++q) {
+        const int R = rl.rad[q] > 1 ? rl.rad[q] : 1;
+        if (lp > 1) off += (R - 1) * lp;
+        lp *= R;
+    }
+    return off;
 }

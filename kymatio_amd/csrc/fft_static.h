@@ -35,7 +35,15 @@ KYM_HD KYM_INL int kym_rev_s(int p) {
     return value;
 }
 
-template <int R, bool INV, int N, int LP, int NTR, int ES, int TS, bool TFAST, int NT, class T, bool TWL = false>
+// The twiddle tw[i] of a table copied to LDS (TWL), or entry p of the per-pass
+// table FftLen::ptw in global memory.
+template <bool TWL, class T>
+KYM_HD KYM_INL cpx<T> tw_s(const cpx<T>* tw, int i, int p) {
+    if constexpr (TWL) return tw[i];
+    else return kym_ldg(tw + p);
+}
+
+template <int R, bool INV, int N, int LP, int NTR, int ES, int TS, bool TFAST, int NT, class T, bool TWL = false, int OFF = 0>
 KYM_HD KYM_INL void dit_pass_s(cpx<T>* buf, const cpx<T>* tw, int tid) {
     constexpr int NB = N / R, L = LP * R, TSTEP = N / L, TOTAL = NB * NTR, ST = LP * ES;
     for (int f = tid; f < TOTAL; f += NT) {
@@ -51,7 +59,7 @@ KYM_HD KYM_INL void dit_pass_s(cpx<T>* buf, const cpx<T>* tw, int tid) {
             if (j != 0) {
 #pragma unroll
                 for (int m = 1; m < R; ++m) {
-                    const cpx<T> w = tw_at<TWL>(tw, j * m * TSTEP);
+                    const cpx<T> w = tw_s<TWL>(tw, j * m * TSTEP, OFF + (m - 1) * LP + j);
                     v[m] = INV ? cmulc(v[m], w) : cmul(v[m], w);
                 }
             }
@@ -62,7 +70,7 @@ KYM_HD KYM_INL void dit_pass_s(cpx<T>* buf, const cpx<T>* tw, int tid) {
     }
 }
 
-template <int R, bool INV, int N, int L, int NTR, int ES, int TS, bool TFAST, int NT, class T, bool TWL = false>
+template <int R, bool INV, int N, int L, int NTR, int ES, int TS, bool TFAST, int NT, class T, bool TWL = false, int OFF = 0>
 KYM_HD KYM_INL void dif_pass_s(cpx<T>* buf, const cpx<T>* tw, int tid) {
     constexpr int NB = N / R, LS = L / R, TSTEP = N / L, TOTAL = NB * NTR, ST = LS * ES;
     for (int f = tid; f < TOTAL; f += NT) {
@@ -79,7 +87,7 @@ KYM_HD KYM_INL void dif_pass_s(cpx<T>* buf, const cpx<T>* tw, int tid) {
             if (j != 0) {
 #pragma unroll
                 for (int m = 1; m < R; ++m) {
-                    const cpx<T> w = tw_at<TWL>(tw, j * m * TSTEP);
+                    const cpx<T> w = tw_s<TWL>(tw, j * m * TSTEP, OFF + (m - 1) * LS + j);
                     v[m] = INV ? cmulc(v[m], w) : cmul(v[m], w);
                 }
             }
@@ -97,7 +105,7 @@ KYM_HD KYM_INL void fft_dit_s(cpx<T>* buf, const cpx<T>* tw, int tid) {
     static_assert(rl.ok, "unsupported static FFT length");
     if constexpr (Q < rl.nrad) {
         constexpr int R = rl.rad[Q];
-        dit_pass_s<R, INV, N, LP, NTR, ES, TS, TFAST, NT, T, TWL>(buf, tw, tid);
+        dit_pass_s<R, INV, N, LP, NTR, ES, TS, TFAST, NT, T, TWL, kym_ptw_off(rl, Q)>(buf, tw, tid);
         wg_barrier();
         fft_dit_s<INV, N, NTR, ES, TS, TFAST, NT, TWL, T, Q + 1, LP * R>(buf, tw, tid);
     }
@@ -113,7 +121,7 @@ KYM_HD KYM_INL void fft_dif_s(cpx<T>* buf, const cpx<T>* tw, int tid) {
     constexpr int q = (Q < 0) ? rl.nrad - 1 : Q;
     if constexpr (q >= QMIN && L > 1) {
         constexpr int R = rl.rad[q];
-        dif_pass_s<R, INV, N, L, NTR, ES, TS, TFAST, NT, T, TWL>(buf, tw, tid);
+        dif_pass_s<R, INV, N, L, NTR, ES, TS, TFAST, NT, T, TWL, kym_ptw_off(rl, q)>(buf, tw, tid);
         wg_barrier();
         if constexpr (q > QMIN) fft_dif_s<INV, N, NTR, ES, TS, TFAST, NT, TWL, T, q - 1, L / R, QMIN>(buf, tw, tid);
     }
@@ -239,4 +247,68 @@ KYM_HD KYM_INL void dit_first_pass_real_s(cpx<T>* buf, int tid, LOAD load) {
         }
     }
     wg_barrier();
+}
+
+// ---------------------------------------------------------------- padded line
+// One transform of a power-of-two length whose element i sits at pad16(i) =
+// i + i / 16 in LDS.  In place, the later DIF passes (and earlier DIT ones)
+// step through LDS at strides of 16 and 256 elements, which fall on 2 of 32
+// bank pairs; with one element of padding in 16, consecutive lanes of every
+// pass touch different banks (two lanes share one at worst).
+KYM_HD KYM_INL constexpr int pad16(int i) { return i + (i >> 4); }
+
+template <int R, bool INV, bool DIT, int N, int LS, int OFF, int NT, class T>
+KYM_HD KYM_INL void pad_pass(cpx<T>* buf, const cpx<T>* ptw, int tid) {
+    constexpr int L = LS * R;
+    // element m of a butterfly lies m ST further on where LS keeps the padding
+    // linear, else its place is computed
+    constexpr bool LIN = LS % 16 == 0 || (LS == 1 && 16 % R == 0);
+    constexpr int ST = LS % 16 == 0 ? LS + LS / 16 : 1;
+    KYM_UNROLL_DEV
+    for (int f = tid; f < N / R; f += NT) {
+        const int b = f / LS, j = f - b * LS, i0 = b * L + j;
+        cpx<T>* p = LIN ? buf + pad16(i0) : buf;
+        cpx<T> v[R], w[R];
+        if constexpr (LS > 1) {
+#pragma unroll
+            for (int m = 1; m < R; ++m) w[m] = kym_ldg(ptw + OFF + (m - 1) * LS + j);
+        }
+#pragma unroll
+        for (int m = 0; m < R; ++m) v[m] = LIN ? p[m * ST] : p[pad16(i0 + m * LS)];
+        if constexpr (DIT && LS > 1) {
+#pragma unroll
+            for (int m = 1; m < R; ++m) v[m] = INV ? cmulc(v[m], w[m]) : cmul(v[m], w[m]);
+        }
+        dft_r<R, INV>(v);
+        if constexpr (!DIT && LS > 1) {
+#pragma unroll
+            for (int m = 1; m < R; ++m) v[m] = INV ? cmulc(v[m], w[m]) : cmul(v[m], w[m]);
+        }
+#pragma unroll
+        for (int m = 0; m < R; ++m) (LIN ? p[m * ST] : p[pad16(i0 + m * LS)]) = v[m];
+    }
+    wg_barrier();
+}
+
+template <bool INV, int N, int NT, class T, int Q = 0, int LP = 1>
+KYM_HD KYM_INL void pad_dit(cpx<T>* buf, const cpx<T>* ptw, int tid) {
+    constexpr RadList rl = kym_factor_list(N);
+    static_assert(rl.ok && (N & (N - 1)) == 0, "power-of-two lengths");
+    if constexpr (Q < rl.nrad) {
+        constexpr int R = rl.rad[Q];
+        pad_pass<R, INV, true, N, LP, kym_ptw_off(rl, Q), NT, T>(buf, ptw, tid);
+        pad_dit<INV, N, NT, T, Q + 1, LP * R>(buf, ptw, tid);
+    }
+}
+
+template <bool INV, int N, int NT, class T, int Q = -1, int L = N>
+KYM_HD KYM_INL void pad_dif(cpx<T>* buf, const cpx<T>* ptw, int tid) {
+    constexpr RadList rl = kym_factor_list(N);
+    static_assert(rl.ok && (N & (N - 1)) == 0, "power-of-two lengths");
+    constexpr int q = Q < 0 ? rl.nrad - 1 : Q;
+    if constexpr (L > 1) {
+        constexpr int R = rl.rad[q];
+        pad_pass<R, INV, false, N, L / R, kym_ptw_off(rl, q), NT, T>(buf, ptw, tid);
+        if constexpr (q > 0) pad_dif<INV, N, NT, T, q - 1, L / R>(buf, ptw, tid);
+    }
 }

@@ -9,8 +9,9 @@ __global__ void __launch_bounds__(NT) k_scat1d(Scat1DArgs<T> a) {
     const int task = xcd_task(blockIdx.x, gridDim.x);
     if (task >= a.ntask) return;
     cpx<T>* lds = reinterpret_cast<cpx<T>*>(kym_smem1d);
-    if constexpr (KIND == 0) body_node1d<T, 7>(a, task, lds, threadIdx.x, NT);
-    else if constexpr (KIND == 1) body_bwd_node1d<T, 7>(a, task, lds, threadIdx.x, NT);
+    // power-of-two lengths only: no odd radices
+    if constexpr (KIND == 0) body_node1d<T, 2>(a, task, lds, threadIdx.x, NT);
+    else if constexpr (KIND == 1) body_bwd_node1d<T, 2>(a, task, lds, threadIdx.x, NT);
     else body_bwd_fold1d<T>(a, task, threadIdx.x, NT);
 }
 
@@ -20,6 +21,14 @@ __global__ void __launch_bounds__(NT) k_node1d_spec(Scat1DArgs<T> a) {
     const int task = xcd_task(blockIdx.x, gridDim.x);
     if (task >= a.ntask) return;
     node1d_spec_body<T, SPEC, false>(a, task, reinterpret_cast<cpx<T>*>(kym_smem1d_ns), threadIdx.x);
+}
+
+template <class T, int SPEC, int NT>
+__global__ void __launch_bounds__(NT) k_bwd_node1d_spec(Scat1DArgs<T> a) {
+    extern __shared__ __attribute__((aligned(16))) char kym_smem1d_bns[];
+    const int task = xcd_task(blockIdx.x, gridDim.x);
+    if (task >= a.ntask) return;
+    bwd_node1d_spec_body<T, SPEC, false>(a, task, reinterpret_cast<cpx<T>*>(kym_smem1d_bns), threadIdx.x);
 }
 
 template <class T>
@@ -33,6 +42,18 @@ Scat1DKernel<T> pick_node1d_spec(int id) {
     case sid: return k_node1d_spec<T, sid, nt>;
         KYM_NODE1D_SPECS(KYM_N1_K)
 #undef KYM_N1_K
+        default: return nullptr;
+    }
+}
+
+template <class T>
+Scat1DKernel<T> pick_bwd_node1d_spec(int id) {
+    if constexpr (sizeof(T) != 4) return nullptr;
+    else switch (id) {
+#define KYM_B1_K(sid, nn, nt) \
+    case sid: return k_bwd_node1d_spec<T, sid, nt>;
+        KYM_NODE1D_SPECS(KYM_B1_K)
+#undef KYM_B1_K
         default: return nullptr;
     }
 }

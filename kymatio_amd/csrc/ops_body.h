@@ -287,7 +287,7 @@ KYM_HD void filter_ifft_body_s(const FilterIfftArgs& o, const FftLen<T>& fl, lon
         lds[q] = acc * inv_k;
     }
     wg_barrier();
-    fft_dif_s<true, NN, M, 1, NN, false, NT>(lds, fl.tw, tid);
+    fft_dif_s<true, NN, M, 1, NN, false, NT>(lds, fl.ptw, tid);
     const T inv_n = T(1) / T(NN);
     for (int q = tid; q < m * NN; q += NT) {
         int t, p;
@@ -427,7 +427,7 @@ KYM_HD void freq_scatter_body_s(const FreqScatterArgs& o, long long blk, cpx<T>*
         X[t * N + kym_ldg(fN.irev + a)] = v;
     }
     wg_barrier();
-    fft_dit_s<false, N, M, 1, N, false, NT>(X, fN.tw, tid);
+    fft_dit_s<false, N, M, 1, N, false, NT>(X, fN.ptw, tid);
     for (int w = 0; w < o.nf; ++w) {
         const int k = o.k[w], n = N / k;
         const T* f = static_cast<const T*>(o.f[w]);
@@ -447,9 +447,9 @@ KYM_HD void freq_scatter_body_s(const FreqScatterArgs& o, long long blk, cpx<T>*
         wg_barrier();
         const FftLen<T>& fl = *static_cast<const FftLen<T>*>(o.lenn[w]);
         if constexpr (N == 88) {
-            if (n == 88) fft_dif_s<true, 88, M, 1, 88, false, NT>(P, fl.tw, tid);
-            else if (n == 44) fft_dif_s<true, 44, M, 1, 44, false, NT>(P, fl.tw, tid);
-            else fft_dif_s<true, 22, M, 1, 22, false, NT>(P, fl.tw, tid);
+            if (n == 88) fft_dif_s<true, 88, M, 1, 88, false, NT>(P, fl.ptw, tid);
+            else if (n == 44) fft_dif_s<true, 44, M, 1, 44, false, NT>(P, fl.ptw, tid);
+            else fft_dif_s<true, 22, M, 1, 22, false, NT>(P, fl.ptw, tid);
         }
         const T inv_n = T(1) / T(n);
         T* y = static_cast<T*>(o.y[w]);
@@ -625,7 +625,7 @@ KYM_HD void lowpass_body_s(const LowpassArgs& o, const FftLen<T>& fN, const FftL
         lds[u * N + kym_ldg(fN.irev + e)] = {va, vb};
     }
     wg_barrier();
-    fft_dit_s<false, N, M2, 1, N, false, NT>(lds, fN.tw, tid);
+    fft_dit_s<false, N, M2, 1, N, false, NT>(lds, fN.ptw, tid);
     cpx<T>* P = lds + M2 * N;
     const T inv_2k = T(1) / T(2 * K);
     for (int q = tid; q < M * NN; q += NT) {
@@ -647,7 +647,7 @@ KYM_HD void lowpass_body_s(const LowpassArgs& o, const FftLen<T>& fN, const FftL
         P[q] = acc * inv_2k;
     }
     wg_barrier();
-    fft_dif_s<true, NN, M, 1, NN, false, NT>(P, fn.tw, tid);
+    fft_dif_s<true, NN, M, 1, NN, false, NT>(P, fn.ptw, tid);
     const T inv_n = T(1) / T(NN);
     for (int q = tid; q < m * NN; q += NT) {
         const int t = q / NN, p = q - t * NN;
@@ -673,7 +673,7 @@ KYM_HD void lowpass_body_sv(const LowpassArgs& o, const FftLen<T>& fN, const Fft
         lds[t * N + kym_ldg(fN.irev + e)] = {kym_ldg(x + (ob * N + e) * S + s0 + t), T(0)};
     }
     wg_barrier();
-    fft_dit_s<false, N, M, 1, N, false, NT>(lds, fN.tw, tid);
+    fft_dit_s<false, N, M, 1, N, false, NT>(lds, fN.ptw, tid);
     cpx<T>* P = lds + M * N;
     const T inv_k = T(1) / T(K);
     for (int q = tid; q < M * NN; q += NT) {
@@ -690,7 +690,7 @@ KYM_HD void lowpass_body_sv(const LowpassArgs& o, const FftLen<T>& fN, const Fft
         P[q] = acc * inv_k;
     }
     wg_barrier();
-    fft_dif_s<true, NN, M, 1, NN, false, NT>(P, fn.tw, tid);
+    fft_dif_s<true, NN, M, 1, NN, false, NT>(P, fn.ptw, tid);
     const T inv_n = T(1) / T(NN);
     for (int q = tid; q < M * NN; q += NT) {
         const int p = q / M, t = q - p * M;

@@ -102,7 +102,7 @@ struct LenTable {
     // Writes FftLen array + tables into the blob; returns offset of the array.
     bool emit(Blob& b, size_t* lens_off, std::string* err) const {
         std::vector<FftLen<T>> fl(ns.size());
-        std::vector<size_t> tw_off(ns.size()), rev_off(ns.size()), irev_off(ns.size());
+        std::vector<size_t> tw_off(ns.size()), ptw_off(ns.size()), rev_off(ns.size()), irev_off(ns.size());
         for (size_t i = 0; i < ns.size(); ++i) {
             const int n = ns[i];
             FftLen<T>& f = fl[i];
@@ -125,6 +125,22 @@ struct LenTable {
             kym_twiddles(n, re.data(), im.data());
             cpx<T>* tw = b.at<cpx<T>>(tw_off[i]);
             for (int t = 0; t < n; ++t) tw[t] = {(T)re[t], (T)im[t]};
+            RadList rl;
+            rl.nrad = f.nrad;
+            for (int q = 0; q < f.nrad; ++q) rl.rad[q] = f.rad[q];
+            ptw_off[i] = b.add(sizeof(cpx<T>) * (kym_ptw_off(rl, f.nrad) + 1));
+            cpx<T>* pt = b.at<cpx<T>>(ptw_off[i]);
+            for (int q = 0, lp = 1; q < f.nrad; ++q) {
+                const int R = f.rad[q] > 1 ? f.rad[q] : 1;
+                f.poff[q] = kym_ptw_off(rl, q);
+                if (lp > 1)
+                    for (int m = 1; m < R; ++m)
+                        for (int j = 0; j < lp; ++j) {
+                            const int t = j * m * (n / (lp * R));
+                            pt[f.poff[q] + (m - 1) * lp + j] = {(T)re[t], (T)im[t]};
+                        }
+                lp *= R;
+            }
             kym_rev_map(n, f.rad, f.nrad, b.at<int>(rev_off[i]));
             const int* rv = b.at<int>(rev_off[i]);
             int* iv = b.at<int>(irev_off[i]);
@@ -134,11 +150,13 @@ struct LenTable {
         FftLen<T>* dst = b.at<FftLen<T>>(*lens_off);
         for (size_t i = 0; i < ns.size(); ++i) {
             fl[i].tw = reinterpret_cast<const cpx<T>*>(tw_off[i]);
+            fl[i].ptw = reinterpret_cast<const cpx<T>*>(ptw_off[i]);
             fl[i].rev = reinterpret_cast<const int*>(rev_off[i]);
             fl[i].irev = reinterpret_cast<const int*>(irev_off[i]);
             dst[i] = fl[i];
             const size_t rec = *lens_off + i * sizeof(FftLen<T>);
             b.reloc.push_back(rec + offsetof(FftLen<T>, tw));
+            b.reloc.push_back(rec + offsetof(FftLen<T>, ptw));
             b.reloc.push_back(rec + offsetof(FftLen<T>, rev));
             b.reloc.push_back(rec + offsetof(FftLen<T>, irev));
         }

@@ -62,47 +62,14 @@ struct Scat1DArgs {
     T* gx;
 };
 
-// Output of one path from the spectrum / modulus in LDS.
-template <class T, int MAXP>
-KYM_HD void leaf1d(const Scat1DArgs<T>& a, const Node1D& nd, const cpx<T>* U, int n, int img, cpx<T>* B, int tid,
-                   int nth) {
-    T* o = a.out + (long long)img * a.out_row + nd.out_off;
-    if (a.mode == AVG1_GLOBAL) {
-        if (tid == 0) o[0] = U[0].re;
-        return;
-    }
-    const int kk = nd.leaf_k, nl = n / kk;
-    const T* phi = a.filt + a.filt_off[nd.leaf_filt];
-    const T inv_k = T(1) / T(kk);
-    for (int i = tid; i < nl; i += nth) {
-        cpx<T> acc = {T(0), T(0)};
-#pragma unroll 8
-        for (int q = 0; q < kk; ++q) {  // unrolled: several filter loads in flight
-            const cpx<T> u = U[i + q * nl];
-            const T f = kym_ldg(phi + i + q * nl);
-            acc.re += u.re * f;
-            acc.im += u.im * f;
-        }
-        B[i] = acc * inv_k;
-    }
-    wg_barrier();
-    // the low-passed path has length N_pad >> max(res, log2_stride) = nl
-    const int lr = nd.res > a.log2_stride ? nd.res : a.log2_stride;
-    const FftLen<T>& fB = a.lens[a.len[lr]];
-    fft_dif<true, MAXP>(B, fB, Batch{1, 1, nl, false}, tid, nth);
-    const int s = a.ind_start[a.log2_stride], e = a.ind_end[a.log2_stride];
-    const T inv_n = T(1) / T(nl);
-    for (int p = tid; p < nl; p += nth) {
-        const int t = fB.rev[p];
-        if (t >= s && t < e) o[t - s] = B[p].re * inv_n;
-    }
-    wg_barrier();
-}
-
 // FFT of a node's length: run-time (Dyn1D) or compile-time (Stat1D, length
-// N and NT threads; the same factorisation and digit-reversed order).
+// N and NT threads; the same factorisation and digit-reversed order).  at(i) is
+// where element i of the transform sits in LDS, elems(n) the elements that n
+// of them take.
 template <class T, int MAXP>
 struct Dyn1D {
+    KYM_HD KYM_INL int at(int i) const { return i; }
+    KYM_HD KYM_INL int elems(int n) const { return n; }
     KYM_HD KYM_INL void inv(cpx<T>* b, const FftLen<T>& fl, int tid, int nth) const {
         fft_dif<true, MAXP>(b, fl, Batch{1, 1, fl.n, false}, tid, nth);
     }
@@ -113,13 +80,70 @@ struct Dyn1D {
 
 template <class T, int N, int NT>
 struct Stat1D {
+    KYM_HD KYM_INL int at(int i) const { return pad16(i); }
+    KYM_HD KYM_INL int elems(int n) const { return pad16(n); }
     KYM_HD KYM_INL void inv(cpx<T>* b, const FftLen<T>& fl, int tid, int) const {
-        fft_dif_s<true, N, 1, 1, N, false, NT>(b, fl.tw, tid);
+        pad_dif<true, N, NT, T>(b, fl.ptw, tid);
     }
     KYM_HD KYM_INL void fwd(cpx<T>* b, const FftLen<T>& fl, int tid, int) const {
-        fft_dit_s<false, N, 1, 1, N, false, NT>(b, fl.tw, tid);
+        pad_dit<false, N, NT, T>(b, fl.ptw, tid);
     }
 };
+
+// LDS elements after the node's line: the leaf's line of nl points, or the
+// nth partial sums it is reduced from.
+KYM_HD KYM_INL int leaf1d_elems(int nl, int nth) { return nl > nth ? nl : nth; }
+
+// Output of one path from the spectrum / modulus in LDS.
+template <class T, int MAXP, class F>
+KYM_HD KYM_INL void leaf1d(const F& ff, const Scat1DArgs<T>& a, const Node1D& nd, const cpx<T>* U, int n, int img,
+                           cpx<T>* B, int tid, int nth) {
+    T* o = a.out + (long long)img * a.out_row + nd.out_off;
+    if (a.mode == AVG1_GLOBAL) {
+        if (tid == 0) o[0] = U[0].re;
+        return;
+    }
+    const int kk = nd.leaf_k;
+    // the low-passed path has length N_pad >> max(res, log2_stride) = nl
+    const int lr = nd.res > a.log2_stride ? nd.res : a.log2_stride;
+    const FftLen<T>& fB = a.lens[a.len[lr]];
+    const FInt nl = fB.size();
+    const T* phi = a.filt + a.filt_off[nd.leaf_filt];
+    const T inv_k = T(1) / T(kk);
+    // S threads per output point (powers of two), each an S-th of the aliases:
+    // 64 aliases of 128 points kept 384 of 512 threads waiting otherwise
+    int S = 1;
+    while (2 * S * nl <= nth && 2 * S <= kk) S *= 2;
+    for (int q = tid; q < S * nl; q += nth) {
+        const int s = q / nl, i = q - s * nl;
+        cpx<T> acc = {T(0), T(0)};
+#pragma unroll 4
+        for (int al = s; al < kk; al += S) {  // unrolled: several filter loads in flight
+            const cpx<T> u = U[ff.at(i + al * nl)];
+            const T f = kym_ldg(phi + i + al * nl);
+            acc.re += u.re * f;
+            acc.im += u.im * f;
+        }
+        B[q] = acc * inv_k;
+    }
+    wg_barrier();
+    if (S > 1) {
+        for (int i = tid; i < nl; i += nth) {  // nl < nth: one point per thread
+            cpx<T> acc = B[i];
+            for (int s = 1; s < S; ++s) acc = acc + B[i + s * nl];
+            B[i] = acc;
+        }
+        wg_barrier();
+    }
+    fft_dif<true, MAXP>(B, fB, Batch{1, 1, nl, false}, tid, nth);
+    const int s = a.ind_start[a.log2_stride], e = a.ind_end[a.log2_stride];
+    const T inv_n = T(1) / T(nl);
+    for (int p = tid; p < nl; p += nth) {
+        const int t = kym_ldg(fB.rev + p);
+        if (t >= s && t < e) o[t - s] = B[p].re * inv_n;
+    }
+    wg_barrier();
+}
 
 template <class T, int MAXP, class F>
 KYM_HD KYM_INL void node1d_body(const F& ff, const Scat1DArgs<T>& a, int task, cpx<T>* lds, int tid, int nth) {
@@ -133,8 +157,8 @@ KYM_HD KYM_INL void node1d_body(const F& ff, const Scat1DArgs<T>& a, int task, c
     if (nd.order == 0) {
         const T* xin = a.x + (long long)img * a.N;
         copy_batched<8>(
-            n, [&](int p) { return kym_ldg(xin + reflect_index(fl.rev[p] - a.pad_left, a.N)); },
-            [&](int p, T v) { lds[p] = {v, T(0)}; }, tid, nth);
+            n, [&](int p) { return kym_ldg(xin + reflect_index(kym_ldg(fl.rev + p) - a.pad_left, a.N)); },
+            [&](int p, T v) { lds[ff.at(p)] = {v, T(0)}; }, tid, nth);
         if (a.mode == AVG1_NONE) {
             // S_0 = U_0 unpadded = the input itself
             const int s = a.ind_start[0], e = a.ind_end[0];
@@ -178,8 +202,8 @@ KYM_HD KYM_INL void node1d_body(const F& ff, const Scat1DArgs<T>& a, int task, c
                     m.im -= u.im * fm2;
                 }
             }
-            lds[i] = d * inv_k;
-            if (im != i) lds[im] = m * inv_k;
+            lds[ff.at(i)] = d * inv_k;
+            if (im != i) lds[ff.at(im)] = m * inv_k;
         }
         wg_barrier();
         ff.inv(lds, fl, tid, nth);
@@ -187,12 +211,13 @@ KYM_HD KYM_INL void node1d_body(const F& ff, const Scat1DArgs<T>& a, int task, c
         const int s = a.ind_start[nd.unpad_res], e = a.ind_end[nd.unpad_res];
         cpx<T>* sv = (a.save && nd.save >= 0) ? wsi + nd.save : nullptr;
         for (int p = tid; p < n; p += nth) {
-            const cpx<T> v = lds[p];
+            cpx<T>& c = lds[ff.at(p)];
+            const cpx<T> v = c;
             if (sv) sv[p] = v;
             const T m = kym_sqrt(v.re * v.re + v.im * v.im) * inv_n;
-            lds[p] = {m, T(0)};
+            c = {m, T(0)};
             if (a.mode == AVG1_NONE) {
-                const int t = fl.rev[p];
+                const int t = kym_ldg(fl.rev + p);
                 if (t >= s && t < e) o[t - s] = m;
             }
         }
@@ -201,9 +226,9 @@ KYM_HD KYM_INL void node1d_body(const F& ff, const Scat1DArgs<T>& a, int task, c
     }
     if (nd.slot >= 0) {
         cpx<T>* dst = wsi + nd.slot;
-        for (int i = tid; i < n; i += nth) dst[i] = lds[i];
+        for (int i = tid; i < n; i += nth) dst[i] = lds[ff.at(i)];
     }
-    if (a.mode != AVG1_NONE) leaf1d<T, MAXP>(a, nd, lds, n, img, lds + n, tid, nth);
+    if (a.mode != AVG1_NONE) leaf1d<T, MAXP>(ff, a, nd, lds, n, img, lds + ff.elems(n), tid, nth);
 }
 
 template <class T, int MAXP>
@@ -211,7 +236,7 @@ KYM_HD void body_node1d(const Scat1DArgs<T>& a, int task, cpx<T>* lds, int tid, 
     node1d_body<T, MAXP>(Dyn1D<T, MAXP>(), a, task, lds, tid, nth);
 }
 
-// Compile-time specialisations X(id, N, threads) of the forward node (FP32):
+// Compile-time specialisations X(id, N, threads) of the nodes, forward and backward (FP32):
 // a launch uses one when its nodes' length matches (threads follow the
 // plan's rule max(64, min(1024, N / 16))).
 #define KYM_NODE1D_SPECS(X) \
@@ -236,7 +261,7 @@ inline int node1d_spec_id(int n, int threads) {
 template <class T, int SPEC, bool EMU>
 KYM_HD KYM_INL void node1d_spec_body(const Scat1DArgs<T>& a, int task, cpx<T>* lds, int tid) {
 #define KYM_N1_BODY(sid, nn, nt) \
-    if constexpr (SPEC == sid) node1d_body<T, 7>(Stat1D<T, nn, (EMU ? 1 : nt)>(), a, task, lds, tid, EMU ? 1 : nt);
+    if constexpr (SPEC == sid) node1d_body<T, 2>(Stat1D<T, nn, (EMU ? 1 : nt)>(), a, task, lds, tid, EMU ? 1 : nt);
     KYM_NODE1D_SPECS(KYM_N1_BODY)
 #undef KYM_N1_BODY
 }
@@ -259,8 +284,8 @@ KYM_HD void dispatch_node1d_spec(int id, const Scat1DArgs<T>& a, int task, cpx<T
 //   dL/dm = Re(n ifft(dL/dU)) (+ dS on the unpadded window without averaging,
 //           + dS everywhere with global averaging)
 //   dL/du = dL/dm u / |u|,  dL/dX = fft(dL/du) / n;  root: dL/dpad(x) = dL/dm.
-template <class T, int MAXP>
-KYM_HD void body_bwd_node1d(const Scat1DArgs<T>& a, int task, cpx<T>* lds, int tid, int nth) {
+template <class T, int MAXP, class F>
+KYM_HD KYM_INL void bwd_node1d_body(const F& ff, const Scat1DArgs<T>& a, int task, cpx<T>* lds, int tid, int nth) {
     const int il = task / a.ngroup, gi = task - il * a.ngroup;
     const int img = a.img0 + il;
     const Node1D& nd = a.nodes[a.group[gi]];
@@ -269,7 +294,7 @@ KYM_HD void body_bwd_node1d(const Scat1DArgs<T>& a, int task, cpx<T>* lds, int t
     cpx<T>* wsi = a.ws + il * a.ws_sig;
     const T* d = a.dS + (long long)img * a.out_row + nd.out_off;
     // leaf gradient (local average) into B
-    cpx<T>* B = lds + n;
+    cpx<T>* B = lds + ff.elems(n);
     int nl = 1, kk = 1;
     if (a.mode == AVG1_LOCAL) {
         kk = nd.leaf_k;
@@ -278,7 +303,7 @@ KYM_HD void body_bwd_node1d(const Scat1DArgs<T>& a, int task, cpx<T>* lds, int t
         const FftLen<T>& fB = a.lens[a.len[lr]];
         const int s = a.ind_start[a.log2_stride], e = a.ind_end[a.log2_stride];
         for (int p = tid; p < nl; p += nth) {
-            const int t = fB.rev[p];
+            const int t = kym_ldg(fB.rev + p);
             B[p] = {(t >= s && t < e) ? d[t - s] : T(0), T(0)};
         }
         wg_barrier();
@@ -287,45 +312,89 @@ KYM_HD void body_bwd_node1d(const Scat1DArgs<T>& a, int task, cpx<T>* lds, int t
     const bool has_u_grad = (a.mode == AVG1_LOCAL) || (nd.child_end > nd.child_begin);
     const T* phi = a.mode == AVG1_LOCAL ? a.filt + a.filt_off[nd.leaf_filt] : nullptr;
     const T sc_leaf = T(1) / (T(nl) * T(kk));
-    for (int i = tid; i < n; i += nth) {
-        cpx<T> acc = {T(0), T(0)};
-        if (phi) {
-            const cpx<T> gy = B[i % nl];
-            acc = {gy.re * phi[i] * sc_leaf, gy.im * phi[i] * sc_leaf};
+    // E points per thread, two children at a time: 4 E loads in flight (the
+    // root sums some sixty children in one workgroup per signal)
+    constexpr int E = 4;
+    for (int i0 = tid; i0 < n; i0 += E * nth) {
+        int ix[E];
+        cpx<T> acc[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            ix[e] = i0 + e * nth < n ? i0 + e * nth : i0;
+            acc[e] = {T(0), T(0)};
+            if (phi) {
+                const cpx<T> gy = B[ix[e] & (nl - 1)];  // lengths are powers of two
+                const T ph = kym_ldg(phi + ix[e]) * sc_leaf;
+                acc[e] = {gy.re * ph, gy.im * ph};
+            }
         }
-#pragma unroll 4
-        for (int c = nd.child_begin; c < nd.child_end; ++c) {  // unrolled: several loads in flight
+#pragma unroll 2
+        for (int c = nd.child_begin; c < nd.child_end; ++c) {
             const Node1D& cn = a.nodes[c];
-            const int nc = a.n[cn.res];
-            const T fv = kym_ldg(a.filt + a.filt_off[cn.filt] + i) / T(cn.k);
-            const cpx<T> gx = kym_ldg(wsi + cn.gsave + (i % nc));
-            acc.re += gx.re * fv;
-            acc.im += gx.im * fv;
+            const int nm = a.n[cn.res] - 1;
+            const T* f = a.filt + a.filt_off[cn.filt];
+            const cpx<T>* g = wsi + cn.gsave;
+            const T inv_k = T(1) / T(cn.k);  // a power of two: exact
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const T fv = kym_ldg(f + ix[e]) * inv_k;
+                const cpx<T> gx = kym_ldg(g + (ix[e] & nm));
+                acc[e].re += gx.re * fv;
+                acc[e].im += gx.im * fv;
+            }
         }
-        lds[i] = acc;
+#pragma unroll
+        for (int e = 0; e < E; ++e)
+            if (i0 + e * nth < n) lds[ff.at(ix[e])] = acc[e];
     }
     wg_barrier();
-    if (has_u_grad) fft_dif<true, MAXP>(lds, fl, Batch{1, 1, n, false}, tid, nth);
+    if (has_u_grad) ff.inv(lds, fl, tid, nth);
     // direct terms on dL/dm (positions p hold natural index rev[p])
     const int us = a.ind_start[nd.unpad_res], ue = a.ind_end[nd.unpad_res];
     for (int p = tid; p < n; p += nth) {
-        T gm = has_u_grad ? lds[p].re : T(0);
-        const int t = fl.rev[p];
+        cpx<T>& c = lds[ff.at(p)];
+        T gm = has_u_grad ? c.re : T(0);
+        const int t = kym_ldg(fl.rev + p);
         if (a.mode == AVG1_NONE && t >= us && t < ue) gm += d[t - us];
         if (a.mode == AVG1_GLOBAL) gm += d[0];
         if (nd.order == 0) {
             reinterpret_cast<T*>(wsi + nd.gpad)[t] = gm;
         } else {
-            const cpx<T> u = wsi[nd.save + p];
+            const cpx<T> u = kym_ldg(wsi + nd.save + p);
             const T mag = kym_sqrt(u.re * u.re + u.im * u.im);
-            lds[p] = mag > T(0) ? cpx<T>{u.re * (gm / mag), u.im * (gm / mag)} : cpx<T>{T(0), T(0)};
+            c = mag > T(0) ? cpx<T>{u.re * (gm / mag), u.im * (gm / mag)} : cpx<T>{T(0), T(0)};
         }
     }
     if (nd.order == 0) return;
     wg_barrier();
-    fft_dit<false, MAXP>(lds, fl, Batch{1, 1, n, false}, tid, nth);
+    ff.fwd(lds, fl, tid, nth);
     const T inv_n = T(1) / T(n);
-    for (int i = tid; i < n; i += nth) wsi[nd.gsave + i] = lds[i] * inv_n;
+    for (int i = tid; i < n; i += nth) wsi[nd.gsave + i] = lds[ff.at(i)] * inv_n;
+}
+
+template <class T, int MAXP>
+KYM_HD void body_bwd_node1d(const Scat1DArgs<T>& a, int task, cpx<T>* lds, int tid, int nth) {
+    bwd_node1d_body<T, MAXP>(Dyn1D<T, MAXP>(), a, task, lds, tid, nth);
+}
+
+template <class T, int SPEC, bool EMU>
+KYM_HD KYM_INL void bwd_node1d_spec_body(const Scat1DArgs<T>& a, int task, cpx<T>* lds, int tid) {
+#define KYM_B1_BODY(sid, nn, nt)                                                                         \
+    if constexpr (SPEC == sid)                                                                           \
+        bwd_node1d_body<T, 2>(Stat1D<T, nn, (EMU ? 1 : nt)>(), a, task, lds, tid, EMU ? 1 : nt);
+    KYM_NODE1D_SPECS(KYM_B1_BODY)
+#undef KYM_B1_BODY
+}
+
+template <class T, bool EMU>
+KYM_HD void dispatch_bwd_node1d_spec(int id, const Scat1DArgs<T>& a, int task, cpx<T>* lds, int tid) {
+    switch (id) {
+#define KYM_B1_CASE(sid, nn, nt) \
+    case sid: bwd_node1d_spec_body<T, sid, EMU>(a, task, lds, tid); break;
+        KYM_NODE1D_SPECS(KYM_B1_CASE)
+#undef KYM_B1_CASE
+        default: break;
+    }
 }
 
 // Reflect-pad adjoint (1D).  task -> signal.

@@ -13,7 +13,7 @@ struct Launch1D {
     int ngroup, threads, res;
     size_t lds_bytes;
     long long model_bytes;  // algorithmic bytes per signal (stage-boundary model)
-    int spec = -1;          // compile-time node specialisation (FP32 forward), or -1
+    int spec = -1;          // compile-time node specialisation (FP32), or -1
 };
 
 struct Scat1DDesc {
@@ -211,11 +211,21 @@ struct Scat1DPlan {
             l.res = n0.res;
             const int len0 = n[n0.res];
             l.threads = std::max(64, std::min(1024, len0 / 16));
-            l.lds_bytes = (size_t)(len0 + (local ? len0 / std::max(n0.leaf_k, 1) : 0)) * cs;
-            // lds must cover every node of the group (same res => same length, leaf <= node)
-            for (int id : ids) {
-                const Node1D& nd = nodes[id];
-                l.lds_bytes = std::max(l.lds_bytes, (size_t)(n[nd.res] + (local ? n[nd.res] / nd.leaf_k : 0)) * cs);
+            // the node's line, then the leaf's (or the partial sums it is reduced from)
+            auto lds_of = [&](int line) {
+                size_t m = 0;
+                for (int id : ids) {
+                    const Node1D& nd = nodes[id];
+                    m = std::max(m, (size_t)(line + (local ? leaf1d_elems(n[nd.res] / std::max(nd.leaf_k, 1),
+                                                                           l.threads) : 0)) * cs);
+                }
+                return m;
+            };
+            l.lds_bytes = lds_of(len0);
+            // a compile-time length where its padded line fits
+            if (kind <= 1 && sizeof(T) == 4 && lds_of(pad16(len0)) <= lds_limit) {
+                l.spec = node1d_spec_id(len0, l.threads);
+                if (l.spec >= 0) l.lds_bytes = lds_of(pad16(len0));
             }
             long long mb = 0;
             for (int id : ids) {
@@ -223,7 +233,6 @@ struct Scat1DPlan {
                 mb += (nd.order == 0 ? 4ll * N + 16ll * N_pad : 40ll * n[nd.res]) + leaf_model;
             }
             l.model_bytes = mb;
-            if (kind == 0 && sizeof(T) == 4) l.spec = node1d_spec_id(len0, l.threads);
             launches.push_back(l);
             max_lds = std::max(max_lds, l.lds_bytes);
         };

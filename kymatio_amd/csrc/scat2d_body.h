@@ -674,12 +674,12 @@ struct StatGeom {
         fft_dit_s<false, H, W, W, 1, true, NT, true>(b, twH, tid);
     }
     KYM_HD KYM_INL void leaf_inv2d(cpx<T>* b, int tid, int) const {
-        fft_dif_s<true, WJ, HJ, 1, WJ, false, NT>(b, fWJ->tw, tid);
-        fft_dif_s<true, HJ, WJ, WJ, 1, true, NT>(b, fHJ->tw, tid);
+        fft_dif_s<true, WJ, HJ, 1, WJ, false, NT>(b, fWJ->ptw, tid);
+        fft_dif_s<true, HJ, WJ, WJ, 1, true, NT>(b, fHJ->ptw, tid);
     }
     KYM_HD KYM_INL void leaf_fwd2d(cpx<T>* b, int tid, int) const {
-        fft_dit_s<false, WJ, HJ, 1, WJ, false, NT>(b, fWJ->tw, tid);
-        fft_dit_s<false, HJ, WJ, WJ, 1, true, NT>(b, fHJ->tw, tid);
+        fft_dit_s<false, WJ, HJ, 1, WJ, false, NT>(b, fWJ->ptw, tid);
+        fft_dit_s<false, HJ, WJ, WJ, 1, true, NT>(b, fHJ->ptw, tid);
     }
 };
 
