@@ -665,11 +665,13 @@ static int upload1d(Scat1DPlan<T>& p, void** dblob) {
     KYM_HIP_TRY(hipMalloc(dblob, bytes));
     p.blob.relocate((uintptr_t)*dblob);
     KYM_HIP_TRY(hipMemcpy(*dblob, p.blob.bytes.data(), bytes, hipMemcpyHostToDevice));
-    for (const std::vector<Launch1D>* ls : {&p.launches, &p.bwd_launches})
+    // the device's limit, not this plan's need: plans share the kernels
+    for (const std::vector<Launch1D>* ls : {&p.launches, &p.bwd_launches, &p.merged, &p.bwd_merged})
         for (const Launch1D& l : *ls)
             if (l.lds_bytes > 65536)
                 KYM_HIP_TRY(hipFuncSetAttribute((const void*)pick_scat1d<T>(l.threads, l.kind, l.spec),
-                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)l.lds_bytes));
+                                                hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                (int)device_lds_limit()));
     return KYM_OK;
 }
 
@@ -770,9 +772,12 @@ static int run1d(const Scat1DPlan<T>& p, int mode, const void* x, const void* fi
     if (chunk < 1) return fail(KYM_ERR_VALUE, "workspace too small for one signal");
     if (chunk > batch) chunk = batch;
     if (mode != 0 && chunk < batch) return fail(KYM_ERR_VALUE, "training workspace must hold the whole batch");
-    const std::vector<Launch1D>& launches = mode == 2 ? p.bwd_launches : p.launches;
+    // few signals: one launch per order, on the caller's stream
+    const bool merged = chunk >= batch && !(prof && prof->enabled) && p.merged_fits(batch);
+    const std::vector<Launch1D>& launches =
+        merged ? (mode == 2 ? p.bwd_merged : p.merged) : mode == 2 ? p.bwd_launches : p.launches;
     // inference chunks rotate over the plan's streams as in run2d
-    const int ns = chunk_streams(cs, streams, mode, batch, &chunk);
+    const int ns = merged ? 1 : chunk_streams(cs, streams, mode, batch, &chunk);
     int rc = chunk_fork(cs, ns, stream);
     if (rc != KYM_OK) return rc;
     int k = 0;

@@ -231,7 +231,7 @@ extern "C" int kym_emu_scat2d_forward(int M, int N, int J, int L, int max_order,
     return emu_forward2d<double>(M, N, J, L, max_order, pre_pad, lds_limit, x, filt, out, batch, chunk, info);
 }
 
-extern "C" int kym_emu_scat1d_forward(int N, int N_pad, int pad_left, int log2_stride, int average_mode,
+static int emu_scat1d(bool merged, int N, int N_pad, int pad_left, int log2_stride, int average_mode,
                                       int oversampling, int max_order, int n_psi1, const int* psi1_j,
                                       const int* psi1_nlev, int n_psi2, const int* psi2_j, const int* psi2_nlev,
                                       int phi_nlev, const int* ind_start, const int* ind_end, int n_ind, int dtype,
@@ -261,7 +261,8 @@ extern "C" int kym_emu_scat1d_forward(int N, int N_pad, int pad_left, int log2_s
         std::vector<cpx<T>> ws((size_t)(stride * batch) + 1);
         std::vector<cpx<T>> lds(p.max_lds / sizeof(cpx<T>) + 1);
         for (int phase = 0; phase < (train ? 1 + nbwd : 1); ++phase)
-            for (const Launch1D& l : (phase ? p.bwd_launches : p.launches)) {
+            for (const Launch1D& l : (phase ? (merged ? p.bwd_merged : p.bwd_launches)
+                                            : (merged ? p.merged : p.launches))) {
                 Scat1DArgs<T> a = p.args(l, base);
                 a.x = static_cast<const T*>(x);
                 a.filt = static_cast<const T*>(filt);
@@ -274,7 +275,9 @@ extern "C" int kym_emu_scat1d_forward(int N, int N_pad, int pad_left, int log2_s
                 a.img0 = 0;
                 a.ntask = (int)(batch * l.ngroup);
                 for (int t = 0; t < a.ntask; ++t) {
-                    if (l.kind == 0 && l.spec >= 0) dispatch_node1d_spec<T, true>(l.spec, a, t, lds.data(), 0);
+                    if (l.spec == KYM_N1_ANY && l.kind == 0) node1d_any_body<T, 0, true>(a, t, lds.data(), 0);
+                    else if (l.spec == KYM_N1_ANY && l.kind == 1) node1d_any_body<T, 1, true>(a, t, lds.data(), 0);
+                    else if (l.kind == 0 && l.spec >= 0) dispatch_node1d_spec<T, true>(l.spec, a, t, lds.data(), 0);
                     else if (l.kind == 1 && l.spec >= 0) dispatch_bwd_node1d_spec<T, true>(l.spec, a, t, lds.data(), 0);
                     else if (l.kind == 0) body_node1d<T, 31>(a, t, lds.data(), 0, 1);
                     else if (l.kind == 1) body_bwd_node1d<T, 31>(a, t, lds.data(), 0, 1);
@@ -288,6 +291,27 @@ extern "C" int kym_emu_scat1d_forward(int N, int N_pad, int pad_left, int log2_s
 }
 
 // Per-op FFT (kym_op_fft) on the host: same launch sequence and bodies.
+extern "C" int kym_emu_scat1d_forward(int N, int N_pad, int pad_left, int log2_stride, int average_mode,
+                                      int oversampling, int max_order, int n_psi1, const int* psi1_j,
+                                      const int* psi1_nlev, int n_psi2, const int* psi2_j, const int* psi2_nlev,
+                                      int phi_nlev, const int* ind_start, const int* ind_end, int n_ind, int dtype,
+                                      const void* x, const void* filt, void* out, long long batch,
+                                      long long* info, const void* dS, void* gx, int nbwd) {
+    return emu_scat1d(false, N, N_pad, pad_left, log2_stride, average_mode, oversampling, max_order, n_psi1, psi1_j, psi1_nlev, n_psi2,
+                      psi2_j, psi2_nlev, phi_nlev, ind_start, ind_end, n_ind, dtype, x, filt, out, batch, info, dS, gx, nbwd);
+}
+
+// The same by the merged launches (one per order).
+extern "C" int kym_emu_scat1d_merged(int N, int N_pad, int pad_left, int log2_stride, int average_mode,
+                                      int oversampling, int max_order, int n_psi1, const int* psi1_j,
+                                      const int* psi1_nlev, int n_psi2, const int* psi2_j, const int* psi2_nlev,
+                                      int phi_nlev, const int* ind_start, const int* ind_end, int n_ind, int dtype,
+                                      const void* x, const void* filt, void* out, long long batch,
+                                      long long* info, const void* dS, void* gx, int nbwd) {
+    return emu_scat1d(true, N, N_pad, pad_left, log2_stride, average_mode, oversampling, max_order, n_psi1, psi1_j, psi1_nlev, n_psi2,
+                      psi2_j, psi2_nlev, phi_nlev, ind_start, ind_end, n_ind, dtype, x, filt, out, batch, info, dS, gx, nbwd);
+}
+
 template <class T>
 static int emu_op_fft(const void* x, void* y, void* work, long long batch, int H, int W, int kind, long long lds_cap) {
     LenTable<T> lt;

@@ -31,6 +31,14 @@ __global__ void __launch_bounds__(NT) k_bwd_node1d_spec(Scat1DArgs<T> a) {
     bwd_node1d_spec_body<T, SPEC, false>(a, task, reinterpret_cast<cpx<T>*>(kym_smem1d_bns), threadIdx.x);
 }
 
+template <class T, int KIND>
+__global__ void __launch_bounds__(1024) k_node1d_any(Scat1DArgs<T> a) {
+    extern __shared__ __attribute__((aligned(16))) char kym_smem1d_any[];
+    const int task = xcd_task(blockIdx.x, gridDim.x);
+    if (task >= a.ntask) return;
+    node1d_any_body<T, KIND, false>(a, task, reinterpret_cast<cpx<T>*>(kym_smem1d_any), threadIdx.x);
+}
+
 template <class T>
 using Scat1DKernel = void (*)(Scat1DArgs<T>);
 

@@ -19,6 +19,7 @@ Scat2DKernel<float> kym_pick_pass_spec_f32(int kind, int id);
 Scat1DKernel<float> kym_pick1d_f32(int threads, int kind);
 Scat1DKernel<float> kym_pick_node1d_spec_f32(int id);
 Scat1DKernel<float> kym_pick_bwd_node1d_spec_f32(int id);
+Scat1DKernel<float> kym_pick_any1d_f32(int kind);
 Scat1DKernel<double> kym_pick1d_f64(int threads, int kind);
 
 // pclass: 7, 17 or 31 (kym_prime_class of the plan's largest odd prime);
@@ -43,6 +44,7 @@ inline Scat2DKernel<T> pick_scat2d(int kind, int threads, int pclass, int spec =
 template <class T>
 inline Scat1DKernel<T> pick_scat1d(int threads, int kind = 0, int spec = -1) {
     if constexpr (sizeof(T) == 4) {
+        if (spec == KYM_N1_ANY && kind <= 1) return kym_pick_any1d_f32(kind);
         if (spec >= 0 && kind == 0) return kym_pick_node1d_spec_f32(spec);
         if (spec >= 0 && kind == 1) return kym_pick_bwd_node1d_spec_f32(spec);
         return kym_pick1d_f32(threads, kind);

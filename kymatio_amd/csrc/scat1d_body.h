@@ -90,9 +90,18 @@ struct Stat1D {
     }
 };
 
-// LDS elements after the node's line: the leaf's line of nl points, or the
-// nth partial sums it is reduced from.
-KYM_HD KYM_INL int leaf1d_elems(int nl, int nth) { return nl > nth ? nl : nth; }
+// Threads of a node's workgroup by its length, and the threads per output
+// point (powers of two) that share its low-pass sum: 64 aliases of 128 points
+// kept 384 of 512 threads waiting otherwise.  The split follows the sizes
+// alone, so that a node's sums do not depend on the launch it runs in.
+KYM_HD KYM_INL constexpr int node1d_threads(int n) { return n / 16 < 64 ? 64 : n / 16 > 1024 ? 1024 : n / 16; }
+KYM_HD KYM_INL constexpr int leaf1d_split(int n, int nl) {
+    int S = 1;
+    while (2 * S * nl <= node1d_threads(n) && 2 * S * nl <= n) S *= 2;
+    return S;
+}
+// LDS elements after the node's line: the leaf's line of nl points as S partial sums.
+KYM_HD KYM_INL constexpr int leaf1d_elems(int n, int nl) { return nl * leaf1d_split(n, nl); }
 
 // Output of one path from the spectrum / modulus in LDS.
 template <class T, int MAXP, class F>
@@ -110,10 +119,7 @@ KYM_HD KYM_INL void leaf1d(const F& ff, const Scat1DArgs<T>& a, const Node1D& nd
     const FInt nl = fB.size();
     const T* phi = a.filt + a.filt_off[nd.leaf_filt];
     const T inv_k = T(1) / T(kk);
-    // S threads per output point (powers of two), each an S-th of the aliases:
-    // 64 aliases of 128 points kept 384 of 512 threads waiting otherwise
-    int S = 1;
-    while (2 * S * nl <= nth && 2 * S <= kk) S *= 2;
+    const int S = leaf1d_split(n, nl);
     for (int q = tid; q < S * nl; q += nth) {
         const int s = q / nl, i = q - s * nl;
         cpx<T> acc = {T(0), T(0)};
@@ -128,7 +134,7 @@ KYM_HD KYM_INL void leaf1d(const F& ff, const Scat1DArgs<T>& a, const Node1D& nd
     }
     wg_barrier();
     if (S > 1) {
-        for (int i = tid; i < nl; i += nth) {  // nl < nth: one point per thread
+        for (int i = tid; i < nl; i += nth) {
             cpx<T> acc = B[i];
             for (int s = 1; s < S; ++s) acc = acc + B[i + s * nl];
             B[i] = acc;
@@ -249,7 +255,7 @@ KYM_HD void body_node1d(const Scat1DArgs<T>& a, int task, cpx<T>* lds, int tid, 
     X(6, 256, 64)           \
     X(7, 128, 64)
 
-inline int node1d_spec_id(int n, int threads) {
+KYM_HD KYM_INL int node1d_spec_id(int n, int threads) {
 #define KYM_N1_MATCH(id, nn, nt) \
     if (n == nn && threads == nt) return id;
     KYM_NODE1D_SPECS(KYM_N1_MATCH)
@@ -415,5 +421,30 @@ KYM_HD void body_bwd_fold1d(const Scat1DArgs<T>& a, int task, int tid, int nth) 
                 for (int t = ((a.pad_left - i) % T_ + T_) % T_; t < P; t += T_) acc += gp[t];
         }
         gx[i] = acc;
+    }
+}
+
+// A node of any length in one workgroup (FP32; launches that mix lengths):
+// the compiled body of its length on the first node1d_threads(n) threads, the
+// very code of a launch of that length alone, so that results do not depend on
+// which launch a node ran in.  The other threads start beyond every loop and
+// only meet the barriers.
+#define KYM_N1_ANY 1000  // Launch1D::spec of such a launch
+template <class T, int KIND, bool EMU>
+KYM_HD KYM_INL void node1d_any_body(const Scat1DArgs<T>& a, int task, cpx<T>* lds, int tid) {
+    const Node1D& nd = a.nodes[a.group[task % a.ngroup]];
+    const int n = a.n[nd.res], nt = EMU ? 1 : node1d_threads(n);
+    if (tid >= nt) tid = 1 << 28;
+    switch (node1d_spec_id(n, node1d_threads(n))) {
+#define KYM_NA_CASE(sid, nn, nnt)                                                     \
+    case sid:                                                                        \
+        if constexpr (KIND == 0) node1d_spec_body<T, sid, EMU>(a, task, lds, tid);   \
+        else bwd_node1d_spec_body<T, sid, EMU>(a, task, lds, tid);                   \
+        break;
+        KYM_NODE1D_SPECS(KYM_NA_CASE)
+#undef KYM_NA_CASE
+        default:
+            if constexpr (KIND == 0) body_node1d<T, 2>(a, task, lds, tid, nt);
+            else body_bwd_node1d<T, 2>(a, task, lds, tid, nt);
     }
 }

@@ -40,6 +40,11 @@ struct Scat1DPlan {
     int C = 0, pclass = 7;
     LenTable<T> lens;
     std::vector<Launch1D> launches, bwd_launches;
+    // the same nodes with one launch per order, every length in it
+    // (node1d_any_body): for batches whose nodes all fit the GPU at once, where a
+    // forward is the latency of its launches one after the other (3 against 11
+    // per chunk, and one chunk); see merged_fits
+    std::vector<Launch1D> merged, bwd_merged;
     long long ws_sig_train = 0;
     Blob blob;
     size_t off_nodes = 0, off_lens = 0, off_filt = 0, max_lds = 0;
@@ -200,7 +205,7 @@ struct Scat1DPlan {
         launches.clear();
         max_lds = 0;
         const long long leaf_model = local ? 16ll * (N_pad >> ls) + 4ll * Tlocal : 4;
-        auto push = [&](const std::vector<int>& ids, int kind) {
+        auto push = [&](const std::vector<int>& ids, int kind, bool mixed = false) {
             if (ids.empty()) return;
             Launch1D l;
             l.kind = kind;
@@ -209,23 +214,27 @@ struct Scat1DPlan {
             l.ngroup = (int)ids.size();
             const Node1D& n0 = nodes[ids[0]];
             l.res = n0.res;
-            const int len0 = n[n0.res];
-            l.threads = std::max(64, std::min(1024, len0 / 16));
-            // the node's line, then the leaf's (or the partial sums it is reduced from)
-            auto lds_of = [&](int line) {
+            int len0 = n[n0.res];  // mixed: the longest line
+            for (int id : ids) len0 = std::max(len0, n[nodes[id].res]);
+            // mixed launches have CUs to spare: half the points per thread
+            l.threads = node1d_threads(len0);
+            // a node's line (padded: the compiled lengths), then the leaf's
+            // partial sums
+            auto lds_of = [&](bool pad) {
                 size_t m = 0;
                 for (int id : ids) {
-                    const Node1D& nd = nodes[id];
-                    m = std::max(m, (size_t)(line + (local ? leaf1d_elems(n[nd.res] / std::max(nd.leaf_k, 1),
-                                                                           l.threads) : 0)) * cs);
+                    const int nn = n[nodes[id].res];
+                    const int line = pad && node1d_spec_id(nn, node1d_threads(nn)) >= 0 ? pad16(nn) : nn;
+                    const int leaf = local ? leaf1d_elems(nn, nn / std::max(nodes[id].leaf_k, 1)) : 0;
+                    m = std::max(m, (size_t)(line + leaf) * cs);
                 }
                 return m;
             };
-            l.lds_bytes = lds_of(len0);
-            // a compile-time length where its padded line fits
-            if (kind <= 1 && sizeof(T) == 4 && lds_of(pad16(len0)) <= lds_limit) {
-                l.spec = node1d_spec_id(len0, l.threads);
-                if (l.spec >= 0) l.lds_bytes = lds_of(pad16(len0));
+            l.lds_bytes = lds_of(false);
+            // compile-time lengths where the padded lines fit
+            if (kind <= 1 && sizeof(T) == 4 && lds_of(true) <= lds_limit) {
+                l.spec = mixed ? KYM_N1_ANY : node1d_spec_id(len0, l.threads);
+                if (l.spec >= 0) l.lds_bytes = lds_of(true);
             }
             long long mb = 0;
             for (int id : ids) {
@@ -258,7 +267,41 @@ struct Scat1DPlan {
         launches.back().threads = 256;
         launches.back().lds_bytes = 0;
         bwd_launches = launches;
+        auto by_order = [&](int order) {
+            std::vector<int> ids;
+            for (size_t i = 0; i < nodes.size(); ++i)
+                if (nodes[i].order == order) ids.push_back((int)i);
+            return ids;
+        };
+        launches.clear();
+        for (int order = 0; order <= max_order; ++order) push(by_order(order), 0, true);
+        merged = launches;
+        launches.clear();
+        for (int order = max_order; order >= 0; --order) push(by_order(order), 1, true);
+        launches.push_back(bwd_launches.back());  // the pad fold
+        bwd_merged = launches;
         launches = fwd;
+        // FP32: only with the compiled bodies, whose results are those of the
+        // per-length launches to the last bit
+        mixed_ok = true;
+        for (const std::vector<Launch1D>* ls : {&merged, &bwd_merged})
+            for (const Launch1D& l : *ls)
+                if (l.kind <= 1) mixed_ok = mixed_ok && (sizeof(T) == 8 || l.spec == KYM_N1_ANY);
+        return true;
+    }
+
+    bool mixed_ok = true;
+
+    // Whether every workgroup of the merged launches over `batch` signals is
+    // resident at once (256 CUs of 160 KB LDS and 2048 threads).  Beyond that
+    // the per-length launches with their compiled kernels are faster.
+    bool merged_fits(long long batch) const {
+        if (!mixed_ok) return false;
+        for (const std::vector<Launch1D>* ls : {&merged, &bwd_merged})
+            for (const Launch1D& l : *ls) {
+                const long long per_cu = std::min(160ll * 1024 / (long long)std::max(l.lds_bytes, (size_t)1), 2048ll / l.threads);
+                if (l.kind != 2 && batch * l.ngroup > 256 * per_cu) return false;
+            }
         return true;
     }
 

@@ -123,13 +123,13 @@ class Emu:
                      'bwd_spec_launches': info[7], 'col_pair_launches': info[8]}
 
 
-def emu_scat1d(emu, module, x, dtype=np.float32, dS=None, nbwd=1):
+def emu_scat1d(emu, module, x, dtype=np.float32, dS=None, nbwd=1, merged=False):
     """Run the 1D bodies in the CPU harness with the setup of a (CPU)
     Scattering1D module; with dS, also the backward (returns S, C, dL/dx)."""
     m = module
     modes = {'local': 0, False: 1, 'global': 2}
     i32 = lambda v: (ctypes.c_int * max(len(v), 1))(*v)
-    f = emu.lib.kym_emu_scat1d_forward
+    f = emu.lib.kym_emu_scat1d_merged if merged else emu.lib.kym_emu_scat1d_forward
     f.argtypes = ([ctypes.c_int] * 8 + [ctypes.c_void_p] * 2 + [ctypes.c_int] + [ctypes.c_void_p] * 2
                   + [ctypes.c_int] + [ctypes.c_void_p] * 2 + [ctypes.c_int, ctypes.c_int]
                   + [ctypes.c_void_p] * 3 + [ctypes.c_longlong, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,

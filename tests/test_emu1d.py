@@ -81,3 +81,23 @@ def test_backward_matches_autograd_through_oracle(emu, kw):
     assert np.abs(out - flat.detach().numpy()).max() <= 1e-12 * np.abs(flat.detach().numpy()).max()
     g = xt.grad.numpy()
     assert np.abs(gx - g).max() <= 1e-11 * np.abs(g).max()
+
+
+@pytest.mark.parametrize('J,N,Q,kw', [(3, 64, 2, {}), (6, 512, 8, {}), (5, 1000, (4, 2), {}), (6, 512, 8, {'T': 'global'}),
+                                      (6, 512, 8, {'T': 0, 'out_type': 'list'}), (5, 1024, 4, {'max_order': 1}),
+                                      (4, 700, 8, {'stride': 4})])
+@pytest.mark.parametrize('dtype', [np.float32, np.float64])
+def test_merged_launches_match(emu, J, N, Q, kw, dtype):
+    """One launch per order (few signals) against one per length, forward and
+    backward: the same node arithmetic with other workgroups and FFT kernels."""
+    S = Scattering1D(J, N, Q, **kw)
+    rng = np.random.default_rng(J * N)
+    x = rng.standard_normal((2, N)).astype(dtype)
+    out, C = emu_scat1d(emu, S, x, dtype)
+    w = rng.standard_normal(out.shape).astype(dtype)
+    out, _, gx = emu_scat1d(emu, S, x, dtype, dS=w)
+    om, _, gm = emu_scat1d(emu, S, x, dtype, dS=w, merged=True)
+    eps = np.finfo(dtype).eps
+    # rounding of transforms of up to 2^12 points and of sums over the nodes
+    assert np.abs(om - out).max() <= 40 * eps * np.abs(out).max()
+    assert np.abs(gm - gx).max() <= 400 * eps * np.abs(gx).max()

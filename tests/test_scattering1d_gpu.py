@@ -147,3 +147,18 @@ def test_shape_errors():
         Scattering1D(6, (5, 6), 8)
     with pytest.raises(ValueError, match='1-tuple'):
         Scattering1D(6, 1.5, 8)
+
+
+@pytest.mark.parametrize('J,N,Q,B', [(5, 1000, 4, 200), (6, 4096, 8, 40), (3, 300, 1, 500)])
+def test_small_batches_match_large(J, N, Q, B):
+    """Batches whose nodes fit the GPU at once take one launch per order, others
+    one per length: the same coefficients and gradients."""
+    sc = Scattering1D(J, N, Q).to(DEV)
+    x = torch.randn(B, N, device=DEV, generator=torch.Generator(DEV).manual_seed(N)).requires_grad_()
+    y = sc(x)
+    w = torch.randn(y.shape, device=DEV, generator=torch.Generator(DEV).manual_seed(1))
+    g, = torch.autograd.grad(y, x, w)
+    y2 = torch.cat([sc(x[i:i + 2]) for i in range(0, B, 2)])
+    g2, = torch.autograd.grad(y2, x, w)
+    assert (y - y2).abs().max() <= 5e-6 * y.abs().max()
+    assert (g - g2).abs().max() <= 5e-5 * g.abs().max()
