@@ -337,6 +337,16 @@ int kym_op_harmonic_products(const void* U, const void* F, void* out, long long 
                              void* stream);
 int kym_op_modulus_rotation_sum(const void* x, void* y, long long batch, int nm, long long n, long long ystride,
                                 int dtype, void* stream);
+/* Both, and the inverse 3D transform between them, for ng scales of one
+ * order l: dest (group g, image b, at g * dstride + b * M N O) =
+ * sqrt(sum_m |ifft3(U[b] F[g, m])|^2), F's group g at g * fstride complex
+ * elements.  work: B ng nm M N O complex elements.  Status 5 where a plane
+ * N x O or a block of lines along M does not fit one workgroup. */
+int kym_op_harmonic_step(const void* U, const void* F, void* work, void* dest, long long B, int ng, int nm, int M, int N,
+                         int O, long long fstride, long long dstride, int dtype, void* stream);
+/* Complex transform along the first axis of (B, M, S), x may equal y;
+ * inverse with 1/M. */
+int kym_op_fft_axis0(const void* x, void* y, long long B, int M, long long S, int inverse, int dtype, void* stream);
 /* compute_integrals (kymatio/scattering3d/backend/torch_backend.py:126-151):
  * out[b, q] = sum over the n elements of x[b] of x^powers[q], q < npow <= 8
  * (accumulated in FP64, stored in the dtype). */

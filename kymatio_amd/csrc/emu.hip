@@ -502,3 +502,46 @@ extern "C" int kym_emu_op_fft(const void* x, void* y, void* work, long long batc
     if (dtype == 0) return emu_op_fft<float>(x, y, work, batch, H, W, kind, lds_cap);
     return emu_op_fft<double>(x, y, work, batch, H, W, kind, lds_cap);
 }
+
+// The 3D steps (kym_op_harmonic_step with one group stride, kym_op_fft_axis0).
+template <class T>
+static int emu_harmonic(const void* U, const void* F, void* work, void* dest, long long B, int ng, int nm, int M, int N,
+                        int O, long long fstride, long long dstride) {
+    LenTable<T> lt;
+    const int lM = lt.add(M), lN = lt.add(N), lO = lt.add(O);
+    Blob b;
+    size_t off = 0;
+    if (!lt.emit(b, &off, &g_emu_error)) return KYM_ERR_UNSUPPORTED;
+    b.relocate((uintptr_t)b.bytes.data());
+    const FftLen<T>* lens = b.at<FftLen<T>>(off);
+    HarmonicArgs o = {U, F, work, dest, B, fstride, dstride, ng, nm, M, N, O, 0, 0};
+    o.cb = axis0_cols(M, N * O);
+    o.ncb = (N * O + o.cb - 1) / o.cb;
+    std::vector<cpx<T>> lds((size_t)std::max(N * plane_stride(O), M * o.cb));
+    for (long long k = 0; k < B * ng * nm * M; ++k)
+        harmonic_plane_body<T, 31>(o, lens[lN], lens[lO], k, lds.data(), 0, 1);
+    for (long long k = 0; k < B * ng * o.ncb; ++k)
+        harmonic_cols_body<T, 31, KYM_HARM_E * 256>(o, lens[lM], k, lds.data(), 0, 1);
+    return 0;
+}
+
+extern "C" int kym_emu_op_harmonic_step(const void* U, const void* F, void* work, void* dest, long long B, int ng,
+                                        int nm, int M, int N, int O, long long fstride, long long dstride, int dtype) {
+    if (dtype == 0) return emu_harmonic<float>(U, F, work, dest, B, ng, nm, M, N, O, fstride, dstride);
+    return emu_harmonic<double>(U, F, work, dest, B, ng, nm, M, N, O, fstride, dstride);
+}
+
+extern "C" int kym_emu_op_fft_axis0(const void* x, void* y, long long B, int M, int S, int inverse) {
+    LenTable<double> lt;
+    const int lM = lt.add(M);
+    Blob b;
+    size_t off = 0;
+    if (!lt.emit(b, &off, &g_emu_error)) return KYM_ERR_UNSUPPORTED;
+    b.relocate((uintptr_t)b.bytes.data());
+    const int cb = axis0_cols(M, S), ncb = (S + cb - 1) / cb;
+    std::vector<cpx<double>> lds((size_t)M * cb);
+    for (long long k = 0; k < B * ncb; ++k)
+        fft_axis0_body<double, 31>((const cpx<double>*)x, (cpx<double>*)y, S, cb, ncb, inverse,
+                                   b.at<FftLen<double>>(off)[lM], k, lds.data(), 0, 1);
+    return 0;
+}

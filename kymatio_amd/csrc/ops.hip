@@ -129,10 +129,21 @@ __global__ void __launch_bounds__(256) k_integrals(const T* x, T* out, long long
     const T* xb = x + b * n;
     double acc[KYM_MAX_POWERS];
     for (int q = 0; q < KYM_MAX_POWERS; ++q) acc[q] = 0.0;
-    for (long long i = threadIdx.x; i < n; i += blockDim.x) {
-        const double v = (double)xb[i];
-        for (int q = 0; q < pw.n; ++q) acc[q] += pow(v, pw.p[q]);
+    // the usual powers without pow (exact but for its last bit; the library
+    // call took 158 us for 192 fields of 32^3, most of it here), four loads in
+    // flight
+    auto power = [&](double v, double p) { return p == 1.0 ? v : p == 2.0 ? v * v : p == 0.5 ? sqrt(v) : pow(v, p); };
+    long long i = threadIdx.x;
+    for (; i + 3 * blockDim.x < n; i += 4 * blockDim.x) {
+        T v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = xb[i + u * blockDim.x];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            for (int q = 0; q < pw.n; ++q) acc[q] += power((double)v[u], pw.p[q]);
     }
+    for (; i < n; i += blockDim.x)
+        for (int q = 0; q < pw.n; ++q) acc[q] += power((double)xb[i], pw.p[q]);
     for (int q = 0; q < pw.n; ++q) part[q][threadIdx.x] = acc[q];
     __syncthreads();
     for (int w = blockDim.x / 2; w > 0; w >>= 1) {
@@ -617,6 +628,134 @@ extern "C" int kym_op_harmonic_products(const void* U, const void* F, void* out,
     hipStream_t s = (hipStream_t)stream;
     if (dtype == KYM_F32) return launch_harmonic_products<float>(U, F, out, batch, nm, n, s);
     if (dtype == KYM_F64) return launch_harmonic_products<double>(U, F, out, batch, nm, n, s);
+    return bad_dtype();
+}
+
+// ------------------------------------------------------------ 3D steps
+template <class T, int MAXP, int NT>
+__global__ void __launch_bounds__(NT) k_harm_plane(HarmonicArgs o, const FftLen<T>* lens, int lN, int lO) {
+    extern __shared__ __attribute__((aligned(16))) char kym_smem_hp[];
+    harmonic_plane_body<T, MAXP>(o, lens[lN], lens[lO], blockIdx.x, reinterpret_cast<cpx<T>*>(kym_smem_hp), threadIdx.x,
+                                 NT);
+}
+
+template <class T, int MAXP>
+__global__ void __launch_bounds__(256) k_harm_cols(HarmonicArgs o, const FftLen<T>* lens, int lM) {
+    extern __shared__ __attribute__((aligned(16))) char kym_smem_hc[];
+    harmonic_cols_body<T, MAXP, KYM_HARM_E>(o, lens[lM], blockIdx.x, reinterpret_cast<cpx<T>*>(kym_smem_hc),
+                                            threadIdx.x, 256);
+}
+
+template <class T, int MAXP>
+__global__ void __launch_bounds__(256) k_fft_axis0(const cpx<T>* x, cpx<T>* y, int S, int cb, int ncb, int inv,
+                                                   const FftLen<T>* lens, int lM) {
+    extern __shared__ __attribute__((aligned(16))) char kym_smem_a0[];
+    fft_axis0_body<T, MAXP>(x, y, S, cb, ncb, inv, lens[lM], blockIdx.x, reinterpret_cast<cpx<T>*>(kym_smem_a0),
+                            threadIdx.x, 256);
+}
+
+template <class T, int MAXP>
+static const void* pick_harm_plane(int nt) {
+    switch (nt) {
+        case 64: return (const void*)k_harm_plane<T, MAXP, 64>;
+        case 128: return (const void*)k_harm_plane<T, MAXP, 128>;
+        case 256: return (const void*)k_harm_plane<T, MAXP, 256>;
+        case 512: return (const void*)k_harm_plane<T, MAXP, 512>;
+        default: return (const void*)k_harm_plane<T, MAXP, 1024>;
+    }
+}
+
+template <class T, int MAXP>
+static int harmonic_step_p(HarmonicArgs o, hipStream_t s) {
+    OpTables tp, tm;
+    int rc = op_tables<T>(o.N, o.O, &tp);
+    if (rc == KYM_OK) rc = op_tables<T>(o.M, 1, &tm);
+    if (rc != KYM_OK) return rc;
+    const FftLen<T>* lp = reinterpret_cast<const FftLen<T>*>((char*)tp.dev + tp.lens_off);
+    const FftLen<T>* lm = reinterpret_cast<const FftLen<T>*>((char*)tm.dev + tm.lens_off);
+    const size_t lds = (size_t)o.N * plane_stride(o.O) * sizeof(cpx<T>);
+    const int S = o.N * o.O;
+    o.cb = axis0_cols(o.M, S);
+    o.ncb = (S + o.cb - 1) / o.cb;
+    const long long planes = o.B * o.ng * o.nm * o.M, cols = o.B * o.ng * o.ncb;
+    // a plane and a block of columns each within one workgroup
+    if (lds > op_lds_limit() || (long long)o.M * o.cb > KYM_HARM_E * 256) return KYM_ERR_UNSUPPORTED;
+    if (planes > 0x7fffffffll || cols > 0x7fffffffll) return KYM_ERR_UNSUPPORTED;
+    const int nt = plane_threads(S);
+    const void* k = pick_harm_plane<T, MAXP>(nt);
+    if (lds > 65536)
+        OPS_HIP_TRY(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)op_lds_limit()));
+    void* a[4] = {&o, &lp, &tp.lH, &tp.lW};
+    OPS_HIP_TRY(hipLaunchKernel(k, dim3((unsigned)planes), dim3(nt), a, lds, s));
+    hipLaunchKernelGGL((k_harm_cols<T, MAXP>), dim3((unsigned)cols), dim3(256), (size_t)o.M * o.cb * sizeof(cpx<T>), s, o,
+                       lm, tm.lH);
+    OPS_HIP_TRY(hipGetLastError());
+    return KYM_OK;
+}
+
+template <class T>
+static int harmonic_step(const HarmonicArgs& o, hipStream_t s) {
+    const int c = std::max(op_pclass(o.N, o.O), op_pclass(o.M));
+    return c <= 7 ? harmonic_step_p<T, 7>(o, s) : c <= 17 ? harmonic_step_p<T, 17>(o, s) : harmonic_step_p<T, 31>(o, s);
+}
+
+// A product of the extents that fits the kernels' 32-bit plane and column indices.
+static bool harmonic_sizes_ok(long long M, long long N, long long O) {
+    return M >= 1 && N >= 1 && O >= 1 && M <= 2048 && N <= 20480 && O <= 20480 && N * O <= (1ll << 28);
+}
+
+extern "C" int kym_op_harmonic_step(const void* U, const void* F, void* work, void* dest, long long B, int ng, int nm,
+                                    int M, int N, int O, long long fstride, long long dstride, int dtype,
+                                    void* stream) {
+    if (ng < 1 || nm < 1) return kym_ops_fail(KYM_ERR_VALUE, "at least one filter per (l, j)");
+    if (B <= 0) return KYM_OK;
+    if (!U || !F || !work || !dest) return kym_ops_fail(KYM_ERR_VALUE, "null device pointer");
+    if (dtype != KYM_F32 && dtype != KYM_F64) return bad_dtype();
+    int rc = KYM_ERR_UNSUPPORTED;
+    if (harmonic_sizes_ok(M, N, O)) {
+        const HarmonicArgs o = {U, F, work, dest, B, fstride, dstride, ng, nm, M, N, O, 0, 0};
+        rc = dtype == KYM_F32 ? harmonic_step<float>(o, (hipStream_t)stream) : harmonic_step<double>(o, (hipStream_t)stream);
+    }
+    if (rc == KYM_ERR_UNSUPPORTED)
+        return kym_ops_fail(rc, "kym_op_harmonic_step: a plane or a line does not fit one workgroup");
+    return rc;
+}
+
+template <class T, int MAXP>
+static int fft_axis0_p(const void* x, void* y, long long B, int M, int S, int inv, hipStream_t s) {
+    OpTables t;
+    const int rc = op_tables<T>(M, 1, &t);
+    if (rc != KYM_OK) return rc;
+    const int cb = axis0_cols(M, S), ncb = (S + cb - 1) / cb;
+    const size_t lds = (size_t)M * cb * sizeof(cpx<T>);
+    if (lds > op_lds_limit()) return kym_ops_fail(KYM_ERR_UNSUPPORTED, "FFT length too large for LDS");
+    if (B * ncb > 0x7fffffffll) return kym_ops_fail(KYM_ERR_VALUE, "batch too large");
+    if (lds > 65536)
+        OPS_HIP_TRY(hipFuncSetAttribute((const void*)k_fft_axis0<T, MAXP>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                        (int)op_lds_limit()));
+    hipLaunchKernelGGL((k_fft_axis0<T, MAXP>), dim3((unsigned)(B * ncb)), dim3(256), lds, s, (const cpx<T>*)x, (cpx<T>*)y,
+                       S, cb, ncb, inv, reinterpret_cast<const FftLen<T>*>((char*)t.dev + t.lens_off), t.lH);
+    OPS_HIP_TRY(hipGetLastError());
+    return KYM_OK;
+}
+
+template <class T>
+static int fft_axis0(const void* x, void* y, long long B, int M, int S, int inv, hipStream_t s) {
+    switch (op_pclass(M)) {
+        case 7: return fft_axis0_p<T, 7>(x, y, B, M, S, inv, s);
+        case 17: return fft_axis0_p<T, 17>(x, y, B, M, S, inv, s);
+        default: return fft_axis0_p<T, 31>(x, y, B, M, S, inv, s);
+    }
+}
+
+extern "C" int kym_op_fft_axis0(const void* x, void* y, long long B, int M, long long S, int inverse, int dtype,
+                                void* stream) {
+    if (B <= 0 || S <= 0) return KYM_OK;
+    if (M < 1 || S > 0x7fffffffll) return kym_ops_fail(KYM_ERR_VALUE, "invalid length");
+    if (!x || !y) return kym_ops_fail(KYM_ERR_VALUE, "null device pointer");
+    hipStream_t s = (hipStream_t)stream;
+    if (dtype == KYM_F32) return fft_axis0<float>(x, y, B, M, (int)S, inverse != 0, s);
+    if (dtype == KYM_F64) return fft_axis0<double>(x, y, B, M, (int)S, inverse != 0, s);
     return bad_dtype();
 }
 

@@ -1,7 +1,7 @@
 """3D HIP backend namespace (op names and checks of
 kymatio/scattering3d/backend/torch_backend.py:59-151): the 3D FFTs are the 2D
-HIP transform over the last two axes followed by the 1D HIP transform over
-the first (after a transpose); products, moduli and integrals are HIP
+HIP transform over the last two axes followed by the HIP transform of the
+strided lines along the first; products, moduli and integrals are HIP
 kernels."""
 import ctypes
 
@@ -12,14 +12,12 @@ from ...backend.torch_backend import TorchBackend, _dt, _gpu, _ptr
 
 
 def _fft_axis0(x, kind):
-    """1D transform over M of (B, M, N, O, 2)."""
+    """1D transform over M of (B, M, N, O, 2), in place."""
     B, M, N, O, _ = x.shape
-    xt = x.reshape(B, M, N * O, 2).transpose(1, 2).contiguous()  # (B, N O, M, 2)
-    yt = torch.empty_like(xt)
     with torch.cuda.device(x.device):
-        _lib.check(_lib.lib().kym_op_fft(_ptr(xt), _ptr(yt), None, B * N * O, M, 1, kind, _dt(x), 0,
-                                          _lib.stream_of(x.device)))
-    return yt.transpose(1, 2).reshape(B, M, N, O, 2).contiguous()
+        _lib.check(_lib.lib().kym_op_fft_axis0(_ptr(x), _ptr(x), B, M, N * O, int(kind == 1), _dt(x),
+                                                _lib.stream_of(x.device)))
+    return x
 
 
 def _fft3(x, kind):

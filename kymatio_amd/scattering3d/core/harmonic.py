@@ -3,15 +3,15 @@
 The reference walks l, j1 (and j2 > j1) and, inside, every m of the order-l
 wavelets one op at a time: cdgmm3d, ifft, modulus_rotation per m, then one
 integral per path (kymatio/scattering3d/core/scattering3d.py:24-75).  Here
-each (l, j) step is three launches over all m and all images together:
+each step of one l is two launches over all j, m and images together:
 
-    products  (B, 2l+1, n) = U_hat (B, n) x psi_{l, j, m} (2l+1, n)   kym_op_harmonic_products
-    inverse   3D FFT of the B (2l+1) volumes                          backend.ifft
-    modulus   (B, n) = the chained rotation modulus over m            kym_op_modulus_rotation_sum
+    planes    products U_hat psi_{l, j, m} and their 2D inverse over (N, O)
+    lines     inverse along M, then the chained rotation modulus over m
 
-and the moduli of every (path, l) land in one field array of layout
-(paths, L + 1, B, n), so one kym_op_integrals launch computes every output
-and the result is that array's integrals moved to (B, paths, L + 1, P).
+(kym_op_harmonic_step, for every j of a parent at once) and the moduli of
+every (path, l) land in one field array of layout (paths, L + 1, B, n), so
+one kym_op_integrals launch computes every output and the result is that
+array's integrals moved to (B, paths, L + 1, P).
 Path order per l is the reference's: all first-order j1, then the pairs
 (j1, j2 > j1) in j1-major order; outputs interleave l inside each path
 (scattering3d.py:64-73).
@@ -52,6 +52,24 @@ class _Launcher:
                                                        self.stream))
         return out
 
+    def step(self, U_hat, F, nm, dest, vol, dstride):
+        """dest[g] (B, n), dstride elements apart = the moduli of scale g of F
+        (ng, 2l + 1, ...) over its first nm filters; False where the volume
+        does not fit the fused kernels.  Scales are taken together up to 256 MB
+        of planes between the two kernels (the MALL)."""
+        B, ng, n = U_hat.shape[0], F.shape[0], vol[0] * vol[1] * vol[2]
+        fs = F.stride(0) // 2
+        each = B * nm * n * 2
+        per = max(1, min(ng, (256 << 20) // max(each * U_hat.element_size(), 1)))
+        work = torch.empty(per * each, dtype=U_hat.dtype, device=self.device)
+        for g in range(0, ng, per):
+            rc = self.lib.kym_op_harmonic_step(_ptr(U_hat), _ptr(F[g]), _ptr(work), _ptr(dest[g]), B, min(per, ng - g),
+                                               nm, vol[0], vol[1], vol[2], fs, dstride, self.code, self.stream)
+            if rc == 5 and g == 0:
+                return False
+            _lib.check(rc)
+        return True
+
     def rotation_modulus(self, Y, dest):
         """Y: (B, nm, M, N, O, 2) -> dest (B, n) (a contiguous block of the field array)."""
         B, nm = Y.shape[0], Y.shape[1]
@@ -80,20 +98,27 @@ def harmonic_scattering(x, bank, J, L, max_order, rotation_covariant, powers, ba
     run = _Launcher(x.device, x.dtype)
     fields = torch.empty((len(paths), L + 1, B, n), dtype=x.dtype, device=x.device)
 
-    def modulus_of(U_hat, l, j, dest):
-        F = bank[l][j] if rotation_covariant else bank[l][j][:1]
-        run.rotation_modulus(backend.ifft(run.products(U_hat, F).reshape((-1,) + vol + (2,))).reshape(
-            (B, F.shape[0]) + vol + (2,)), dest)
+    nm_all = [bank[l].shape[1] for l in range(L + 1)]
+    rows = fields.shape[1] * B * n  # field elements between paths
+
+    def moduli(U_hat, l, j0, ng, path0):
+        """The moduli of scales j0 .. j0 + ng - 1 of order l into the fields of
+        paths path0, path0 + 1, ..."""
+        nm = nm_all[l] if rotation_covariant else 1
+        if run.step(U_hat, bank[l][j0:j0 + ng], nm, fields[path0:path0 + ng, l], vol, rows):
+            return
+        for g in range(ng):  # volumes whose planes do not fit a workgroup
+            F = bank[l][j0 + g][:nm]
+            run.rotation_modulus(backend.ifft(run.products(U_hat, F).reshape((-1,) + vol + (2,))).reshape(
+                (B, nm) + vol + (2,)), fields[path0 + g, l])
 
     U0_hat = backend.rfft(x)
     for l in range(L + 1):
-        for j1 in range(J + 1):
-            first = fields[slot[(j1,)], l]
-            modulus_of(U0_hat, l, j1, first)
-            if max_order > 1 and j1 < J:
-                U1_hat = backend.rfft(first.reshape((B,) + vol + (1,)))
-                for j2 in range(j1 + 1, J + 1):
-                    modulus_of(U1_hat, l, j2, fields[slot[(j1, j2)], l])
+        moduli(U0_hat, l, 0, J + 1, slot[(0,)])
+        if max_order > 1:
+            for j1 in range(J):
+                U1_hat = backend.rfft(fields[slot[(j1,)], l].reshape((B,) + vol + (1,)))
+                moduli(U1_hat, l, j1 + 1, J - j1, slot[(j1, j1 + 1)])
     S = run.integrals(fields.reshape(-1, n), powers).reshape(len(paths), L + 1, B, len(powers))
     return S.permute(2, 0, 1, 3).contiguous().to(torch.float32)
 

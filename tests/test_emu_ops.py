@@ -355,3 +355,38 @@ def test_freq_scatter_compiled(emu, T, c):
         ref = np.abs(np.fft.ifft((X * g.astype(np.float64)[None, :, None]).reshape(B, k, n, T).mean(axis=1), axis=1))
         got = y[:B * n * T].reshape(B, n, T)
         assert np.abs(got - ref).max() <= 2e-6 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize('M,N,O,ng,nm', [(8, 16, 4, 2, 3), (5, 6, 7, 1, 1), (32, 12, 20, 1, 5), (1, 9, 33, 2, 2),
+                                         (34, 3, 1, 1, 7)])
+@pytest.mark.parametrize('dtype', [np.float32, np.float64])
+def test_harmonic_step(emu, M, N, O, ng, nm, dtype):
+    """sqrt(sum_m |ifft3(U F_gm)|^2) against numpy in 64 bits, and the
+    transform along the first axis."""
+    rng = np.random.default_rng(M * N + O)
+    B = 2
+    c = np.complex64 if dtype == np.float32 else np.complex128
+    z = lambda *s: (rng.standard_normal(s) + 1j * rng.standard_normal(s)).astype(c)
+    U, F = z(B, M, N, O), z(ng, nm + 1, M, N, O)  # one filter more per group than is used
+    vol = M * N * O
+    work = np.zeros(B * ng * nm * vol, c)
+    dest = np.zeros((ng, 3, B, vol), dtype)  # groups three fields apart
+    f = emu.lib.kym_emu_op_harmonic_step
+    P, LL, I = ctypes.c_void_p, ctypes.c_longlong, ctypes.c_int
+    f.argtypes, f.restype = [P] * 4 + [LL] + [I] * 5 + [LL, LL, I], I
+    assert f(U.ctypes.data, F.ctypes.data, work.ctypes.data, dest.ctypes.data, B, ng, nm, M, N, O, (nm + 1) * vol,
+             3 * B * vol, 0 if dtype == np.float32 else 1) == 0
+    u = np.fft.ifftn(U[None, :, None].astype(np.complex128) * F[:, None, :nm], axes=(-3, -2, -1))
+    ref = np.sqrt((np.abs(u) ** 2).sum(2)).reshape(ng, B, vol)
+    # log2(vol) butterfly levels and nm squares
+    tol = 8 * (np.log2(vol) + nm) * np.finfo(dtype).eps
+    assert np.abs(dest[:, 0] - ref).max() <= tol * ref.max()
+    assert not dest[:, 1:].any()
+    x = U.astype(np.complex128)
+    g = emu.lib.kym_emu_op_fft_axis0
+    g.argtypes, g.restype = [P, P, LL, I, I, I], I
+    for inv in (0, 1):
+        y = x.copy()
+        assert g(y.ctypes.data, y.ctypes.data, B, M, N * O, inv) == 0
+        r = (np.fft.ifft if inv else np.fft.fft)(x, axis=1)
+        assert np.abs(y - r).max() <= 1e-14 * M * np.abs(x).max()

@@ -156,3 +156,25 @@ def test_numpy_and_sklearn_3d():
     t = Sk3D(J=int(d['J']), shape=x.shape[1:], L=int(d['L']),
              integral_powers=d['integral_powers']).transform(x.reshape(x.shape[0], -1))
     assert np.allclose(t, Sx.reshape(x.shape[0], -1))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('shape,B', [((32, 32, 32), 3), ((8, 64, 20), 2), ((20, 12, 9), 1), ((6, 160, 150), 1),
+                                     ((17, 22, 26), 2), ((1, 8, 8), 1)])
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float64])
+def test_moduli_match_64_bits(shape, B, dtype):
+    """First- and second-order integrals against torch.fft in 64 bits, for
+    planes within a workgroup and ((160, 150)) beyond one."""
+    J, L = 1, 2
+    S = HarmonicScattering3D(J=J, shape=shape, L=L, integral_powers=(1., 2.)).to(dtype).to(DEV)
+    x = torch.rand((B,) + shape, device=DEV, dtype=dtype, generator=torch.Generator(DEV).manual_seed(B))
+    out = S(x).double().cpu()
+    dim = (-3, -2, -1)
+    bank = [torch.view_as_complex(f.double().cpu()) for f in S.filters]
+    mod = lambda U, l, j: torch.fft.ifftn(U[:, None] * bank[l][j][None], dim=dim).abs().square().sum(1).sqrt()
+    U0 = torch.fft.fftn(x.double().cpu(), dim=dim)
+    for l in range(L + 1):
+        u = [mod(U0, l, j) for j in range(J + 1)]
+        u.append(mod(torch.fft.fftn(u[0], dim=dim), l, 1))
+        ref = torch.stack([torch.stack([v.sum(dim), v.square().sum(dim)], -1) for v in u], 1)
+        assert ((out[:, :, l] - ref).abs() <= 2e-6 * ref.abs() + 1e-9 * ref.abs().max()).all()
