@@ -257,16 +257,19 @@ KYM_HD KYM_INL void dit_first_pass_real_s(cpx<T>* buf, int tid, LOAD load) {
 // pass touch different banks (two lanes share one at worst).
 KYM_HD KYM_INL constexpr int pad16(int i) { return i + (i >> 4); }
 
-template <int R, bool INV, bool DIT, int N, int LS, int OFF, int NT, class T>
-KYM_HD KYM_INL void pad_pass(cpx<T>* buf, const cpx<T>* ptw, int tid) {
+// NTR lines lie pad16(N) apart.
+template <int R, bool INV, bool DIT, int N, int LS, int OFF, int NT, class T, int NTR = 1>
+KYM_HD KYM_INL void pad_pass(cpx<T>* buf0, const cpx<T>* ptw, int tid) {
     constexpr int L = LS * R;
     // element m of a butterfly lies m ST further on where LS keeps the padding
     // linear, else its place is computed
     constexpr bool LIN = LS % 16 == 0 || (LS == 1 && 16 % R == 0);
     constexpr int ST = LS % 16 == 0 ? LS + LS / 16 : 1;
     KYM_UNROLL_DEV
-    for (int f = tid; f < N / R; f += NT) {
-        const int b = f / LS, j = f - b * LS, i0 = b * L + j;
+    for (int f = tid; f < NTR * (N / R); f += NT) {
+        const int t = f / (N / R), u = f - t * (N / R);
+        cpx<T>* buf = buf0 + t * pad16(N);
+        const int b = u / LS, j = u - b * LS, i0 = b * L + j;
         cpx<T>* p = LIN ? buf + pad16(i0) : buf;
         cpx<T> v[R], w[R];
         if constexpr (LS > 1) {
@@ -290,25 +293,25 @@ KYM_HD KYM_INL void pad_pass(cpx<T>* buf, const cpx<T>* ptw, int tid) {
     wg_barrier();
 }
 
-template <bool INV, int N, int NT, class T, int Q = 0, int LP = 1>
+template <bool INV, int N, int NT, class T, int NTR = 1, int Q = 0, int LP = 1>
 KYM_HD KYM_INL void pad_dit(cpx<T>* buf, const cpx<T>* ptw, int tid) {
     constexpr RadList rl = kym_factor_list(N);
     static_assert(rl.ok && (N & (N - 1)) == 0, "power-of-two lengths");
     if constexpr (Q < rl.nrad) {
         constexpr int R = rl.rad[Q];
-        pad_pass<R, INV, true, N, LP, kym_ptw_off(rl, Q), NT, T>(buf, ptw, tid);
-        pad_dit<INV, N, NT, T, Q + 1, LP * R>(buf, ptw, tid);
+        pad_pass<R, INV, true, N, LP, kym_ptw_off(rl, Q), NT, T, NTR>(buf, ptw, tid);
+        pad_dit<INV, N, NT, T, NTR, Q + 1, LP * R>(buf, ptw, tid);
     }
 }
 
-template <bool INV, int N, int NT, class T, int Q = -1, int L = N>
+template <bool INV, int N, int NT, class T, int NTR = 1, int Q = -1, int L = N>
 KYM_HD KYM_INL void pad_dif(cpx<T>* buf, const cpx<T>* ptw, int tid) {
     constexpr RadList rl = kym_factor_list(N);
     static_assert(rl.ok && (N & (N - 1)) == 0, "power-of-two lengths");
     constexpr int q = Q < 0 ? rl.nrad - 1 : Q;
     if constexpr (L > 1) {
         constexpr int R = rl.rad[q];
-        pad_pass<R, INV, false, N, L / R, kym_ptw_off(rl, q), NT, T>(buf, ptw, tid);
-        if constexpr (q > 0) pad_dif<INV, N, NT, T, q - 1, L / R>(buf, ptw, tid);
+        pad_pass<R, INV, false, N, L / R, kym_ptw_off(rl, q), NT, T, NTR>(buf, ptw, tid);
+        if constexpr (q > 0) pad_dif<INV, N, NT, T, NTR, q - 1, L / R>(buf, ptw, tid);
     }
 }

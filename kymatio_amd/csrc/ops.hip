@@ -511,7 +511,7 @@ static int freq_scatter_op(const void* x, void* const* ys, const void* const* fs
         o.k[i] = ks[i];
         mp = std::max(mp, kym_max_odd_prime(N / ks[i]));
     }
-    const size_t lds = (size_t)2 * o.m * N * sizeof(cpx<T>);
+    const size_t lds = (size_t)2 * o.m * line_stride(N, o.m) * sizeof(cpx<T>);
     if (lds > op_lds_limit()) return kym_ops_fail(KYM_ERR_UNSUPPORTED, "transform length too large for LDS");
     const long long nblk = B * o.nt_blk;
     if (nblk > 0x7fffffffll) return kym_ops_fail(KYM_ERR_VALUE, "batch too large");

@@ -330,6 +330,11 @@ inline int filter_ifft_spec_id(int n, long long batch, const FilterIfftArgs& o, 
     return -1;
 }
 
+// LDS row stride of m lines of n points that are filled and read across lines
+// (lane t to line t): odd, so the lines start on different banks.  At 88
+// points 32 lanes met 4 banks.
+KYM_HD KYM_INL constexpr int line_stride(int n, int m) { return m > 1 ? n | 1 : n; }
+
 // Frequency scattering of one (b, t-block) in one workgroup: the rows x[b][a][t]
 // (a < A along the log-frequency axis, t < T; real (c = 1) or complex
 // (c = 2)), zero-padded to N along a, are transformed along a; then for every
@@ -358,28 +363,33 @@ KYM_HD void freq_scatter_body(const FreqScatterArgs& o, long long blk, cpx<T>* l
     const int t0 = (int)(blk - b * o.nt_blk) * m;
     const int mm = (TT - t0 < m) ? TT - t0 : m;
     cpx<T>* X = lds;
-    cpx<T>* P = lds + (long long)m * N;
+    const int sN = line_stride(N, m);
+    const FInt dm = fast_int(m), dmm = fast_int(mm);
+    cpx<T>* P = lds + m * sN;
     // rows t of the block along a, each value at its digit-reversed slot
     for (int i = tid; i < m * N; i += nth) {
-        const int a = i / m, t = i - a * m;
+        const int a = i / dm, t = i - a * m;
         cpx<T> v = {T(0), T(0)};
         if (a < A && t < mm) {
             const long long src = (b * A + a) * (long long)TT + t0 + t;
             if (o.c == 2) v = kym_ldg(static_cast<const cpx<T>*>(o.x) + src);
             else v = {kym_ldg(static_cast<const T*>(o.x) + src), T(0)};
         }
-        X[t * N + kym_ldg(fN.irev + a)] = v;
+        X[t * sN + kym_ldg(fN.irev + a)] = v;
     }
     wg_barrier();
-    fft_dit<false, MAXP>(X, fN, Batch{m, 1, N, false}, tid, nth);
+    fft_dit<false, MAXP>(X, fN, Batch{m, 1, sN, false}, tid, nth);
     wg_barrier();
     for (int w = 0; w < o.nf; ++w) {
-        const int k = o.k[w], n = N / k;
+        const FftLen<T>& fl = *static_cast<const FftLen<T>*>(o.lenn[w]);
+        const int k = o.k[w];
+        const FInt n = fl.size();
+        const int sn = line_stride(n, m);
         const T* f = static_cast<const T*>(o.f[w]);
         const T inv_k = T(1) / T(k);
         for (int q = tid; q < m * n; q += nth) {
             const int t = q / n, p = q - t * n;
-            const cpx<T>* xr = X + t * N + p;
+            const cpx<T>* xr = X + t * sN + p;
             cpx<T> acc = {T(0), T(0)};
             for (int a = 0; a < k; ++a) {
                 const T fv = kym_ldg(f + p + a * n);
@@ -387,17 +397,16 @@ KYM_HD void freq_scatter_body(const FreqScatterArgs& o, long long blk, cpx<T>* l
                 acc.re += v.re * fv;
                 acc.im += v.im * fv;
             }
-            P[q] = acc * inv_k;
+            P[t * sn + p] = acc * inv_k;
         }
         wg_barrier();
-        const FftLen<T>& fl = *static_cast<const FftLen<T>*>(o.lenn[w]);
-        fft_dif<true, MAXP>(P, fl, Batch{m, 1, n, false}, tid, nth);
+        fft_dif<true, MAXP>(P, fl, Batch{m, 1, sn, false}, tid, nth);
         wg_barrier();
         const T inv_n = T(1) / T(n);
         T* y = static_cast<T*>(o.y[w]);
         for (int q = tid; q < mm * n; q += nth) {
-            const int p = q / mm, t = q - p * mm;
-            const cpx<T> v = P[t * n + kym_ldg(fl.irev + p)];
+            const int p = q / dmm, t = q - p * mm;
+            const cpx<T> v = P[t * sn + kym_ldg(fl.irev + p)];
             y[(b * n + p) * (long long)TT + t0 + t] = kym_sqrt(v.re * v.re + v.im * v.im) * inv_n;
         }
         wg_barrier();
@@ -407,6 +416,7 @@ KYM_HD void freq_scatter_body(const FreqScatterArgs& o, long long blk, cpx<T>* l
 // freq_scatter_body with N and the t-values per workgroup M fixed at compile
 // time (static passes) and the output lengths N / k among 88, 44 and 22 as
 // compiled (freq_scatter_spec_ok).  Same arithmetic.
+template <int K> struct ConstK { static constexpr int value = K; };
 template <class T, int N, int M, int NT>
 KYM_HD void freq_scatter_body_s(const FreqScatterArgs& o, long long blk, cpx<T>* lds, int tid) {
     const FftLen<T>& fN = *static_cast<const FftLen<T>*>(o.lenN);
@@ -415,7 +425,8 @@ KYM_HD void freq_scatter_body_s(const FreqScatterArgs& o, long long blk, cpx<T>*
     const int t0 = (int)(blk - b * o.nt_blk) * M;
     const int mm = (TT - t0 < M) ? TT - t0 : M;
     cpx<T>* X = lds;
-    cpx<T>* P = lds + M * N;
+    constexpr int sN = line_stride(N, M);
+    cpx<T>* P = lds + M * sN;
     for (int i = tid; i < M * N; i += NT) {
         const int a = i / M, t = i - a * M;
         cpx<T> v = {T(0), T(0)};
@@ -424,41 +435,45 @@ KYM_HD void freq_scatter_body_s(const FreqScatterArgs& o, long long blk, cpx<T>*
             if (o.c == 2) v = kym_ldg(static_cast<const cpx<T>*>(o.x) + src);
             else v = {kym_ldg(static_cast<const T*>(o.x) + src), T(0)};
         }
-        X[t * N + kym_ldg(fN.irev + a)] = v;
+        X[t * sN + kym_ldg(fN.irev + a)] = v;
     }
     wg_barrier();
-    fft_dit_s<false, N, M, 1, N, false, NT>(X, fN.ptw, tid);
-    for (int w = 0; w < o.nf; ++w) {
-        const int k = o.k[w], n = N / k;
+    fft_dit_s<false, N, M, 1, sN, false, NT>(X, fN.ptw, tid);
+    // one wavelet with its output length fixed: n = N / k
+    auto wavelet = [&](int w, auto kc) {
+        constexpr int K = decltype(kc)::value, n = N / K, sn = line_stride(n, M);
         const T* f = static_cast<const T*>(o.f[w]);
-        const T inv_k = T(1) / T(k);
+        const T inv_k = T(1) / T(K);
         for (int q = tid; q < M * n; q += NT) {
             const int t = q / n, p = q - t * n;
-            const cpx<T>* xr = X + t * N + p;
+            const cpx<T>* xr = X + t * sN + p;
             cpx<T> acc = {T(0), T(0)};
-            for (int a = 0; a < k; ++a) {
+#pragma unroll
+            for (int a = 0; a < K; ++a) {
                 const T fv = kym_ldg(f + p + a * n);
                 const cpx<T> v = xr[a * n];
                 acc.re += v.re * fv;
                 acc.im += v.im * fv;
             }
-            P[q] = acc * inv_k;
+            P[t * sn + p] = acc * inv_k;
         }
         wg_barrier();
         const FftLen<T>& fl = *static_cast<const FftLen<T>*>(o.lenn[w]);
-        if constexpr (N == 88) {
-            if (n == 88) fft_dif_s<true, 88, M, 1, 88, false, NT>(P, fl.ptw, tid);
-            else if (n == 44) fft_dif_s<true, 44, M, 1, 44, false, NT>(P, fl.ptw, tid);
-            else fft_dif_s<true, 22, M, 1, 22, false, NT>(P, fl.ptw, tid);
-        }
+        fft_dif_s<true, n, M, 1, sn, false, NT>(P, fl.ptw, tid);
         const T inv_n = T(1) / T(n);
-        T* y = static_cast<T*>(o.y[w]);
-        for (int q = tid; q < mm * n; q += NT) {
-            const int p = q / mm, t = q - p * mm;
-            const cpx<T> v = P[t * n + kym_ldg(fl.irev + p)];
-            y[(b * n + p) * (long long)TT + t0 + t] = kym_sqrt(v.re * v.re + v.im * v.im) * inv_n;
+        T* y = static_cast<T*>(o.y[w]) + b * n * (long long)TT + t0;
+        for (int q = tid; q < M * n; q += NT) {
+            const int p = q / M, t = q - p * M;
+            if (t >= mm) continue;
+            const cpx<T> v = P[t * sn + kym_ldg(fl.irev + p)];
+            y[p * (long long)TT + t] = kym_sqrt(v.re * v.re + v.im * v.im) * inv_n;
         }
         wg_barrier();
+    };
+    for (int w = 0; w < o.nf; ++w) {
+        if (o.k[w] == 1) wavelet(w, ConstK<1>());
+        else if (o.k[w] == 2) wavelet(w, ConstK<2>());
+        else wavelet(w, ConstK<4>());
     }
 }
 
@@ -522,7 +537,9 @@ struct LowpassArgs {
 template <class T, int MAXP = 31>
 KYM_HD void lowpass_body(const LowpassArgs& o, const FftLen<T>& fN, const FftLen<T>& fn, long long blk, cpx<T>* lds,
                          int tid, int nth) {
-    const int N = o.N, n = o.n, k = o.k, S = o.S;
+    const FInt N = fN.size(), n = fn.size();
+    const int k = o.k, S = o.S;
+    const int sN = line_stride(N, o.nrow), sn = line_stride(n, o.nrow);
     long long ob;
     int s0, m;
     if (S == 1) {
@@ -534,6 +551,7 @@ KYM_HD void lowpass_body(const LowpassArgs& o, const FftLen<T>& fN, const FftLen
         s0 = (int)(blk - ob * o.nsb) * o.nrow;
         m = (S - s0 < o.nrow) ? S - s0 : o.nrow;
     }
+    const FInt dm = fast_int(m);
     const T* x = static_cast<const T*>(o.x);
     const T* f = static_cast<const T*>(o.f);
     T* y = static_cast<T*>(o.y);
@@ -545,22 +563,22 @@ KYM_HD void lowpass_body(const LowpassArgs& o, const FftLen<T>& fN, const FftLen
         if (S == 1) {
             t = i / N;
             e = i - t * N;
-            src = (ob + t) * N + e;
+            src = (ob + t) * (int)N + e;
         } else {
-            e = i / m;
+            e = i / dm;
             t = i - e * m;
-            src = (ob * N + e) * S + s0 + t;
+            src = (ob * (int)N + e) * S + s0 + t;
         }
-        lds[t * N + fN.irev[e]] = {kym_ldg(x + src), T(0)};
+        lds[t * sN + kym_ldg(fN.irev + e)] = {kym_ldg(x + src), T(0)};
     }
     wg_barrier();
-    fft_dit<false, MAXP>(lds, fN, Batch{m, 1, N, false}, tid, nth);
+    fft_dit<false, MAXP>(lds, fN, Batch{m, 1, sN, false}, tid, nth);
     wg_barrier();
-    cpx<T>* P = lds + (long long)o.nrow * N;
+    cpx<T>* P = lds + o.nrow * sN;
     const T inv_k = T(1) / T(k);
     for (int q = tid; q < m * n; q += nth) {
         const int t = q / n, p = q - t * n;
-        const cpx<T>* X = lds + t * N + p;
+        const cpx<T>* X = lds + t * sN + p;
         cpx<T> acc = {T(0), T(0)};
         int a = 0;
         for (; a + 7 < k; a += 8) {  // the filter loads of a round issued together
@@ -580,10 +598,10 @@ KYM_HD void lowpass_body(const LowpassArgs& o, const FftLen<T>& fN, const FftLen
             acc.re += v.re * w;
             acc.im += v.im * w;
         }
-        P[q] = acc * inv_k;
+        P[t * sn + p] = acc * inv_k;
     }
     wg_barrier();
-    fft_dif<true, MAXP>(P, fn, Batch{m, 1, n, false}, tid, nth);
+    fft_dif<true, MAXP>(P, fn, Batch{m, 1, sn, false}, tid, nth);
     wg_barrier();
     const T inv_n = T(1) / T(n);
     for (int q = tid; q < m * n; q += nth) {
@@ -592,13 +610,13 @@ KYM_HD void lowpass_body(const LowpassArgs& o, const FftLen<T>& fN, const FftLen
         if (S == 1) {
             t = q / n;
             p = q - t * n;
-            dst = (ob + t) * n + p;
+            dst = (ob + t) * (int)n + p;
         } else {
-            p = q / m;
+            p = q / dm;
             t = q - p * m;
-            dst = (ob * n + p) * S + s0 + t;
+            dst = (ob * (int)n + p) * S + s0 + t;
         }
-        y[dst] = P[t * n + fn.irev[p]].re * inv_n;
+        y[dst] = P[t * sn + kym_ldg(fn.irev + p)].re * inv_n;
     }
 }
 
@@ -612,7 +630,7 @@ KYM_HD void lowpass_body(const LowpassArgs& o, const FftLen<T>& fN, const FftLen
 template <class T, int N, int NN, int NT>
 KYM_HD void lowpass_body_s(const LowpassArgs& o, const FftLen<T>& fN, const FftLen<T>& fn, long long blk,
                            cpx<T>* lds, int tid) {
-    constexpr int M = 8192 / N, M2 = M / 2, K = N / NN;
+    constexpr int M = 8192 / N, M2 = M / 2, K = N / NN, sN = pad16(N), sn = pad16(NN);
     const long long ob = blk * M;
     const int m = (int)((o.outer - ob < M) ? o.outer - ob : M);
     const T* x = static_cast<const T*>(o.x);
@@ -622,36 +640,36 @@ KYM_HD void lowpass_body_s(const LowpassArgs& o, const FftLen<T>& fN, const FftL
         const int u = i / N, e = i - u * N;
         const T va = u < m ? kym_ldg(x + (ob + u) * N + e) : T(0);
         const T vb = u + M2 < m ? kym_ldg(x + (ob + u + M2) * N + e) : T(0);
-        lds[u * N + kym_ldg(fN.irev + e)] = {va, vb};
+        lds[u * sN + pad16(kym_ldg(fN.irev + e))] = {va, vb};
     }
     wg_barrier();
-    fft_dit_s<false, N, M2, 1, N, false, NT>(lds, fN.ptw, tid);
-    cpx<T>* P = lds + M2 * N;
+    pad_dit<false, N, NT, T, M2>(lds, fN.ptw, tid);
+    cpx<T>* P = lds + M2 * sN;
     const T inv_2k = T(1) / T(2 * K);
     for (int q = tid; q < M * NN; q += NT) {
         const int t = q / NN, p = q - t * NN;
         const bool second = t >= M2;
-        const cpx<T>* Z = lds + (second ? t - M2 : t) * N;
+        const cpx<T>* Z = lds + (second ? t - M2 : t) * sN;
         cpx<T> acc = {T(0), T(0)};
 #pragma unroll 8
         for (int a = 0; a < K; ++a) {
             const int i = p + a * NN;
             const T w = kym_ldg(f + i);
-            const cpx<T> z = Z[i], zm = Z[i == 0 ? 0 : N - i];
+            const cpx<T> z = Z[pad16(i)], zm = Z[pad16(i == 0 ? 0 : N - i)];
             // 2 A = (z.re + zm.re, z.im - zm.im); 2 B = (z.im + zm.im, zm.re - z.re)
             const T re = second ? z.im + zm.im : z.re + zm.re;
             const T im = second ? zm.re - z.re : z.im - zm.im;
             acc.re += re * w;
             acc.im += im * w;
         }
-        P[q] = acc * inv_2k;
+        P[t * sn + pad16(p)] = acc * inv_2k;
     }
     wg_barrier();
-    fft_dif_s<true, NN, M, 1, NN, false, NT>(P, fn.ptw, tid);
+    pad_dif<true, NN, NT, T, M>(P, fn.ptw, tid);
     const T inv_n = T(1) / T(NN);
     for (int q = tid; q < m * NN; q += NT) {
         const int t = q / NN, p = q - t * NN;
-        y[(ob + t) * NN + p] = P[t * NN + kym_ldg(fn.irev + p)].re * inv_n;
+        y[(ob + t) * NN + p] = P[t * sn + pad16(kym_ldg(fn.irev + p))].re * inv_n;
     }
 }
 
@@ -661,7 +679,7 @@ KYM_HD void lowpass_body_s(const LowpassArgs& o, const FftLen<T>& fN, const FftL
 template <class T, int N, int NN, int M, int NT>
 KYM_HD void lowpass_body_sv(const LowpassArgs& o, const FftLen<T>& fN, const FftLen<T>& fn, long long blk,
                             cpx<T>* lds, int tid) {
-    constexpr int K = N / NN;
+    constexpr int K = N / NN, sN = line_stride(N, M), sn = line_stride(NN, M);
     const int S = o.S, nsb = S / M;
     const long long ob = blk / nsb;
     const int s0 = (int)(blk - ob * nsb) * M;
@@ -670,15 +688,15 @@ KYM_HD void lowpass_body_sv(const LowpassArgs& o, const FftLen<T>& fN, const Fft
     T* y = static_cast<T*>(o.y);
     for (int i = tid; i < M * N; i += NT) {
         const int e = i / M, t = i - e * M;
-        lds[t * N + kym_ldg(fN.irev + e)] = {kym_ldg(x + (ob * N + e) * S + s0 + t), T(0)};
+        lds[t * sN + kym_ldg(fN.irev + e)] = {kym_ldg(x + (ob * N + e) * S + s0 + t), T(0)};
     }
     wg_barrier();
-    fft_dit_s<false, N, M, 1, N, false, NT>(lds, fN.ptw, tid);
-    cpx<T>* P = lds + M * N;
+    fft_dit_s<false, N, M, 1, sN, false, NT>(lds, fN.ptw, tid);
+    cpx<T>* P = lds + M * sN;
     const T inv_k = T(1) / T(K);
     for (int q = tid; q < M * NN; q += NT) {
         const int t = q / NN, p = q - t * NN;
-        const cpx<T>* X = lds + t * N + p;
+        const cpx<T>* X = lds + t * sN + p;
         cpx<T> acc = {T(0), T(0)};
 #pragma unroll
         for (int a = 0; a < K; ++a) {
@@ -687,14 +705,14 @@ KYM_HD void lowpass_body_sv(const LowpassArgs& o, const FftLen<T>& fN, const Fft
             acc.re += v.re * w;
             acc.im += v.im * w;
         }
-        P[q] = acc * inv_k;
+        P[t * sn + p] = acc * inv_k;
     }
     wg_barrier();
-    fft_dif_s<true, NN, M, 1, NN, false, NT>(P, fn.ptw, tid);
+    fft_dif_s<true, NN, M, 1, sn, false, NT>(P, fn.ptw, tid);
     const T inv_n = T(1) / T(NN);
     for (int q = tid; q < M * NN; q += NT) {
         const int p = q / M, t = q - p * M;
-        y[(ob * NN + p) * S + s0 + t] = P[t * NN + kym_ldg(fn.irev + p)].re * inv_n;
+        y[(ob * NN + p) * S + s0 + t] = P[t * sn + kym_ldg(fn.irev + p)].re * inv_n;
     }
 }
 
@@ -726,7 +744,8 @@ inline int lowpass_spec_id(int N, int n, int S, int* rows) {
 // Complex elements of LDS of a compile-time low-pass: two lines per
 // transform for contiguous lines (S = 1), one per line along a stride.
 inline long long lowpass_spec_lds(int N, int n, int S, int M) {
-    return S == 1 ? (long long)(M / 2) * N + (long long)M * n : (long long)M * (N + n);
+    return S == 1 ? (long long)(M / 2) * pad16(N) + (long long)M * pad16(n)
+                  : (long long)M * (line_stride(N, M) + line_stride(n, M));
 }
 
 template <class T, int SPEC, bool EMU>
@@ -763,7 +782,7 @@ inline long long lowpass_shape(int N, int n, int S, long long outer, int* rows, 
         *nblk = (outer + m - 1) / m;
     }
     *rows = (int)m;
-    return m * (N + n);
+    return m * (line_stride(N, (int)m) + line_stride(n, (int)m));
 }
 
 // Pass kernels for transforms that do not fit: axis 1 = rows (along W),
