@@ -220,9 +220,9 @@ __global__ void __launch_bounds__(256) k_freq_scatter(FreqScatterArgs o) {
 }
 
 template <class T>
-__global__ void __launch_bounds__(256) k_freq_scatter_s88(FreqScatterArgs o) {
+__global__ void __launch_bounds__(KYM_FS_THREADS) k_freq_scatter_s88(FreqScatterArgs o) {
     extern __shared__ __attribute__((aligned(16))) char kym_smem_fss[];
-    freq_scatter_body_s<T, 88, 32, 256>(o, blockIdx.x, reinterpret_cast<cpx<T>*>(kym_smem_fss), threadIdx.x);
+    freq_scatter_body_s<T, 88, 32, KYM_FS_THREADS>(o, blockIdx.x, reinterpret_cast<cpx<T>*>(kym_smem_fss), threadIdx.x);
 }
 
 template <class T, int NN, int M>
@@ -232,7 +232,7 @@ __global__ void __launch_bounds__(256) k_filter_ifft_s(FilterIfftArgs o, const F
 }
 
 template <class T, int SPEC>
-__global__ void __launch_bounds__(256) k_lowpass_s(LowpassArgs o, const FftLen<T>* lens, int lN, int ln) {
+__global__ void __launch_bounds__(KYM_LP_THREADS) k_lowpass_s(LowpassArgs o, const FftLen<T>* lens, int lN, int ln) {
     extern __shared__ __attribute__((aligned(16))) char kym_smem_lps[];
     lowpass_spec_body<T, SPEC, false>(o, lens[lN], lens[ln], blockIdx.x, reinterpret_cast<cpx<T>*>(kym_smem_lps),
                                       threadIdx.x);
@@ -475,7 +475,7 @@ static int lowpass_op(const void* x, const void* f, void* y, long long outer, in
         if (nblk > 0x7fffffffll) return kym_ops_fail(KYM_ERR_VALUE, "batch too large");
         LowpassArgs o = {x, f, y, outer, N, S, k, n, M, S == 1 ? 1 : S / M};
         void* args[] = {&o, (void*)&lens, &t.lH, &t.lW};
-        OPS_HIP_TRY(hipLaunchKernel(kern, dim3((unsigned)nblk), dim3(256), args, lds, s));
+        OPS_HIP_TRY(hipLaunchKernel(kern, dim3((unsigned)nblk), dim3(KYM_LP_THREADS), args, lds, s));
         return KYM_OK;
     }
     switch (op_pclass(N, N / k)) {
@@ -518,10 +518,11 @@ static int freq_scatter_op(const void* x, void* const* ys, const void* const* fs
     const void* kern = kym_prime_class(mp) == 7    ? (const void*)k_freq_scatter<T, 7>
                        : kym_prime_class(mp) == 17 ? (const void*)k_freq_scatter<T, 17>
                                                    : (const void*)k_freq_scatter<T, 31>;
-    if (sizeof(T) == 4 && freq_scatter_spec_ok(o)) kern = (const void*)k_freq_scatter_s88<T>;
+    const bool spec = sizeof(T) == 4 && freq_scatter_spec_ok(o);
+    if (spec) kern = (const void*)k_freq_scatter_s88<T>;
     if (lds > 65536) OPS_HIP_TRY(hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     void* args[] = {&o};
-    OPS_HIP_TRY(hipLaunchKernel(kern, dim3((unsigned)nblk), dim3(256), args, lds, s));
+    OPS_HIP_TRY(hipLaunchKernel(kern, dim3((unsigned)nblk), dim3(spec ? KYM_FS_THREADS : 256), args, lds, s));
     return KYM_OK;
 }
 

@@ -335,6 +335,12 @@ inline int filter_ifft_spec_id(int n, long long batch, const FilterIfftArgs& o, 
 // points 32 lanes met 4 banks.
 KYM_HD KYM_INL constexpr int line_stride(int n, int m) { return m > 1 ? n | 1 : n; }
 
+// Threads of the compile-time frequency scatter and low-passes.
+#ifndef KYM_FS_THREADS
+#define KYM_FS_THREADS 512
+#define KYM_LP_THREADS 512
+#endif
+
 // Frequency scattering of one (b, t-block) in one workgroup: the rows x[b][a][t]
 // (a < A along the log-frequency axis, t < T; real (c = 1) or complex
 // (c = 2)), zero-padded to N along a, are transformed along a; then for every
@@ -753,8 +759,8 @@ KYM_HD KYM_INL void lowpass_spec_body(const LowpassArgs& o, const FftLen<T>& fN,
                                       cpx<T>* lds, int tid) {
 #define KYM_LP_BODY(id, nn, n2, mm, sv)                                                          \
     if constexpr (SPEC == id) {                                                                  \
-        if constexpr (sv) lowpass_body_sv<T, nn, n2, mm, (EMU ? 1 : 256)>(o, fN, fn, blk, lds, tid); \
-        else lowpass_body_s<T, nn, n2, (EMU ? 1 : 256)>(o, fN, fn, blk, lds, tid);               \
+        if constexpr (sv) lowpass_body_sv<T, nn, n2, mm, (EMU ? 1 : KYM_LP_THREADS)>(o, fN, fn, blk, lds, tid); \
+        else lowpass_body_s<T, nn, n2, (EMU ? 1 : KYM_LP_THREADS)>(o, fN, fn, blk, lds, tid);               \
     }
     KYM_LOWPASS_SPECS(KYM_LP_BODY)
 #undef KYM_LP_BODY
