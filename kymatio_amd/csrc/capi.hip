@@ -295,7 +295,7 @@ static int launch_call(const Scat2DPlan<T>& p, const Launch2D& l, int mode, cons
     if (ntask > (1ll << 30)) return fail(KYM_ERR_VALUE, "too many tasks in one launch");
     a.ntask = (int)ntask;
     c->grid = (unsigned)((ntask + 7) / 8 * 8);
-    const bool many = l.many_threads && ntask > KYM_MANY_TASKS;
+    const bool many = l.many_threads && ntask > l.many_tasks;
     const int threads = many ? l.many_threads : l.threads;
     c->threads = (unsigned)threads;
     c->lds = l.lds_bytes;

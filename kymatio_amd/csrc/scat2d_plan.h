@@ -20,8 +20,8 @@ struct Launch2D {
     int spec;               // compile-time specialisation id, -1 = run-time sizes
     int pair = 0;           // 1: a task is a sibling pair (group lists 2 ngroup node ids)
     // small LDS nodes: threads (and specialisation) of a launch of more than
-    // KYM_MANY_TASKS workgroups, 0 = the same
-    int many_threads = 0, many_spec = -1;
+    // many_tasks workgroups, 0 = the same
+    int many_threads = 0, many_spec = -1, many_tasks = 0;
 };
 
 // Workgroups from which a launch of small nodes uses one wave per node.  Up to
@@ -33,6 +33,12 @@ struct Launch2D {
 #define KYM_MANY_TASKS 2048
 // Points up to which one wave per node is used.
 #define KYM_WAVE_NODE 640
+// Run-time-sized nodes of 2048 to 4095 points: 512 threads up to two
+// workgroups a CU (what their 105 registers allow at once), 256 beyond, where
+// four independent workgroups wait less for each other's barriers than two of
+// twice the threads (48 images of 224 x 224 J=3: 1103 -> 1053 us; 6 of 150 x
+// 203 J=4, 400 nodes a launch: 221 us against 224).
+#define KYM_MANY_MEDIUM 512
 
 // Tuning choices of a plan (0 = the built-in heuristic).  Any non-default
 // choice turns the compile-time specialisations off for what it affects.
@@ -368,14 +374,21 @@ struct Scat2DPlan {
         launches.clear();
         max_lds = 0;
         max_threads = 256;
-        // one wave per node where the launch's nodes are small and many
+        // fewer threads per node where the launch's nodes are small and many
         auto many_waves = [&](Launch2D& l) {
             const size_t elems = (size_t)H[l.res] * W[l.res];
-            if (tune.node_threads || elems > KYM_WAVE_NODE || l.pair) return;
+            if (tune.node_threads || l.pair) return;
+            if (l.spec < 0 && elems >= 2048 && elems < 4096) {
+                l.many_threads = 256;
+                l.many_tasks = KYM_MANY_MEDIUM;
+                return;
+            }
+            if (elems > KYM_WAVE_NODE) return;
             int nt = 0;
             const int sid = l.spec >= 0 ? node_spec_id(H[l.res], W[l.res], H[J], W[J], 64, &nt, 0) : -1;
             if (l.spec >= 0 && sid < 0) return;
             l.many_threads = 64;
+            l.many_tasks = KYM_MANY_TASKS;
             l.many_spec = sid;
         };
         auto add_group = [&](const std::vector<int>& ids) {
