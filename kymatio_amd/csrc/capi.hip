@@ -147,7 +147,7 @@ static int upload_and_prepare(Scat2DPlan<T>& p, void** dblob) {
     KYM_HIP_TRY(hipMemcpy(*dblob, p.blob.bytes.data(), bytes, hipMemcpyHostToDevice));
     for (const std::vector<Launch2D>* ls : {&p.launches, &p.bwd_launches})
         for (const Launch2D& l : *ls) {
-            Scat2DKernel<T> k = pick_scat2d<T>(l.kind, l.threads, p.pclass, l.spec);
+            Scat2DKernel<T> k = pick_scat2d<T>(l.kind, l.threads, l.pclass, l.spec);
             if (!k) return fail(KYM_ERR_UNSUPPORTED, "no kernel for launch kind");
             if (l.lds_bytes > 65536)
                 KYM_HIP_TRY(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -299,7 +299,7 @@ static int launch_call(const Scat2DPlan<T>& p, const Launch2D& l, int mode, cons
     const int threads = many ? l.many_threads : l.threads;
     c->threads = (unsigned)threads;
     c->lds = l.lds_bytes;
-    c->k = pick_scat2d<T>(l.kind, threads, p.pclass, many ? l.many_spec : l.spec);
+    c->k = pick_scat2d<T>(l.kind, threads, l.pclass, many ? l.many_spec : l.spec);
     if (!c->k) return fail(KYM_ERR_UNSUPPORTED, "no kernel for launch kind");
     c->a = a;
     return KYM_OK;

@@ -227,6 +227,25 @@ KYM_HD KYM_INL void dif_pass(cpx<T>* buf, const FftLen<T>& fl, const cpx<T>* tw,
     }
 }
 
+// The radices a kernel is built for: every one up to MAXP, or (MAXP = 100 + p)
+// those up to 7 and the prime p.
+template <int MAXP>
+KYM_HD constexpr bool kym_has_radix(int R) { return MAXP > 100 ? R <= 7 || R == MAXP - 100 : R <= MAXP; }
+
+// The passes of large radices as functions, for kernels with every radix up to
+// 31 (a node whose two lengths have different primes from 19 up), which would
+// hold each of them four to six times (246 KB of code).
+template <int R, bool INV, bool TWL, class T>
+KYM_HD __attribute__((noinline)) void dit_pass_call(cpx<T>* buf, const FftLen<T>& fl, const cpx<T>* tw, int q, int Lp,
+                                                    const Batch& bt, unsigned mtr, int tid, int nth) {
+    dit_pass<R, INV, TWL, T>(buf, fl, tw, q, Lp, bt, mtr, tid, nth);
+}
+template <int R, bool INV, bool TWL, class T>
+KYM_HD __attribute__((noinline)) void dif_pass_call(cpx<T>* buf, const FftLen<T>& fl, const cpx<T>* tw, int q, int L,
+                                                    const Batch& bt, unsigned mtr, int tid, int nth) {
+    dif_pass<R, INV, TWL, T>(buf, fl, tw, q, L, bt, mtr, tid, nth);
+}
+
 // Radix dispatch.  MAXP is the largest odd prime the kernel is built for, so a
 // kernel only carries the butterflies its plan can use (large odd radices
 // cost registers for every path through the kernel).
@@ -236,16 +255,16 @@ KYM_HD KYM_INL void dif_pass(cpx<T>* buf, const FftLen<T>& fl, const cpx<T>* tw,
         case 4: { CALL(4); } break;                                      \
         case 8: { CALL(8); } break;                                      \
         case 16: { CALL(16); } break;                                    \
-        case 3: if constexpr (MAXP >= 3) { CALL(3); } break;         \
-        case 5: if constexpr (MAXP >= 5) { CALL(5); } break;         \
-        case 7: if constexpr (MAXP >= 7) { CALL(7); } break;         \
-        case 11: if constexpr (MAXP >= 11) { CALL(11); } break;      \
-        case 13: if constexpr (MAXP >= 13) { CALL(13); } break;      \
-        case 17: if constexpr (MAXP >= 17) { CALL(17); } break;      \
-        case 19: if constexpr (MAXP >= 19) { CALL(19); } break;      \
-        case 23: if constexpr (MAXP >= 23) { CALL(23); } break;      \
-        case 29: if constexpr (MAXP >= 29) { CALL(29); } break;      \
-        case 31: if constexpr (MAXP >= 31) { CALL(31); } break;      \
+        case 3: if constexpr (kym_has_radix<MAXP>(3)) { CALL(3); } break;    \
+        case 5: if constexpr (kym_has_radix<MAXP>(5)) { CALL(5); } break;    \
+        case 7: if constexpr (kym_has_radix<MAXP>(7)) { CALL(7); } break;    \
+        case 11: if constexpr (kym_has_radix<MAXP>(11)) { CALL(11); } break;    \
+        case 13: if constexpr (kym_has_radix<MAXP>(13)) { CALL(13); } break;    \
+        case 17: if constexpr (kym_has_radix<MAXP>(17)) { CALL(17); } break;    \
+        case 19: if constexpr (kym_has_radix<MAXP>(19)) { CALL(19); } break;    \
+        case 23: if constexpr (kym_has_radix<MAXP>(23)) { CALL(23); } break;    \
+        case 29: if constexpr (kym_has_radix<MAXP>(29)) { CALL(29); } break;    \
+        case 31: if constexpr (kym_has_radix<MAXP>(31)) { CALL(31); } break;    \
         default: break;                                              \
     }
 
@@ -262,6 +281,26 @@ KYM_HD KYM_INL int kym_max_odd_prime(int n) {
 // Kernel families by prime set: 2-only/3/5/7 -> 7, up to 17 -> 17, up to 31 -> 31.
 KYM_HD KYM_INL int kym_prime_class(int maxp) { return maxp <= 7 ? 7 : maxp <= 17 ? 17 : 31; }
 
+// The family of kernels for lengths 2^i a and 2^i b: also 100 + p where
+// 19 <= p <= 31 is the only prime above 7 in them.  A kernel that holds the
+// radix-19 to -31 butterflies together needs 246 KB of code and up to 250
+// registers with spills; with one of them, 70 KB and the registers of that one.
+// J=3, each before and after: 32 x 136^2 (19) 770 -> 361 us, 16 x 170^2 (23)
+// 725 -> 318, 16 x 220^2 (29) 1149 -> 528, 16 x 235^2 (31) 1306 -> 616, FP64
+// 4 x 141^2 676 -> 292; 16 x 136x170 (19 and 23, every radix, large ones in
+// functions) 495 -> 353.
+inline int kym_plan_class(int a, int b) {
+    int only = 0, maxp = 1;
+    for (int v : {a, b})
+        for (int p = 3; p <= 31; p += 2)
+            while (v % p == 0) {
+                v /= p;
+                maxp = p > maxp ? p : maxp;
+                if (p > 7) only = only == 0 || only == p ? p : -1;
+            }
+    return only >= 19 ? 100 + only : kym_prime_class(maxp);
+}
+
 // Full DIT transform (digit-reversed in, natural out); barrier after each pass.
 // TWL: tw is fl's twiddle table copied to LDS (else fl.ptw is read).
 template <bool INV, int MAXP, bool TWL = false, class T>
@@ -271,7 +310,9 @@ KYM_HD KYM_INL void fft_dit(cpx<T>* buf, const FftLen<T>& fl, const Batch& bt, i
     const unsigned mtr = bt.tfast ? div_magic(bt.ntr) : 0;
     for (int q = 0; q < fl.nrad; ++q) {
         const int R = fl.rad[q];
-#define KYM_DIT_CALL(RR) dit_pass<RR, INV, TWL, T>(buf, fl, tw, q, Lp, bt, mtr, tid, nth)
+#define KYM_DIT_CALL(RR)                                                                 \
+    if constexpr (MAXP == 31 && RR >= 11) dit_pass_call<RR, INV, TWL, T>(buf, fl, tw, q, Lp, bt, mtr, tid, nth); \
+    else dit_pass<RR, INV, TWL, T>(buf, fl, tw, q, Lp, bt, mtr, tid, nth)
         KYM_RADIX_SWITCH(R, KYM_DIT_CALL)
 #undef KYM_DIT_CALL
         Lp *= R;
@@ -287,7 +328,10 @@ KYM_HD KYM_INL void fft_dif(cpx<T>* buf, const FftLen<T>& fl, const Batch& bt, i
     const unsigned mtr = bt.tfast ? div_magic(bt.ntr) : 0;
     for (int q = fl.nrad - 1; q >= 0; --q) {
         const int R = fl.rad[q];
-#define KYM_DIF_CALL(RR) dif_pass<RR, INV, TWL, T>(buf, fl, tw, q, L, bt, mtr, tid, nth); L = div_by(L, div_magic(RR))
+#define KYM_DIF_CALL(RR)                                                                 \
+    if constexpr (MAXP == 31 && RR >= 11) dif_pass_call<RR, INV, TWL, T>(buf, fl, tw, q, L, bt, mtr, tid, nth); \
+    else dif_pass<RR, INV, TWL, T>(buf, fl, tw, q, L, bt, mtr, tid, nth);                 \
+    L = div_by(L, div_magic(RR))
         KYM_RADIX_SWITCH(R, KYM_DIF_CALL)
 #undef KYM_DIF_CALL
         wg_barrier();

@@ -10,9 +10,17 @@ template <class T> using Scat1DKernel = void (*)(Scat1DArgs<T>);
 Scat2DKernel<float> kym_pick2d_f32_p7(int kind, int threads);
 Scat2DKernel<float> kym_pick2d_f32_p17(int kind, int threads);
 Scat2DKernel<float> kym_pick2d_f32_p31(int kind, int threads);
+Scat2DKernel<float> kym_pick2d_f32_p119(int kind, int threads);
+Scat2DKernel<float> kym_pick2d_f32_p123(int kind, int threads);
+Scat2DKernel<float> kym_pick2d_f32_p129(int kind, int threads);
+Scat2DKernel<float> kym_pick2d_f32_p131(int kind, int threads);
 Scat2DKernel<double> kym_pick2d_f64_p7(int kind, int threads);
 Scat2DKernel<double> kym_pick2d_f64_p17(int kind, int threads);
 Scat2DKernel<double> kym_pick2d_f64_p31(int kind, int threads);
+Scat2DKernel<double> kym_pick2d_f64_p119(int kind, int threads);
+Scat2DKernel<double> kym_pick2d_f64_p123(int kind, int threads);
+Scat2DKernel<double> kym_pick2d_f64_p129(int kind, int threads);
+Scat2DKernel<double> kym_pick2d_f64_p131(int kind, int threads);
 Scat2DKernel<float> kym_pick_node_spec_f32(int id);
 Scat2DKernel<float> kym_pick_bwd_node_spec_f32(int id);
 Scat2DKernel<float> kym_pick_pass_spec_f32(int kind, int id);
@@ -22,22 +30,29 @@ Scat1DKernel<float> kym_pick_bwd_node1d_spec_f32(int id);
 Scat1DKernel<float> kym_pick_any1d_f32(int kind);
 Scat1DKernel<double> kym_pick1d_f64(int threads, int kind);
 
-// pclass: 7, 17 or 31 (kym_prime_class of the plan's largest odd prime);
+// pclass: 7, 17, 31 or 100 + p (kym_plan_class);
 // spec >= 0 selects a compile-time specialisation of the node or pass kernel.
 template <class T>
 inline Scat2DKernel<T> pick_scat2d(int kind, int threads, int pclass, int spec = -1) {
+#define KYM_PICK_FAMILY(tag)                                                  \
+    switch (pclass) {                                                         \
+        case 7: return kym_pick2d_##tag##_p7(kind, threads);                  \
+        case 17: return kym_pick2d_##tag##_p17(kind, threads);                \
+        case 119: return kym_pick2d_##tag##_p119(kind, threads);              \
+        case 123: return kym_pick2d_##tag##_p123(kind, threads);              \
+        case 129: return kym_pick2d_##tag##_p129(kind, threads);              \
+        case 131: return kym_pick2d_##tag##_p131(kind, threads);              \
+        default: return kym_pick2d_##tag##_p31(kind, threads);                \
+    }
     if constexpr (sizeof(T) == 4) {
         if (spec >= 0 && kind == K2_LDS_NODE) return kym_pick_node_spec_f32(spec);
         if (spec >= 0 && kind == K2B_NODE) return kym_pick_bwd_node_spec_f32(spec);
         if (spec >= 0) return kym_pick_pass_spec_f32(kind, spec);
-        if (pclass <= 7) return kym_pick2d_f32_p7(kind, threads);
-        if (pclass <= 17) return kym_pick2d_f32_p17(kind, threads);
-        return kym_pick2d_f32_p31(kind, threads);
+        KYM_PICK_FAMILY(f32)
     } else {
-        if (pclass <= 7) return kym_pick2d_f64_p7(kind, threads);
-        if (pclass <= 17) return kym_pick2d_f64_p17(kind, threads);
-        return kym_pick2d_f64_p31(kind, threads);
+        KYM_PICK_FAMILY(f64)
     }
+#undef KYM_PICK_FAMILY
 }
 
 // spec >= 0 (FP32 nodes) selects a compile-time specialisation.

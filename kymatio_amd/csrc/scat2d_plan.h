@@ -18,6 +18,7 @@ struct Launch2D {
     int res;                // resolution of the launch's nodes
     long long model_bytes;  // algorithmic HBM bytes per image (stage-boundary model)
     int spec;               // compile-time specialisation id, -1 = run-time sizes
+    int pclass = 7;         // radix family of the kernel (kym_plan_class)
     int pair = 0;           // 1: a task is a sibling pair (group lists 2 ngroup node ids)
     // small LDS nodes: threads (and specialisation) of a launch of more than
     // many_tasks workgroups, 0 = the same
@@ -84,7 +85,6 @@ struct Scat2DPlan {
     size_t off_nodes = 0, off_lens = 0, off_filt = 0;
     size_t max_lds = 0;
     int max_threads = 256;
-    int pclass = 7;  // prime class of the kernels (largest odd radix family)
 
     int phi_index(int r) const { return r; }
     int psi_index(int n1, int level) const { return psi_base[n1] + level; }
@@ -201,11 +201,6 @@ struct Scat2DPlan {
         }
         oh = H[J] - 2;
         ow = W[J] - 2;
-        {
-            int mp = 1;
-            for (int r = 0; r <= J; ++r) mp = std::max(mp, std::max(kym_max_odd_prime(H[r]), kym_max_odd_prime(W[r])));
-            pclass = kym_prime_class(mp);
-        }
         // filters
         filt_off.clear(); filt_h.clear(); filt_w.clear();
         long long off = 0;
@@ -425,6 +420,18 @@ struct Scat2DPlan {
                 if (leaf_here) mb += leaf_model;
             }
             l.model_bytes = mb;
+            // a pass needs the radices of its own direction only, a node both
+            // (halving a length keeps its odd primes)
+            switch (kind) {
+                case K2_ICOL: case K2_ICOL_PAIR: case K2_FWD_COLS: case K2_LEAF_ICOL: case K2B_GCOLS: case K2B_GFCOLS:
+                    l.pclass = kym_plan_class(H[0], 1);
+                    break;
+                case K2_ROOT_ROWS: case K2_ROWS_MOD: case K2_LEAF_ROWS: case K2B_GROWS:
+                    l.pclass = kym_plan_class(W[0], 1);
+                    break;
+                case K2_FIR_COLS: case K2_FOLD: case K2B_FOLD: break;  // no transform
+                default: l.pclass = kym_plan_class(H[0], W[0]);
+            }
             l.spec = -1;
             launches.push_back(l);
             max_lds = std::max(max_lds, lds);

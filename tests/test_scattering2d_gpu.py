@@ -212,3 +212,28 @@ def test_many_small_nodes_match_few(shape, J, B):
     # the same butterflies in the same order, only spread over other threads
     assert (many - few).abs().max() <= 1e-6 * few.abs().max()
     assert (gmany - gfew).abs().max() <= 1e-5 * gfew.abs().max()
+
+
+@pytest.mark.parametrize('lds', [0, 8192], ids=['lds', 'multipass'])
+@pytest.mark.parametrize('shape', [(68, 12), (12, 84), (108, 108), (20, 116), (60, 44), (68, 116), (84, 36)],
+                         ids=['19x5', '5x23', '29x29', '7x31', '17x13', '19x31', '23x11'])
+def test_prime_lengths(shape, lds):
+    """Padded lengths 4 p and 4 q: each family of radices, alone and mixed,
+    forward in both types and the FP64 gradient, against the oracle."""
+    sc = Scattering2D(2, shape, L=2).to(DEV)
+    sc.lds_limit = lds
+    ref = scat2d.Scattering2DTorchCPU(2, shape, L=2, dtype=torch.float64)
+    x = torch.randn((2,) + shape, dtype=torch.float64, generator=torch.Generator().manual_seed(shape[0]))
+    xr = x.clone().requires_grad_()
+    want = ref(xr)
+    w = torch.randn(want.shape, dtype=torch.float64, generator=torch.Generator().manual_seed(1))
+    gw, = torch.autograd.grad((want * w).sum(), xr)
+    out = sc(x.float().to(DEV)).cpu().numpy()
+    assert channel_rel_err(out, want.detach().numpy()) <= RTOL_CHANNEL
+    sd = Scattering2D(2, shape, L=2).double().to(DEV)
+    sd.lds_limit = 2 * lds  # a double's line takes twice the bytes; the backward needs its leaf in LDS
+    xd = x.to(DEV).requires_grad_()
+    got = sd(xd)
+    gd, = torch.autograd.grad((got * w.to(DEV)).sum(), xd)
+    assert (got.detach().cpu() - want.detach()).abs().max() <= 1e-12 * want.abs().max()
+    assert torch.allclose(gd.cpu(), gw, rtol=1e-10, atol=1e-12 * gw.abs().max().item())
