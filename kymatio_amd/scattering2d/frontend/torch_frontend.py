@@ -55,8 +55,10 @@ class ScatteringTorch2D(ScatteringTorch, ScatteringBase):
         self._n_filters = n
 
     def _filter_buffers(self):
-        bufs = dict(self.named_buffers())
-        return [bufs['tensor' + str(i)] for i in range(self._n_filters)]
+        # the module's own table: named_buffers() walks the module tree and hashes
+        # every buffer to drop duplicates, 8 us of a 37 us call (32 x 32, J = 2)
+        bufs = self._buffers
+        return [bufs['tensor%d' % i] for i in range(self._n_filters)]
 
     def load_filters(self):
         """(phi, psi) dicts pointing at the module buffers
@@ -138,13 +140,13 @@ class ScatteringTorch2D(ScatteringTorch, ScatteringBase):
             raise RuntimeError("The out_type must be one of 'array' or 'list'.")
         if not getattr(self.backend, 'fused', False):
             return self._scattering_per_op(input)
-        bufs = self._filter_buffers()
-        if input.dtype is not bufs[0].dtype:
+        phi0 = self._buffers['tensor0']
+        if input.dtype is not phi0.dtype:
             raise TypeError('Input and filter must be of the same dtype.')
         _lib.require_device(input)
-        if not bufs[0].is_cuda:
+        if not phi0.is_cuda:
             raise TypeError('Input must be on CPU.')
-        if input.device != bufs[0].device:
+        if input.device != phi0.device:
             raise TypeError('Input and filter must be on the same GPU.')
         batch_shape, sig = input.shape[:-2], input.shape[-2:]
         x = input.reshape((-1,) + tuple(sig))
