@@ -1,6 +1,7 @@
 // Mixed-radix in-place FFT passes over data held in LDS.
 //
-// Length n = r_1 r_2 ... r_K (radices 2, 4, 8, 16 and odd primes 3..31).
+// Length n = r_1 r_2 ... r_K (radices 2, 4, 8, 16, odd primes 3..31, and the
+// products 9 and 15 where a plan asks for them).
 // Two in-place Cooley-Tukey variants share one digit-reversal permutation
 // `rev` (rev[p] = natural index of the element at storage position p):
 //   * DIT, passes r_1 .. r_K: input stored digit-reversed, output natural.
@@ -153,11 +154,64 @@ template <int P, bool INV, class T> KYM_HD KYM_INL void dft_odd(cpx<T>* v) {
     }
 }
 
+template <int R, bool INV, class T> KYM_HD KYM_INL void dft_r(cpx<T>* v);
+
+// R = A B with A and B coprime: the prime-factor algorithm (Good 1958).  Inputs
+// (B n1 + A n2) mod R, outputs k with k = k1 mod A and k = k2 mod B, and no
+// twiddles between the two.
+template <int A, int B, bool INV, class T> KYM_HD KYM_INL void dft_coprime(cpx<T>* v) {
+    constexpr int R = A * B;
+    constexpr int iB = [] { int i = 1; while (i * B % A != 1) ++i; return i; }();
+    constexpr int iA = [] { int i = 1; while (i * A % B != 1) ++i; return i; }();
+    cpx<T> t[R];
+#pragma unroll
+    for (int n2 = 0; n2 < B; ++n2) {
+        cpx<T> u[A];
+#pragma unroll
+        for (int n1 = 0; n1 < A; ++n1) u[n1] = v[(B * n1 + A * n2) % R];
+        dft_r<A, INV>(u);
+#pragma unroll
+        for (int k1 = 0; k1 < A; ++k1) t[k1 * B + n2] = u[k1];
+    }
+#pragma unroll
+    for (int k1 = 0; k1 < A; ++k1) {
+        dft_r<B, INV>(t + k1 * B);
+#pragma unroll
+        for (int k2 = 0; k2 < B; ++k2) v[(k1 * B * iB + k2 * A * iA) % R] = t[k1 * B + k2];
+    }
+}
+
+template <bool INV, class T> KYM_HD KYM_INL void dft9(cpx<T>* v) {
+    // 3 x 3: inner over n1 for each n2, twiddle W9^(n2 k1), outer over n2
+    // cos and sin of 2 pi m / 9, m = 1, 2, 4
+    constexpr double cs[3] = {0.76604444311897803520, 0.17364817766693034885, -0.93969262078590838405};
+    constexpr double sn[3] = {0.64278760968653932632, 0.98480775301220805937, 0.34202014332566873304};
+    cpx<T> t[9];
+#pragma unroll
+    for (int n2 = 0; n2 < 3; ++n2) {
+        cpx<T> u[3] = {v[n2], v[3 + n2], v[6 + n2]};
+        dft_odd<3, INV>(u);
+#pragma unroll
+        for (int k1 = 0; k1 < 3; ++k1) {
+            const int m = n2 * k1 == 4 ? 2 : n2 * k1 - 1;
+            t[k1 * 3 + n2] = n2 * k1 == 0 ? u[k1] : cmul(u[k1], cpx<T>{T(cs[m]), T(INV ? sn[m] : -sn[m])});
+        }
+    }
+#pragma unroll
+    for (int k1 = 0; k1 < 3; ++k1) {
+        dft_odd<3, INV>(t + 3 * k1);
+#pragma unroll
+        for (int k2 = 0; k2 < 3; ++k2) v[k1 + 3 * k2] = t[3 * k1 + k2];
+    }
+}
+
 template <int R, bool INV, class T> KYM_HD KYM_INL void dft_r(cpx<T>* v) {
     if constexpr (R == 2) dft2<INV>(v);
     else if constexpr (R == 4) dft4<INV>(v);
     else if constexpr (R == 8) dft8<INV>(v);
     else if constexpr (R == 16) dft16<INV>(v);
+    else if constexpr (R == 9) dft9<INV>(v);
+    else if constexpr (R == 15) dft_coprime<5, 3, INV>(v);
     else dft_odd<R, INV>(v);
 }
 
@@ -227,10 +281,20 @@ KYM_HD KYM_INL void dif_pass(cpx<T>* buf, const FftLen<T>& fl, const cpx<T>* tw,
     }
 }
 
-// The radices a kernel is built for: every one up to MAXP, or (MAXP = 100 + p)
+// The primes a kernel is built for: every one up to MAXP, or (MAXP = 100 + p)
 // those up to 7 and the prime p.
 template <int MAXP>
 KYM_HD constexpr bool kym_has_radix(int R) { return MAXP > 100 ? R <= 7 || R == MAXP - 100 : R <= MAXP; }
+
+// Radices 9 and 15: in the kernels of the class 7 (kym_factor_list says why),
+// and in the CPU harness, which runs every plan on the bodies of the class 31.
+template <int MAXP> KYM_HD constexpr bool kym_has_products() {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return MAXP == 7;
+#else
+    return true;
+#endif
+}
 
 // The passes of large radices as functions, for kernels with every radix up to
 // 31 (a node whose two lengths have different primes from 19 up), which would
@@ -255,6 +319,8 @@ KYM_HD __attribute__((noinline)) void dif_pass_call(cpx<T>* buf, const FftLen<T>
         case 4: { CALL(4); } break;                                      \
         case 8: { CALL(8); } break;                                      \
         case 16: { CALL(16); } break;                                    \
+        case 9: if constexpr (kym_has_products<MAXP>()) { CALL(9); } break;    \
+        case 15: if constexpr (kym_has_products<MAXP>()) { CALL(15); } break;  \
         case 3: if constexpr (kym_has_radix<MAXP>(3)) { CALL(3); } break;    \
         case 5: if constexpr (kym_has_radix<MAXP>(5)) { CALL(5); } break;    \
         case 7: if constexpr (kym_has_radix<MAXP>(7)) { CALL(7); } break;    \
@@ -343,6 +409,14 @@ KYM_HD KYM_INL void fft_dif(cpx<T>* buf, const FftLen<T>& fl, const Batch& bt, i
 // max_pow2 (16, 8, 4 or 2) caps the power-of-two radices (a tuning choice;
 // 16 is the default every compile-time specialisation assumes).
 // constexpr so compile-time specialisations use exactly the runtime order.
+// products: 15 and 9 in one pass each from 48 points on (shorter lines would
+// leave most of a workgroup's threads without a butterfly), for run-time-sized
+// kernels of the class 7.  A pass over LDS less: 48 x 224^2, J=3 (15 x 16, 15 x
+// 8) 1055 -> 961 us, 16 of them with the gradient 1157 -> 1064, 32 x 128^2 (9 x
+// 16, 9 x 8) 322 -> 309.  Odd radices read a row's first pass without bank
+// conflicts; 6, 10 and 14 were no faster than the passes they saved, and in
+// the kernels up to 17 the added butterflies spilled (6 x 150x203 221 -> 417).
+#define KYM_PRODUCT_MIN_N 48
 struct RadList {
     int n = 0;
     int nrad = 0;
@@ -350,11 +424,20 @@ struct RadList {
     bool ok = false;
 };
 
-KYM_HD constexpr RadList kym_factor_list(int n, int max_pow2 = 16) {
+KYM_HD constexpr RadList kym_factor_list(int n, int max_pow2 = 16, bool products = false) {
     RadList rl;
     rl.n = n;
     int k = 0;
     int m = n;
+    int a = 0;
+    while (m % 2 == 0) { m /= 2; ++a; }
+    const int product[2] = {15, 9};
+    for (int i = 0; products && n >= KYM_PRODUCT_MIN_N && i < 2; ++i)
+        while (m % product[i] == 0) {
+            if (k >= KYM_MAX_RADICES) return rl;
+            rl.rad[k++] = product[i];
+            m /= product[i];
+        }
     const int odd[10] = {3, 5, 7, 11, 13, 17, 19, 23, 29, 31};
     for (int i = 0; i < 10; ++i) {
         const int p = odd[i];
@@ -364,8 +447,6 @@ KYM_HD constexpr RadList kym_factor_list(int n, int max_pow2 = 16) {
             m /= p;
         }
     }
-    int a = 0;
-    while (m % 2 == 0) { m /= 2; ++a; }
     if (m != 1) return rl;
     const int dmax = max_pow2 >= 16 ? 4 : max_pow2 >= 8 ? 3 : max_pow2 >= 4 ? 2 : 1;
     while (a > 0) {
@@ -388,8 +469,8 @@ KYM_HD constexpr RadList kym_factor_list(int n, int max_pow2 = 16) {
     return rl;
 }
 
-inline bool kym_factor(int n, int* rad, int* nrad, int max_pow2 = 16) {
-    const RadList rl = kym_factor_list(n, max_pow2);
+inline bool kym_factor(int n, int* rad, int* nrad, int max_pow2 = 16, bool products = false) {
+    const RadList rl = kym_factor_list(n, max_pow2, products);
     if (!rl.ok) return false;
     for (int i = 0; i < rl.nrad; ++i) rad[i] = rl.rad[i];
     *nrad = rl.nrad;

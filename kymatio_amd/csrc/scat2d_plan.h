@@ -193,6 +193,7 @@ struct Scat2DPlan {
         Np = ((N + (1 << J)) / (1 << J) + 1) * (1 << J);
         top = (Mp - M) / 2;
         left = (Np - N) / 2;
+        lens.products = kym_plan_class(Mp, Np) == 7;  // every kernel of the plan is of the class 7
         for (int r = 0; r <= J; ++r) {
             H[r] = Mp >> r;
             W[r] = Np >> r;

@@ -215,11 +215,14 @@ def test_many_small_nodes_match_few(shape, J, B):
 
 
 @pytest.mark.parametrize('lds', [0, 8192], ids=['lds', 'multipass'])
-@pytest.mark.parametrize('shape', [(68, 12), (12, 84), (108, 108), (20, 116), (60, 44), (68, 116), (84, 36)],
-                         ids=['19x5', '5x23', '29x29', '7x31', '17x13', '19x31', '23x11'])
+@pytest.mark.parametrize('shape', [(68, 12), (12, 84), (108, 108), (20, 116), (60, 44), (68, 116), (84, 36),
+                                   (52, 64), (172, 100), (28, 172)],
+                         ids=['19x5', '5x23', '29x29', '7x31', '17x13', '19x31', '23x11',
+                              '15x18', '45x27', '9x45'])
 def test_prime_lengths(shape, lds):
-    """Padded lengths 4 p and 4 q: each family of radices, alone and mixed,
-    forward in both types and the FP64 gradient, against the oracle."""
+    """Padded lengths 4 p and 4 q: each family of radices, alone and mixed, and
+    products of small primes in one radix (15, 9 from 48 points on): forward
+    in both types and the FP64 gradient, against the oracle."""
     sc = Scattering2D(2, shape, L=2).to(DEV)
     sc.lds_limit = lds
     ref = scat2d.Scattering2DTorchCPU(2, shape, L=2, dtype=torch.float64)
@@ -231,7 +234,7 @@ def test_prime_lengths(shape, lds):
     out = sc(x.float().to(DEV)).cpu().numpy()
     assert channel_rel_err(out, want.detach().numpy()) <= RTOL_CHANNEL
     sd = Scattering2D(2, shape, L=2).double().to(DEV)
-    sd.lds_limit = 2 * lds  # a double's line takes twice the bytes; the backward needs its leaf in LDS
+    sd.lds_limit = 3 * lds  # doubles; the backward needs its leaf (45 x 27 at most) in LDS
     xd = x.to(DEV).requires_grad_()
     got = sd(xd)
     gd, = torch.autograd.grad((got * w.to(DEV)).sum(), xd)
