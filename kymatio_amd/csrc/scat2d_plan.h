@@ -34,11 +34,13 @@ struct Launch2D {
 #define KYM_MANY_TASKS 2048
 // Points up to which one wave per node is used.
 #define KYM_WAVE_NODE 640
-// Run-time-sized nodes of 2048 to 4095 points: 512 threads up to two
-// workgroups a CU (what their 105 registers allow at once), 256 beyond, where
-// four independent workgroups wait less for each other's barriers than two of
-// twice the threads (48 images of 224 x 224 J=3: 1103 -> 1053 us; 6 of 150 x
-// 203 J=4, 400 nodes a launch: 221 us against 224).
+// Run-time-sized nodes of 2048 points up to what 256 threads stage (5120; FP64,
+// whose node fills half the LDS, 4095): 512 threads up to two workgroups a CU
+// (what their 105 registers allow at once), 256 beyond, where four independent
+// workgroups wait less for each other's barriers than two of twice the threads
+// (48 images of 224 x 224 J=3, 60 x 60 nodes: 1103 -> 1053 us; 64 of 112 x 112
+// J=3, 64 x 64 nodes: 451 -> 409; 6 of 150 x 203 J=4, 400 nodes a launch: 221 us
+// against 224).
 #define KYM_MANY_MEDIUM 512
 
 // Tuning choices of a plan (0 = the built-in heuristic).  Any non-default
@@ -371,10 +373,11 @@ struct Scat2DPlan {
         max_lds = 0;
         max_threads = 256;
         // fewer threads per node where the launch's nodes are small and many
+        const size_t medium = sizeof(T) == 4 ? KYM_STAGE_MAX * 256 : 4095;
         auto many_waves = [&](Launch2D& l) {
             const size_t elems = (size_t)H[l.res] * W[l.res];
             if (tune.node_threads || l.pair) return;
-            if (l.spec < 0 && elems >= 2048 && elems < 4096) {
+            if (l.spec < 0 && elems >= 2048 && elems <= medium) {
                 l.many_threads = 256;
                 l.many_tasks = KYM_MANY_MEDIUM;
                 return;

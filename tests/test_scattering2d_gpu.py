@@ -198,10 +198,10 @@ def test_list_output_meta():
         assert torch.equal(o['coef'], arr[:, c])
 
 
-@pytest.mark.parametrize('shape,J,B', [((32, 32), 2, 80), ((28, 34), 2, 70), ((24, 24), 3, 130)])
+@pytest.mark.parametrize('shape,J,B', [((32, 32), 2, 80), ((28, 34), 2, 70), ((24, 24), 3, 130), ((60, 60), 2, 80)])
 def test_many_small_nodes_match_few(shape, J, B):
     """Launches of more than 2048 small nodes run them one wave each, smaller
-    launches with 256 threads: the same coefficients and gradients."""
+    launches with 256 threads (nodes of up to 5120 points: 256 and 512): the same coefficients and gradients."""
     sc = Scattering2D(J, shape).to(DEV)
     x = torch.randn((B,) + shape, device=DEV, generator=torch.Generator(DEV).manual_seed(B)).requires_grad_()
     w = torch.randn(sc(x[:1]).shape[1:], device=DEV, generator=torch.Generator(DEV).manual_seed(1))
