@@ -70,10 +70,12 @@ def build_emu():
 
 
 def main(argv):
-    if '--hip-only' not in argv:
-        build_emu()
-    if '--emu-only' not in argv:
-        build_product()
+    from concurrent.futures import ThreadPoolExecutor
+    # one source of two minutes beside the other units
+    parts = [build_emu] * ('--hip-only' not in argv) + [build_product] * ('--emu-only' not in argv)
+    with ThreadPoolExecutor(2) as ex:
+        for f in [ex.submit(p) for p in parts]:
+            f.result()
 
 
 if __name__ == '__main__':
