@@ -55,7 +55,8 @@ int kym_scat2d_create(int M, int N, int J, int L, int max_order, int pre_pad, in
  * big-node column block, big-node row block, big-node pass threads (a
  * compiled choice for these sizes and blocks), streams (1: the inference
  * forward runs its chunks one after the other on the caller's stream; S in
- * 2..4, default 2: the workspace is split in S parts and chunks rotate over
+ * 2..4, default 2, or 1 for a batch of fewer than 9 million node points: the
+ * workspace is split in S parts and chunks rotate over
  * the caller's stream and S - 1 streams of the plan, joined back to the
  * caller's stream before kym_scat2d_forward's work ends; forward_train and
  * backward split the batch in S chunks the same way, each image's saved
@@ -218,7 +219,8 @@ int kym_scat1d_forward(void* plan, const void* x, const void* filt, void* out, l
 /* Inference chunks in flight for kym_scat1d_forward (no counterpart in the
  * reference; a scheduling choice): 1 = one after the other on the caller's
  * stream, S in 2..4 = the workspace split in S parts and chunks rotating over
- * the caller's stream and S - 1 streams of the plan; 0 = default 2.  Results
+ * the caller's stream and S - 1 streams of the plan; 0 = default 2, or 1 for
+ * a batch of fewer than 20 million node points.  Results
  * do not depend on it. */
 int kym_scat1d_set_streams(void* plan, int streams);
 

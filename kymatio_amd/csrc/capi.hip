@@ -90,15 +90,28 @@ struct ChunkStreams {
     }
 };
 
-// Streams a chunked inference call uses: `want` (0 = 2) reduced until every
-// stream gets a chunk.  The chunk then fits one stream's share of the
+// Node points of a call from which it is split over two streams by default.
+// The fork and join cost the host two event records and waits, the device two
+// waits between queues, 20 to 50 us a call; the second stream gains where a
+// launch's tail leaves the chip idle for as long.  One stream against two:
+// 92 images of 17 x 17 J=1 (0.3 million points) 28 against 75 us, 32 of 64 x 64
+// J=3 (7.3) 89 against 105, 8 of 128 x 128 J=4 with the gradient (7.9) 417
+// against 442, FP64 4 of 224 x 224 J=3 (8.2) 529 against 563, 6 of 150 x 203
+// J=4 (9.1) 221 against 218, 4 of 256 x 256 J=3 (10.5) 201 against 194, 16 (42) 407 against 387; 1D, whose launches are
+// fewer: 105 signals of 3608 J=7 (7.5) 226 against 430, 64 of 4096 J=6 Q=8 (17)
+// 254 against 264, 128 (35) 332 against 322.
+#define KYM_STREAM_POINTS_2D 9000000
+#define KYM_STREAM_POINTS_1D 20000000
+
+// Streams a chunked call uses: `want` (0 = 2, or 1 for a call of fewer than
+// `enough` of its `points`) reduced until every stream gets a chunk.  The chunk then fits one stream's share of the
 // workspace, with the chunk count a multiple of the stream count and the
 // chunks as even as that allows (256 over 3 streams: 6 chunks of <= 43, not
 // 85, 85, 85, 1).
-static int chunk_streams(const ChunkStreams* cs, int want, int mode, long long batch, long long* chunk) {
-    int ns = want == 0 ? 2 : want;
+static int chunk_streams(const ChunkStreams* cs, int want, long long points, long long enough, long long batch,
+                         long long* chunk) {
+    int ns = want != 0 ? want : points < enough ? 1 : 2;
     if (!cs || !cs->aux[0]) ns = 1;
-    (void)mode;
     while (ns > 1 && (*chunk < ns || batch <= *chunk / ns * (ns - 1))) --ns;
     if (ns > 1) {
         const long long part = *chunk / ns;
@@ -327,7 +340,7 @@ static int chunk_of(const Scat2DPlan<T>& p, int mode, long long batch, long long
 
 // mode 0: inference forward (batch in chunks); 1: training forward (saves
 // u, whole batch in the workspace); 2: backward from the saved workspace.
-// With S streams (tune.streams, 0 = 2; at least S images) chunk k runs on
+// With S streams (tune.streams, 0 = 2 or 1, chunk_streams; at least S images) chunk k runs on
 // stream k mod S.  Inference splits the workspace in S parts and chunk k
 // uses part k mod S, so chunk k + S reuses a part only after chunk k on the
 // same stream; training keeps image i's state at image offset i of the
@@ -342,7 +355,7 @@ static int run2d(const Scat2DPlan<T>& p, int mode, const void* x, const void* fi
     int rc = chunk_of(p, mode, batch, ws_bytes, &chunk, &img_elems);
     if (rc != KYM_OK) return rc;
     const std::vector<Launch2D>& launches = mode == 2 ? p.bwd_launches : p.launches;
-    const int ns = chunk_streams(cs, p.tune.streams, mode, batch, &chunk);
+    const int ns = chunk_streams(cs, p.tune.streams, batch * p.points, KYM_STREAM_POINTS_2D, batch, &chunk);
     rc = chunk_fork(cs, ns, stream);
     if (rc != KYM_OK) return rc;
     int k = 0;
@@ -777,7 +790,7 @@ static int run1d(const Scat1DPlan<T>& p, int mode, const void* x, const void* fi
     const std::vector<Launch1D>& launches =
         merged ? (mode == 2 ? p.bwd_merged : p.merged) : mode == 2 ? p.bwd_launches : p.launches;
     // inference chunks rotate over the plan's streams as in run2d
-    const int ns = merged ? 1 : chunk_streams(cs, streams, mode, batch, &chunk);
+    const int ns = merged ? 1 : chunk_streams(cs, streams, batch * p.points, KYM_STREAM_POINTS_1D, batch, &chunk);
     int rc = chunk_fork(cs, ns, stream);
     if (rc != KYM_OK) return rc;
     int k = 0;

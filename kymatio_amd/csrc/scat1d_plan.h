@@ -46,6 +46,7 @@ struct Scat1DPlan {
     // per chunk, and one chunk); see merged_fits
     std::vector<Launch1D> merged, bwd_merged;
     long long ws_sig_train = 0;
+    long long points = 0;  // of all nodes of a signal
     Blob blob;
     size_t off_nodes = 0, off_lens = 0, off_filt = 0, max_lds = 0;
 
@@ -155,6 +156,8 @@ struct Scat1DPlan {
         for (auto& nd : nodes)
             if (nd.parent >= 0) has_children[nd.parent] = 1;
         ws_sig = 0;
+        points = 0;
+        for (const auto& nd : nodes) points += n[nd.res];
         const long long align = 256 / (long long)sizeof(cpx<T>);
         for (size_t i = 0; i < nodes.size(); ++i) {
             nodes[i].slot = has_children[i] ? ws_sig : -1;

@@ -74,6 +74,7 @@ struct Scat2DPlan {
     // the same without the gin slots (which come last): a workspace that holds
     // only this runs without the K2_FOLD launches, every node gathering itself
     long long ws_img_base = 0;
+    long long points = 0;  // of all nodes of an image
     std::vector<Launch2D> launches;
     // training: forward with saving, then the backward launches
     long long ws_img_train = 0;  // complex elements per image (layout extends the inference one)
@@ -324,6 +325,8 @@ struct Scat2DPlan {
         }
         // gathered inputs of LDS nodes with a deep periodisation (K2_FOLD)
         ws_img_base = ws_img;
+        points = 0;
+        for (const auto& nd : nodes) points += (long long)H[nd.res] * W[nd.res];
         for (auto& nd : nodes) {
             nd.gin = -1;
             if (nd.big || nd.order == 0 || nd.k < KYM_FOLD_MIN_K || W[nd.res] > KYM_FOLD_THREADS ||

@@ -55,7 +55,7 @@ class Scat1DPlanHandle:
         self.filter_offsets, self.path_len = list(fo), list(pl)
 
     def set_streams(self, streams):
-        """Inference chunks in flight (0 = default 2; kym_scat1d_set_streams)."""
+        """Inference chunks in flight (0 = default: 2, or 1 for small batches; kym_scat1d_set_streams)."""
         _lib.check(self._lib.kym_scat1d_set_streams(self._h, int(streams)))
 
     def forward(self, x, filt, out, batch, ws):
@@ -101,7 +101,8 @@ class ScatteringTorch1D(ScatteringTorch, ScatteringBase):
         self._packed = {}
         self.signals_per_chunk = None
         self.lds_limit = 0
-        self.streams = 0  # inference chunks in flight on the device (0 = the library's default, 2)
+        # inference chunks in flight on the device (0 = the library's default: 2, or 1 for small batches)
+        self.streams = 0
 
     # ------------------------------------------------------------ setup
     def build(self):

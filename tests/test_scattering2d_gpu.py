@@ -240,3 +240,23 @@ def test_prime_lengths(shape, lds):
     gd, = torch.autograd.grad((got * w.to(DEV)).sum(), xd)
     assert (got.detach().cpu() - want.detach()).abs().max() <= 1e-12 * want.abs().max()
     assert torch.allclose(gd.cpu(), gw, rtol=1e-10, atol=1e-12 * gw.abs().max().item())
+
+
+@pytest.mark.parametrize('B', [1, 2, 39, 40])
+def test_streams_either_side_of_the_line(B):
+    """Batches of fewer than 9 million node points (227,600 an image here, 39
+    images) stay on the caller's stream, larger ones take two: the same
+    coefficients and gradients as with one and two streams asked for."""
+    x = torch.randn(B, 64, 64, device=DEV, generator=torch.Generator(DEV).manual_seed(B)).requires_grad_()
+    res = []
+    for streams in (0, 1, 2):
+        sc = Scattering2D(3, (64, 64)).to(DEV)
+        sc.tune = [0, 0, 0, 0, 0, streams] if streams else None
+        out = sc(x * 1.0)
+        g, = torch.autograd.grad((out * out).sum(), x)
+        with torch.no_grad():
+            res.append((out.detach(), g, sc(x * 1.0)))
+    for r in res[1:]:
+        # the same butterflies, possibly spread over other threads
+        for a, b, tol in zip(r, res[0], (1e-6, 1e-5, 1e-6)):
+            assert (a - b).abs().max() <= tol * b.abs().max()
