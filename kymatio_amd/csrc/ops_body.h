@@ -940,9 +940,12 @@ KYM_HD void harmonic_plane_body(const HarmonicArgs& o, const FftLen<T>& fN, cons
     fft_dif<true, MAXP>(lds, fO, Batch{N, 1, ws, false}, tid, nth);
     fft_dif<true, MAXP>(lds, fN, Batch{O, ws, 1, true}, tid, nth);
     cpx<T>* y = static_cast<cpx<T>*>(o.Y) + blk * n;
+    // each transform is scaled by its own length, before any square is formed:
+    // FP32 moduli hold to 1.8e19, not to that over the volume's points
+    const T inv_n = T(1) / T(n);
     for (int i = tid; i < n; i += nth) {
         const int r = i / O, x = i - r * O;
-        y[i] = lds[kym_ldg(fN.irev + r) * ws + kym_ldg(fO.irev + x)];
+        y[i] = lds[kym_ldg(fN.irev + r) * ws + kym_ldg(fO.irev + x)] * inv_n;
     }
 }
 
@@ -958,6 +961,7 @@ KYM_HD void harmonic_cols_body(const HarmonicArgs& o, const FftLen<T>& fM, long 
     const FInt nc = fast_int(S - c0 < o.cb ? S - c0 : o.cb);
     const int total = M * nc;
     const cpx<T>* y = static_cast<const cpx<T>*>(o.Y) + bg * o.nm * ((long long)M * S) + c0;
+    const T inv_m = T(1) / T(M);
     T acc[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) acc[e] = T(0);
@@ -979,19 +983,18 @@ KYM_HD void harmonic_cols_body(const HarmonicArgs& o, const FftLen<T>& fM, long 
 #pragma unroll
         for (int e = 0; e < E; ++e)
             if (tid + e * nth < total) {
-                const cpx<T> u = lds[tid + e * nth];
+                const cpx<T> u = lds[tid + e * nth] * inv_m;
                 acc[e] += u.re * u.re + u.im * u.im;
             }
         wg_barrier();
     }
-    const T inv_n = T(1) / (T(M) * T(S));
     T* d = static_cast<T*>(o.dest) + g * o.dstride + b * ((long long)M * S) + c0;
 #pragma unroll
     for (int e = 0; e < E; ++e) {
         const int i = tid + e * nth;
         if (i < total) {
             const int p = i / nc, c = i - p * nc;
-            d[(long long)kym_ldg(fM.rev + p) * S + c] = kym_sqrt(acc[e]) * inv_n;
+            d[(long long)kym_ldg(fM.rev + p) * S + c] = kym_sqrt(acc[e]);
         }
     }
 }

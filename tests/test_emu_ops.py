@@ -390,3 +390,22 @@ def test_harmonic_step(emu, M, N, O, ng, nm, dtype):
         assert g(y.ctypes.data, y.ctypes.data, B, M, N * O, inv) == 0
         r = (np.fft.ifft if inv else np.fft.fft)(x, axis=1)
         assert np.abs(y - r).max() <= 1e-14 * M * np.abs(x).max()
+
+
+@pytest.mark.parametrize('M,N,O', [(8, 16, 4), (17, 6, 10)])
+def test_harmonic_step_large_magnitudes(emu, M, N, O):
+    """FP32 moduli of 1e18 stay finite: their squares fit, those of the
+    transform before its 1 / (M N O) would not."""
+    rng = np.random.default_rng(M)
+    vol, nm = M * N * O, 3
+    u = 1e18 * (rng.uniform(-1, 1, (1, M, N, O)) + 1j * rng.uniform(-1, 1, (1, M, N, O)))
+    U = np.fft.fftn(u, axes=(-3, -2, -1)).astype(np.complex64)
+    F = np.ones((nm, vol), np.complex64)
+    work, dest = np.zeros(nm * vol, np.complex64), np.zeros(vol, np.float32)
+    f = emu.lib.kym_emu_op_harmonic_step
+    P, LL, I = ctypes.c_void_p, ctypes.c_longlong, ctypes.c_int
+    f.argtypes, f.restype = [P] * 4 + [LL] + [I] * 5 + [LL, LL, I], I
+    assert f(U.ctypes.data, F.ctypes.data, work.ctypes.data, dest.ctypes.data, 1, 1, nm, M, N, O, nm * vol, vol, 0) == 0
+    ref = np.sqrt(nm) * np.abs(np.fft.ifftn(U.astype(np.complex128), axes=(-3, -2, -1))).reshape(-1)
+    tol = 8 * (np.log2(vol) + nm) * np.finfo(np.float32).eps  # as in test_harmonic_step
+    assert np.abs(dest - ref).max() <= tol * ref.max()

@@ -178,3 +178,15 @@ def test_moduli_match_64_bits(shape, B, dtype):
         u.append(mod(torch.fft.fftn(u[0], dim=dim), l, 1))
         ref = torch.stack([torch.stack([v.sum(dim), v.square().sum(dim)], -1) for v in u], 1)
         assert ((out[:, :, l] - ref).abs() <= 2e-6 * ref.abs() + 1e-9 * ref.abs().max()).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('shape', [(32, 32, 32), (4, 160, 150)])
+def test_large_magnitudes_scale(shape):
+    """Every step up to the integral of power 1 is homogeneous of degree one,
+    and a power of two changes no mantissa: S(2^46 x) = 2^46 S(x) as long as
+    the squares of the moduli fit FP32 (they are at most 2^97 here)."""
+    S = HarmonicScattering3D(J=1, shape=shape, L=2, integral_powers=(1.,)).to(DEV)
+    x = torch.rand((2,) + shape, device=DEV, generator=torch.Generator(DEV).manual_seed(3))
+    c = 2. ** 46
+    assert torch.allclose(S(c * x), c * S(x), rtol=1e-6, atol=0)
