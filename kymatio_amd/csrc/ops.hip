@@ -132,7 +132,9 @@ __global__ void __launch_bounds__(256) k_integrals(const T* x, T* out, long long
     // the usual powers without pow (exact but for its last bit; the library
     // call took 158 us for 192 fields of 32^3, most of it here), four loads in
     // flight
-    auto power = [&](double v, double p) { return p == 1.0 ? v : p == 2.0 ? v * v : p == 0.5 ? sqrt(v) : pow(v, p); };
+    auto power = [&](double v, double p) {
+        return p == 1.0 ? v : p == 2.0 ? v * v : p == 0.5 && v >= 0.0 ? sqrt(v) : pow(v, p);  // pow(-inf, 0.5) = inf
+    };
     long long i = threadIdx.x;
     for (; i + 3 * blockDim.x < n; i += 4 * blockDim.x) {
         T v[4];

@@ -190,3 +190,17 @@ def test_large_magnitudes_scale(shape):
     x = torch.rand((2,) + shape, device=DEV, generator=torch.Generator(DEV).manual_seed(3))
     c = 2. ** 46
     assert torch.allclose(S(c * x), c * S(x), rtol=1e-6, atol=0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float64])
+def test_integrals_of_special_values(dtype):
+    """The integrals' powers of infinities and signed zeros are those of C's
+    pow: pow(-inf, 0.5) = inf, pow(-0, 0.5) = +0, a negative root is NaN."""
+    powers = (0.5, 1., 2.)
+    rows = [[np.inf, 1.], [-np.inf, 4.], [-0., 0.25], [-1., 4.], [np.nan, 4.]]
+    x = torch.tensor(rows, dtype=dtype).reshape(len(rows), 2, 1, 1)
+    out = backend.compute_integrals(x.to(DEV), powers).cpu().numpy()
+    with np.errstate(invalid='ignore'):
+        ref = np.stack([np.power(np.float64(rows), p).sum(1) for p in powers], 1)
+    assert np.array_equal(out, ref.astype(np.float32), equal_nan=True)
