@@ -27,7 +27,10 @@ PRODUCT_UNITS = [('kpass2d.hip', [], 'kpass2d.o'), ('kspec2d.hip', [], 'kspec2d.
                  ('ops.hip', [], 'ops.o'), ('decoder.hip', [], 'decoder.o')] + [
     ('kinst2d.hip', ['-DKYM_T=%s' % T, '-DKYM_P=%d' % P, '-DKYM_PICK=kym_pick2d_%s_p%d' % (tag, P)],
      'kinst2d_%s_p%d.o' % (tag, P))
-    for tag, T in (('f32', 'float'), ('f64', 'double')) for P in (31, 131, 129, 123, 119, 17, 7)]
+    for tag, T in (('f32', 'float'), ('f64', 'double')) for P in (31, 131, 129, 123, 119, 17, 7)] + [
+    ('kinst2d.hip', ['-DKYM_T=%s' % T, '-DKYM_P=%d' % P, '-DKYM_PICK=kym_pick2d_%s_g%d' % (tag, P),
+                     '-DKYM_GLOBAL_TW_ONLY'], 'kinst2d_%s_g%d.o' % (tag, P))
+    for tag, T in (('f32', 'float'), ('f64', 'double')) for P in (31, 17, 7)]
 EMU_SOURCES = ['emu.hip']
 BUILD_DIR = os.path.join(HERE, '_build')
 

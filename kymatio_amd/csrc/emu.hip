@@ -31,6 +31,51 @@ static void emu_spec(const Launch2D& l, const Scat2DArgs<T>& a, int t, cpx<T>* l
     }
 }
 
+// A launch of run-time sizes, with or without its twiddles in LDS.
+template <class T>
+static void emu_body(const Launch2D& l, const Scat2DArgs<T>& a, int t, cpx<T>* lds) {
+    if (l.kind >= K2B_NODE) {
+        if (l.global_tw) dispatch_bwd2d<T, 31, false>(l.kind, a, t, lds, 0, 1);
+        else dispatch_bwd2d<T, 31>(l.kind, a, t, lds, 0, 1);
+    } else {
+        if (l.global_tw) dispatch_body2d<T, 31, false>(l.kind, a, t, lds, 0, 1);
+        else dispatch_body2d<T, 31>(l.kind, a, t, lds, 0, 1);
+    }
+}
+
+// Placement of a plan: info = {LDS bytes of its largest launch, big nodes,
+// launches with twiddles in global memory, workspace bytes per image, those of
+// the launches that are nodes}.
+template <class T>
+static int emu_plan2d(int M, int N, int J, int L, long long lds_limit, const int* tune, int ntune, long long* info) {
+    Scat2DPlan<T> p;
+    int* fields[7] = {&p.tune.max_pow2, &p.tune.node_threads, &p.tune.col_block, &p.tune.row_block,
+                      &p.tune.pass_threads, &p.tune.streams, &p.tune.pair};
+    for (int i = 0; i < ntune && i < 7; ++i)
+        if (tune[i] != 0) *fields[i] = tune[i];
+    KymError e = {0, ""};
+    if (!p.build(M, N, J, L, 2, 0, (size_t)lds_limit, &e)) {
+        g_emu_error = e.msg;
+        return e.code;
+    }
+    info[0] = info[1] = info[2] = info[4] = 0;
+    for (const std::vector<Launch2D>* ls : {&p.launches, &p.bwd_launches})
+        for (const Launch2D& l : *ls) {
+            info[0] = std::max(info[0], (long long)l.lds_bytes);
+            info[2] += l.global_tw;
+            info[4] += l.global_tw && (l.kind == K2_LDS_NODE || l.kind == K2B_NODE);
+        }
+    for (const Node2D& nd : p.nodes) info[1] += nd.big;
+    info[3] = p.ws_img * (long long)sizeof(cpx<T>);
+    return 0;
+}
+
+extern "C" int kym_emu_scat2d_plan(int M, int N, int J, int L, int dtype, long long lds_limit, const int* tune,
+                                   int ntune, long long* info) {
+    if (dtype == 0) return emu_plan2d<float>(M, N, J, L, lds_limit, tune, ntune, info);
+    return emu_plan2d<double>(M, N, J, L, lds_limit, tune, ntune, info);
+}
+
 template <class T>
 static int emu_forward2d(int M, int N, int J, int L, int max_order, int pre_pad, long long lds_limit, const void* x,
                          const void* filt, void* out, long long batch, long long chunk, long long* info,
@@ -84,7 +129,7 @@ static int emu_forward2d(int M, int N, int J, int L, int max_order, int pre_pad,
             a.ntask = nimg * l.ngroup * l.nblk;
             for (int t = 0; t < a.ntask; ++t) {
                 if (l.spec >= 0) emu_spec(l, a, t, lds.data());
-                else dispatch_body2d<T, 31>(l.kind, a, t, lds.data(), 0, 1);
+                else emu_body(l, a, t, lds.data());
             }
         }
     }
@@ -135,9 +180,8 @@ static int emu_train2d(int M, int N, int J, int L, int max_order, int pre_pad, l
                     dispatch_bwd_pass_spec<T, K2B_GROWS, true>(l.spec, a, t, lds.data(), 0);
                 else if (l.kind == K2B_GFCOLS && l.spec >= 0)
                     dispatch_bwd_pass_spec<T, K2B_GFCOLS, true>(l.spec, a, t, lds.data(), 0);
-                else if (l.kind >= K2B_NODE) dispatch_bwd2d<T, 31>(l.kind, a, t, lds.data(), 0, 1);
-                else if (l.spec >= 0) emu_spec(l, a, t, lds.data());
-                else dispatch_body2d<T, 31>(l.kind, a, t, lds.data(), 0, 1);
+                else if (l.kind < K2B_NODE && l.spec >= 0) emu_spec(l, a, t, lds.data());
+                else emu_body(l, a, t, lds.data());
             }
         }
     }

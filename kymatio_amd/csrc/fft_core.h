@@ -355,6 +355,9 @@ KYM_HD KYM_INL int kym_prime_class(int maxp) { return maxp <= 7 ? 7 : maxp <= 17
 // 725 -> 318, 16 x 220^2 (29) 1149 -> 528, 16 x 235^2 (31) 1306 -> 616, FP64
 // 4 x 141^2 676 -> 292; 16 x 136x170 (19 and 23, every radix, large ones in
 // functions) 495 -> 353.
+// KYM_GLOBAL_TW + 7, 17 or 31: the kernels that read their twiddles from global
+// memory, for the few sizes whose data leaves no room in LDS.
+#define KYM_GLOBAL_TW 200
 inline int kym_plan_class(int a, int b) {
     int only = 0, maxp = 1;
     for (int v : {a, b})

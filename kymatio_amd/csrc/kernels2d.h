@@ -11,14 +11,14 @@ __device__ KYM_INL int xcd_task(int bid, int nblocks) {
     return (bid & 7) * per + (bid >> 3);
 }
 
-template <class T, int KIND, int NT, int MAXP>
+template <class T, int KIND, int NT, int MAXP, bool TWL = true>
 __global__ void __launch_bounds__(NT, 2) k_scat2d(Scat2DArgs<T> a) {
     extern __shared__ __attribute__((aligned(16))) char kym_smem2d[];
     const int task = xcd_task(blockIdx.x, gridDim.x);
     if (task >= live_tasks(a)) return;
     cpx<T>* lds = reinterpret_cast<cpx<T>*>(kym_smem2d);
-    if constexpr (KIND >= K2B_NODE) dispatch_bwd2d<T, MAXP>(KIND, a, task, lds, threadIdx.x, NT);
-    else dispatch_body2d<T, MAXP>(KIND, a, task, lds, threadIdx.x, NT);
+    if constexpr (KIND >= K2B_NODE) dispatch_bwd2d<T, MAXP, TWL>(KIND, a, task, lds, threadIdx.x, NT);
+    else dispatch_body2d<T, MAXP, TWL>(KIND, a, task, lds, threadIdx.x, NT);
 }
 
 template <class T, int SPEC, int NT>
@@ -129,6 +129,24 @@ Scat2DKernel<T> pick_scat2d_p(int kind, int threads) {
         case K2B_GROWS: return k_scat2d<T, K2B_GROWS, 256, MAXP>;
         case K2B_GFCOLS: return k_scat2d<T, K2B_GFCOLS, 256, MAXP>;
         case K2B_FOLD: return k_scat2d<T, K2B_FOLD, 256, MAXP>;
+        default: return nullptr;
+    }
+}
+
+// The kernels of launches whose LDS has no room for the twiddles
+// (Launch2D::global_tw); nodes on 1024 threads only.
+template <class T, int MAXP>
+Scat2DKernel<T> pick_scat2d_global_tw(int kind, int threads) {
+    switch (kind) {
+        case K2_LDS_NODE: return threads == 1024 ? k_scat2d<T, K2_LDS_NODE, 1024, MAXP, false> : nullptr;
+        case K2_ROOT_ROWS: return k_scat2d<T, K2_ROOT_ROWS, 256, MAXP, false>;
+        case K2_ICOL: return k_scat2d<T, K2_ICOL, 256, MAXP, false>;
+        case K2_ROWS_MOD: return k_scat2d<T, K2_ROWS_MOD, 256, MAXP, false>;
+        case K2_FWD_COLS: return k_scat2d<T, K2_FWD_COLS, 256, MAXP, false>;
+        case K2B_NODE: return threads == 1024 ? k_scat2d<T, K2B_NODE, 1024, MAXP, false> : nullptr;
+        case K2B_GCOLS: return k_scat2d<T, K2B_GCOLS, 256, MAXP, false>;
+        case K2B_GROWS: return k_scat2d<T, K2B_GROWS, 256, MAXP, false>;
+        case K2B_GFCOLS: return k_scat2d<T, K2B_GFCOLS, 256, MAXP, false>;
         default: return nullptr;
     }
 }

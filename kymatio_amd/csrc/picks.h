@@ -14,6 +14,9 @@ Scat2DKernel<float> kym_pick2d_f32_p119(int kind, int threads);
 Scat2DKernel<float> kym_pick2d_f32_p123(int kind, int threads);
 Scat2DKernel<float> kym_pick2d_f32_p129(int kind, int threads);
 Scat2DKernel<float> kym_pick2d_f32_p131(int kind, int threads);
+Scat2DKernel<float> kym_pick2d_f32_g7(int kind, int threads);
+Scat2DKernel<float> kym_pick2d_f32_g17(int kind, int threads);
+Scat2DKernel<float> kym_pick2d_f32_g31(int kind, int threads);
 Scat2DKernel<double> kym_pick2d_f64_p7(int kind, int threads);
 Scat2DKernel<double> kym_pick2d_f64_p17(int kind, int threads);
 Scat2DKernel<double> kym_pick2d_f64_p31(int kind, int threads);
@@ -21,6 +24,9 @@ Scat2DKernel<double> kym_pick2d_f64_p119(int kind, int threads);
 Scat2DKernel<double> kym_pick2d_f64_p123(int kind, int threads);
 Scat2DKernel<double> kym_pick2d_f64_p129(int kind, int threads);
 Scat2DKernel<double> kym_pick2d_f64_p131(int kind, int threads);
+Scat2DKernel<double> kym_pick2d_f64_g7(int kind, int threads);
+Scat2DKernel<double> kym_pick2d_f64_g17(int kind, int threads);
+Scat2DKernel<double> kym_pick2d_f64_g31(int kind, int threads);
 Scat2DKernel<float> kym_pick_node_spec_f32(int id);
 Scat2DKernel<float> kym_pick_bwd_node_spec_f32(int id);
 Scat2DKernel<float> kym_pick_pass_spec_f32(int kind, int id);
@@ -30,7 +36,7 @@ Scat1DKernel<float> kym_pick_bwd_node1d_spec_f32(int id);
 Scat1DKernel<float> kym_pick_any1d_f32(int kind);
 Scat1DKernel<double> kym_pick1d_f64(int threads, int kind);
 
-// pclass: 7, 17, 31 or 100 + p (kym_plan_class);
+// pclass: 7, 17, 31 or 100 + p (kym_plan_class), or KYM_GLOBAL_TW + 7, 17 or 31;
 // spec >= 0 selects a compile-time specialisation of the node or pass kernel.
 template <class T>
 inline Scat2DKernel<T> pick_scat2d(int kind, int threads, int pclass, int spec = -1) {
@@ -42,6 +48,9 @@ inline Scat2DKernel<T> pick_scat2d(int kind, int threads, int pclass, int spec =
         case 123: return kym_pick2d_##tag##_p123(kind, threads);              \
         case 129: return kym_pick2d_##tag##_p129(kind, threads);              \
         case 131: return kym_pick2d_##tag##_p131(kind, threads);              \
+        case KYM_GLOBAL_TW + 7: return kym_pick2d_##tag##_g7(kind, threads);  \
+        case KYM_GLOBAL_TW + 17: return kym_pick2d_##tag##_g17(kind, threads); \
+        case KYM_GLOBAL_TW + 31: return kym_pick2d_##tag##_g31(kind, threads); \
         default: return kym_pick2d_##tag##_p31(kind, threads);                \
     }
     if constexpr (sizeof(T) == 4) {

@@ -578,7 +578,9 @@ KYM_HD KYM_INL T fir_sum(const T* src, int stride, int n, int base, const T* c, 
 // registers (see stage_modulus): the plan keeps H W <= KYM_STAGE_MAX * threads.
 #define KYM_STAGE_MAX 20
 
-template <class T, int MAXP>
+// TWL: the twiddles of H and W are in LDS (twH, twW), else the transforms read
+// FftLen::ptw (nodes whose field leaves no room for the tables).
+template <class T, int MAXP, bool TWL>
 struct DynGeom {
     static constexpr int STAGE = KYM_STAGE_MAX;
     // modulus / restaging as separate sweeps (stage_modulus, restage_complex)
@@ -588,7 +590,6 @@ struct DynGeom {
     const FftLen<T>* fW;
     const FftLen<T>* fHJ;
     const FftLen<T>* fWJ;
-    // twiddle tables of H and W in LDS (load_twiddles)
     const cpx<T>* twH;
     const cpx<T>* twW;
     KYM_HD const int* revH() const { return fH->rev; }
@@ -598,12 +599,12 @@ struct DynGeom {
     KYM_HD int rh(int p) const { return kym_ldg(fH->rev + p); }
     KYM_HD int rw(int p) const { return kym_ldg(fW->rev + p); }
     KYM_HD KYM_INL void inv2d(cpx<T>* b, int tid, int nth) const {
-        fft_dif<true, MAXP, true>(b, *fW, Batch{H, 1, W, false}, tid, nth, twW);
-        fft_dif<true, MAXP, true>(b, *fH, Batch{W, W, 1, true}, tid, nth, twH);
+        fft_dif<true, MAXP, TWL>(b, *fW, Batch{H, 1, W, false}, tid, nth, twW);
+        fft_dif<true, MAXP, TWL>(b, *fH, Batch{W, W, 1, true}, tid, nth, twH);
     }
     KYM_HD KYM_INL void fwd2d(cpx<T>* b, int tid, int nth) const {
-        fft_dit<false, MAXP, true>(b, *fW, Batch{H, 1, W, false}, tid, nth, twW);
-        fft_dit<false, MAXP, true>(b, *fH, Batch{W, W, 1, true}, tid, nth, twH);
+        fft_dit<false, MAXP, TWL>(b, *fW, Batch{H, 1, W, false}, tid, nth, twW);
+        fft_dit<false, MAXP, TWL>(b, *fH, Batch{W, W, 1, true}, tid, nth, twH);
     }
     KYM_HD KYM_INL void leaf_inv2d(cpx<T>* b, int tid, int nth) const {
         fft_dif<true, MAXP>(b, *fWJ, Batch{HJ, 1, WJ, false}, tid, nth);
@@ -1155,27 +1156,29 @@ KYM_HD KYM_INL void load_twiddles(cpx<T>* tw, const FftLen<T>* fh, const FftLen<
     wg_barrier();
 }
 
-// tw: LDS for the twiddles of the node's sizes (nullptr: a body that
-// transforms leaves only).
-template <class T, int MAXP>
-KYM_HD DynGeom<T, MAXP> dyn_geom(const Scat2DArgs<T>& a, int r, cpx<T>* tw, int tid, int nth) {
+// tw (TWL): LDS for the twiddles of the node's sizes.
+template <class T, int MAXP, bool TWL>
+KYM_HD DynGeom<T, MAXP, TWL> dyn_geom(const Scat2DArgs<T>& a, int r, cpx<T>* tw, int tid, int nth) {
     const int J = a.J;
     const FftLen<T>* fH = &a.lens[a.lenH[r]];
     const FftLen<T>* fW = &a.lens[a.lenW[r]];
     const FftLen<T>* fHJ = &a.lens[a.lenH[J]];
     const FftLen<T>* fWJ = &a.lens[a.lenW[J]];
-    if (tw) load_twiddles(tw, fH, fW, fH->n, fW->n, tid, nth);
-    return DynGeom<T, MAXP>{fH->size(), fW->size(), fHJ->size(), fWJ->size(), fH, fW, fHJ, fWJ,
-                            tw + (fH->n != fW->n ? fW->n : 0), tw};
+    const cpx<T>* twH = nullptr;
+    if constexpr (TWL) {
+        load_twiddles(tw, fH, fW, fH->n, fW->n, tid, nth);
+        twH = tw + (fH->n != fW->n ? fW->n : 0);
+    }
+    return DynGeom<T, MAXP, TWL>{fH->size(), fW->size(), fHJ->size(), fWJ->size(), fH, fW, fHJ, fWJ, twH, tw};
 }
 
-// A whole node in LDS (after its twiddles).  task -> (image of chunk, node of group).
-template <class T, int MAXP>
+// A whole node in LDS (TWL: after its twiddles).  task -> (image of chunk, node of group).
+template <class T, int MAXP, bool TWL>
 KYM_HD KYM_INL void body_lds_node(const Scat2DArgs<T>& a, int task, cpx<T>* lds, int tid, int nth) {
     const int il = task / a.ngroup, gi = task - il * a.ngroup;
     const Node2D& nd = a.nodes[a.group[gi]];
-    const auto g = dyn_geom<T, MAXP>(a, nd.res, lds, tid, nth);
-    node_body(a, g, nd, il, lds + kym_tw_elems(g.H, g.W), tid, nth);
+    const auto g = dyn_geom<T, MAXP, TWL>(a, nd.res, lds, tid, nth);
+    node_body(a, g, nd, il, lds + (TWL ? kym_tw_elems(g.H, g.W) : 0), tid, nth);
 }
 
 // The same with compile-time sizes (the plan only selects it when the
@@ -1305,7 +1308,7 @@ KYM_HD void body_leaf(const Scat2DArgs<T>& a, int task, cpx<T>* lds, int tid, in
     const int r = nd.res;
     const cpx<T>* U = a.ws + il * a.ws_img + nd.slot;
     const T* phi = a.filt + a.filt_off[nd.leaf_filt];
-    leaf_body(a, dyn_geom<T, MAXP>(a, r, nullptr, tid, nth), U, phi, nd.leaf_k, nd.leaf_ch, a.img0 + il, lds, tid, nth);
+    leaf_body(a, dyn_geom<T, MAXP, false>(a, r, nullptr, tid, nth), U, phi, nd.leaf_k, nd.leaf_ch, a.img0 + il, lds, tid, nth);
 }
 
 // ------------------------------------------------------------------ pass FFTs
@@ -1847,31 +1850,39 @@ KYM_HD KYM_INL int pass_twiddles(const Scat2DArgs<T>& a, cpx<T>* lds, int tid, i
     return pass_tw_elems(f.n);
 }
 
-template <class T, int MAXP>
+// The pass with or without its twiddles in LDS (COLS: of H, else of W).
+template <bool TWL, bool COLS, class T, int MAXP, class F>
+KYM_HD KYM_INL void with_dyn_pass(const Scat2DArgs<T>& a, cpx<T>* lds, int tid, int nth, F body) {
+    const int n = TWL ? pass_twiddles<COLS>(a, lds, tid, nth) : 0;
+    body(DynPass<T, MAXP, TWL>{TWL ? lds : nullptr}, lds + n);
+}
+
+// TWL: the launch's LDS holds the twiddles of its sizes (Launch2D::global_tw).
+template <class T, int MAXP, bool TWL = true>
 KYM_HD KYM_INL void dispatch_body2d(int kind, const Scat2DArgs<T>& a, int task, cpx<T>* lds, int tid, int nth) {
     switch (kind) {
-        case K2_LDS_NODE: body_lds_node<T, MAXP>(a, task, lds, tid, nth); break;
+        case K2_LDS_NODE: body_lds_node<T, MAXP, TWL>(a, task, lds, tid, nth); break;
         case K2_LEAF: body_leaf<T, MAXP>(a, task, lds, tid, nth); break;
-        case K2_ROOT_ROWS: {
-            const int n = pass_twiddles<false>(a, lds, tid, nth);
-            body_root_rows<T>(DynPass<T, MAXP, true>{lds}, a, task, lds + n, tid, nth);
+        case K2_ROOT_ROWS:
+            with_dyn_pass<TWL, false, T, MAXP>(a, lds, tid, nth, [&](auto fp, cpx<T>* l) {
+                body_root_rows<T>(fp, a, task, l, tid, nth);
+            });
             break;
-        }
-        case K2_ICOL: {
-            const int n = pass_twiddles<true>(a, lds, tid, nth);
-            body_icol<T>(DynPass<T, MAXP, true>{lds}, a, task, lds + n, tid, nth);
+        case K2_ICOL:
+            with_dyn_pass<TWL, true, T, MAXP>(a, lds, tid, nth, [&](auto fp, cpx<T>* l) {
+                body_icol<T>(fp, a, task, l, tid, nth);
+            });
             break;
-        }
-        case K2_ROWS_MOD: {
-            const int n = pass_twiddles<false>(a, lds, tid, nth);
-            body_rows_mod<T>(DynPass<T, MAXP, true>{lds}, a, task, lds + n, tid, nth);
+        case K2_ROWS_MOD:
+            with_dyn_pass<TWL, false, T, MAXP>(a, lds, tid, nth, [&](auto fp, cpx<T>* l) {
+                body_rows_mod<T>(fp, a, task, l, tid, nth);
+            });
             break;
-        }
-        case K2_FWD_COLS: {
-            const int n = pass_twiddles<true>(a, lds, tid, nth);
-            body_fwd_cols<T>(DynPass<T, MAXP, true>{lds}, a, task, lds + n, tid, nth);
+        case K2_FWD_COLS:
+            with_dyn_pass<TWL, true, T, MAXP>(a, lds, tid, nth, [&](auto fp, cpx<T>* l) {
+                body_fwd_cols<T>(fp, a, task, l, tid, nth);
+            });
             break;
-        }
         case K2_LEAF_ICOL: body_leaf_icol<T, MAXP>(a, task, lds, tid, nth); break;
         case K2_LEAF_ROWS: body_leaf_rows<T, MAXP>(a, task, lds, tid, nth); break;
         case K2_FIR_COLS: body_fir_cols<T, MAXP>(a, task, lds, tid, nth); break;

@@ -320,12 +320,12 @@ KYM_HD KYM_INL void bwd_node_body(const Scat2DArgs<T>& a, const G& g, const Node
     for (int i = tid; i < n; i += nth) gs[i] = lds[i] * inv_n;
 }
 
-template <class T, int MAXP>
-KYM_HD void body_bwd_node(const Scat2DArgs<T>& a, int task, cpx<T>* lds, int tid, int nth) {
+template <class T, int MAXP, bool TWL>
+KYM_HD KYM_INL void body_bwd_node(const Scat2DArgs<T>& a, int task, cpx<T>* lds, int tid, int nth) {
     const int il = task / a.ngroup, gi = task - il * a.ngroup;
     const Node2D& nd = a.nodes[a.group[gi]];
-    const auto g = dyn_geom<T, MAXP>(a, nd.res, lds, tid, nth);
-    bwd_node_body(a, g, nd, il, lds + kym_tw_elems(g.H, g.W), tid, nth);
+    const auto g = dyn_geom<T, MAXP, TWL>(a, nd.res, lds, tid, nth);
+    bwd_node_body(a, g, nd, il, lds + (TWL ? kym_tw_elems(g.H, g.W) : 0), tid, nth);
 }
 
 // A node's backward with compile-time sizes (FP32): twiddles of both lengths
@@ -370,7 +370,7 @@ template <class T, int MAXP>
 KYM_HD void body_bwd_leafg(const Scat2DArgs<T>& a, int task, cpx<T>* lds, int tid, int nth) {
     const int il = task / a.ngroup, gi = task - il * a.ngroup;
     const Node2D& nd = a.nodes[a.group[gi]];
-    const auto g = dyn_geom<T, MAXP>(a, nd.res, nullptr, tid, nth);
+    const auto g = dyn_geom<T, MAXP, false>(a, nd.res, nullptr, tid, nth);
     leaf_grad(a, g, nd, a.img0 + il, lds, tid, nth);
     cpx<T>* dst = a.ws + il * a.ws_img + nd.gslot;
     for (int i = tid; i < g.HJ * g.WJ; i += nth) dst[i] = lds[i];
@@ -547,26 +547,26 @@ KYM_HD void body_bwd_fold(const Scat2DArgs<T>& a, int task, cpx<T>* lds, int tid
 
 enum Kind2DBwd { K2B_NODE = 16, K2B_LEAFG, K2B_GCOLS, K2B_GROWS, K2B_GFCOLS, K2B_FOLD };
 
-template <class T, int MAXP>
+template <class T, int MAXP, bool TWL = true>
 KYM_HD KYM_INL void dispatch_bwd2d(int kind, const Scat2DArgs<T>& a, int task, cpx<T>* lds, int tid, int nth) {
     switch (kind) {
-        case K2B_NODE: body_bwd_node<T, MAXP>(a, task, lds, tid, nth); break;
+        case K2B_NODE: body_bwd_node<T, MAXP, TWL>(a, task, lds, tid, nth); break;
         case K2B_LEAFG: body_bwd_leafg<T, MAXP>(a, task, lds, tid, nth); break;
-        case K2B_GCOLS: {
-            const int n = pass_twiddles<true>(a, lds, tid, nth);
-            body_bwd_gcols<T>(DynPass<T, MAXP, true>{lds}, a, task, lds + n, tid, nth);
+        case K2B_GCOLS:
+            with_dyn_pass<TWL, true, T, MAXP>(a, lds, tid, nth, [&](auto fp, cpx<T>* l) {
+                body_bwd_gcols<T>(fp, a, task, l, tid, nth);
+            });
             break;
-        }
-        case K2B_GROWS: {
-            const int n = pass_twiddles<false>(a, lds, tid, nth);
-            body_bwd_grows<T>(DynPass<T, MAXP, true>{lds}, a, task, lds + n, tid, nth);
+        case K2B_GROWS:
+            with_dyn_pass<TWL, false, T, MAXP>(a, lds, tid, nth, [&](auto fp, cpx<T>* l) {
+                body_bwd_grows<T>(fp, a, task, l, tid, nth);
+            });
             break;
-        }
-        case K2B_GFCOLS: {
-            const int n = pass_twiddles<true>(a, lds, tid, nth);
-            body_bwd_gfcols<T>(DynPass<T, MAXP, true>{lds}, a, task, lds + n, tid, nth);
+        case K2B_GFCOLS:
+            with_dyn_pass<TWL, true, T, MAXP>(a, lds, tid, nth, [&](auto fp, cpx<T>* l) {
+                body_bwd_gfcols<T>(fp, a, task, l, tid, nth);
+            });
             break;
-        }
         case K2B_FOLD: body_bwd_fold<T, MAXP>(a, task, lds, tid, nth); break;
         default: break;
     }

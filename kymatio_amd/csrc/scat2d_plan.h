@@ -19,6 +19,7 @@ struct Launch2D {
     long long model_bytes;  // algorithmic HBM bytes per image (stage-boundary model)
     int spec;               // compile-time specialisation id, -1 = run-time sizes
     int pclass = 7;         // radix family of the kernel (kym_plan_class)
+    bool global_tw = false; // no room for the twiddles beside the data: read from global memory
     int pair = 0;           // 1: a task is a sibling pair (group lists 2 ngroup node ids)
     // small LDS nodes: threads (and specialisation) of a launch of more than
     // many_tasks workgroups, 0 = the same
@@ -289,6 +290,7 @@ struct Scat2DPlan {
             }
             return b;
         };
+        const bool wide_nodes = tune.node_threads == 0 || tune.node_threads == 1024;
         ws_img = 0;
         for (size_t i = 0; i < nodes.size(); ++i) {
             Node2D& nd = nodes[i];
@@ -302,9 +304,17 @@ struct Scat2DPlan {
                 specs && sizeof(T) == 4 &&
                 node_spec_id(H[nd.res], W[nd.res], H[J], W[J], node_threads(elems), &spec_threads, 0) >= 0 &&
                 node_lds(nd) + cs * kym_tw_elems(H[nd.res], W[nd.res]) <= lds_limit;
-            const size_t tw = cs * kym_tw_elems(H[nd.res], W[nd.res]);
+            // a field that fits the LDS by itself reads its twiddles from global
+            // memory, on 1024 threads, where a launch holds the first and the second
+            // order: 16 images of 144 x 488 J=3, 128 x 160 nodes, 825 us as passes,
+            // 531 so.  The first order alone, 8 nodes an image, leaves CUs idle that
+            // passes fill: 16 of 112 x 144 J=3 177 us as passes, 191 so.
+            const bool wide = wide_nodes && nd.res > 0 && max_order == 2;
+            const size_t tw = wide ? 0 : cs * kym_tw_elems(H[nd.res], W[nd.res]);
             const bool fits = node_lds(nd) + tw <= lds_limit &&
-                              (!fir || elems <= (size_t)KYM_STAGE_MAX * node_threads(elems) || spec_fit);
+                              (!fir || elems <= (size_t)KYM_STAGE_MAX * node_threads(elems) || spec_fit ||
+                               (wide && node_lds(nd) + cs * kym_tw_elems(H[nd.res], W[nd.res]) > lds_limit &&
+                                elems <= (size_t)KYM_STAGE_MAX * 1024));
             if (fits) { nd.big = 0; nd.leaf_mode = ((elems + leaf_elems) * cs + tw <= lds_limit) ? 0 : 1; }
             else { nd.big = 1; nd.leaf_mode = (leaf_elems * cs <= lds_limit) ? 1 : 2; }
             nd.fir = fir ? (nd.big ? 2 : 1) : 0;
@@ -379,7 +389,7 @@ struct Scat2DPlan {
         const size_t medium = sizeof(T) == 4 ? KYM_STAGE_MAX * 256 : 4095;
         auto many_waves = [&](Launch2D& l) {
             const size_t elems = (size_t)H[l.res] * W[l.res];
-            if (tune.node_threads || l.pair) return;
+            if (tune.node_threads || l.pair || l.global_tw) return;
             if (l.spec < 0 && elems >= 2048 && elems <= medium) {
                 l.many_threads = 256;
                 l.many_tasks = KYM_MANY_MEDIUM;
@@ -443,6 +453,17 @@ struct Scat2DPlan {
             launches.push_back(l);
             max_lds = std::max(max_lds, lds);
             max_threads = std::max(max_threads, threads);
+        };
+        // `tw` bytes of twiddles in front of the last launch's `lds` bytes, or,
+        // where they don't fit, the kernels that read them from global memory
+        auto add_twiddles = [&](size_t lds, size_t tw) {
+            Launch2D& l = launches.back();
+            l.global_tw = lds + tw > lds_limit;
+            l.lds_bytes = l.global_tw ? lds : lds + tw;
+            if (l.global_tw) l.pclass = KYM_GLOBAL_TW + (l.pclass > 100 ? 31 : l.pclass);
+            if (l.global_tw && (l.kind == K2_LDS_NODE || l.kind == K2B_NODE)) l.threads = 1024;
+            max_lds = std::max(max_lds, l.lds_bytes);
+            max_threads = std::max(max_threads, l.threads);
         };
         const size_t pass_budget = std::min(lds_limit, (size_t)64 * 1024);
         bool no_pass_spec = false;  // a tuned pass thread count with no compiled kernel
@@ -541,10 +562,12 @@ struct Scat2DPlan {
                         return;
                     }
                 }
-                push(K2_LDS_NODE, ids, 1, 0, node_threads(elems), lds + cs * kym_tw_elems(H[r], W[r]));
+                push(K2_LDS_NODE, ids, 1, 0, node_threads(elems), 0);
+                add_twiddles(lds, cs * kym_tw_elems(H[r], W[r]));
                 int nt = 0;
                 const int sid = node_spec_id(H[r], W[r], H[J], W[J], tune.node_threads, &nt, 0);
-                if (specs && sizeof(T) == 4 && sid >= 0 && (n0.fir == 1 || n0.leaf_mode == 0)) {
+                if (specs && sizeof(T) == 4 && sid >= 0 && (n0.fir == 1 || n0.leaf_mode == 0) &&
+                    !launches.back().global_tw) {
                     launches.back().spec = sid;
                     launches.back().threads = nt;
                 }
@@ -567,7 +590,8 @@ struct Scat2DPlan {
                 if (tune.pass_threads && tune.pass_threads != 256 && psid < 0) no_pass_spec = true;
                 auto pass = [&](int kind, int nblk, int blk, size_t lds) {
                     const bool cols = kind == K2_ICOL || kind == K2_FWD_COLS;
-                    push(kind, ids, nblk, blk, 256, lds + cs * pass_tw_elems(cols ? H[r] : W[r]));
+                    push(kind, ids, nblk, blk, 256, 0);
+                    add_twiddles(lds, cs * pass_tw_elems(cols ? H[r] : W[r]));
                     const size_t tw = cs * kym_tw_elems(H[r], W[r]);
                     if (psid >= 0 && lds + tw <= lds_limit) {
                         launches.back().spec = psid;
@@ -663,11 +687,12 @@ struct Scat2DPlan {
             if (!leafg.empty()) push(K2B_LEAFG, leafg, 1, 0, node_threads(leaf_elems), leaf_elems * cs);
             if (!n0.big) {
                 const size_t lds = (elems + (n0.leaf_mode == 0 ? leaf_elems : 0)) * cs;
-                push(K2B_NODE, ids, 1, 0, node_threads(elems), lds + cs * kym_tw_elems(H[r], W[r]));
+                push(K2B_NODE, ids, 1, 0, node_threads(elems), 0);
+                add_twiddles(lds, cs * kym_tw_elems(H[r], W[r]));
                 // compile-time sizes as in the forward (one node per workgroup)
                 int nt = 0;
                 const int sid = node_spec_id(H[r], W[r], H[J], W[J], tune.node_threads, &nt, 0);
-                if (specs && sizeof(T) == 4 && sid >= 0) {
+                if (specs && sizeof(T) == 4 && sid >= 0 && !launches.back().global_tw) {
                     launches.back().spec = sid;
                     launches.back().threads = nt;
                 }
@@ -695,7 +720,8 @@ struct Scat2DPlan {
                     if (psid < 0 && !tune.col_block && !tune.row_block && (psid = spec_for(8, 8)) >= 0) cb = rb = 8;
                 }
                 auto bpass = [&](int kind, int nblk, int blk, size_t lds) {
-                    push(kind, ids, nblk, blk, 256, lds + cs * pass_tw_elems(kind == K2B_GROWS ? W[r] : H[r]));
+                    push(kind, ids, nblk, blk, 256, 0);
+                    add_twiddles(lds, cs * pass_tw_elems(kind == K2B_GROWS ? W[r] : H[r]));
                     const size_t tw = cs * kym_tw_elems(H[r], W[r]);
                     if (psid >= 0 && lds + tw <= lds_limit) {
                         launches.back().spec = psid;

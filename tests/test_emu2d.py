@@ -164,3 +164,54 @@ def test_fold_pass_matches_gathers(emu, shape, J, L, dt):
     assert rc == 0
     # k^2 <= 256 products per point in another order: sqrt(256) eps of the largest term
     assert channel_rel_err(out, ref) < (1e-5 if dt == np.float32 else 1e-13)
+
+
+def _placement(emu, shape, J, L, dt, lds_limit=160 * 1024, tune=()):
+    info = (ctypes.c_longlong * 5)()
+    t = (ctypes.c_int * 7)(*tune)
+    rc = emu.lib.kym_emu_scat2d_plan(shape[0], shape[1], J, L, 0 if dt == np.float32 else 1,
+                                     ctypes.c_longlong(lds_limit), t, len(tune), info)
+    assert rc == 0, emu.lib.kym_emu_last_error().decode()
+    return dict(zip(('lds', 'big', 'global_tw', 'ws', 'global_tw_nodes'), info))
+
+
+@pytest.mark.parametrize('shape,J,dt,tune,big', [
+    ((16, 8192), 3, np.float32, (), None), ((16, 9000), 3, np.float32, (), None),  # one row and its table: 175, 191 KB
+    ((20, 9228), 4, np.float64, (), None),
+    ((512, 512), 6, np.float32, (16, 0, 32), None), ((256, 256), 5, np.float32, (16, 0, 64), None),
+    ((300, 300), 3, np.float64, (16, 0, 32, 32), None),
+    # nodes that fill the LDS by themselves stay in one workgroup, but for those of resolution 0
+    ((144, 488), 3, np.float32, (), 9), ((96, 384), 2, np.float64, (), 9),
+    ((72, 440), 3, np.float64, (), 9)])
+def test_launches_fit_the_workgroup(emu, shape, J, dt, tune, big):
+    """Every launch stays within the LDS, twiddles included."""
+    p = _placement(emu, shape, J, 8, dt, tune=tune)
+    assert p['lds'] <= 160 * 1024
+    assert p['global_tw'] > 0
+    assert big is None or p['big'] == big
+
+
+@pytest.mark.parametrize('shape,J,L,dt,limits', [
+    ((40, 40), 3, 3, np.float32, (8840, 7608)), ((20, 24), 2, 3, np.float64, (8696, 4952)),
+    ((33, 31), 3, 2, np.float32, (6744, 6520)), ((45, 30), 1, 2, np.float64, (9240,))])
+def test_twiddles_in_global_memory(emu, shape, J, L, dt, limits):
+    """Launches whose LDS has no room for their twiddles, nodes and passes,
+    forward and backward, against the default placement."""
+    from tests.helpers import emu_train2d
+    _, f = _filters(shape, J, L, dt)
+    rng = np.random.default_rng(J)
+    x = rng.standard_normal((2,) + shape).astype(dt)
+    ref, _ = emu.scat2d(x, J, shape, f, L=L)
+    w = rng.standard_normal(ref.shape).astype(dt)
+    _, gref = emu_train2d(emu, x, J, shape, f, w, L=L)
+    eps = 1e-5 if dt == np.float32 else 1e-12
+    nodes = passes = 0
+    for lim in limits:
+        p = _placement(emu, shape, J, L, dt, lim)
+        assert p['global_tw'] and p['lds'] <= lim
+        nodes += p['global_tw_nodes']
+        passes += p['global_tw'] - p['global_tw_nodes']
+        out, gx = emu_train2d(emu, x, J, shape, f, w, L=L, lds_limit=lim, nbwd=2)
+        assert channel_rel_err(out, ref) <= eps
+        assert np.abs(gx - gref).max() <= eps * np.abs(gref).max()
+    assert passes and (nodes or J == 1)

@@ -260,3 +260,28 @@ def test_streams_either_side_of_the_line(B):
         # the same butterflies, possibly spread over other threads
         for a, b, tol in zip(r, res[0], (1e-6, 1e-5, 1e-6)):
             assert (a - b).abs().max() <= tol * b.abs().max()
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float64])
+@pytest.mark.parametrize('shape,J,lds', [((16, 8192), 3, 0), ((144, 488), 3, 0), ((72, 440), 3, 0), ((96, 384), 2, 0),
+                                         ((40, 40), 3, 8840), ((40, 40), 3, 7608), ((20, 24), 2, 8696),
+                                         ((20, 24), 2, 4952), ((33, 31), 3, 6520), ((45, 30), 1, 9240)])
+def test_data_that_fills_the_lds(shape, J, lds, dtype):
+    """Lines and nodes that leave no room in LDS for their twiddles (in one
+    type or the other), forward and gradient, against the FP64 oracle."""
+    sc = Scattering2D(J, shape, L=2).to(dtype).to(DEV)
+    sc.lds_limit = lds
+    ref = scat2d.Scattering2DTorchCPU(J, shape, L=2, dtype=torch.float64)
+    x = torch.randn((2,) + shape, generator=torch.Generator().manual_seed(J)).to(dtype)
+    xr = x.double().requires_grad_()
+    want = ref(xr)
+    w = torch.randn(want.shape, dtype=torch.float64, generator=torch.Generator().manual_seed(1)).to(dtype)
+    gw, = torch.autograd.grad((want * w.double()).sum(), xr)
+    xg = x.to(DEV).requires_grad_()
+    got = sc(xg)
+    gx, = torch.autograd.grad((got * w.to(DEV)).sum(), xg)
+    tol = RTOL_CHANNEL if dtype == torch.float32 else 1e-12
+    assert channel_rel_err(got.detach().cpu().numpy(), want.detach().numpy()) <= tol
+    if dtype == torch.float32 and shape == (16, 8192):
+        return  # some |u| of so many is small enough that u / |u| has three digits in FP32, in plain torch too
+    assert (gx.cpu().double() - gw).abs().max() <= (1e-5 if dtype == torch.float32 else 1e-11) * gw.abs().max()
