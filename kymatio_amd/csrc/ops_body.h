@@ -332,8 +332,13 @@ inline int filter_ifft_spec_id(int n, long long batch, const FilterIfftArgs& o, 
 
 // LDS row stride of m lines of n points that are filled and read across lines
 // (lane t to line t): odd, so the lines start on different banks.  At 88
-// points 32 lanes met 4 banks.
-KYM_HD KYM_INL constexpr int line_stride(int n, int m) { return m > 1 ? n | 1 : n; }
+// points 32 lanes met 4 banks.  Lines of fewer than 8 points stay packed: the
+// padding would be a quarter of the LDS and more (2 points in FP64: 192 KB).
+KYM_HD KYM_INL constexpr int line_stride(int n, int m) { return m > 1 && n >= 8 ? n | 1 : n; }
+// The same for low-passes, whose contiguous lines (S = 1) are filled and read
+// along the line and stay packed: two lines of 2048 points padded let three
+// workgroups share a CU instead of four (4096 lines, k = 4: 71 against 64 us).
+KYM_HD KYM_INL constexpr int lowpass_stride(int n, int m, int S) { return S > 1 ? line_stride(n, m) : n; }
 
 // Threads of the compile-time frequency scatter and low-passes.
 #ifndef KYM_FS_THREADS
@@ -545,7 +550,7 @@ KYM_HD void lowpass_body(const LowpassArgs& o, const FftLen<T>& fN, const FftLen
                          int tid, int nth) {
     const FInt N = fN.size(), n = fn.size();
     const int k = o.k, S = o.S;
-    const int sN = line_stride(N, o.nrow), sn = line_stride(n, o.nrow);
+    const int sN = lowpass_stride(N, o.nrow, S), sn = lowpass_stride(n, o.nrow, S);
     long long ob;
     int s0, m;
     if (S == 1) {
@@ -788,7 +793,7 @@ inline long long lowpass_shape(int N, int n, int S, long long outer, int* rows, 
         *nblk = (outer + m - 1) / m;
     }
     *rows = (int)m;
-    return m * (line_stride(N, (int)m) + line_stride(n, (int)m));
+    return m * (lowpass_stride(N, (int)m, S) + lowpass_stride(n, (int)m, S));
 }
 
 // Pass kernels for transforms that do not fit: axis 1 = rows (along W),

@@ -252,3 +252,22 @@ def test_freq_scatter_equals_op_sequence(c):
         seq = B1.modulus(B1.swap_time_frequency(B1.filter_ifft(X_hat, f, k, 'complex')))
         assert y.shape == seq.shape
         assert (y - seq).abs().max().item() <= 1e-6 * seq.abs().max().item()
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float64])
+@pytest.mark.parametrize('N', [1, 2, 3, 4, 6, 8, 9])
+def test_short_frequency_axes_over_long_times(N, dtype):
+    """Frequency axes of a few points over 5000 times fill a workgroup with up
+    to 4096 lines: freq_scatter and lowpass against torch.fft in 64 bits."""
+    g = torch.Generator(DEV).manual_seed(N)
+    x = torch.randn(2, N, 5000, 1, device=DEV, dtype=dtype, generator=g)
+    f = torch.rand(N, 1, device=DEV, dtype=dtype, generator=g)
+    k = 2 if N % 2 == 0 else 1
+    X = torch.fft.fft(x[..., 0].double().cpu(), dim=1) * f.double().cpu()[None]
+    fold = torch.fft.ifft(X.reshape(2, k, N // k, 5000).mean(1), dim=1)
+    tol = 16 * torch.finfo(dtype).eps * X.abs().max()  # at most four radices, nine terms a sum
+    low = B1.lowpass(x, f, k, -3)
+    assert (low[..., 0].double().cpu() - fold.real).abs().max() <= tol
+    for y, kk in zip(B1.freq_scatter(x, [f, f], [k, 1], N), (k, 1)):
+        ref = torch.fft.ifft(X.reshape(2, kk, N // kk, 5000).mean(1), dim=1).abs()
+        assert (y[..., 0].double().cpu() - ref).abs().max() <= tol
