@@ -158,14 +158,20 @@ static int upload_and_prepare(Scat2DPlan<T>& p, void** dblob) {
     KYM_HIP_TRY(hipMalloc(dblob, bytes));
     p.blob.relocate((uintptr_t)*dblob);
     KYM_HIP_TRY(hipMemcpy(*dblob, p.blob.bytes.data(), bytes, hipMemcpyHostToDevice));
+    // every kernel that launch_call may pick, for the device's limit and not
+    // this plan's need: plans share the kernels (a launch beyond the limit is
+    // refused here)
+    const size_t lim = device_lds_limit();
     for (const std::vector<Launch2D>* ls : {&p.launches, &p.bwd_launches})
-        for (const Launch2D& l : *ls) {
-            Scat2DKernel<T> k = pick_scat2d<T>(l.kind, l.threads, l.pclass, l.spec);
-            if (!k) return fail(KYM_ERR_UNSUPPORTED, "no kernel for launch kind");
-            if (l.lds_bytes > 65536)
-                KYM_HIP_TRY(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                (int)l.lds_bytes));
-        }
+        for (const Launch2D& l : *ls)
+            for (int many = 0; many <= (l.many_threads != 0); ++many) {
+                Scat2DKernel<T> k = pick_scat2d<T>(l.kind, many ? l.many_threads : l.threads, l.pclass,
+                                                   many ? l.many_spec : l.spec);
+                if (!k) return fail(KYM_ERR_UNSUPPORTED, "no kernel for launch kind");
+                if (l.lds_bytes > 65536)
+                    KYM_HIP_TRY(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                    (int)std::max(l.lds_bytes, lim)));
+            }
     return KYM_OK;
 }
 

@@ -285,3 +285,22 @@ def test_data_that_fills_the_lds(shape, J, lds, dtype):
     if dtype == torch.float32 and shape == (16, 8192):
         return  # some |u| of so many is small enough that u / |u| has three digits in FP32, in plain torch too
     assert (gx.cpu().double() - gw).abs().max() <= (1e-5 if dtype == torch.float32 else 1e-11) * gw.abs().max()
+
+
+@pytest.mark.parametrize('shape,J,B', [((224, 224), 3, 6), ((58, 58), 1, 70), ((116, 116), 2, 20)])
+def test_many_medium_nodes_in_doubles(shape, J, B):
+    """FP64 nodes of 2048 to 4095 points and over 64 KB, on 256 threads in
+    launches of more than 512, on 512 in smaller ones, with a plan of smaller
+    needs of the same kernels made in between: the same outputs and gradients."""
+    sc = Scattering2D(J, shape).double().to(DEV)
+    x = torch.randn((B,) + shape, device=DEV, dtype=torch.float64,
+                    generator=torch.Generator(DEV).manual_seed(B)).requires_grad_()
+    few = torch.cat([sc(x[i:i + 1]) for i in range(B)])
+    w = torch.randn(few.shape[1:], device=DEV, dtype=torch.float64, generator=torch.Generator(DEV).manual_seed(1))
+    gfew, = torch.autograd.grad((few * w).sum(), x)
+    Scattering2D(1, (46, 46)).double().to(DEV)(x[:1, :46, :46].detach().contiguous())
+    many = sc(x)
+    gmany, = torch.autograd.grad((many * w).sum(), x)
+    # the same butterflies in the same order, only spread over other threads
+    assert (many - few).abs().max() <= 1e-14 * few.abs().max()
+    assert (gmany - gfew).abs().max() <= 1e-13 * gfew.abs().max()
