@@ -275,6 +275,13 @@ extern "C" int kym_emu_scat2d_forward(int M, int N, int J, int L, int max_order,
     return emu_forward2d<double>(M, N, J, L, max_order, pre_pad, lds_limit, x, filt, out, batch, chunk, info);
 }
 
+// LDS limit of the 1D plans made from here on, and what the last one needs.
+static long long g_lds1d = 160 * 1024, g_need1d = 0;
+extern "C" void kym_emu_scat1d_lds(long long limit, long long* need) {
+    if (limit > 0) g_lds1d = limit;
+    if (need) *need = g_need1d;
+}
+
 static int emu_scat1d(bool merged, int N, int N_pad, int pad_left, int log2_stride, int average_mode,
                                       int oversampling, int max_order, int n_psi1, const int* psi1_j,
                                       const int* psi1_nlev, int n_psi2, const int* psi2_j, const int* psi2_nlev,
@@ -287,10 +294,11 @@ static int emu_scat1d(bool merged, int N, int N_pad, int pad_left, int log2_stri
         using T = decltype(tag);
         Scat1DPlan<T> p;
         KymError e = {0, ""};
-        if (!p.build(d, 160 * 1024, &e)) {
+        if (!p.build(d, (size_t)g_lds1d, &e)) {
             g_emu_error = e.msg;
             return e.code;
         }
+        g_need1d = (long long)p.max_lds;
         p.blob.relocate((uintptr_t)p.blob.bytes.data());
         const uintptr_t base = (uintptr_t)p.blob.bytes.data();
         if (info) {

@@ -48,6 +48,7 @@ struct Scat1DArgs {
     int len[KYM_MAX_RES1], n[KYM_MAX_RES1];
     int ind_start[KYM_MAX_RES1], ind_end[KYM_MAX_RES1];
     int mode, log2_stride;
+    int split;  // low-pass sums shared by leaf1d_split threads
     const T* x;
     int N, pad_left;
     const T* filt;
@@ -119,7 +120,7 @@ KYM_HD KYM_INL void leaf1d(const F& ff, const Scat1DArgs<T>& a, const Node1D& nd
     const FInt nl = fB.size();
     const T* phi = a.filt + a.filt_off[nd.leaf_filt];
     const T inv_k = T(1) / T(kk);
-    const int S = leaf1d_split(n, nl);
+    const int S = a.split ? leaf1d_split(n, nl) : 1;
     for (int q = tid; q < S * nl; q += nth) {
         const int s = q / nl, i = q - s * nl;
         cpx<T> acc = {T(0), T(0)};

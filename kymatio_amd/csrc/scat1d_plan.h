@@ -38,6 +38,7 @@ struct Scat1DPlan {
     std::vector<int> out_len;  // per output path, in output order
     long long out_row = 0, ws_sig = 0;
     int C = 0, pclass = 7;
+    int split = 1;  // the leaves' partial sums (leaf1d_split) fit everywhere
     LenTable<T> lens;
     std::vector<Launch1D> launches, bwd_launches;
     // the same nodes with one launch per order, every length in it
@@ -196,6 +197,12 @@ struct Scat1DPlan {
                 return false;
             }
         }
+        // under a caller's smaller limit every sum stays with one thread
+        split = 1;
+        for (auto& nd : nodes) {
+            const int nn = n[nd.res];
+            if (local && (size_t)(nn + leaf1d_elems(nn, nn / std::max(nd.leaf_k, 1))) * cs > lds_limit) split = 0;
+        }
         // blob
         blob = Blob();
         std::string err;
@@ -228,7 +235,8 @@ struct Scat1DPlan {
                 for (int id : ids) {
                     const int nn = n[nodes[id].res];
                     const int line = pad && node1d_spec_id(nn, node1d_threads(nn)) >= 0 ? pad16(nn) : nn;
-                    const int leaf = local ? leaf1d_elems(nn, nn / std::max(nodes[id].leaf_k, 1)) : 0;
+                    const int nl = nn / std::max(nodes[id].leaf_k, 1);
+                    const int leaf = !local ? 0 : split ? leaf1d_elems(nn, nl) : nl;
                     m = std::max(m, (size_t)(line + leaf) * cs);
                 }
                 return m;
@@ -319,7 +327,7 @@ struct Scat1DPlan {
             a.len[r] = len[r]; a.n[r] = n[r];
             a.ind_start[r] = ind_start[r]; a.ind_end[r] = ind_end[r];
         }
-        a.mode = mode; a.log2_stride = log2_stride;
+        a.mode = mode; a.log2_stride = log2_stride; a.split = split;
         a.N = N; a.pad_left = pad_left;
         a.ws_sig = ws_sig; a.out_row = out_row;
         return a;

@@ -1,6 +1,8 @@
 """1D workgroup bodies run single-threaded on the CPU (libkymatio_emu.so)
 against the reference fixture, the golden vectors and the oracle, in every
 averaging mode."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -101,3 +103,35 @@ def test_merged_launches_match(emu, J, N, Q, kw, dtype):
     # rounding of transforms of up to 2^12 points and of sums over the nodes
     assert np.abs(om - out).max() <= 40 * eps * np.abs(out).max()
     assert np.abs(gm - gx).max() <= 400 * eps * np.abs(gx).max()
+
+
+@pytest.mark.parametrize('J,N,Q,kw', [(6, 512, 8, {}), (5, 1000, (4, 2), {}), (4, 700, 8, {'stride': 4})])
+@pytest.mark.parametrize('dtype', [np.float32, np.float64])
+def test_plans_keep_a_callers_lds_limit(emu, J, N, Q, kw, dtype):
+    """Under the smallest limit that a plan is made for (its longest node and
+    leaf), no launch asks for more, and the results are the same."""
+    S = Scattering1D(J, N, Q, **kw)
+    rng = np.random.default_rng(J * N)
+    x = rng.standard_normal((2, N)).astype(dtype)
+    w = rng.standard_normal(emu_scat1d(emu, S, x, dtype)[0].shape).astype(dtype)
+    ref, _, gref = emu_scat1d(emu, S, x, dtype, dS=w)
+    cs = 2 * np.dtype(dtype).itemsize
+    limit = (S._N_padded + (S._N_padded >> S.log2_stride)) * cs
+    lds = emu.lib.kym_emu_scat1d_lds
+    lds.argtypes, lds.restype = [ctypes.c_longlong, ctypes.c_void_p], None
+    need = ctypes.c_longlong()
+    eps = np.finfo(dtype).eps
+    try:
+        lds(limit - 8, None)
+        with pytest.raises(RuntimeError, match='does not fit'):
+            emu_scat1d(emu, S, x, dtype)
+        lds(limit, None)
+        for merged in (False, True):
+            out, _, gx = emu_scat1d(emu, S, x, dtype, dS=w, merged=merged)
+            lds(0, ctypes.byref(need))
+            assert need.value <= limit
+            # as in test_merged_launches_match
+            assert np.abs(out - ref).max() <= 40 * eps * np.abs(ref).max()
+            assert np.abs(gx - gref).max() <= 400 * eps * np.abs(gref).max()
+    finally:
+        lds(160 * 1024, None)
