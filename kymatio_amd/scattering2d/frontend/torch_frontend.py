@@ -110,19 +110,32 @@ class ScatteringTorch2D(ScatteringTorch, ScatteringBase):
         self._packed[key] = (stamp, packed)
         return packed
 
-    def _chunk(self, plan, batch):
+    def _chunk(self, plan, batch, least=4):
         """Images per launch chunk: images_per_chunk if set, else as many as a
         256 MB workspace holds (the MALL), balanced so that all chunks are
-        equally full; but four where fewer fit and 2 GB hold them: two images
-        a launch fill the GPU better than residency helps (8 images of 512 x
-        512, J = 6, 118 MB each: 2 / 4 / 8 per chunk 3190 / 2819 / 2847 us)."""
+        equally full; but `least` where fewer fit and 2 GB hold them: four images
+        a launch fill the GPU better than residency helps.  8 images, 1 / 2 / 4
+        per chunk: 512 x 512 J = 5 3894 / 2597 / 2208 us, 500 x 510 J = 5 3501 /
+        2216 / 1833, 480 x 640 J = 6 5238 / 3830 / 3393, 1000 x 1000 J = 6 12538 /
+        10596 / 10286, FP64 300 x 300 J = 4 5580 / 3092 / 1915."""
         if self.images_per_chunk:
             return max(1, min(batch, int(self.images_per_chunk)))
         per = plan.ws_bytes_per_image
-        cap = max(1, (256 << 20) // max(per, 1), min(4, (2 << 30) // max(per, 1)))
+        cap = max(1, (256 << 20) // max(per, 1), min(least, (2 << 30) // max(per, 1)))
         cap = min(batch, cap)
         nchunks = -(-batch // cap)
         return -(-batch // nchunks)
+
+    def _workspace(self, plan, batch, device):
+        """A forward's workspace: `_chunk` images, or without the four images a
+        launch where memory has no room for them."""
+        try:
+            return torch.empty(self._chunk(plan, batch) * plan.ws_bytes_per_image, dtype=torch.uint8, device=device)
+        except torch.OutOfMemoryError:
+            chunk = self._chunk(plan, batch, least=1)
+            if chunk == self._chunk(plan, batch):
+                raise
+            return torch.empty(chunk * plan.ws_bytes_per_image, dtype=torch.uint8, device=device)
 
     def scattering(self, input):
         if not torch.is_tensor(input):
@@ -168,8 +181,7 @@ class ScatteringTorch2D(ScatteringTorch, ScatteringBase):
         out = torch.empty((B, plan.C, plan.oh, plan.ow), dtype=dtype, device=device)
         if B == 0:
             return out
-        chunk = self._chunk(plan, B)
-        ws = torch.empty(chunk * plan.ws_bytes_per_image, dtype=torch.uint8, device=device)
+        ws = self._workspace(plan, B, device)
         with torch.cuda.device(device):
             plan.forward(x, filt, out, B, ws)
         return out

@@ -104,3 +104,34 @@ def test_1d_validation():
         sc._check_runtime_args()
     with pytest.raises(ValueError, match='stride must be a power of two'):
         Scattering1D(6, 512, 8, stride=3).log2_stride
+
+
+@pytest.mark.parametrize('mb,batch,want,tight', [(118, 8, 4, 2), (600, 8, 3, 1), (3000, 5, 1, 1), (60, 64, 4, 4),
+                                                  (10, 64, 22, 22), (118, 1, 1, 1)])
+def test_workspace_falls_back_where_memory_is_short(monkeypatch, mb, batch, want, tight):
+    """The images of a launch chunk, and that a device without room for four
+    of them runs with what 256 MB hold."""
+    plan = namedtuple('plan', ['ws_bytes_per_image'])(mb << 20)
+    sc = Scattering2D(2, (32, 32))
+    asked = []
+
+    def empty(n, dtype, device):
+        asked.append(n // (mb << 20))
+        if room is not None and n > room:
+            raise torch.OutOfMemoryError('out of memory')
+
+    with monkeypatch.context() as m:
+        m.setattr(torch, 'empty', empty)
+        room = None
+        sc._workspace(plan, batch, 'cpu')
+        assert asked == [want]
+        room, asked[:] = tight * (mb << 20), []
+        sc._workspace(plan, batch, 'cpu')
+        assert asked == ([want] if want == tight else [want, tight])
+        room = 0
+        with pytest.raises(torch.OutOfMemoryError):
+            sc._workspace(plan, batch, 'cpu')
+        sc.images_per_chunk, asked[:] = 3, []
+        with pytest.raises(torch.OutOfMemoryError):
+            sc._workspace(plan, batch, 'cpu')
+        assert asked == [min(3, batch)]
