@@ -45,7 +45,7 @@ static void emu_body(const Launch2D& l, const Scat2DArgs<T>& a, int t, cpx<T>* l
 
 // Placement of a plan: info = {LDS bytes of its largest launch, big nodes,
 // launches with twiddles in global memory, workspace bytes per image, those of
-// the launches that are nodes}.
+// the launches that are nodes, nodes with a gathered input}.
 template <class T>
 static int emu_plan2d(int M, int N, int J, int L, long long lds_limit, const int* tune, int ntune, long long* info) {
     Scat2DPlan<T> p;
@@ -58,14 +58,17 @@ static int emu_plan2d(int M, int N, int J, int L, long long lds_limit, const int
         g_emu_error = e.msg;
         return e.code;
     }
-    info[0] = info[1] = info[2] = info[4] = 0;
+    info[0] = info[1] = info[2] = info[4] = info[5] = 0;
     for (const std::vector<Launch2D>* ls : {&p.launches, &p.bwd_launches})
         for (const Launch2D& l : *ls) {
             info[0] = std::max(info[0], (long long)l.lds_bytes);
             info[2] += l.global_tw;
             info[4] += l.global_tw && (l.kind == K2_LDS_NODE || l.kind == K2B_NODE);
         }
-    for (const Node2D& nd : p.nodes) info[1] += nd.big;
+    for (const Node2D& nd : p.nodes) {
+        info[1] += nd.big;
+        info[5] += nd.gin >= 0;
+    }
     info[3] = p.ws_img * (long long)sizeof(cpx<T>);
     return 0;
 }

@@ -72,7 +72,7 @@ struct Scat2DPlan {
     // tree
     std::vector<Node2D> nodes;
     long long ws_img = 0;  // complex elements of workspace per image
-    // the same without the gin slots (which come last): a workspace that holds
+    // the same without the gin slots at the end, if any: a workspace that holds
     // only this runs without the K2_FOLD launches, every node gathering itself
     long long ws_img_base = 0;
     long long points = 0;  // of all nodes of an image
@@ -309,7 +309,10 @@ struct Scat2DPlan {
             // order: 16 images of 144 x 488 J=3, 128 x 160 nodes, 825 us as passes,
             // 531 so.  The first order alone, 8 nodes an image, leaves CUs idle that
             // passes fill: 16 of 112 x 144 J=3 177 us as passes, 191 so.
-            const bool wide = wide_nodes && nd.res > 0 && max_order == 2;
+            // Nor where some of them gather deeply by themselves (rows too long for
+            // K2_FOLD): 2 of 240 x 4000 J=6, 40 x 512 nodes, 4097 us against 4365.
+            const bool wide = wide_nodes && nd.res > 0 && max_order == 2 &&
+                              (W[nd.res] <= KYM_FOLD_THREADS || (1 << nd.res) < KYM_FOLD_MIN_K);
             const size_t tw = wide ? 0 : cs * kym_tw_elems(H[nd.res], W[nd.res]);
             const bool fits = node_lds(nd) + tw <= lds_limit &&
                               (!fir || elems <= (size_t)KYM_STAGE_MAX * node_threads(elems) || spec_fit ||
@@ -333,18 +336,36 @@ struct Scat2DPlan {
             const long long align = 256 / (long long)cs;
             ws_img = (ws_img + align - 1) / align * align;
         }
-        // gathered inputs of LDS nodes with a deep periodisation (K2_FOLD)
+        // gathered inputs of LDS nodes with a deep periodisation (K2_FOLD), in
+        // the slots of second-order big nodes of lower resolutions: nothing reads
+        // those after the launches of their resolution, which come before.  (4
+        // images of 480 x 480 J=5 in 64 MB, which hold one image and no more: 3715
+        // us with gathers in the nodes.)  Without such slots, at the end.
         ws_img_base = ws_img;
         points = 0;
         for (const auto& nd : nodes) points += (long long)H[nd.res] * W[nd.res];
+        std::vector<std::pair<long long, long long>> done[KYM_MAX_RES];  // free [begin, end) per resolution
+        for (const auto& nd : nodes)
+            if (nd.big && nd.order == 2)
+                done[nd.res].push_back({nd.slot, nd.slot + (long long)H[nd.res] * W[nd.res]});
         for (auto& nd : nodes) {
             nd.gin = -1;
             if (nd.big || nd.order == 0 || nd.k < KYM_FOLD_MIN_K || W[nd.res] > KYM_FOLD_THREADS ||
                 fold_lds(nd.res) > lds_limit)
                 continue;
-            nd.gin = ws_img;
             const long long align = 256 / (long long)cs;
-            ws_img = (ws_img + (long long)H[nd.res] * W[nd.res] + align - 1) / align * align;
+            const long long need = ((long long)H[nd.res] * W[nd.res] + align - 1) / align * align;
+            for (int r = 0; r < nd.res && nd.gin < 0; ++r)
+                for (auto& f : done[r])
+                    if (f.second - f.first >= need) {
+                        nd.gin = f.first;
+                        f.first += need;
+                        break;
+                    }
+            if (nd.gin < 0) {
+                nd.gin = ws_img;
+                ws_img += need;
+            }
         }
         // training layout: save slot (u) and gsave slot (dL/dX) for every non-root node,
         // leaf dL/dY slot where the leaf is not formed in the node kernel, and

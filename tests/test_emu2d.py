@@ -167,12 +167,12 @@ def test_fold_pass_matches_gathers(emu, shape, J, L, dt):
 
 
 def _placement(emu, shape, J, L, dt, lds_limit=160 * 1024, tune=()):
-    info = (ctypes.c_longlong * 5)()
+    info = (ctypes.c_longlong * 6)()
     t = (ctypes.c_int * 7)(*tune)
     rc = emu.lib.kym_emu_scat2d_plan(shape[0], shape[1], J, L, 0 if dt == np.float32 else 1,
                                      ctypes.c_longlong(lds_limit), t, len(tune), info)
     assert rc == 0, emu.lib.kym_emu_last_error().decode()
-    return dict(zip(('lds', 'big', 'global_tw', 'ws', 'global_tw_nodes'), info))
+    return dict(zip(('lds', 'big', 'global_tw', 'ws', 'global_tw_nodes', 'gathered'), info))
 
 
 @pytest.mark.parametrize('shape,J,dt,tune,big', [
@@ -215,3 +215,34 @@ def test_twiddles_in_global_memory(emu, shape, J, L, dt, limits):
         assert channel_rel_err(out, ref) <= eps
         assert np.abs(gx - gref).max() <= eps * np.abs(gref).max()
     assert passes and (nodes or J == 1)
+
+
+def test_gathered_inputs_take_finished_slots(emu):
+    """Large images' deep gathers cost no workspace: 480 x 480 J=5 still fits the
+    64 MB of a call without allocations, 512 x 512 J=6 takes what its slots take."""
+    p = _placement(emu, (480, 480), 5, 8, np.float32)
+    assert p['gathered'] > 0 and p['ws'] <= 64 << 20
+    p = _placement(emu, (512, 512), 6, 8, np.float32)
+    assert p['gathered'] > 0 and p['ws'] <= 113 << 20  # 119 MB with slots of their own
+
+
+@pytest.mark.parametrize('shape,J,L,dt,lds', [((120, 130), 4, 2, np.float32, 36000), ((100, 96), 5, 1, np.float32, 34000),
+                                              ((120, 96), 4, 2, np.float64, 70000)])
+def test_fold_into_finished_slots(emu, shape, J, L, dt, lds):
+    """Gathered inputs in the slots of finished second-order big nodes, against
+    the placement without big nodes, forward and backward."""
+    from tests.helpers import emu_train2d
+    p = _placement(emu, shape, J, L, dt, lds)
+    assert p['gathered'] > 0 and p['big'] > 1 + 2 * L  # second-order ones among the big nodes
+    _, f = _filters(shape, J, L, dt)
+    rng = np.random.default_rng(J * L)
+    x = rng.standard_normal((2,) + shape).astype(dt)
+    ref, _ = emu.scat2d(x, J, shape, f, L=L)
+    w = rng.standard_normal(ref.shape).astype(dt)
+    _, gref = emu_train2d(emu, x, J, shape, f, w, L=L)
+    out, _ = emu.scat2d(x, J, shape, f, L=L, lds_limit=lds, chunk=1)
+    eps = 1e-5 if dt == np.float32 else 1e-12
+    assert channel_rel_err(out, ref) <= eps
+    out, gx = emu_train2d(emu, x, J, shape, f, w, L=L, lds_limit=lds, nbwd=2)
+    assert channel_rel_err(out, ref) <= eps
+    assert np.abs(gx - gref).max() <= eps * np.abs(gref).max()
