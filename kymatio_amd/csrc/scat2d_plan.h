@@ -128,7 +128,10 @@ struct Scat2DPlan {
     }
 
     size_t fold_lds(int r) const {
-        return (size_t)KYM_FOLD_TILE * KYM_FOLD_TILE * fold_stripe(W[r]) * sizeof(cpx<T>);
+        return fold_direct(r) ? 0 : (size_t)KYM_FOLD_TILE * KYM_FOLD_TILE * fold_stripe(W[r]) * sizeof(cpx<T>);
+    }
+    bool fold_direct(int r) const {
+        return W[r] > KYM_FOLD_THREADS && (size_t)KYM_FOLD_TILE * KYM_FOLD_TILE * W[r] * sizeof(cpx<T>) > lds_limit;
     }
 
     // Tiles of the fold launch of resolution r: siblings under wavelets of one
@@ -157,6 +160,7 @@ struct Scat2DPlan {
             for (int p0 = 0; p0 < nset; p0 += P)
                 for (int q0 = 0; q0 < nch; q0 += F) {
                     FoldTile t = {};
+                    t.direct = fold_direct(r);
                     t.res = r; t.k = nodes[sets[s][0]].k; t.np = P; t.nf = F;
                     for (int p = 0; p < P; ++p) {
                         t.parent[p] = par[s + p0 + p];
@@ -309,10 +313,7 @@ struct Scat2DPlan {
             // order: 16 images of 144 x 488 J=3, 128 x 160 nodes, 825 us as passes,
             // 531 so.  The first order alone, 8 nodes an image, leaves CUs idle that
             // passes fill: 16 of 112 x 144 J=3 177 us as passes, 191 so.
-            // Nor where some of them gather deeply by themselves (rows too long for
-            // K2_FOLD): 2 of 240 x 4000 J=6, 40 x 512 nodes, 4097 us against 4365.
-            const bool wide = wide_nodes && nd.res > 0 && max_order == 2 &&
-                              (W[nd.res] <= KYM_FOLD_THREADS || (1 << nd.res) < KYM_FOLD_MIN_K);
+            const bool wide = wide_nodes && nd.res > 0 && max_order == 2;
             const size_t tw = wide ? 0 : cs * kym_tw_elems(H[nd.res], W[nd.res]);
             const bool fits = node_lds(nd) + tw <= lds_limit &&
                               (!fir || elems <= (size_t)KYM_STAGE_MAX * node_threads(elems) || spec_fit ||
@@ -350,9 +351,7 @@ struct Scat2DPlan {
                 done[nd.res].push_back({nd.slot, nd.slot + (long long)H[nd.res] * W[nd.res]});
         for (auto& nd : nodes) {
             nd.gin = -1;
-            if (nd.big || nd.order == 0 || nd.k < KYM_FOLD_MIN_K || W[nd.res] > KYM_FOLD_THREADS ||
-                fold_lds(nd.res) > lds_limit)
-                continue;
+            if (nd.big || nd.order == 0 || nd.k < KYM_FOLD_MIN_K || fold_lds(nd.res) > lds_limit) continue;
             const long long align = 256 / (long long)cs;
             const long long need = ((long long)H[nd.res] * W[nd.res] + align - 1) / align * align;
             for (int r = 0; r < nd.res && nd.gin < 0; ++r)

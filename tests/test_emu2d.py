@@ -246,3 +246,24 @@ def test_fold_into_finished_slots(emu, shape, J, L, dt, lds):
     out, gx = emu_train2d(emu, x, J, shape, f, w, L=L, lds_limit=lds, nbwd=2)
     assert channel_rel_err(out, ref) <= eps
     assert np.abs(gx - gref).max() <= eps * np.abs(gref).max()
+
+
+@pytest.mark.parametrize('shape,J,L,dt', [((24, 2280), 4, 2, np.float32), ((20, 4576), 4, 1, np.float32),
+                                          ((24, 2280), 4, 3, np.float64), ((20, 4576), 4, 1, np.float64),
+                                          ((16, 5600), 4, 1, np.float64)])
+def test_fold_pass_over_long_rows(emu, shape, J, L, dt):
+    """Deeply periodised rows of 288, 576 and (beyond the LDS) 704 points, more
+    than the fold pass's threads, against the nodes gathering by themselves."""
+    assert _placement(emu, shape, J, L, dt)['gathered'] == L + L * L
+    Mp, Np = compute_padding(shape[0], shape[1], J)
+    f = pack_filters_2d(filter_bank(Mp, Np, J, L)).astype(dt)
+    x = np.random.default_rng(L).standard_normal((2,) + shape).astype(dt)
+    out, _ = emu.scat2d(x, J, shape, f, L=L)
+    g = emu.with_taps(f, J, shape, L)
+    ref = np.zeros_like(out)
+    fn = emu.lib.kym_emu_scat2d_forward_nofold
+    fn.argtypes, fn.restype = emu.lib.kym_emu_scat2d_forward.argtypes, ctypes.c_int
+    i9 = (ctypes.c_longlong * 9)()
+    assert fn(shape[0], shape[1], J, L, 2, 0, 0 if dt == np.float32 else 1, 160 * 1024, x.ctypes.data, g.ctypes.data,
+              ref.ctypes.data, 2, 0, i9) == 0
+    assert channel_rel_err(out, ref) < (1e-5 if dt == np.float32 else 1e-13)  # as in test_fold_pass_matches_gathers

@@ -304,3 +304,22 @@ def test_many_medium_nodes_in_doubles(shape, J, B):
     # the same butterflies in the same order, only spread over other threads
     assert (many - few).abs().max() <= 1e-14 * few.abs().max()
     assert (gmany - gfew).abs().max() <= 1e-13 * gfew.abs().max()
+
+
+@pytest.mark.parametrize('shape,L', [((24, 2280), 3), ((24, 2280), 4), ((20, 4576), 2), ((16, 5600), 2)])
+def test_deep_averages_of_long_rows(shape, L):
+    """J = 4 with rows of 288, 576 and 704 points at the deepest resolution: forward
+    in both types and the FP64 gradient against the FP64 oracle."""
+    ref = scat2d.Scattering2DTorchCPU(4, shape, L=L, dtype=torch.float64)
+    x = torch.randn((3,) + shape, dtype=torch.float64, generator=torch.Generator().manual_seed(L))
+    xr = x.clone().requires_grad_()
+    want = ref(xr)
+    w = torch.randn(want.shape, dtype=torch.float64, generator=torch.Generator().manual_seed(1))
+    gw, = torch.autograd.grad((want * w).sum(), xr)
+    out = Scattering2D(4, shape, L=L).to(DEV)(x.float().to(DEV)).cpu().numpy()
+    assert channel_rel_err(out, want.detach().numpy()) <= RTOL_CHANNEL
+    xd = x.to(DEV).requires_grad_()
+    got = Scattering2D(4, shape, L=L).double().to(DEV)(xd)
+    gd, = torch.autograd.grad((got * w.to(DEV)).sum(), xd)
+    assert (got.detach().cpu() - want.detach()).abs().max() <= 1e-12 * want.abs().max()
+    assert (gd.cpu() - gw).abs().max() <= 1e-11 * gw.abs().max()
