@@ -296,7 +296,14 @@ template <int MAXP> KYM_HD constexpr bool kym_has_products() {
 #endif
 }
 
-// The passes of large radices as functions, for kernels with every radix up to
+// MAXP of kernels with every radix up to 31 inline: the per-op transforms, low-
+// passes and the frequency scatter, which hold each pass once or twice.  Inline
+// and in functions: 512 x 14384 points 81 and 104 us, 64 x 124 x 116 48 and 72,
+// FP64 64 x 58 x 62 23 and 55, low-passes of 4096 lines of 1984 points 74 and 109,
+// frequency scatters to 92 points 33 and 45.
+#define KYM_ALL_PRIMES 32
+
+// The passes of large radices as functions, for the 2D kernels with every radix up to
 // 31 (a node whose two lengths have different primes from 19 up), which would
 // hold each of them four to six times (246 KB of code).
 template <int R, bool INV, bool TWL, class T>

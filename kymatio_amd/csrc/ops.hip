@@ -352,7 +352,13 @@ static int fft_op(const void* x, void* y, void* work, long long batch, int H, in
     switch (op_pclass(H, W)) {
         case 7: return fft_op_p<T, 7>(x, y, work, batch, H, W, kind, s, lds_cap);
         case 17: return fft_op_p<T, 17>(x, y, work, batch, H, W, kind, s, lds_cap);
-        default: return fft_op_p<T, 31>(x, y, work, batch, H, W, kind, s, lds_cap);
+        case 31:
+            // lines in FP64, whose inline radices take most registers: 1024 of 1216
+            // points 31 us by functions, 36 inline; 512 of 5888 57 and 56
+            if constexpr (sizeof(T) == 8)
+                if (W == 1 && H <= 2048) return fft_op_p<T, 31>(x, y, work, batch, H, W, kind, s, lds_cap);
+            [[fallthrough]];
+        default: return fft_op_p<T, KYM_ALL_PRIMES>(x, y, work, batch, H, W, kind, s, lds_cap);
     }
 }
 
@@ -425,6 +431,8 @@ static int filter_ifft_op(const void* x, const void* f, void* y, long long batch
     switch (op_pclass((int)(N / k))) {
         case 7: return filter_ifft_op_p<T, 7>(x, f, y, batch, N, k, mode, rl, s);
         case 17: return filter_ifft_op_p<T, 17>(x, f, y, batch, N, k, mode, rl, s);
+        // passes in functions leave the alias sums the registers that inline radices
+        // take: 4096 rows of 608 points from 1216 28 us, inline 69
         default: return filter_ifft_op_p<T, 31>(x, f, y, batch, N, k, mode, rl, s);
     }
 }
@@ -483,7 +491,7 @@ static int lowpass_op(const void* x, const void* f, void* y, long long outer, in
     switch (op_pclass(N, N / k)) {
         case 7: return lowpass_op_p<T, 7>(x, f, y, outer, N, S, k, s);
         case 17: return lowpass_op_p<T, 17>(x, f, y, outer, N, S, k, s);
-        default: return lowpass_op_p<T, 31>(x, f, y, outer, N, S, k, s);
+        default: return lowpass_op_p<T, KYM_ALL_PRIMES>(x, f, y, outer, N, S, k, s);
     }
 }
 
@@ -519,7 +527,7 @@ static int freq_scatter_op(const void* x, void* const* ys, const void* const* fs
     if (nblk > 0x7fffffffll) return kym_ops_fail(KYM_ERR_VALUE, "batch too large");
     const void* kern = kym_prime_class(mp) == 7    ? (const void*)k_freq_scatter<T, 7>
                        : kym_prime_class(mp) == 17 ? (const void*)k_freq_scatter<T, 17>
-                                                   : (const void*)k_freq_scatter<T, 31>;
+                                                   : (const void*)k_freq_scatter<T, KYM_ALL_PRIMES>;
     const bool spec = sizeof(T) == 4 && freq_scatter_spec_ok(o);
     if (spec) kern = (const void*)k_freq_scatter_s88<T>;
     if (lds > 65536) OPS_HIP_TRY(hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
@@ -698,6 +706,7 @@ static int harmonic_step_p(HarmonicArgs o, hipStream_t s) {
 
 template <class T>
 static int harmonic_step(const HarmonicArgs& o, hipStream_t s) {
+    // as for filter_ifft: 4 volumes of 38^3, whole transform 567 us, inline 905
     const int c = std::max(op_pclass(o.N, o.O), op_pclass(o.M));
     return c <= 7 ? harmonic_step_p<T, 7>(o, s) : c <= 17 ? harmonic_step_p<T, 17>(o, s) : harmonic_step_p<T, 31>(o, s);
 }
@@ -747,7 +756,7 @@ static int fft_axis0(const void* x, void* y, long long B, int M, int S, int inv,
     switch (op_pclass(M)) {
         case 7: return fft_axis0_p<T, 7>(x, y, B, M, S, inv, s);
         case 17: return fft_axis0_p<T, 17>(x, y, B, M, S, inv, s);
-        default: return fft_axis0_p<T, 31>(x, y, B, M, S, inv, s);
+        default: return fft_axis0_p<T, KYM_ALL_PRIMES>(x, y, B, M, S, inv, s);
     }
 }
 

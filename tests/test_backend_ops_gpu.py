@@ -271,3 +271,35 @@ def test_short_frequency_axes_over_long_times(N, dtype):
     for y, kk in zip(B1.freq_scatter(x, [f, f], [k, 1], N), (k, 1)):
         ref = torch.fft.ifft(X.reshape(2, kk, N // kk, 5000).mean(1), dim=1).abs()
         assert (y[..., 0].double().cpu() - ref).abs().max() <= tol
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float64])
+@pytest.mark.parametrize('p', [19, 23, 29, 31])
+def test_large_primes_in_the_ops(p, dtype):
+    """Transforms, low-passes and frequency scattering of lengths with a prime
+    from 19 up (their kernels hold every radix) against torch.fft in 64 bits."""
+    g = torch.Generator(DEV).manual_seed(p)
+    rnd = lambda *s: torch.randn(*s, device=DEV, dtype=dtype, generator=g)
+    z = lambda t: torch.view_as_complex(t.double().cpu())
+    # p products a radix-p butterfly, each with the rounding of its sum
+    tol = 4 * p * torch.finfo(dtype).eps
+    for n in (p, 2 * p, 32 * p, 16 * p * 3):
+        x = rnd(5, n, 2)
+        for y, ref in ((B1.cfft(x), torch.fft.fft(z(x))), (B1.ifft(x), torch.fft.ifft(z(x)))):
+            assert (z(y) - ref).abs().max() <= tol * ref.abs().max()
+    x = rnd(3, 2 * p, 4 * p, 2)
+    ref = torch.fft.ifft2(z(x))
+    assert (z(B2.ifft(x)) - ref).abs().max() <= tol * ref.abs().max()
+    x, f = rnd(2, 4 * p, 64, 1), rnd(4 * p, 1)
+    fold = lambda X, k: torch.fft.ifft(X.reshape(2, k, 4 * p // k, 64).mean(1), dim=1)
+    X = torch.fft.fft(x[..., 0].double().cpu(), dim=1) * f.double().cpu()[None]
+    low = B1.lowpass(x, f, 2, -3)[..., 0].double().cpu()
+    assert (low - fold(X, 2).real).abs().max() <= tol * fold(X, 2).abs().max()
+    for y, k in zip(B1.freq_scatter(x, [f, f, f], [1, 2, 4], 4 * p), (1, 2, 4)):
+        ref = fold(X, k).abs()
+        assert (y[..., 0].double().cpu() - ref).abs().max() <= tol * ref.max()
+    x = rnd(3, 4, 16 * p, 1)
+    f = rnd(16 * p, 1)
+    X = torch.fft.fft(x[..., 0].double().cpu()) * f[:, 0].double().cpu()
+    ref = torch.fft.ifft(X.reshape(3, 4, 4, 4 * p).mean(2)).real
+    assert (B1.lowpass(x, f, 4, -2)[..., 0].double().cpu() - ref).abs().max() <= tol * X.abs().max() / (4 * p) ** .5
