@@ -152,3 +152,18 @@ def test_autotuned_mixed_workload(per_size):
             err = channel_rel_err(out[s].cpu().numpy(), ref.cpu().numpy())
             print('side %d (%d images, tuning %s): rel err vs default plan %.3e' % (s, x.shape[0], mx.tuning[s], err))
             assert err < RTOL_CHANNEL
+
+
+def test_chunks_of_a_size_are_equally_full(per_size):
+    """A size laid out for 36 images in a budget of ten of them: four chunks of
+    nine, with the same coefficients over several replays."""
+    groups = _images({64: 20})
+    want = per_size[64](groups[64])
+    per = per_size[64]._plan(want.device, torch.float32).ws_bytes_per_image
+    mx = MixedScattering2D(autotune=False, ws_budget=10 * per)
+    for _ in range(3):
+        out = mx.forward_grouped(groups)[64]
+        assert (out - want).abs().max() <= 1e-6 * want.abs().max()
+        want = per_size[64](groups[64])
+    buf, = mx._state[2]
+    assert buf['n'] == 36 and buf['ws'].numel() == 9 * per
