@@ -226,7 +226,8 @@ struct Scat1DPlan {
             l.res = n0.res;
             int len0 = n[n0.res];  // mixed: the longest line
             for (int id : ids) len0 = std::max(len0, n[nodes[id].res]);
-            // mixed launches have CUs to spare: half the points per thread
+            // the threads of the longest line; shorter ones of a mixed launch use their
+            // own number of them (node1d_any_body)
             l.threads = node1d_threads(len0);
             // a node's line (padded: the compiled lengths), then the leaf's
             // partial sums
@@ -292,8 +293,8 @@ struct Scat1DPlan {
         launches.push_back(bwd_launches.back());  // the pad fold
         bwd_merged = launches;
         launches = fwd;
-        // FP32: only with the compiled bodies, whose results are those of the
-        // per-length launches to the last bit
+        // FP32: only with the compiled bodies, whose results (forward and backward)
+        // are those of the per-length launches to the last bit
         mixed_ok = true;
         for (const std::vector<Launch1D>* ls : {&merged, &bwd_merged})
             for (const Launch1D& l : *ls)

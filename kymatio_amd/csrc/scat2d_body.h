@@ -255,48 +255,36 @@ KYM_HD KYM_INL bool herm_point(int p, int H, int W, D W1, int* y, int* x) {
 // For NF filters fs[i] and 0 < y, 0 < x: d[i] += sum u fs[i] at (y, x) and
 // m[i] += sum conj(u') fs[i] at the mirror (H - y, W - x).  The mirror of
 // alias (a, b) reads the point's alias (K-1-a, K-1-b), so alias rows
-// {a, K-1-a} and column chunks {c, NC-1-c} (CH = min(K, 4) columns each) are
-// taken together: at most 16 parent values are live at a time.
+// {a, K-1-a} are taken together: at most 8 parent values are live at a time.
 template <int K, int NF, class T>
-KYM_HD KYM_INL void herm_block(cpx<T>* d, cpx<T>* m, const cpx<T>* U, const T* const* fs, int H, int W, int y, int x,
-                               int a0, int c0) {
-    constexpr int CH = K < 4 ? K : 4, NC = K / CH;
-    const int Wp = W * K, ym = H - y, xm = W - x, a1 = K - 1 - a0, c1 = NC - 1 - c0;
-    const bool two_a = a1 != a0, two_c = c1 != c0;
-    cpx<T> u[2][2][CH];
+KYM_HD KYM_INL void herm_rows(cpx<T>* d, cpx<T>* m, const cpx<T>* U, const T* const* fs, int H, int W, int y, int x,
+                              int a0) {
+    const int Wp = W * K, ym = H - y, xm = W - x, a1 = K - 1 - a0;
+    const bool two = a1 != a0;
+    cpx<T> u[2][K];
 #pragma unroll
     for (int r = 0; r < 2; ++r)
 #pragma unroll
-        for (int q = 0; q < 2; ++q)
-#pragma unroll
-            for (int e = 0; e < CH; ++e) {
-                if ((r && !two_a) || (q && !two_c)) {
-                    u[r][q][e] = u[r && two_a][q && two_c][e];
-                } else {
-                    const int al = r ? a1 : a0, b = (q ? c1 : c0) * CH + e;
-                    u[r][q][e] = kym_ldg(U + (y + al * H) * Wp + x + b * W);
-                }
-            }
+        for (int e = 0; e < K; ++e)
+            u[r][e] = r && !two ? u[0][e] : kym_ldg(U + (y + (r ? a1 : a0) * H) * Wp + x + e * W);
 #pragma unroll
     for (int i = 0; i < NF; ++i) {
         const T* f = fs[i];
 #pragma unroll
         for (int r = 0; r < 2; ++r)
 #pragma unroll
-            for (int q = 0; q < 2; ++q)
-#pragma unroll
-                for (int e = 0; e < CH; ++e) {
-                    if ((r && !two_a) || (q && !two_c)) continue;
-                    const int al = r ? a1 : a0, b = (q ? c1 : c0) * CH + e;
-                    const cpx<T> v = u[r][q][e];                   // alias (al, b) of (y, x)
-                    const cpx<T> w = u[1 - r][1 - q][CH - 1 - e];  // alias (al, b) of the mirror, conjugated
-                    const T fd = kym_ldg(f + (y + al * H) * Wp + x + b * W);
-                    const T fm = kym_ldg(f + (ym + al * H) * Wp + xm + b * W);
-                    d[i].re += v.re * fd;
-                    d[i].im += v.im * fd;
-                    m[i].re += w.re * fm;
-                    m[i].im -= w.im * fm;
-                }
+            for (int e = 0; e < K; ++e) {
+                if (r && !two) continue;
+                const int al = r ? a1 : a0;
+                const cpx<T> v = u[r][e];              // alias (al, e) of (y, x)
+                const cpx<T> w = u[1 - r][K - 1 - e];  // alias (al, e) of the mirror, conjugated
+                const T fd = kym_ldg(f + (y + al * H) * Wp + x + e * W);
+                const T fm = kym_ldg(f + (ym + al * H) * Wp + xm + e * W);
+                d[i].re += v.re * fd;
+                d[i].im += v.im * fd;
+                m[i].re += w.re * fm;
+                m[i].im -= w.im * fm;
+            }
     }
 }
 
@@ -305,7 +293,7 @@ KYM_HD KYM_INL void herm_gather(cpx<T>* d, cpx<T>* m, const cpx<T>* U, const T* 
                                 int x) {
     static_assert(K <= 4, "deeper periodisations are not gathered by mirror pairs");
 #pragma unroll
-    for (int a0 = 0; a0 < (K + 1) / 2; ++a0) herm_block<K, NF>(d, m, U, fs, H, W, y, x, a0, 0);
+    for (int a0 = 0; a0 < (K + 1) / 2; ++a0) herm_rows<K, NF>(d, m, U, fs, H, W, y, x, a0);
 }
 
 // dst[y W + x] = scale P_K(U f)[y][x] for the whole H x W child.

@@ -162,3 +162,26 @@ def test_small_batches_match_large(J, N, Q, B):
     g2, = torch.autograd.grad(y2, x, w)
     assert (y - y2).abs().max() <= 5e-6 * y.abs().max()
     assert (g - g2).abs().max() <= 5e-5 * g.abs().max()
+
+
+@pytest.mark.parametrize('J,N,Q', [(3, 300, 1), (5, 1000, 4), (6, 4096, 8)])
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float64])
+def test_launch_routes_agree_to_the_bit(J, N, Q, dtype):
+    """A batch with more first-order nodes than the GPU holds workgroups (256
+    CUs, at most 32 each) takes a launch per length, two signals take one per
+    order, and a forward in chunks one per length again: the same bits."""
+    sc = Scattering1D(J, N, Q).to(dtype).to(DEV)
+    B = 256 * 32 // len(sc.psi1_f) + 1
+    x = torch.randn(B, N, device=DEV, dtype=dtype, generator=torch.Generator(DEV).manual_seed(N)).requires_grad_()
+    y = sc(x)
+    w = torch.randn(y.shape, device=DEV, dtype=dtype, generator=torch.Generator(DEV).manual_seed(1))
+    g, = torch.autograd.grad(y, x, w)
+    few = slice(0, B, 41)
+    xs = x[few].detach().contiguous().requires_grad_()
+    for i in range(0, xs.shape[0], 2):
+        yi = sc(xs[i:i + 2])
+        gi, = torch.autograd.grad(yi, xs, w[few][i:i + 2])
+        assert torch.equal(yi, y[few][i:i + 2]) and torch.equal(gi[i:i + 2], g[few][i:i + 2])
+    with torch.no_grad():
+        sc.signals_per_chunk = 3
+        assert torch.equal(sc(xs[:10]), y[few][:10])
