@@ -332,6 +332,7 @@ static int emu_scat1d(bool merged, int N, int N_pad, int pad_left, int log2_stri
                 for (int t = 0; t < a.ntask; ++t) {
                     if (l.spec == KYM_N1_ANY && l.kind == 0) node1d_any_body<T, 0, true>(a, t, lds.data(), 0);
                     else if (l.spec == KYM_N1_ANY && l.kind == 1) node1d_any_body<T, 1, true>(a, t, lds.data(), 0);
+                    else if (l.spec == KYM_N1_NOSPLIT) body_node1d<T, 31, false>(a, t, lds.data(), 0, 1);
                     else if (l.kind == 0 && l.spec >= 0) dispatch_node1d_spec<T, true>(l.spec, a, t, lds.data(), 0);
                     else if (l.kind == 1 && l.spec >= 0) dispatch_bwd_node1d_spec<T, true>(l.spec, a, t, lds.data(), 0);
                     else if (l.kind == 0) body_node1d<T, 31>(a, t, lds.data(), 0, 1);

@@ -12,6 +12,7 @@ __global__ void __launch_bounds__(NT) k_scat1d(Scat1DArgs<T> a) {
     // power-of-two lengths only: no odd radices
     if constexpr (KIND == 0) body_node1d<T, 2>(a, task, lds, threadIdx.x, NT);
     else if constexpr (KIND == 1) body_bwd_node1d<T, 2>(a, task, lds, threadIdx.x, NT);
+    else if constexpr (KIND == 3) body_node1d<T, 2, false>(a, task, lds, threadIdx.x, NT);
     else body_bwd_fold1d<T>(a, task, threadIdx.x, NT);
 }
 
@@ -79,5 +80,6 @@ template <class T>
 Scat1DKernel<T> pick_scat1d_nt(int threads, int kind) {
     if (kind == 1) return pick_scat1d_k<T, 1>(threads);
     if (kind == 2) return k_scat1d<T, 256, 2>;
+    if (kind == 3) return pick_scat1d_k<T, 3>(threads);
     return pick_scat1d_k<T, 0>(threads);
 }

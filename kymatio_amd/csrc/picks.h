@@ -67,6 +67,7 @@ inline Scat2DKernel<T> pick_scat2d(int kind, int threads, int pclass, int spec =
 // spec >= 0 (FP32 nodes) selects a compile-time specialisation.
 template <class T>
 inline Scat1DKernel<T> pick_scat1d(int threads, int kind = 0, int spec = -1) {
+    if (spec == KYM_N1_NOSPLIT && kind == 0) kind = 3, spec = -1;
     if constexpr (sizeof(T) == 4) {
         if (spec == KYM_N1_ANY && kind <= 1) return kym_pick_any1d_f32(kind);
         if (spec >= 0 && kind == 0) return kym_pick_node1d_spec_f32(spec);

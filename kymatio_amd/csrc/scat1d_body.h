@@ -48,7 +48,6 @@ struct Scat1DArgs {
     int len[KYM_MAX_RES1], n[KYM_MAX_RES1];
     int ind_start[KYM_MAX_RES1], ind_end[KYM_MAX_RES1];
     int mode, log2_stride;
-    int split;  // low-pass sums shared by leaf1d_split threads
     const T* x;
     int N, pad_left;
     const T* filt;
@@ -104,8 +103,10 @@ KYM_HD KYM_INL constexpr int leaf1d_split(int n, int nl) {
 // LDS elements after the node's line: the leaf's line of nl points as S partial sums.
 KYM_HD KYM_INL constexpr int leaf1d_elems(int n, int nl) { return nl * leaf1d_split(n, nl); }
 
-// Output of one path from the spectrum / modulus in LDS.
-template <class T, int MAXP, class F>
+// Output of one path from the spectrum / modulus in LDS.  SPLIT = false: every
+// sum by one thread, where the partial sums have no room (a compile-time choice:
+// read from the node or the arguments, it cost 3 signals of 1000 J=5 1%).
+template <class T, int MAXP, bool SPLIT, class F>
 KYM_HD KYM_INL void leaf1d(const F& ff, const Scat1DArgs<T>& a, const Node1D& nd, const cpx<T>* U, int n, int img,
                            cpx<T>* B, int tid, int nth) {
     T* o = a.out + (long long)img * a.out_row + nd.out_off;
@@ -120,7 +121,7 @@ KYM_HD KYM_INL void leaf1d(const F& ff, const Scat1DArgs<T>& a, const Node1D& nd
     const FInt nl = fB.size();
     const T* phi = a.filt + a.filt_off[nd.leaf_filt];
     const T inv_k = T(1) / T(kk);
-    const int S = a.split ? leaf1d_split(n, nl) : 1;
+    const int S = SPLIT ? leaf1d_split(n, nl) : 1;
     for (int q = tid; q < S * nl; q += nth) {
         const int s = q / nl, i = q - s * nl;
         cpx<T> acc = {T(0), T(0)};
@@ -152,7 +153,7 @@ KYM_HD KYM_INL void leaf1d(const F& ff, const Scat1DArgs<T>& a, const Node1D& nd
     wg_barrier();
 }
 
-template <class T, int MAXP, class F>
+template <class T, int MAXP, bool SPLIT = true, class F>
 KYM_HD KYM_INL void node1d_body(const F& ff, const Scat1DArgs<T>& a, int task, cpx<T>* lds, int tid, int nth) {
     const int il = task / a.ngroup, gi = task - il * a.ngroup;
     const int img = a.img0 + il;
@@ -235,12 +236,12 @@ KYM_HD KYM_INL void node1d_body(const F& ff, const Scat1DArgs<T>& a, int task, c
         cpx<T>* dst = wsi + nd.slot;
         for (int i = tid; i < n; i += nth) dst[i] = lds[ff.at(i)];
     }
-    if (a.mode != AVG1_NONE) leaf1d<T, MAXP>(ff, a, nd, lds, n, img, lds + ff.elems(n), tid, nth);
+    if (a.mode != AVG1_NONE) leaf1d<T, MAXP, SPLIT>(ff, a, nd, lds, n, img, lds + ff.elems(n), tid, nth);
 }
 
-template <class T, int MAXP>
+template <class T, int MAXP, bool SPLIT = true>
 KYM_HD void body_node1d(const Scat1DArgs<T>& a, int task, cpx<T>* lds, int tid, int nth) {
-    node1d_body<T, MAXP>(Dyn1D<T, MAXP>(), a, task, lds, tid, nth);
+    node1d_body<T, MAXP, SPLIT>(Dyn1D<T, MAXP>(), a, task, lds, tid, nth);
 }
 
 // Compile-time specialisations X(id, N, threads) of the nodes, forward and backward (FP32):
@@ -431,6 +432,8 @@ KYM_HD void body_bwd_fold1d(const Scat1DArgs<T>& a, int task, int tid, int nth) 
 // which launch a node ran in.  The other threads start beyond every loop and
 // only meet the barriers.
 #define KYM_N1_ANY 1000  // Launch1D::spec of such a launch
+// Launch1D::spec of forward nodes whose partial sums do not fit a caller's LDS limit
+#define KYM_N1_NOSPLIT 1001
 template <class T, int KIND, bool EMU>
 KYM_HD KYM_INL void node1d_any_body(const Scat1DArgs<T>& a, int task, cpx<T>* lds, int tid) {
     const Node1D& nd = a.nodes[a.group[task % a.ngroup]];

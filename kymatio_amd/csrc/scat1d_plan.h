@@ -244,7 +244,8 @@ struct Scat1DPlan {
             };
             l.lds_bytes = lds_of(false);
             // compile-time lengths where the padded lines fit
-            if (kind <= 1 && sizeof(T) == 4 && lds_of(true) <= lds_limit) {
+            if (kind == 0 && !split) l.spec = KYM_N1_NOSPLIT;
+            else if (kind <= 1 && sizeof(T) == 4 && lds_of(true) <= lds_limit) {
                 l.spec = mixed ? KYM_N1_ANY : node1d_spec_id(len0, l.threads);
                 if (l.spec >= 0) l.lds_bytes = lds_of(true);
             }
@@ -328,7 +329,7 @@ struct Scat1DPlan {
             a.len[r] = len[r]; a.n[r] = n[r];
             a.ind_start[r] = ind_start[r]; a.ind_end[r] = ind_end[r];
         }
-        a.mode = mode; a.log2_stride = log2_stride; a.split = split;
+        a.mode = mode; a.log2_stride = log2_stride;
         a.N = N; a.pad_left = pad_left;
         a.ws_sig = ws_sig; a.out_row = out_row;
         return a;

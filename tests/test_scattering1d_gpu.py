@@ -185,3 +185,23 @@ def test_launch_routes_agree_to_the_bit(J, N, Q, dtype):
     with torch.no_grad():
         sc.signals_per_chunk = 3
         assert torch.equal(sc(xs[:10]), y[few][:10])
+
+
+@pytest.mark.parametrize('J,N,Q,kw', [(6, 512, 8, {}), (5, 1000, 4, {}), (6, 4096, 8, {'stride': 16})])
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float64])
+def test_smallest_lds_limit(J, N, Q, kw, dtype):
+    """The smallest limit that a plan is made for (its longest node and leaf),
+    where no thread shares a low-pass sum: the results of the default plan."""
+    x = torch.randn(5, N, device=DEV, dtype=dtype, generator=torch.Generator(DEV).manual_seed(N)).requires_grad_()
+    res = []
+    for limited in (False, True):
+        sc = Scattering1D(J, N, Q, **kw).to(dtype).to(DEV)
+        if limited:
+            sc.lds_limit = (sc._N_padded + (sc._N_padded >> sc.log2_stride)) * 2 * x.element_size()
+        y = sc(x)
+        w = torch.randn(y.shape, device=DEV, dtype=dtype, generator=torch.Generator(DEV).manual_seed(1))
+        res.append((y.detach(), torch.autograd.grad(y, x, w)[0]))
+    eps = torch.finfo(dtype).eps
+    # rounding of transforms of up to 2^13 points and of sums over the nodes
+    assert (res[1][0] - res[0][0]).abs().max() <= 40 * eps * res[0][0].abs().max()
+    assert (res[1][1] - res[0][1]).abs().max() <= 400 * eps * res[0][1].abs().max()
