@@ -97,17 +97,19 @@ struct ChunkStreams {
 // 92 images of 17 x 17 J=1 (0.3 million points) 28 against 75 us, 32 of 64 x 64
 // J=3 (7.3) 89 against 105, 8 of 128 x 128 J=4 with the gradient (7.9) 417
 // against 442, FP64 4 of 224 x 224 J=3 (8.2) 529 against 563, 6 of 150 x 203
-// J=4 (9.1) 221 against 218, 4 of 256 x 256 J=3 (10.5) 201 against 194, 16 (42) 407 against 387; 1D, whose launches are
-// fewer: 105 signals of 3608 J=7 (7.5) 226 against 430, 64 of 4096 J=6 Q=8 (17)
-// 254 against 264, 128 (35) 332 against 322.
+// J=4 (9.1) 221 against 218, 4 of 256 x 256 J=3 (10.5) 201 against 194, 16 (42)
+// 407 against 387; 1D, whose launches are fewer: 105 signals of 3608 J=7 (7.5) 226
+// against 430, 64 of 4096 J=6 Q=8 (17) 254 against 264, 128 (35) 332 against 322.
+// Next to the lines the choices differ by 1 to 4%, so they are no sharper than
+// that.
 #define KYM_STREAM_POINTS_2D 9000000
 #define KYM_STREAM_POINTS_1D 20000000
 
 // Streams a chunked call uses: `want` (0 = 2, or 1 for a call of fewer than
-// `enough` of its `points`) reduced until every stream gets a chunk.  The chunk then fits one stream's share of the
-// workspace, with the chunk count a multiple of the stream count and the
-// chunks as even as that allows (256 over 3 streams: 6 chunks of <= 43, not
-// 85, 85, 85, 1).
+// `enough` of its `points`) reduced until every stream gets a chunk.  The chunk
+// then fits one stream's share of the workspace, with the chunk count a multiple
+// of the stream count and the chunks as even as that allows (256 over 3 streams:
+// 6 chunks of <= 43, not 85, 85, 85, 1).
 static int chunk_streams(const ChunkStreams* cs, int want, long long points, long long enough, long long batch,
                          long long* chunk) {
     int ns = want != 0 ? want : points < enough ? 1 : 2;

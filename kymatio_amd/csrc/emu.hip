@@ -346,7 +346,7 @@ static int emu_scat1d(bool merged, int N, int N_pad, int pad_left, int log2_stri
     return run(double(0));
 }
 
-// Per-op FFT (kym_op_fft) on the host: same launch sequence and bodies.
+// The 1D plan's launches (one per length and order) on the host.
 extern "C" int kym_emu_scat1d_forward(int N, int N_pad, int pad_left, int log2_stride, int average_mode,
                                       int oversampling, int max_order, int n_psi1, const int* psi1_j,
                                       const int* psi1_nlev, int n_psi2, const int* psi2_j, const int* psi2_nlev,
@@ -368,6 +368,7 @@ extern "C" int kym_emu_scat1d_merged(int N, int N_pad, int pad_left, int log2_st
                       psi2_j, psi2_nlev, phi_nlev, ind_start, ind_end, n_ind, dtype, x, filt, out, batch, info, dS, gx, nbwd);
 }
 
+// Per-op FFT (kym_op_fft) on the host: same launch sequence and bodies.
 template <class T>
 static int emu_op_fft(const void* x, void* y, void* work, long long batch, int H, int W, int kind, long long lds_cap) {
     LenTable<T> lt;

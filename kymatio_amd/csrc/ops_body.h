@@ -340,7 +340,12 @@ KYM_HD KYM_INL constexpr int line_stride(int n, int m) { return m > 1 && n >= 8 
 // workgroups share a CU instead of four (4096 lines, k = 4: 71 against 64 us).
 KYM_HD KYM_INL constexpr int lowpass_stride(int n, int m, int S) { return S > 1 ? line_stride(n, m) : n; }
 
-// Threads of the compile-time frequency scatter and low-passes.
+// Threads of the compile-time frequency scatter and low-passes: 64 signals of
+// 4096, J=6 Q=8, whole transform 2231 us, on 256 threads 2633.  The run-time-sized
+// kernels keep 256.  Low-passes on 512: 4096 lines of 2048 points, k = 4, 64 -> 73
+// us, of 1984 74 -> 109, of 512 23 -> 21.  Frequency scatters on 512: 50 rows of 128
+// times to 64 points 30 -> 23 us, 90 of 256 to 120 36 -> 28, but 60 to 76 30 -> 45 and
+// 70 to 92 33 -> 49, where radices 19 and 23 take the registers of eight waves.
 #ifndef KYM_FS_THREADS
 #define KYM_FS_THREADS 512
 #define KYM_LP_THREADS 512

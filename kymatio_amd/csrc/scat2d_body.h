@@ -97,7 +97,6 @@ struct FirAxis {
 #define KYM_FOLD_TILE 4
 struct FoldTile {
     int res, k, np, nf;
-    int direct;  // rows of one stripe beyond the LDS: sums stored by their threads
     int parent[KYM_FOLD_TILE];
     int child[KYM_FOLD_TILE * KYM_FOLD_TILE];
 };
@@ -453,8 +452,7 @@ KYM_HD KYM_INL void gather_whole(cpx<T>* dst, const cpx<T>* U, const T* f, int H
 #define KYM_FOLD_THREADS 256
 // Rows of more than 256 points are one stripe, several columns a thread (8
 // images of 40 x 3000 J=4, 380-point rows: 1391 us, 1640 with gathers in the
-// nodes).  Their sums are whole and need no LDS, which they take as a way to
-// contiguous stores while it fits (1441 us without).
+// nodes), in tiles that fit the LDS.
 KYM_HD KYM_INL constexpr int fold_stripe(int W) {
     return W > KYM_FOLD_THREADS ? W : W * (KYM_FOLD_THREADS / W);
 }
@@ -470,7 +468,6 @@ KYM_HD KYM_INL void fold_tile(const Scat2DArgs<T>& a, const FoldTile& tl, cpx<T>
 #pragma unroll
     for (int q = 0; q < F; ++q) f[q] = a.filt + a.filt_off[a.nodes[tl.child[q]].filt] + (long long)y0 * Wp;
     const int rstep = H * Wp;
-    const T scale = T(1) / T(k * k);
     for (int t = tid; t < stripe; t += nth) {
         cpx<T> acc[P][F];
 #pragma unroll
@@ -507,13 +504,10 @@ KYM_HD KYM_INL void fold_tile(const Scat2DArgs<T>& a, const FoldTile& tl, cpx<T>
 #pragma unroll
         for (int p = 0; p < P; ++p)
 #pragma unroll
-            for (int q = 0; q < F; ++q) {
-                if (tl.direct) wsi[a.nodes[tl.child[p * F + q]].gin + (long long)y0 * W + t] = acc[p][q] * scale;
-                else part[(p * F + q) * stripe + t] = acc[p][q];
-            }
+            for (int q = 0; q < F; ++q) part[(p * F + q) * stripe + t] = acc[p][q];
     }
-    if (tl.direct) return;
     wg_barrier();
+    const T scale = T(1) / T(k * k);
     for (int i = tid; i < P * F * W; i += nth) {
         const int pq = i / W, x = i - pq * W;
         const cpx<T>* s = part + pq * stripe + x;

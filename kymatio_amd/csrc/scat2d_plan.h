@@ -127,11 +127,17 @@ struct Scat2DPlan {
         return f;
     }
 
-    size_t fold_lds(int r) const {
-        return fold_direct(r) ? 0 : (size_t)KYM_FOLD_TILE * KYM_FOLD_TILE * fold_stripe(W[r]) * sizeof(cpx<T>);
+    // Parents (and wavelets) of a fold tile of resolution r at most: four, or for
+    // rows of more than a thread a column what fits the LDS; 0: no fold pass.
+    int fold_width(int r) const {
+        for (int w = KYM_FOLD_TILE; w >= 1; --w) {
+            if ((size_t)w * w * fold_stripe(W[r]) * sizeof(cpx<T>) <= lds_limit) return w;
+            if (W[r] <= KYM_FOLD_THREADS) break;
+        }
+        return 0;
     }
-    bool fold_direct(int r) const {
-        return W[r] > KYM_FOLD_THREADS && (size_t)KYM_FOLD_TILE * KYM_FOLD_TILE * W[r] * sizeof(cpx<T>) > lds_limit;
+    size_t fold_lds(int r) const {
+        return (size_t)fold_width(r) * fold_width(r) * fold_stripe(W[r]) * sizeof(cpx<T>);
     }
 
     // Tiles of the fold launch of resolution r: siblings under wavelets of one
@@ -146,7 +152,12 @@ struct Scat2DPlan {
             if (par.empty() || par.back() != nd.parent) { par.push_back(nd.parent); sets.emplace_back(); }
             sets.back().push_back((int)i);
         }
-        auto width = [](int n) { return n % 4 == 0 ? 4 : n % 3 == 0 ? 3 : n % 2 == 0 ? 2 : 1; };
+        const int most = fold_width(r);
+        auto width = [&](int n) {
+            int w = most;
+            while (n % w) --w;
+            return w;
+        };
         std::vector<FoldTile> tiles;
         for (size_t s = 0; s < sets.size();) {
             // parents of one scale: consecutive sets whose first children have one filter
@@ -160,7 +171,6 @@ struct Scat2DPlan {
             for (int p0 = 0; p0 < nset; p0 += P)
                 for (int q0 = 0; q0 < nch; q0 += F) {
                     FoldTile t = {};
-                    t.direct = fold_direct(r);
                     t.res = r; t.k = nodes[sets[s][0]].k; t.np = P; t.nf = F;
                     for (int p = 0; p < P; ++p) {
                         t.parent[p] = par[s + p0 + p];
@@ -351,7 +361,7 @@ struct Scat2DPlan {
                 done[nd.res].push_back({nd.slot, nd.slot + (long long)H[nd.res] * W[nd.res]});
         for (auto& nd : nodes) {
             nd.gin = -1;
-            if (nd.big || nd.order == 0 || nd.k < KYM_FOLD_MIN_K || fold_lds(nd.res) > lds_limit) continue;
+            if (nd.big || nd.order == 0 || nd.k < KYM_FOLD_MIN_K || fold_width(nd.res) == 0) continue;
             const long long align = 256 / (long long)cs;
             const long long need = ((long long)H[nd.res] * W[nd.res] + align - 1) / align * align;
             for (int r = 0; r < nd.res && nd.gin < 0; ++r)

@@ -6,7 +6,8 @@ integral per path (kymatio/scattering3d/core/scattering3d.py:24-75).  Here
 each step of one l is two launches over all j, m and images together:
 
     planes    products U_hat psi_{l, j, m} and their 2D inverse over (N, O)
-    lines     inverse along M, then the chained rotation modulus over m
+    lines     inverse along M, then the root of the squares' sum over m (what
+              the chained rotation modulus computes, with one rounding)
 
 (kym_op_harmonic_step, for every j of a parent at once) and the moduli of
 every (path, l) land in one field array of layout (paths, L + 1, B, n), so

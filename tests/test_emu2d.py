@@ -250,9 +250,9 @@ def test_fold_into_finished_slots(emu, shape, J, L, dt, lds):
 
 @pytest.mark.parametrize('shape,J,L,dt', [((24, 2280), 4, 2, np.float32), ((20, 4576), 4, 1, np.float32),
                                           ((24, 2280), 4, 3, np.float64), ((20, 4576), 4, 1, np.float64),
-                                          ((16, 5600), 4, 1, np.float64)])
+                                          ((16, 5600), 4, 4, np.float64)])
 def test_fold_pass_over_long_rows(emu, shape, J, L, dt):
-    """Deeply periodised rows of 288, 576 and (beyond the LDS) 704 points, more
+    """Deeply periodised rows of 288, 576 and (in smaller tiles) 704 points, more
     than the fold pass's threads, against the nodes gathering by themselves."""
     assert _placement(emu, shape, J, L, dt)['gathered'] == L + L * L
     Mp, Np = compute_padding(shape[0], shape[1], J)
