@@ -373,7 +373,7 @@ static int run2d(const Scat2DPlan<T>& p, int mode, const void* x, const void* fi
         const hipStream_t st = si ? cs->aux[si - 1] : stream;
         void* wsk = static_cast<char*>(ws) + (mode == 0 ? si * chunk : i0) * img_elems * (long long)sizeof(cpx<T>);
         for (const Launch2D& l : launches) {
-            if (l.kind == K2_FOLD && mode == 0 && img_elems < p.ws_img) continue;
+            if (l.is_fold() && mode == 0 && img_elems < p.ws_img) continue;
             Launch2DCall<T> c;
             rc = launch_call(p, l, mode, x, filt, out, dS, gx, img_elems, wsk, i0, nimg, base, &c);
             if (rc != KYM_OK) return rc;
@@ -568,7 +568,7 @@ static int add_plan_chain(hipGraph_t g, const Scat2DPlan<T>& p, const void* x, c
     for (long long i0 = 0; i0 < batch; i0 += chunk) {
         const int nimg = (int)std::min(chunk, batch - i0);
         for (const Launch2D& l : p.launches) {
-            if (l.kind == K2_FOLD && img_elems < p.ws_img) continue;
+            if (l.is_fold() && img_elems < p.ws_img) continue;
             Launch2DCall<T> c;
             rc = launch_call(p, l, 0, x, filt, out, nullptr, nullptr, img_elems, ws, i0, nimg, base, &c);
             if (rc != KYM_OK) return rc;

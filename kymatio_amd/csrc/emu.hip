@@ -120,7 +120,7 @@ static int emu_forward2d(int M, int N, int J, int L, int max_order, int pre_pad,
     for (long long i0 = 0; i0 < batch; i0 += chunk) {
         const int nimg = (int)std::min(chunk, batch - i0);
         for (const Launch2D& l : p.launches) {
-            if (l.kind == K2_FOLD && !folds) continue;
+            if (l.is_fold() && !folds) continue;
             Scat2DArgs<T> a = p.args(l, base);
             a.ws_img = ws_img;
             a.fold = folds;

@@ -123,6 +123,7 @@ Scat2DKernel<T> pick_scat2d_p(int kind, int threads) {
         case K2_LEAF_ROWS: return k_scat2d<T, K2_LEAF_ROWS, 256, MAXP>;
         case K2_FIR_COLS: return k_scat2d<T, K2_FIR_COLS, 256, MAXP>;
         case K2_FOLD: return k_scat2d<T, K2_FOLD, KYM_FOLD_THREADS, 7>;  // no transform in it
+        case K2_FOLD_LONG: return k_scat2d<T, K2_FOLD_LONG, KYM_FOLD_THREADS, 7>;
         case K2B_NODE: return pick_scat2d_nt<T, K2B_NODE, MAXP>(threads);
         case K2B_LEAFG: return pick_scat2d_nt<T, K2B_LEAFG, MAXP>(threads);
         case K2B_GCOLS: return k_scat2d<T, K2B_GCOLS, 256, MAXP>;

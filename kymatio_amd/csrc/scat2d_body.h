@@ -452,15 +452,18 @@ KYM_HD KYM_INL void gather_whole(cpx<T>* dst, const cpx<T>* U, const T* f, int H
 #define KYM_FOLD_THREADS 256
 // Rows of more than 256 points are one stripe, several columns a thread (8
 // images of 40 x 3000 J=4, 380-point rows: 1391 us, 1640 with gathers in the
-// nodes), in tiles that fit the LDS.
+// nodes), in tiles that fit the LDS: K2_FOLD_LONG, a kernel of its own (in one,
+// 26 images of 178 x 178 J=5 681 us instead of 678, 4 of 182 x 182 J=4 192 instead
+// of 190).
 KYM_HD KYM_INL constexpr int fold_stripe(int W) {
     return W > KYM_FOLD_THREADS ? W : W * (KYM_FOLD_THREADS / W);
 }
 
-template <int P, int F, class T>
+template <int P, int F, bool LONG, class T>
 KYM_HD KYM_INL void fold_tile(const Scat2DArgs<T>& a, const FoldTile& tl, cpx<T>* wsi, int y0, cpx<T>* part, int tid,
                               int nth) {
-    const int H = a.H[tl.res], W = a.W[tl.res], k = tl.k, Wp = W * k, stripe = fold_stripe(W);
+    const int H = a.H[tl.res], W = a.W[tl.res], k = tl.k, Wp = W * k;
+    const int stripe = LONG ? W : W * (KYM_FOLD_THREADS / W);
     const cpx<T>* U[P];
     const T* f[F];
 #pragma unroll
@@ -518,7 +521,7 @@ KYM_HD KYM_INL void fold_tile(const Scat2DArgs<T>& a, const FoldTile& tl, cpx<T>
 }
 
 // task -> (image, tile, output row).
-template <class T>
+template <class T, bool LONG>
 KYM_HD void body_fold(const Scat2DArgs<T>& a, int task, cpx<T>* lds, int tid, int nth) {
     const int per = a.ngroup * a.nblk;
     const int il = task / per, rem = task - il * per;
@@ -526,13 +529,13 @@ KYM_HD void body_fold(const Scat2DArgs<T>& a, int task, cpx<T>* lds, int tid, in
     const FoldTile& tl = reinterpret_cast<const FoldTile*>(a.group)[gi];
     cpx<T>* wsi = a.ws + il * a.ws_img;
     switch (tl.np * 8 + tl.nf) {  // the plan's tiles: P x F with P = F or P = 1
-        case 8 * 4 + 4: fold_tile<4, 4>(a, tl, wsi, y0, lds, tid, nth); break;
-        case 8 * 3 + 3: fold_tile<3, 3>(a, tl, wsi, y0, lds, tid, nth); break;
-        case 8 * 2 + 2: fold_tile<2, 2>(a, tl, wsi, y0, lds, tid, nth); break;
-        case 8 * 1 + 4: fold_tile<1, 4>(a, tl, wsi, y0, lds, tid, nth); break;
-        case 8 * 1 + 3: fold_tile<1, 3>(a, tl, wsi, y0, lds, tid, nth); break;
-        case 8 * 1 + 2: fold_tile<1, 2>(a, tl, wsi, y0, lds, tid, nth); break;
-        default: fold_tile<1, 1>(a, tl, wsi, y0, lds, tid, nth); break;
+        case 8 * 4 + 4: fold_tile<4, 4, LONG>(a, tl, wsi, y0, lds, tid, nth); break;
+        case 8 * 3 + 3: fold_tile<3, 3, LONG>(a, tl, wsi, y0, lds, tid, nth); break;
+        case 8 * 2 + 2: fold_tile<2, 2, LONG>(a, tl, wsi, y0, lds, tid, nth); break;
+        case 8 * 1 + 4: fold_tile<1, 4, LONG>(a, tl, wsi, y0, lds, tid, nth); break;
+        case 8 * 1 + 3: fold_tile<1, 3, LONG>(a, tl, wsi, y0, lds, tid, nth); break;
+        case 8 * 1 + 2: fold_tile<1, 2, LONG>(a, tl, wsi, y0, lds, tid, nth); break;
+        default: fold_tile<1, 1, LONG>(a, tl, wsi, y0, lds, tid, nth); break;
     }
 }
 
@@ -1781,7 +1784,7 @@ inline int pass_spec_id(int H, int W, int cb, int rb, int want_threads, int* thr
 
 enum Kind2D {
     K2_LDS_NODE = 0, K2_LEAF, K2_ROOT_ROWS, K2_ICOL, K2_ROWS_MOD, K2_FWD_COLS, K2_LEAF_ICOL, K2_LEAF_ROWS, K2_FIR_COLS,
-    K2_ICOL_PAIR, K2_FOLD
+    K2_ICOL_PAIR, K2_FOLD, K2_FOLD_LONG
 };
 
 template <class T, int KIND, class P>
@@ -1879,7 +1882,8 @@ KYM_HD KYM_INL void dispatch_body2d(int kind, const Scat2DArgs<T>& a, int task, 
         case K2_LEAF_ICOL: body_leaf_icol<T, MAXP>(a, task, lds, tid, nth); break;
         case K2_LEAF_ROWS: body_leaf_rows<T, MAXP>(a, task, lds, tid, nth); break;
         case K2_FIR_COLS: body_fir_cols<T, MAXP>(a, task, lds, tid, nth); break;
-        case K2_FOLD: body_fold<T>(a, task, lds, tid, nth); break;
+        case K2_FOLD: body_fold<T, false>(a, task, lds, tid, nth); break;
+        case K2_FOLD_LONG: body_fold<T, true>(a, task, lds, tid, nth); break;
         default: break;
     }
 }

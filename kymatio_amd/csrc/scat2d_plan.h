@@ -24,6 +24,7 @@ struct Launch2D {
     // small LDS nodes: threads (and specialisation) of a launch of more than
     // many_tasks workgroups, 0 = the same
     int many_threads = 0, many_spec = -1, many_tasks = 0;
+    bool is_fold() const { return kind == K2_FOLD || kind == K2_FOLD_LONG; }
 };
 
 // Workgroups from which a launch of small nodes uses one wave per node.  Up to
@@ -476,7 +477,7 @@ struct Scat2DPlan {
                 case K2_ROOT_ROWS: case K2_ROWS_MOD: case K2_LEAF_ROWS: case K2B_GROWS:
                     l.pclass = kym_plan_class(W[0], 1);
                     break;
-                case K2_FIR_COLS: case K2_FOLD: case K2B_FOLD: break;  // no transform
+                case K2_FIR_COLS: case K2_FOLD: case K2_FOLD_LONG: case K2B_FOLD: break;  // no transform
                 default: l.pclass = kym_plan_class(H[0], W[0]);
             }
             l.spec = -1;
@@ -552,7 +553,7 @@ struct Scat2DPlan {
             const size_t elems = (size_t)H[r] * W[r];
             const std::vector<FoldTile> tiles = n0.big ? std::vector<FoldTile>() : fold_tiles(r);
             if (!tiles.empty()) {
-                push(K2_FOLD, {ids[0]}, H[r], 1, KYM_FOLD_THREADS, fold_lds(r));
+                push(W[r] > KYM_FOLD_THREADS ? K2_FOLD_LONG : K2_FOLD, {ids[0]}, H[r], 1, KYM_FOLD_THREADS, fold_lds(r));
                 Launch2D& lf = launches.back();
                 lf.group_off = blob.add(sizeof(FoldTile) * tiles.size());
                 std::memcpy(blob.at<char>(lf.group_off), tiles.data(), sizeof(FoldTile) * tiles.size());

@@ -33,7 +33,7 @@ class Scat2DPlanHandle:
         self.dtype = dtype
 
     KIND_NAMES = ['lds_node', 'leaf', 'root_rows', 'icol', 'rows_mod', 'fwd_cols', 'leaf_icol', 'leaf_rows',
-                  'fir_cols', 'icol_pair', 'fold']
+                  'fir_cols', 'icol_pair', 'fold', 'fold_long']
 
     def launches(self):
         """Per-launch records: kind, nodes, tasks per node, threads, LDS bytes,
