@@ -123,7 +123,6 @@ Scat2DKernel<T> pick_scat2d_p(int kind, int threads) {
         case K2_LEAF_ROWS: return k_scat2d<T, K2_LEAF_ROWS, 256, MAXP>;
         case K2_FIR_COLS: return k_scat2d<T, K2_FIR_COLS, 256, MAXP>;
         case K2_FOLD: return k_scat2d<T, K2_FOLD, KYM_FOLD_THREADS, 7>;  // no transform in it
-        case K2_FOLD_LONG: return k_scat2d<T, K2_FOLD_LONG, KYM_FOLD_THREADS, 7>;
         case K2B_NODE: return pick_scat2d_nt<T, K2B_NODE, MAXP>(threads);
         case K2B_LEAFG: return pick_scat2d_nt<T, K2B_LEAFG, MAXP>(threads);
         case K2B_GCOLS: return k_scat2d<T, K2B_GCOLS, 256, MAXP>;
@@ -135,7 +134,7 @@ Scat2DKernel<T> pick_scat2d_p(int kind, int threads) {
 }
 
 // The kernels of launches whose LDS has no room for the twiddles
-// (Launch2D::global_tw); nodes on 1024 threads only.
+// (Launch2D::global_tw; nodes on 1024 threads only), and other rare ones.
 template <class T, int MAXP>
 Scat2DKernel<T> pick_scat2d_global_tw(int kind, int threads) {
     switch (kind) {
@@ -144,6 +143,7 @@ Scat2DKernel<T> pick_scat2d_global_tw(int kind, int threads) {
         case K2_ICOL: return k_scat2d<T, K2_ICOL, 256, MAXP, false>;
         case K2_ROWS_MOD: return k_scat2d<T, K2_ROWS_MOD, 256, MAXP, false>;
         case K2_FWD_COLS: return k_scat2d<T, K2_FWD_COLS, 256, MAXP, false>;
+        case K2_FOLD_LONG: return k_scat2d<T, K2_FOLD_LONG, KYM_FOLD_THREADS, 7>;  // no transform in it
         case K2B_NODE: return threads == 1024 ? k_scat2d<T, K2B_NODE, 1024, MAXP, false> : nullptr;
         case K2B_GCOLS: return k_scat2d<T, K2B_GCOLS, 256, MAXP, false>;
         case K2B_GROWS: return k_scat2d<T, K2B_GROWS, 256, MAXP, false>;

@@ -1846,39 +1846,32 @@ KYM_HD KYM_INL int pass_twiddles(const Scat2DArgs<T>& a, cpx<T>* lds, int tid, i
     return pass_tw_elems(f.n);
 }
 
-// The pass with or without its twiddles in LDS (COLS: of H, else of W).
-template <bool TWL, bool COLS, class T, int MAXP, class F>
-KYM_HD KYM_INL void with_dyn_pass(const Scat2DArgs<T>& a, cpx<T>* lds, int tid, int nth, F body) {
-    const int n = TWL ? pass_twiddles<COLS>(a, lds, tid, nth) : 0;
-    body(DynPass<T, MAXP, TWL>{TWL ? lds : nullptr}, lds + n);
-}
-
 // TWL: the launch's LDS holds the twiddles of its sizes (Launch2D::global_tw).
 template <class T, int MAXP, bool TWL = true>
 KYM_HD KYM_INL void dispatch_body2d(int kind, const Scat2DArgs<T>& a, int task, cpx<T>* lds, int tid, int nth) {
     switch (kind) {
         case K2_LDS_NODE: body_lds_node<T, MAXP, TWL>(a, task, lds, tid, nth); break;
         case K2_LEAF: body_leaf<T, MAXP>(a, task, lds, tid, nth); break;
-        case K2_ROOT_ROWS:
-            with_dyn_pass<TWL, false, T, MAXP>(a, lds, tid, nth, [&](auto fp, cpx<T>* l) {
-                body_root_rows<T>(fp, a, task, l, tid, nth);
-            });
+        case K2_ROOT_ROWS: {
+            const int n = TWL ? pass_twiddles<false>(a, lds, tid, nth) : 0;
+            body_root_rows<T>(DynPass<T, MAXP, TWL>{TWL ? lds : nullptr}, a, task, lds + n, tid, nth);
             break;
-        case K2_ICOL:
-            with_dyn_pass<TWL, true, T, MAXP>(a, lds, tid, nth, [&](auto fp, cpx<T>* l) {
-                body_icol<T>(fp, a, task, l, tid, nth);
-            });
+        }
+        case K2_ICOL: {
+            const int n = TWL ? pass_twiddles<true>(a, lds, tid, nth) : 0;
+            body_icol<T>(DynPass<T, MAXP, TWL>{TWL ? lds : nullptr}, a, task, lds + n, tid, nth);
             break;
-        case K2_ROWS_MOD:
-            with_dyn_pass<TWL, false, T, MAXP>(a, lds, tid, nth, [&](auto fp, cpx<T>* l) {
-                body_rows_mod<T>(fp, a, task, l, tid, nth);
-            });
+        }
+        case K2_ROWS_MOD: {
+            const int n = TWL ? pass_twiddles<false>(a, lds, tid, nth) : 0;
+            body_rows_mod<T>(DynPass<T, MAXP, TWL>{TWL ? lds : nullptr}, a, task, lds + n, tid, nth);
             break;
-        case K2_FWD_COLS:
-            with_dyn_pass<TWL, true, T, MAXP>(a, lds, tid, nth, [&](auto fp, cpx<T>* l) {
-                body_fwd_cols<T>(fp, a, task, l, tid, nth);
-            });
+        }
+        case K2_FWD_COLS: {
+            const int n = TWL ? pass_twiddles<true>(a, lds, tid, nth) : 0;
+            body_fwd_cols<T>(DynPass<T, MAXP, TWL>{TWL ? lds : nullptr}, a, task, lds + n, tid, nth);
             break;
+        }
         case K2_LEAF_ICOL: body_leaf_icol<T, MAXP>(a, task, lds, tid, nth); break;
         case K2_LEAF_ROWS: body_leaf_rows<T, MAXP>(a, task, lds, tid, nth); break;
         case K2_FIR_COLS: body_fir_cols<T, MAXP>(a, task, lds, tid, nth); break;

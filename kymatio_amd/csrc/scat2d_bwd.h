@@ -552,21 +552,21 @@ KYM_HD KYM_INL void dispatch_bwd2d(int kind, const Scat2DArgs<T>& a, int task, c
     switch (kind) {
         case K2B_NODE: body_bwd_node<T, MAXP, TWL>(a, task, lds, tid, nth); break;
         case K2B_LEAFG: body_bwd_leafg<T, MAXP>(a, task, lds, tid, nth); break;
-        case K2B_GCOLS:
-            with_dyn_pass<TWL, true, T, MAXP>(a, lds, tid, nth, [&](auto fp, cpx<T>* l) {
-                body_bwd_gcols<T>(fp, a, task, l, tid, nth);
-            });
+        case K2B_GCOLS: {
+            const int n = TWL ? pass_twiddles<true>(a, lds, tid, nth) : 0;
+            body_bwd_gcols<T>(DynPass<T, MAXP, TWL>{TWL ? lds : nullptr}, a, task, lds + n, tid, nth);
             break;
-        case K2B_GROWS:
-            with_dyn_pass<TWL, false, T, MAXP>(a, lds, tid, nth, [&](auto fp, cpx<T>* l) {
-                body_bwd_grows<T>(fp, a, task, l, tid, nth);
-            });
+        }
+        case K2B_GROWS: {
+            const int n = TWL ? pass_twiddles<false>(a, lds, tid, nth) : 0;
+            body_bwd_grows<T>(DynPass<T, MAXP, TWL>{TWL ? lds : nullptr}, a, task, lds + n, tid, nth);
             break;
-        case K2B_GFCOLS:
-            with_dyn_pass<TWL, true, T, MAXP>(a, lds, tid, nth, [&](auto fp, cpx<T>* l) {
-                body_bwd_gfcols<T>(fp, a, task, l, tid, nth);
-            });
+        }
+        case K2B_GFCOLS: {
+            const int n = TWL ? pass_twiddles<true>(a, lds, tid, nth) : 0;
+            body_bwd_gfcols<T>(DynPass<T, MAXP, TWL>{TWL ? lds : nullptr}, a, task, lds + n, tid, nth);
             break;
+        }
         case K2B_FOLD: body_bwd_fold<T, MAXP>(a, task, lds, tid, nth); break;
         default: break;
     }

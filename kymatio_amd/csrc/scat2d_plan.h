@@ -477,7 +477,8 @@ struct Scat2DPlan {
                 case K2_ROOT_ROWS: case K2_ROWS_MOD: case K2_LEAF_ROWS: case K2B_GROWS:
                     l.pclass = kym_plan_class(W[0], 1);
                     break;
-                case K2_FIR_COLS: case K2_FOLD: case K2_FOLD_LONG: case K2B_FOLD: break;  // no transform
+                case K2_FIR_COLS: case K2_FOLD: case K2B_FOLD: break;  // no transform
+                case K2_FOLD_LONG: l.pclass = KYM_GLOBAL_TW + 7; break;
                 default: l.pclass = kym_plan_class(H[0], W[0]);
             }
             l.spec = -1;
