@@ -18,11 +18,15 @@ static int fail(int code, const std::string& msg) {
     return code;
 }
 
+// A failed call's error is taken back from the runtime: the caller gets it as a
+// status, and its next unrelated call would report it again.
 #define KYM_HIP_TRY(expr)                                                                    \
     do {                                                                                     \
         hipError_t _e = (expr);                                                              \
-        if (_e != hipSuccess)                                                                \
+        if (_e != hipSuccess) {                                                              \
+            (void)hipGetLastError();                                                         \
             return fail(KYM_ERR_HIP, std::string(#expr " failed: ") + hipGetErrorString(_e)); \
+        }                                                                                    \
     } while (0)
 
 extern "C" const char* kym_last_error(void) { return g_last_error.c_str(); }

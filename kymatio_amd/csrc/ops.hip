@@ -15,7 +15,10 @@ int kym_ops_fail(int code, const std::string& msg);  // capi.hip
 #define OPS_HIP_TRY(expr)                                                                          \
     do {                                                                                           \
         hipError_t _e = (expr);                                                                    \
-        if (_e != hipSuccess) return kym_ops_fail(KYM_ERR_HIP, std::string(#expr " failed: ") + hipGetErrorString(_e)); \
+        if (_e != hipSuccess) {                                                                    \
+            (void)hipGetLastError();                                                               \
+            return kym_ops_fail(KYM_ERR_HIP, std::string(#expr " failed: ") + hipGetErrorString(_e)); \
+        }                                                                                          \
     } while (0)
 
 static inline unsigned grid_for(long long n, int block) {

@@ -323,3 +323,13 @@ def test_deep_averages_of_long_rows(shape, L):
     gd, = torch.autograd.grad((got * w.to(DEV)).sum(), xd)
     assert (got.detach().cpu() - want.detach()).abs().max() <= 1e-12 * want.abs().max()
     assert (gd.cpu() - gw).abs().max() <= 1e-11 * gw.abs().max()
+
+
+def test_a_refused_plan_leaves_no_error_behind():
+    """A size whose leaf column pass exceeds the LDS (3000 x 40, J = 4) is
+    refused as a plan is made, and nothing else fails afterwards."""
+    sc = Scattering2D(4, (3000, 40)).to(DEV)
+    with pytest.raises(RuntimeError, match='hipFuncSetAttribute'):
+        sc(torch.zeros(1, 3000, 40, device=DEV))
+    assert torch.ones(8, device=DEV).sum().item() == 8
+    assert Scattering2D(2, (32, 32)).to(DEV)(torch.zeros(1, 32, 32, device=DEV)).abs().max().item() == 0
