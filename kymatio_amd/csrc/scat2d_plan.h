@@ -324,7 +324,10 @@ struct Scat2DPlan {
             // order: 16 images of 144 x 488 J=3, 128 x 160 nodes, 825 us as passes,
             // 531 so.  The first order alone, 8 nodes an image, leaves CUs idle that
             // passes fill: 16 of 112 x 144 J=3 177 us as passes, 191 so.
-            const bool wide = wide_nodes && nd.res > 0 && max_order == 2;
+            // So do fewer wavelets: 20 nodes an image (L = 4), one of 144 x 488 with the
+            // gradient 485 us as passes, 508 so, 16 forward 337 and 275; with 72 (L = 8)
+            // 546 and 554, 1085 and 959 (8 with the gradient).
+            const bool wide = wide_nodes && max_order == 2 && nd.res > 0 && L + nd.res * L * L >= 64;
             const size_t tw = wide ? 0 : cs * kym_tw_elems(H[nd.res], W[nd.res]);
             const bool fits = node_lds(nd) + tw <= lds_limit &&
                               (!fir || elems <= (size_t)KYM_STAGE_MAX * node_threads(elems) || spec_fit ||

@@ -192,8 +192,8 @@ def test_launches_fit_the_workgroup(emu, shape, J, dt, tune, big):
 
 
 @pytest.mark.parametrize('shape,J,L,dt,limits', [
-    ((40, 40), 3, 3, np.float32, (8840, 7608)), ((20, 24), 2, 3, np.float64, (8696, 4952)),
-    ((33, 31), 3, 2, np.float32, (6744, 6520)), ((45, 30), 1, 2, np.float64, (9240,))])
+    ((40, 40), 3, 8, np.float32, (8840, 7608)), ((20, 24), 2, 8, np.float64, (8696, 4952)),
+    ((33, 31), 3, 8, np.float32, (6744, 6520)), ((45, 30), 1, 2, np.float64, (9240,))])
 def test_twiddles_in_global_memory(emu, shape, J, L, dt, limits):
     """Launches whose LDS has no room for their twiddles, nodes and passes,
     forward and backward, against the default placement."""
